@@ -130,29 +130,33 @@ int heuristic_tile(int M, int N)
   return best;
 }
 
-// The FP16 / BF16 kernels' tile for shapes the table does not list: the most tiles any CU gets (two 128 x 128 tiles share
-// a CU side by side, but it then takes as long as for both) times the tile's area, over a measured efficiency relative
-// to the 256 x 256 tile (4096^3: 111.6 us in 256 x 256, 127.6 in 128 x 256, 131.9 in 256 x 128, 146.8 in 128 x 128).  Picks
-// the measured best on every shape of the tune driver's list, e.g. 128 x 256 for 2048 x 2560 x 9728 (115 us; 144 in
-// 128 x 128, 182 in 256 x 256) and for 4096 x 2048 x 12288 (184 us; 229 in 256 x 256).
-int heuristic_tile_fp16(int M, int N)
+// The FP16 / BF16 kernels' tile for shapes the table does not list.  A launch takes about
+//   fixed + K / 64 * (full rounds * all + (a round is left over) * one)   microseconds,
+// where a CU holds `per_cu` tiles side by side, works K = 64 of them all in `all` and of a lone one in `one`, and the busiest CU
+// gets ceil(tiles / CUs) tiles.  The constants are fitted to 56 shapes (M, N, K log-uniform in 256 .. 8192 and the benchmark's) x
+// both B layouts on the MI355X; the choice is within 1 % of the best tile on average and 15 % at worst there (the tile a
+// wave-count rule chose before cost 31 % on average with today's kernels' times, 3.4 x at worst: 64 x 64 tiles for 384 x 256 x 3648).
+int heuristic_tile_fp16(int M, int N, int K)
 {
   static const struct {
-    int   id, bm, bn;
-    float eff;
-  } cand[] = {{LLMMM_TILE_256x256, 256, 256, 1.00f}, {LLMMM_TILE_128x256, 128, 256, 0.875f}, {LLMMM_TILE_256x128, 256, 128, 0.85f}, {LLMMM_TILE_128x128, 128, 128, 0.74f}};
-  int   best      = -1;
-  float best_cost = 0.f;
+    int    id, bm, bn, per_cu;
+    double fixed, one, all;
+  } cand[] = {{LLMMM_TILE_256x256, 256, 256, 1, 1.24, 1.295, 1.295}, {LLMMM_TILE_128x256, 128, 256, 1, 0.50, 0.777, 0.777},
+              {LLMMM_TILE_256x128, 256, 128, 1, 0.50, 0.797, 0.797}, {LLMMM_TILE_128x128, 128, 128, 2, 2.57, 0.526, 0.950},
+              {LLMMM_TILE_64x128, 64, 128, 2, 2.83, 0.295, 0.629},   {LLMMM_TILE_64x64, 64, 64, 2, 2.85, 0.182, 0.402}};
+  int    best    = -1;
+  double best_us = 0.;
   for (const auto& c : cand) {
     if (M % c.bm || N % c.bn) continue;
     const long tiles  = (long)(M / c.bm) * (N / c.bn);
-    float      rounds = (float)((tiles + NUM_CUS - 1) / NUM_CUS);
+    const long per    = (tiles + NUM_CUS - 1) / NUM_CUS;  // tiles of the busiest CU
+    double     rounds = per / c.per_cu * c.all + (per % c.per_cu ? c.one : 0.);
     if (c.id == LLMMM_TILE_256x256) {  // a partly filled last round runs in half-size tiles where launch_fp16 can arrange it
       const long tm = M / 256, tn = N / 256, full = tiles / NUM_CUS * NUM_CUS;
-      if (tiles > NUM_CUS && tm > 1 && full % tm == 0 && tn - full / tm > 0 && (tn - full / tm) * tm * 2 <= NUM_CUS) rounds -= 0.5f;
+      if (tiles > NUM_CUS && tm > 1 && full % tm == 0 && tn - full / tm > 0 && (tn - full / tm) * tm * 2 <= NUM_CUS) rounds -= 0.4 * c.one;
     }
-    const float cost = rounds * c.bm * c.bn / c.eff;
-    if (best < 0 || cost < best_cost) best = c.id, best_cost = cost;
+    const double us = c.fixed + K / 64. * rounds;
+    if (best < 0 || us < best_us) best = c.id, best_us = us;
   }
   return best;
 }
@@ -160,6 +164,7 @@ int heuristic_tile_fp16(int M, int N)
 constexpr int MAX_TILE_SPLIT = 8;
 
 bool tile_dims(int tile, int& bm, int& bn);
+bool fp16_only(int tile) { return tile == LLMMM_TILE_64x128 || tile == LLMMM_TILE_64x64; }
 
 // Split-K factor for the MFMA tile kernels: only when the tiles alone leave most of the chip idle -- at most about one
 // workgroup per CU, every split at least two slices long -- and only when the shorter K loop pays for the fp32 planes'
@@ -193,6 +198,7 @@ bool tile_dims(int tile, int& bm, int& bn)
     case LLMMM_TILE_256x128: bm = 256; bn = 128; return true;
     case LLMMM_TILE_128x128: bm = 128; bn = 128; return true;
     case LLMMM_TILE_64x128: bm = 64; bn = 128; return true;  // FP16/BF16 only
+    case LLMMM_TILE_64x64: bm = 64; bn = 64; return true;    // FP16/BF16 only
     case LLMMM_TILE_128x160: bm = 128; bn = 160; return true;  // FP8 only, outputs without 1x128 groups
     default: return false;
   }
@@ -241,7 +247,7 @@ const TuneOverride& tune_override()
         o.skinny.push_back({a, b, c, d});
       // (a tile must divide the shape it is entered for -- an entry that does not would turn a call the heuristic serves
       // into "not aligned"; the one exception is a row tail: fewer than 128 rows in 128 x 128 tiles)
-      else if (n == 6 && !strcmp(kind, "tile") && a > 0 && b > 0 && c > 0 && tile_dims(d, bm, bn) && d != LLMMM_TILE_64x128 && d != LLMMM_TILE_128x160 && e >= 0 &&
+      else if (n == 6 && !strcmp(kind, "tile") && a > 0 && b > 0 && c > 0 && tile_dims(d, bm, bn) && !fp16_only(d) && d != LLMMM_TILE_128x160 && e >= 0 &&
                e <= MAX_SPLIT_K && b % bn == 0 && (a % bm == 0 || (a < 128 && d == LLMMM_TILE_128x128)))
         o.tile.push_back({a, b, c, d, e});
       else if (n == 5 && !strcmp(kind, "fp16") && a > 0 && b > 0 && c > 0 && tile_dims(d, bm, bn) && d != LLMMM_TILE_128x160 && a % bm == 0 && b % bn == 0)
@@ -518,12 +524,7 @@ int llmmm_fp16_gemm_ex(int dtype, const void* A, const void* B, void* C, int M, 
   int tile = cfg ? cfg->tile : LLMMM_TILE_AUTO;
   if (tile == LLMMM_TILE_AUTO) {
     if (!lookup_fp16_tile(M, N, K, &tile)) tile = LLMMM_TILE_AUTO;
-    if (tile == LLMMM_TILE_AUTO) {
-      tile = heuristic_tile_fp16(M, N);
-      // small problems: 128 x 128 tiles on at most half of the CUs -> twice as many 64 x 128 tiles of four 16-row
-      // waves (1024^3: 8.0 instead of 11.3 us; from 160 tiles of 128 x 128 on, the larger tile wins again)
-      if (tile == LLMMM_TILE_128x128 && (long)(M / 128) * (N / 128) <= NUM_CUS / 2) tile = LLMMM_TILE_64x128;
-    }
+    if (tile == LLMMM_TILE_AUTO) tile = heuristic_tile_fp16(M, N, K);
   }
   int bm, bn;
   if (!tile_dims(tile, bm, bn) || tile == LLMMM_TILE_128x160) return fail(LLMMM_ERR_INVALID_ARGUMENT, "unknown tile id %d", tile);
@@ -752,7 +753,7 @@ int llmmm_fp8_gemm_ex(int out_kind, const void* A, const float* As, const void* 
   }
   else {
     int bm, bn;
-    if (!tile_dims(cfg.tile, bm, bn) || cfg.tile == LLMMM_TILE_64x128) return fail(LLMMM_ERR_INVALID_ARGUMENT, "unknown tile id %d", cfg.tile);
+    if (!tile_dims(cfg.tile, bm, bn) || fp16_only(cfg.tile)) return fail(LLMMM_ERR_INVALID_ARGUMENT, "unknown tile id %d", cfg.tile);
     if (cfg.tile == LLMMM_TILE_128x160 && (out_kind == LLMMM_OUT_FP8Q || swiglu)) {
       // its waves straddle the 1x128 groups of the fused quantisation: a tile the library picked itself gives way, one asked for is refused
       if (user && user->tile == LLMMM_TILE_128x160) return fail(LLMMM_ERR_INVALID_ARGUMENT, "the 128 x 160 tile has no fp8 output");
@@ -970,7 +971,7 @@ static int resolve_plane_cfg(const void*& A, const float*& As, const void* Bt, c
     if (M > SKINNY_MAX_M) return fail(LLMMM_ERR_INVALID_ARGUMENT, "the weight-streaming kernel handles M <= %d", SKINNY_MAX_M);
   }
   else {
-    if (!tile_dims(cfg.tile, bm, bn) || cfg.tile == LLMMM_TILE_64x128) return fail(LLMMM_ERR_INVALID_ARGUMENT, "unknown tile id %d", cfg.tile);
+    if (!tile_dims(cfg.tile, bm, bn) || fp16_only(cfg.tile)) return fail(LLMMM_ERR_INVALID_ARGUMENT, "unknown tile id %d", cfg.tile);
     if ((M % bm && !(cfg.tile == LLMMM_TILE_128x128 && M < 128)) || N % bn) return fail(LLMMM_ERR_NOT_ALIGNED, "M or N or K are not aligned.");
     if (user && user->tile != LLMMM_TILE_AUTO && user->split_k <= 0) cfg.split_k = heuristic_tile_split(cfg.tile, M < bm ? bm : M, N, K);
   }
