@@ -92,6 +92,11 @@ def load():
 
 
 lib = load()
+try:
+    from . import _native as native  # noqa: E402  (linked against the library just loaded)
+except ImportError as e:
+    raise ImportError("%s cannot be loaded (%s): build it with `python llmmm_amd/build.py`. There is no fallback path."
+                      % (os.path.join(_HERE, "_native.so"), e)) from None
 
 
 def check(code):

@@ -1,8 +1,8 @@
-"""Builds ``libllmmm.so`` (HIP kernels + C ABI) for gfx950 with hipcc, in-tree.
+"""Builds ``libllmmm.so`` (HIP kernels + C ABI) for gfx950 with hipcc and ``_native.so`` (the Python entry points' host work), in-tree.
 
-``python llmmm_amd/build.py`` (run as a script: importing the package needs the library this
-builds).  hipcc cross-compiles without a GPU; the resulting library sits next to this file so
-that it travels with the source tree.
+``python llmmm_amd/build.py`` (run as a script: importing the package needs the libraries this
+builds).  hipcc cross-compiles without a GPU; the resulting libraries sit next to this file so
+that they travel with the source tree.
 """
 import os
 import subprocess
@@ -13,6 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libllmmm.so")
+BINDING = os.path.join(HERE, "_native.so")
 
 COMMON = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
@@ -46,10 +47,26 @@ def _compile(item):
     return obj, out
 
 
+def _compile_binding():
+    """csrc/binding.cpp: host code only, against the headers of the installed torch and Python (g++)."""
+    import sysconfig
+    import torch
+    obj = os.path.join(OBJ, "binding.o")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+           "-I", sysconfig.get_paths()["include"], "-isystem", os.path.join(os.path.dirname(torch.__file__), "include"),
+           "-c", os.path.join(CSRC, "binding.cpp"), "-o", obj]
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed for binding.cpp:\n" + res.stdout)
+    return obj
+
+
 def build(verbose=False):
     os.makedirs(OBJ, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as pool:
+    with ThreadPoolExecutor(max_workers=5) as pool:
+        binding = pool.submit(_compile_binding)
         results = list(pool.map(_compile, SOURCES.items()))
+        binding = binding.result()
     objs = [o for o, _ in results]
     if verbose:
         for _, out in results:
@@ -59,7 +76,17 @@ def build(verbose=False):
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + res.stdout)
+    _link_binding(binding)
     return LIB
+
+
+def _link_binding(obj):
+    import torch
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-shared", "-o", BINDING, obj, "-L", HERE, "-lllmmm", "-L", torch_lib, "-ltorch_python", "-ltorch_cpu", "-lc10", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("link failed:\n" + res.stdout)
 
 
 def build_dropin_test():

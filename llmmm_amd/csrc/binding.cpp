@@ -1,0 +1,428 @@
+// llmmm_amd._native: the Python entry points' host work -- argument checks, output and workspace allocation, the current stream,
+// the call into the C ABI -- as one CPython extension.
+//
+// What bounds a decode step through these entry points is the host: one decoder layer at M = 1 is nine kernels, about 40 us of GPU
+// time, and took 99 us when every argument went through Python checks and ctypes (about 17 us per call); the same six calls here
+// keep ahead of the GPU (50 us a layer; batched decode at M = 16 / 100: 98 -> 83, 99 -> 73; one product at M = 1: 11.2 -> 6.1; the
+// FP16 product 1024^3: 8.7 -> 6.4).  The checks, their order and the exceptions are those the Python module documents: a CUDA tensor (TypeError),
+// contiguous (ValueError), of a supported type (RuntimeError "T is not supported."), large enough (ValueError).  Outputs are
+// allocated through torch's dispatcher, so its modes see them as they see torch.empty.  No state is kept between calls.
+#include <Python.h>
+
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/Exceptions.h>
+#include <ATen/ATen.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
+
+#include <climits>
+
+#include "../../include/llmmm.h"
+
+namespace {
+
+enum : unsigned { T_F32 = 1, T_F16 = 2, T_BF16 = 4, T_FP8 = 8, T_I32 = 16, T_ANY = 0 };
+
+unsigned type_bit(const at::Tensor& t)
+{
+  switch (t.scalar_type()) {
+    case at::kFloat: return T_F32;
+    case at::kHalf: return T_F16;
+    case at::kBFloat16: return T_BF16;
+    case at::kByte:
+    case at::kFloat8_e4m3fn: return T_FP8;  // e4m3 codes travel as either type
+    case at::kInt: return T_I32;
+    default: return 0;
+  }
+}
+
+struct Refused {};  // a Python exception has been set
+
+[[noreturn]] void refuse(PyObject* type, const char* fmt, ...)
+{
+  va_list ap;
+  va_start(ap, fmt);
+  PyErr_FormatV(type, fmt, ap);
+  va_end(ap);
+  throw Refused();
+}
+[[noreturn]] void not_supported() { refuse(PyExc_RuntimeError, "T is not supported."); }
+
+const at::Tensor& tensor(PyObject* o, const char* what)
+{
+  if (!THPVariable_Check(o)) refuse(PyExc_TypeError, "%s must be a CUDA tensor", what);
+  return THPVariable_Unpack(o);
+}
+
+// The device address of a tensor argument; `types` = the element types it may have (T_ANY: all), `numel` = elements needed.
+void* ptr(PyObject* o, const char* what, unsigned types, int64_t numel)
+{
+  const at::Tensor& t = tensor(o, what);
+  if (!t.is_cuda()) refuse(PyExc_TypeError, "%s must be a CUDA tensor", what);
+  if (!t.is_contiguous()) refuse(PyExc_ValueError, "%s must be contiguous", what);
+  if (types != T_ANY && !(type_bit(t) & types)) not_supported();
+  if (t.numel() < numel) refuse(PyExc_ValueError, "%s holds %lld elements, %lld needed", what, (long long)t.numel(), (long long)numel);
+  return t.data_ptr();
+}
+void* ptr_or_null(PyObject* o, const char* what, unsigned types, int64_t numel) { return o == Py_None ? nullptr : ptr(o, what, types, numel); }
+
+int as_int(PyObject* o)
+{
+  const long v = PyLong_AsLong(o);
+  if (v == -1 && PyErr_Occurred()) throw Refused();
+  if (v < INT_MIN || v > INT_MAX) refuse(PyExc_OverflowError, "%ld does not fit an int", v);
+  return (int)v;
+}
+float as_float(PyObject* o)
+{
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) throw Refused();
+  return (float)v;
+}
+bool as_bool(PyObject* o)
+{
+  const int v = PyObject_IsTrue(o);
+  if (v < 0) throw Refused();
+  return v != 0;
+}
+
+PyObject* current_raw_stream;  // torch._C._cuda_getCurrentRawStream(device index)
+
+// None: torch's current stream; a torch stream: its handle; anything else: the handle as an integer.
+void* as_stream(PyObject* o)
+{
+  if (o == Py_None) {
+    const long device = c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getDevice().index();
+    PyObject*  index  = PyLong_FromLong(device);
+    PyObject*  raw    = index ? PyObject_CallOneArg(current_raw_stream, index) : nullptr;
+    Py_XDECREF(index);
+    if (!raw) throw Refused();
+    void* p = PyLong_AsVoidPtr(raw);
+    Py_DECREF(raw);
+    if (!p && PyErr_Occurred()) throw Refused();
+    return p;
+  }
+  PyObject* handle = PyLong_Check(o) ? nullptr : PyObject_GetAttrString(o, "cuda_stream");
+  if (!handle) PyErr_Clear();
+  PyObject* index = PyNumber_Long(handle ? handle : o);
+  Py_XDECREF(handle);
+  if (!index) throw Refused();
+  void* p = PyLong_AsVoidPtr(index);
+  Py_DECREF(index);
+  if (!p && PyErr_Occurred()) throw Refused();
+  return p;
+}
+
+at::Tensor empty(at::IntArrayRef sizes, at::ScalarType type, const at::Device& device)
+{
+  return at::empty(sizes, at::TensorOptions().dtype(type).device(device));
+}
+int64_t blocks(int64_t n) { return (n + 127) / 128; }
+int64_t whole_blocks(int64_t n) { return n % 128 == 0 ? n / 128 : 0; }
+
+PyObject* tuple2(const at::Tensor& a, const at::Tensor& b)
+{
+  PyObject* r = PyTuple_New(2);
+  if (!r) throw Refused();
+  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(a));
+  PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(b));
+  return r;
+}
+
+// The call itself, without the interpreter lock (a full hardware queue makes a launch wait).  The text of a failure is the calling
+// thread's, so it is fetched before anything else runs.
+template <typename F>
+void call(F&& f)
+{
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = f();
+  Py_END_ALLOW_THREADS
+  if (rc == LLMMM_OK) return;
+  const char *text = llmmm_error_string(rc), *detail = llmmm_last_error();
+  if (rc == LLMMM_ERR_NOT_ALIGNED || rc == LLMMM_ERR_UNSUPPORTED_TYPE)
+    refuse(PyExc_RuntimeError, "%s", *detail ? detail : text);  // the detail is the reference's text for the entry point that failed
+  if (*detail) refuse(PyExc_RuntimeError, "%s: %s", text, detail);
+  refuse(PyExc_RuntimeError, "%s", text);
+}
+
+int hidden_dtype(const at::Tensor& t)
+{
+  switch (type_bit(t)) {
+    case T_F32: return LLMMM_DTYPE_F32;
+    case T_BF16: return LLMMM_DTYPE_BF16;
+    case T_F16: return LLMMM_DTYPE_F16;
+    default: not_supported();
+  }
+}
+void shape2(const at::Tensor& t, const char* what, int& rows, int& cols)
+{
+  if (t.dim() != 2) refuse(PyExc_ValueError, "%s must have two dimensions", what);
+  if (t.size(0) > INT_MAX || t.size(1) > INT_MAX) refuse(PyExc_OverflowError, "%s is too large", what);
+  rows = (int)t.size(0), cols = (int)t.size(1);
+}
+
+// The A operand of an FP8 product by layout: quantised codes with their scales, the fp32 gate_up result [M, 2K], or the host
+// address of an llmmm_a_planes_rmsnorm.
+struct AOperand {
+  const void*  a;
+  const float* as;
+};
+AOperand a_operand(PyObject* A, PyObject* As, int layout, int64_t M, int64_t K)
+{
+  if (layout == LLMMM_FP8_A_PLANES_RMSNORM) {
+    void* p = PyLong_AsVoidPtr(A);
+    if (!p) {
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null A operand");
+      throw Refused();
+    }
+    return {p, nullptr};
+  }
+  if (layout == LLMMM_FP8_A_SWIGLU_F32) return {ptr(A, "A (fp32 gate_up result)", T_F32, M * 2 * K), nullptr};
+  const void* a = ptr(A, "A", T_FP8, M * K);
+  return {a, (const float*)ptr(As, "A_scale_transposed", T_F32, whole_blocks(K) * M)};
+}
+size_t a_workspace_bytes(int layout, int M, int N, int K)
+{
+  if (layout == LLMMM_FP8_A_PLANES_RMSNORM) return llmmm_fp8_planes_rmsnorm_a_workspace(M, N, K);
+  return layout == LLMMM_FP8_A_SWIGLU_F32 ? llmmm_fp8_swiglu_a_workspace(M, N, K) : 0;
+}
+struct Workspace {
+  at::Tensor own;
+  void*      p = nullptr;
+  size_t     n = 0;
+};
+// The caller's workspace, or (`own` >= 0) one of that many bytes, at least 16.
+Workspace workspace(PyObject* o, int64_t own, const at::Device& device)
+{
+  Workspace w;
+  if (o != Py_None) {
+    if (!THPVariable_Check(o)) refuse(PyExc_TypeError, "workspace must be a tensor");
+    const at::Tensor& t = THPVariable_Unpack(o);
+    w.p = t.data_ptr(), w.n = (size_t)t.numel() * t.element_size();
+  }
+  else if (own >= 0) {
+    w.own = empty({own > 16 ? own : 16}, at::kByte, device);
+    w.p = w.own.data_ptr(), w.n = (size_t)w.own.numel();
+  }
+  return w;
+}
+
+// ---------------------------------------------------------------------------------------------- entry points
+typedef PyObject* const* Args;
+
+// (A, B, C or None, b_transposed, tile, stream) -> C
+PyObject* fp16_gemm(Args v)
+{
+  const at::Tensor &A = tensor(v[0], "A"), &B = tensor(v[1], "B");
+  const unsigned    t = type_bit(A);
+  if (t != T_F16 && t != T_BF16) not_supported();
+  int M, K, b0, b1;
+  shape2(A, "A", M, K);
+  shape2(B, "B", b0, b1);
+  const bool bt = as_bool(v[3]);
+  const int  N  = bt ? b0 : b1;
+  if ((bt ? b1 : b0) != K || B.scalar_type() != A.scalar_type()) refuse(PyExc_ValueError, "shape or dtype mismatch between A and B");
+  at::Tensor own;
+  if (v[2] == Py_None) own = empty({M, N}, A.scalar_type(), A.device());
+  const llmmm_gemm_cfg cfg = {as_int(v[4]), 0, 0, 0};
+  const void *         a = ptr(v[0], "A", T_ANY, 0), *b = ptr(v[1], "B", T_ANY, 0);
+  void*                c = own.defined() ? own.data_ptr() : ptr(v[2], "C", t, (int64_t)M * N);
+  void* const          s = as_stream(v[5]);
+  call([&] { return llmmm_fp16_gemm_ex(t == T_F16 ? LLMMM_DTYPE_F16 : LLMMM_DTYPE_BF16, a, b, c, M, N, K, bt ? LLMMM_B_TRANSPOSED : LLMMM_B_ROW_MAJOR, &cfg, s); });
+  if (own.defined()) return THPVariable_Wrap(own);
+  Py_INCREF(v[2]);
+  return v[2];
+}
+
+// (A, B, C, M, N, K, stream): the reference's launcher
+PyObject* fp16_mm(Args v)
+{
+  const at::Tensor &A = tensor(v[0], "A"), &B = tensor(v[1], "B"), &C = tensor(v[2], "C");
+  const unsigned    t = type_bit(A);
+  if ((t != T_F16 && t != T_BF16) || B.scalar_type() != A.scalar_type() || C.scalar_type() != A.scalar_type()) not_supported();
+  const int M = as_int(v[3]), N = as_int(v[4]), K = as_int(v[5]);
+  if (M % 256 || N % 256 || K % 16) refuse(PyExc_RuntimeError, "M or N or K are not aligned.");
+  const void* a = ptr(v[0], "A", T_ANY, (int64_t)M * K);
+  const void* b = ptr(v[1], "B", T_ANY, (int64_t)K * N);
+  void*       c = ptr(v[2], "C", T_ANY, (int64_t)M * N);
+  void* const s = as_stream(v[6]);
+  call([&] { return llmmm_fp16_gemm(t == T_F16 ? LLMMM_DTYPE_F16 : LLMMM_DTYPE_BF16, a, b, c, M, N, K, LLMMM_B_ROW_MAJOR, s); });
+  Py_RETURN_NONE;
+}
+
+int64_t scale_count(int kind, int64_t M, int64_t N)
+{
+  switch (kind) {
+    case LLMMM_QUANT_1x128_T:
+    case LLMMM_QUANT_128x128_T: return blocks(N) * M;
+    case LLMMM_QUANT_1x128: return M * blocks(N);
+    default: return blocks(M) * blocks(N);
+  }
+}
+
+// (x, q, scale, M, N, kind, stream)
+PyObject* quantize_into(Args v)
+{
+  const int    M = as_int(v[3]), N = as_int(v[4]), kind = as_int(v[5]);
+  const float* x = (const float*)ptr(v[0], "x", T_F32, (int64_t)M * N);
+  void*        q = ptr(v[1], "q", T_FP8, (int64_t)M * N);
+  float*       c = (float*)ptr(v[2], "scale", T_F32, scale_count(kind, M, N));
+  void* const  s = as_stream(v[6]);
+  call([&] { return llmmm_quant_fp8(kind, x, q, c, M, N, s); });
+  Py_RETURN_NONE;
+}
+
+// (x, kind, stream) -> (codes, scales); kind 1x128 transposed (activations) or 128x128 (weights)
+PyObject* quantize(Args v)
+{
+  const at::Tensor& X = tensor(v[0], "x");
+  const int         kind = as_int(v[1]);
+  int               M, N;
+  shape2(X, "x", M, N);
+  const at::Tensor q = empty({M, N}, at::kByte, X.device());
+  const at::Tensor c = kind == LLMMM_QUANT_1x128_T ? empty({blocks(N), M}, at::kFloat, X.device()) : empty({blocks(M), blocks(N)}, at::kFloat, X.device());
+  const float*     x = (const float*)ptr(v[0], "x", T_F32, (int64_t)M * N);
+  void* const      s = as_stream(v[2]);
+  call([&] { return llmmm_quant_fp8(kind, x, q.data_ptr(), (float*)c.data_ptr(), M, N, s); });
+  return tuple2(q, c);
+}
+
+// (x, weight, eps, stream) -> (codes, scales)
+PyObject* rmsnorm_quantize(Args v)
+{
+  const at::Tensor& X = tensor(v[0], "x");
+  int               M, K;
+  shape2(X, "x", M, K);
+  const int        code = hidden_dtype(X);
+  const at::Tensor q = empty({M, K}, at::kByte, X.device()), c = empty({blocks(K), M}, at::kFloat, X.device());
+  const void*      x = ptr(v[0], "x", T_ANY, 0);
+  const float*     w = (const float*)ptr(v[1], "weight", T_F32, K);
+  const float      eps = as_float(v[2]);
+  void* const      s   = as_stream(v[3]);
+  call([&] { return llmmm_rmsnorm_quant_fp8(code, x, w, eps, q.data_ptr(), (float*)c.data_ptr(), M, K, s); });
+  return tuple2(q, c);
+}
+
+// (out_kind, A, As, Bt, Bs, C, Cs, M, N, K, workspace, tile, split_k, b_preshuffled, a_layout, stream)
+PyObject* fp8_gemm(Args v)
+{
+  const int      kind = as_int(v[0]), M = as_int(v[7]), N = as_int(v[8]), K = as_int(v[9]), layout = as_int(v[14]);
+  const int64_t  n_out = kind == LLMMM_OUT_FP8Q_SWIGLU ? N / 2 : N;  // SwiGLU halves the width
+  const unsigned types = kind == LLMMM_OUT_F32 ? T_F32 : kind == LLMMM_OUT_BF16 ? T_BF16 : T_FP8;
+  const bool     fp8   = types == T_FP8;
+  const AOperand a     = a_operand(v[1], v[2], layout, M, K);
+  const void*    b     = ptr(v[3], "B_transposed", T_FP8, (int64_t)N * K);
+  const float*   bs    = (const float*)ptr(v[4], "B_scale_transposed", T_F32, blocks(N) * whole_blocks(K));
+  void*          c     = ptr(v[5], "C", types, M * n_out);
+  float*         cs    = fp8 ? (float*)ptr(v[6], "C_scale_transposed", T_F32, blocks(n_out) * M) : nullptr;
+  const Workspace      w   = workspace(v[10], -1, at::Device(at::kCPU));
+  const llmmm_gemm_cfg cfg = {as_int(v[11]), as_int(v[12]), as_bool(v[13]) ? LLMMM_FP8_B_PRESHUFFLED : LLMMM_FP8_B_ROWS, layout};
+  void* const          s   = as_stream(v[15]);
+  call([&] { return llmmm_fp8_gemm_ex(kind, a.a, a.as, b, bs, c, cs, M, N, K, w.p, w.n, &cfg, s); });
+  Py_RETURN_NONE;
+}
+
+// (A, As, Bt, Bs, residual, hidden_out, norm_weight, eps, M, N, K, workspace, tile, split_k, b_preshuffled, a_layout, stream) -> (codes, scales)
+PyObject* fp8_gemm_add_rmsnorm_quant(Args v)
+{
+  const at::Tensor &R = tensor(v[4], "residual"), &H = tensor(v[5], "hidden_out");
+  const int         code = hidden_dtype(R);
+  if (H.scalar_type() != R.scalar_type()) not_supported();
+  const int        M = as_int(v[8]), N = as_int(v[9]), K = as_int(v[10]), layout = as_int(v[15]);
+  const Workspace  w = workspace(
+      v[11], v[11] == Py_None ? (int64_t)(llmmm_fp8_gemm_add_rmsnorm_quant_workspace(M, N, K) + a_workspace_bytes(layout, M, N, K)) : -1, R.device());
+  const at::Tensor q = empty({M, N}, at::kByte, R.device()), c = empty({blocks(N), M}, at::kFloat, R.device());
+  const AOperand   a  = a_operand(v[0], v[1], layout, M, K);
+  const void*      b  = ptr(v[2], "B_transposed", T_FP8, (int64_t)N * K);
+  const float*     bs = (const float*)ptr(v[3], "B_scale_transposed", T_F32, blocks(N) * whole_blocks(K));
+  const void*      r  = ptr(v[4], "residual", T_ANY, (int64_t)M * N);
+  void*            h  = ptr(v[5], "hidden_out", T_ANY, (int64_t)M * N);
+  const float*     nw = (const float*)ptr(v[6], "norm_weight", T_F32, N);
+  const float      eps = as_float(v[7]);
+  const llmmm_gemm_cfg cfg = {as_int(v[12]), as_int(v[13]), as_bool(v[14]) ? LLMMM_FP8_B_PRESHUFFLED : LLMMM_FP8_B_ROWS, layout};
+  void* const          s   = as_stream(v[16]);
+  call([&] {
+    return llmmm_fp8_gemm_add_rmsnorm_quant(a.a, a.as, b, bs, code, r, h, nw, eps, q.data_ptr(), (float*)c.data_ptr(), M, N, K, w.p, w.n, &cfg, s);
+  });
+  return tuple2(q, c);
+}
+
+// (A, As, Bt, Bs, q_norm, k_norm, eps, cos, sin, positions, n_q, n_kv, M, N, K, out_fp8, workspace, tile, split_k, b_preshuffled, a_layout, stream)
+// -> out or (codes, scales)
+PyObject* fp8_gemm_qkv_rope(Args v)
+{
+  const at::Tensor &B = tensor(v[2], "B_transposed"), &T = tensor(v[7], "cos_table");
+  const int         n_q = as_int(v[10]), n_kv = as_int(v[11]), M = as_int(v[12]), N = as_int(v[13]), K = as_int(v[14]), layout = as_int(v[20]);
+  const bool        fp8 = as_bool(v[15]);
+  const Workspace   w = workspace(
+      v[16], v[16] == Py_None ? (int64_t)(llmmm_fp8_gemm_qkv_rope_workspace(M, N, K) + a_workspace_bytes(layout, M, N, K)) : -1, B.device());
+  const at::Tensor out = empty({M, N}, fp8 ? at::kByte : at::kBFloat16, B.device());
+  at::Tensor       sc;
+  if (fp8) sc = empty({blocks(N), M}, at::kFloat, B.device());
+  if (T.dim() < 1 || T.size(0) > INT_MAX) refuse(PyExc_ValueError, "cos_table must have rows");
+  const int      rows = (int)T.size(0);
+  const AOperand a    = a_operand(v[0], v[1], layout, M, K);
+  const void*    b    = ptr(v[2], "B_transposed", T_FP8, (int64_t)N * K);
+  const float*   bs   = (const float*)ptr(v[3], "B_scale_transposed", T_F32, blocks(N) * whole_blocks(K));
+  const float*   qn   = (const float*)ptr_or_null(v[4], "q_norm_weight", T_F32, 128);
+  const float*   kn   = (const float*)ptr_or_null(v[5], "k_norm_weight", T_F32, 128);
+  const float    eps  = as_float(v[6]);
+  const float*   ct   = (const float*)ptr(v[7], "cos_table", T_F32, (int64_t)rows * 64);
+  const float*   st   = (const float*)ptr(v[8], "sin_table", T_F32, (int64_t)rows * 64);
+  const int*     pos  = (const int*)ptr(v[9], "positions", T_I32, M);
+  const llmmm_gemm_cfg cfg = {as_int(v[17]), as_int(v[18]), as_bool(v[19]) ? LLMMM_FP8_B_PRESHUFFLED : LLMMM_FP8_B_ROWS, layout};
+  void* const          s   = as_stream(v[21]);
+  call([&] {
+    return llmmm_fp8_gemm_qkv_rope(fp8 ? LLMMM_OUT_FP8Q : LLMMM_OUT_BF16, a.a, a.as, b, bs, out.data_ptr(), fp8 ? (float*)sc.data_ptr() : nullptr, qn, kn, eps, ct, st,
+                                   rows, pos, n_q, n_kv, M, N, K, w.p, w.n, &cfg, s);
+  });
+  return fp8 ? tuple2(out, sc) : THPVariable_Wrap(out);
+}
+
+// (codes, stream) -> the pre-shuffled image, a new tensor of the same shape and type
+PyObject* preshuffle(Args v)
+{
+  const at::Tensor& Q = tensor(v[0], "src_transposed");
+  int               N, K;
+  shape2(Q, "src_transposed", N, K);
+  const at::Tensor out = at::empty_like(Q);
+  const void*      q   = ptr(v[0], "src_transposed", T_FP8, (int64_t)N * K);
+  void* const      s   = as_stream(v[1]);
+  call([&] { return llmmm_fp8_preshuffle_b(q, out.data_ptr(), N, K, s); });
+  return THPVariable_Wrap(out);
+}
+
+template <PyObject* (*F)(Args), Py_ssize_t COUNT>
+PyObject* entry(PyObject*, Args v, Py_ssize_t n)
+{
+  HANDLE_TH_ERRORS
+  if (n != COUNT) {
+    PyErr_Format(PyExc_TypeError, "%zd arguments expected, got %zd", COUNT, n);
+    return nullptr;
+  }
+  try {
+    return F(v);
+  }
+  catch (const Refused&) {
+    return nullptr;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+#define LLMMM_ENTRY(NAME, COUNT) {#NAME, (PyCFunction)(void*)&entry<NAME, COUNT>, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {LLMMM_ENTRY(fp16_gemm, 6),        LLMMM_ENTRY(fp16_mm, 7),   LLMMM_ENTRY(quantize_into, 7),
+                         LLMMM_ENTRY(quantize, 3),         LLMMM_ENTRY(rmsnorm_quantize, 4),
+                         LLMMM_ENTRY(fp8_gemm, 16),        LLMMM_ENTRY(fp8_gemm_add_rmsnorm_quant, 17),
+                         LLMMM_ENTRY(fp8_gemm_qkv_rope, 22), LLMMM_ENTRY(preshuffle, 2),
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void)
+{
+  PyObject* torch_c  = PyImport_ImportModule("torch._C");
+  current_raw_stream = torch_c ? PyObject_GetAttrString(torch_c, "_cuda_getCurrentRawStream") : nullptr;
+  Py_XDECREF(torch_c);
+  return current_raw_stream ? PyModule_Create(&module) : nullptr;
+}

@@ -3,14 +3,15 @@
 Same names, argument order and error behaviour as the reference's C++ functions
 (``LLMMM::fp16_mm`` src/mm/fp16/mm.h:9-10; the FP8 launchers examples/005.fp8.mm.cu:217-225,
 :547-549, :2467-2476), taking torch CUDA tensors where the reference takes raw device pointers.
-Everything goes through the C ABI of ``libllmmm.so``; torch only owns the memory and the stream.
+Everything goes through the C ABI of ``libllmmm.so``; torch only owns the memory and the stream.  The calls of a
+model's step check and marshal their arguments in ``_native.so`` (csrc/binding.cpp), the others through ctypes here.
 """
 import ctypes
 
 import torch
 
 from . import _lib
-from ._lib import GemmCfg, check, lib
+from ._lib import GemmCfg, check, lib, native as _native
 
 _FP8_DTYPES = (torch.uint8, torch.float8_e4m3fn)
 
@@ -35,14 +36,6 @@ def _ptr(t, what, dtypes=None, numel=None):
     return ctypes.c_void_p(t.data_ptr())
 
 
-def _dtype_code(t):
-    if t.dtype == torch.float16:
-        return _lib.DTYPE_F16
-    if t.dtype == torch.bfloat16:
-        return _lib.DTYPE_BF16
-    raise RuntimeError("T is not supported.")  # src/mm/fp16/mm.cu:15-17
-
-
 # ------------------------------------------------------------------------------------- FP16 / BF16
 def fp16_mm(A, B, C, M, N, K, stream=None):
     """``LLMMM::fp16_mm<T>(A, B, C, M, N, K, stream)`` (src/mm/fp16/mm.cu:6-42).
@@ -51,30 +44,14 @@ def fp16_mm(A, B, C, M, N, K, stream=None):
     Raises RuntimeError("M or N or K are not aligned.") unless M % 256 == 0, N % 256 == 0 and
     K % 16 == 0 (the reference's rule, mm.cu:19-21) and RuntimeError("T is not supported.")
     for other element types.  Asynchronous on ``stream`` (default: torch's current stream)."""
-    code = _dtype_code(A)
-    if B.dtype != A.dtype or C.dtype != A.dtype:
-        raise RuntimeError("T is not supported.")
-    if not (M % 256 == 0 and N % 256 == 0 and K % 16 == 0):
-        raise RuntimeError("M or N or K are not aligned.")
-    check(lib.llmmm_fp16_gemm(code, _ptr(A, "A", numel=M * K), _ptr(B, "B", numel=K * N), _ptr(C, "C", numel=M * N), M, N, K,
-                              _lib.B_ROW_MAJOR, _stream(stream)))
+    _native.fp16_mm(A, B, C, M, N, K, stream)
 
 
 def fp16_gemm(A, B, C=None, b_transposed=False, tile=_lib.TILE_AUTO, stream=None):
     """C = A @ B (or A @ Bt.T when ``b_transposed``) through ``llmmm_fp16_gemm_ex``.
 
     The library's own (wider) shape rule applies: M, N multiples of 128, K of 16."""
-    code = _dtype_code(A)
-    M, K = A.shape
-    N = B.shape[0] if b_transposed else B.shape[1]
-    if (B.shape[1] if b_transposed else B.shape[0]) != K or B.dtype != A.dtype:
-        raise ValueError("shape or dtype mismatch between A and B")
-    if C is None:
-        C = torch.empty((M, N), dtype=A.dtype, device=A.device)
-    cfg = GemmCfg(tile, 0)
-    check(lib.llmmm_fp16_gemm_ex(code, _ptr(A, "A"), _ptr(B, "B"), _ptr(C, "C", (A.dtype,), M * N), M, N, K,
-                                 _lib.B_TRANSPOSED if b_transposed else _lib.B_ROW_MAJOR, ctypes.byref(cfg), _stream(stream)))
-    return C
+    return _native.fp16_gemm(A, B, C, b_transposed, tile, stream)
 
 
 # ------------------------------------------------------------------------------------- FP8 quantiser
@@ -85,43 +62,24 @@ def fp8_blockwise_symmetric_quantization(x, q, scale, M, N, quant_m, quant_n=128
         raise ValueError("QUANT_M must be 1 or 128 and QUANT_N 128")
     kind = {(1, True): _lib.QUANT_1x128_T, (128, False): _lib.QUANT_128x128, (1, False): _lib.QUANT_1x128,
             (128, True): _lib.QUANT_128x128_T}[(quant_m, bool(scale_transpose))]
-    nb = (N + 127) // 128
-    n_scale = nb * M if scale_transpose else ((M + quant_m - 1) // quant_m) * nb
-    check(lib.llmmm_quant_fp8(kind, _ptr(x, "x", (torch.float32,), M * N), _ptr(q, "q", _FP8_DTYPES, M * N),
-                              _ptr(scale, "scale", (torch.float32,), n_scale), M, N, _stream(stream)))
+    _native.quantize_into(x, q, scale, M, N, kind, stream)
 
 
 def quantize_activation(x, stream=None):
     """1x128 quantisation with transposed scales: returns (codes uint8 [M,K], scales [K/128... ceil, M])."""
-    M, K = x.shape
-    q = torch.empty((M, K), dtype=torch.uint8, device=x.device)
-    s = torch.empty(((K + 127) // 128, M), dtype=torch.float32, device=x.device)
-    fp8_blockwise_symmetric_quantization(x, q, s, M, K, 1, 128, True, stream)
-    return q, s
+    return _native.quantize(x, _lib.QUANT_1x128_T, stream)
 
 
 def quantize_weight(wt, stream=None):
     """128x128 quantisation of a transposed weight Wt [N,K]: (codes [N,K], scales [ceil(N/128), ceil(K/128)])."""
-    N, K = wt.shape
-    q = torch.empty((N, K), dtype=torch.uint8, device=wt.device)
-    s = torch.empty(((N + 127) // 128, (K + 127) // 128), dtype=torch.float32, device=wt.device)
-    fp8_blockwise_symmetric_quantization(wt, q, s, N, K, 128, 128, False, stream)
-    return q, s
+    return _native.quantize(wt, _lib.QUANT_128x128, stream)
 
 
 def rmsnorm_quantize_activation(x, weight, eps, stream=None):
     """RMSNorm fused in front of the activation quantiser (the fusion the reference plans, README.md:16):
     x [M,K] float32 / bfloat16 / float16, weight [K] float32 -> (codes uint8 [M,K], scales float32 [K/128, M]) of
     ``x / sqrt(mean(x^2) + eps) * weight``, ready to be the A operand of the FP8 GEMM."""
-    M, K = x.shape
-    code = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16}.get(x.dtype)
-    if code is None:
-        raise RuntimeError("T is not supported.")
-    q = torch.empty((M, K), dtype=torch.uint8, device=x.device)
-    s = torch.empty(((K + 127) // 128, M), dtype=torch.float32, device=x.device)
-    check(lib.llmmm_rmsnorm_quant_fp8(code, _ptr(x, "x"), _ptr(weight, "weight", (torch.float32,), K), ctypes.c_float(eps), _ptr(q, "q"),
-                                      _ptr(s, "scale"), M, K, _stream(stream)))
-    return q, s
+    return _native.rmsnorm_quantize(x, weight, eps, stream)
 
 
 # ------------------------------------------------------------------------------------- FP8 GEMM
@@ -179,18 +137,17 @@ def _a_workspace_bytes(A, M, N, K, a_swiglu):
     return int(lib.llmmm_fp8_swiglu_a_workspace(M, N, K)) if a_swiglu else 0
 
 
+def _a_argument(A, M, K, a_swiglu):
+    """(A argument, a_layout, keep-alive) for the native entry points, which take a :class:`PlanesRmsnorm` as its structure's address."""
+    if isinstance(A, PlanesRmsnorm):
+        st = A.c_struct(M, K)
+        return ctypes.addressof(st), _lib.FP8_A_PLANES_RMSNORM, st
+    return A, _lib.FP8_A_SWIGLU_F32 if a_swiglu else _lib.FP8_A_QUANTISED, None
+
+
 def _fp8_gemm(out_kind, A, As, Bt, Bs, C, Cs, M, N, K, workspace, tile, split_k, stream, b_preshuffled=False, a_swiglu=False):
-    kb = K // 128 if K % 128 == 0 else 0
-    c_dtypes = {_lib.OUT_F32: (torch.float32,), _lib.OUT_BF16: (torch.bfloat16,), _lib.OUT_FP8Q: _FP8_DTYPES, _lib.OUT_FP8Q_SWIGLU: _FP8_DTYPES}[out_kind]
-    n_out = N // 2 if out_kind == _lib.OUT_FP8Q_SWIGLU else N  # SwiGLU halves the width
-    a_p, as_p, a_layout, _keep = _a_operand(A, As, M, K, a_swiglu)
-    b_p = _ptr(Bt, "B_transposed", _FP8_DTYPES, N * K)
-    bs_p = _ptr(Bs, "B_scale_transposed", (torch.float32,), ((N + 127) // 128) * kb)
-    c_p = _ptr(C, "C", c_dtypes, M * n_out)
-    cs_p = _ptr(Cs, "C_scale_transposed", (torch.float32,), ((n_out + 127) // 128) * M) if out_kind in (_lib.OUT_FP8Q, _lib.OUT_FP8Q_SWIGLU) else None
-    ws_p, ws_n = (ctypes.c_void_p(workspace.data_ptr()), workspace.numel() * workspace.element_size()) if workspace is not None else (None, 0)
-    cfg = GemmCfg(tile, split_k, _lib.FP8_B_PRESHUFFLED if b_preshuffled else _lib.FP8_B_ROWS, a_layout)
-    check(lib.llmmm_fp8_gemm_ex(out_kind, a_p, as_p, b_p, bs_p, c_p, cs_p, M, N, K, ws_p, ws_n, ctypes.byref(cfg), _stream(stream)))
+    A, a_layout, _keep = _a_argument(A, M, K, a_swiglu)
+    _native.fp8_gemm(out_kind, A, As, Bt, Bs, C, Cs, M, N, K, workspace, tile, split_k, b_preshuffled, a_layout, stream)
 
 
 def fp8_gemm_blockwise_quant_A_1x128__B_128x128__output_fp32(A, A_scale_transposed, B_transposed, B_scale_transposed, C, M, N, K,
@@ -238,24 +195,9 @@ def fp8_gemm_add_rmsnorm_quant(A, A_scale_transposed, B_transposed, B_scale_tran
     plans, README.md:16): ``hidden_out = residual + A @ B`` (stored in the residual's dtype; may be the same tensor), then
     RMSNorm(hidden_out) * norm_weight quantised 1x128 with transposed scales.  Returns (codes uint8 [M,N], scales float32
     [N/128, M]): the A operand of the next projection, bit-identical to ``rmsnorm_quantize_activation(hidden_out, ...)``."""
-    code = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16}.get(residual.dtype)
-    if code is None or hidden_out.dtype != residual.dtype:
-        raise RuntimeError("T is not supported.")
-    kb = K // 128 if K % 128 == 0 else 0
-    if workspace is None:
-        n = int(lib.llmmm_fp8_gemm_add_rmsnorm_quant_workspace(M, N, K)) + _a_workspace_bytes(A, M, N, K, a_swiglu)
-        workspace = torch.empty(max(n, 16), dtype=torch.uint8, device=residual.device)
-    q = torch.empty((M, N), dtype=torch.uint8, device=residual.device)
-    s = torch.empty(((N + 127) // 128, M), dtype=torch.float32, device=residual.device)
-    a_p, as_p, a_layout, _keep = _a_operand(A, A_scale_transposed, M, K, a_swiglu)
-    cfg = GemmCfg(tile, split_k, _lib.FP8_B_PRESHUFFLED if b_preshuffled else _lib.FP8_B_ROWS, a_layout)
-    check(lib.llmmm_fp8_gemm_add_rmsnorm_quant(
-        a_p, as_p,
-        _ptr(B_transposed, "B_transposed", _FP8_DTYPES, N * K), _ptr(B_scale_transposed, "B_scale_transposed", (torch.float32,), ((N + 127) // 128) * kb),
-        code, _ptr(residual, "residual", numel=M * N), _ptr(hidden_out, "hidden_out", numel=M * N), _ptr(norm_weight, "norm_weight", (torch.float32,), N),
-        ctypes.c_float(eps), _ptr(q, "q"), _ptr(s, "q_scale"), M, N, K, ctypes.c_void_p(workspace.data_ptr()),
-        workspace.numel() * workspace.element_size(), ctypes.byref(cfg), _stream(stream)))
-    return q, s
+    A, a_layout, _keep = _a_argument(A, M, K, a_swiglu)
+    return _native.fp8_gemm_add_rmsnorm_quant(A, A_scale_transposed, B_transposed, B_scale_transposed, residual, hidden_out, norm_weight, eps, M, N, K,
+                                              workspace, tile, split_k, b_preshuffled, a_layout, stream)
 
 
 def fp8_gemm_planes(A, A_scale_transposed, B_transposed, B_scale_transposed, M, N, K, planes=None, stream=None, workspace=None, tile=_lib.TILE_AUTO,
@@ -285,26 +227,9 @@ def fp8_gemm_qkv_rope(A, A_scale_transposed, B_transposed, B_scale_transposed, q
     """The QKV projection with per-head RMSNorm (weights [128] or None) and rotate-half RoPE of the query and key heads fused
     behind it (planned by the reference, README.md:16).  Heads are 128 wide; cos_table / sin_table [rows, 64] float32,
     positions [M] int32.  Returns the bf16 tensor [M,N], or (codes uint8 [M,N], scales float32 [N/128, M]) with out_fp8."""
-    dev = B_transposed.device
-    kb = K // 128 if K % 128 == 0 else 0
-    if workspace is None:
-        n = int(lib.llmmm_fp8_gemm_qkv_rope_workspace(M, N, K)) + _a_workspace_bytes(A, M, N, K, False)
-        workspace = torch.empty(max(n, 16), dtype=torch.uint8, device=dev)
-    out = torch.empty((M, N), dtype=torch.uint8 if out_fp8 else torch.bfloat16, device=dev)
-    sc = torch.empty(((N + 127) // 128, M), dtype=torch.float32, device=dev) if out_fp8 else None
-    rows = cos_table.shape[0]
-    a_p, as_p, a_layout, _keep = _a_operand(A, A_scale_transposed, M, K, False)
-    cfg = GemmCfg(tile, split_k, _lib.FP8_B_PRESHUFFLED if b_preshuffled else _lib.FP8_B_ROWS, a_layout)
-    check(lib.llmmm_fp8_gemm_qkv_rope(
-        _lib.OUT_FP8Q if out_fp8 else _lib.OUT_BF16, a_p, as_p,
-        _ptr(B_transposed, "B_transposed", _FP8_DTYPES, N * K), _ptr(B_scale_transposed, "B_scale_transposed", (torch.float32,), ((N + 127) // 128) * kb),
-        _ptr(out, "out"), _ptr(sc, "out_scale") if out_fp8 else None,
-        _ptr(q_norm_weight, "q_norm_weight", (torch.float32,), 128) if q_norm_weight is not None else None,
-        _ptr(k_norm_weight, "k_norm_weight", (torch.float32,), 128) if k_norm_weight is not None else None, ctypes.c_float(eps),
-        _ptr(cos_table, "cos_table", (torch.float32,), rows * 64), _ptr(sin_table, "sin_table", (torch.float32,), rows * 64), rows,
-        _ptr(positions, "positions", (torch.int32,), M), n_q_heads, n_kv_heads, M, N, K, ctypes.c_void_p(workspace.data_ptr()),
-        workspace.numel() * workspace.element_size(), ctypes.byref(cfg), _stream(stream)))
-    return (out, sc) if out_fp8 else out
+    A, a_layout, _keep = _a_argument(A, M, K, False)
+    return _native.fp8_gemm_qkv_rope(A, A_scale_transposed, B_transposed, B_scale_transposed, q_norm_weight, k_norm_weight, eps, cos_table, sin_table,
+                                     positions, n_q_heads, n_kv_heads, M, N, K, out_fp8, workspace, tile, split_k, b_preshuffled, a_layout, stream)
 
 
 # ------------------------------------------------------------------------------------- offline layout helpers
@@ -327,10 +252,7 @@ def restore_B_layout(dst_transposed, src, N, K, stream=None):
 
 def preshuffle_weight(bq, stream=None):
     """Bt [N,K] e4m3 codes -> a new tensor holding the pre-shuffled image (same shape and dtype)."""
-    N, K = bq.shape
-    out = torch.empty_like(bq)
-    construct_mfma_B_layout(out, bq, N, K, stream)
-    return out
+    return _native.preshuffle(bq, stream)
 
 
 def transpose_matrix__aligned_128(dst, src, M, N, stream=None):
