@@ -132,34 +132,83 @@ __device__ __forceinline__ void tile_coords(int wg, int tiles_m, int tiles_n, in
   tn                = in / gm;
 }
 
-// The value lane (l ^ mask) holds, for mask = 1, 2, 4, 8, 16 or 32 (a compile-time constant at every call site once
-// inlined).  No LDS address computation and, for 1, 2 and 32, no trip through the LDS crossbar at all:
-//   1, 2     DPP quad permutes (a VALU move),
-//   4 .. 16  ds_swizzle in bit-mask mode (xor inside each group of 32 lanes),
-//   32       v_permlane32_swap exchanges the upper 32 lanes of its first register with the lower 32 lanes of its second:
-//            from (v, v) it returns r[0] = the lower half of v in both halves, r[1] = the upper half in both halves.
-__device__ __forceinline__ float wave_xor_get(float v, int mask)
+// mask = 16: v_permlane16_swap exchanges the odd 16-lane rows of its first register with the even rows of its second; from (v, v)
+// it gives a = the even row of each pair in both rows, b = the odd row in both.  mask = 32: v_permlane32_swap, likewise for the
+// halves of the wavefront.
+// (The empty asm keeps them two values: the compiler otherwise takes both results for v and drops the operation on them.)
+struct WavePair {
+  float a, b;
+};
+template <int MASK>
+__device__ __forceinline__ WavePair wave_swap_pair(float v)
+{
+  static_assert(MASK == 16 || MASK == 32, "row or half swap");
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  unsigned       x, y;
+  if constexpr (MASK == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    x = r[0], y = r[1];
+  }
+  else {
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    x = r[0], y = r[1];
+  }
+  asm("" : "+v"(x), "+v"(y));
+  return {__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
+}
+// The value lane (l ^ mask) holds, for mask = 1, 2, 4, 8, 16 or 32.  Register moves only, no trip through the LDS crossbar -- the reductions of the row kernels are chains of these,
+// eleven long, and with ds_swizzle for 4, 8 and 16 (about 60 cycles a step instead of 8) seven of the eleven waited on it:
+//   1, 2     DPP quad permutes,
+//   4        lane l + 4 for the lanes with bit 2 clear, l - 4 for the others: two DPP row shifts with complementary bank masks,
+//   8        a DPP rotation of the 16-lane row by 8,
+//   16, 32   the row and half swaps above.
+template <int MASK>
+__device__ __forceinline__ float wave_xor_get(float v)
 {
   const int iv = __builtin_bit_cast(int, v);
-  switch (mask) {
-    case 1: return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(iv, 0xB1, 0xf, 0xf, true));  // quad_perm [1,0,3,2]
-    case 2: return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(iv, 0x4E, 0xf, 0xf, true));  // quad_perm [2,3,0,1]
-    case 4: return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(iv, (4 << 10) | 0x1f));
-    case 8: return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(iv, (8 << 10) | 0x1f));
-    case 16: return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(iv, (16 << 10) | 0x1f));
-    case 32: {
-      const auto r = __builtin_amdgcn_permlane32_swap((unsigned)iv, (unsigned)iv, false, false);
-      // lanes 0..31 want the upper half (r[1]), lanes 32..63 the lower half (r[0])
-      return __builtin_bit_cast(float, (__lane_id() < 32) ? r[1] : r[0]);
-    }
-    default: return __shfl_xor(v, mask, 64);
+  if constexpr (MASK == 1)
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(iv, 0xB1, 0xf, 0xf, true));  // quad_perm [1,0,3,2]
+  else if constexpr (MASK == 2)
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(iv, 0x4E, 0xf, 0xf, true));  // quad_perm [2,3,0,1]
+  else if constexpr (MASK == 4) {
+    const int up = __builtin_amdgcn_update_dpp(iv, iv, 0x104, 0xf, 0x5, false);                     // row_shl:4 into banks 0 and 2
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, iv, 0x114, 0xf, 0xa, false));  // row_shr:4 into banks 1 and 3
+  }
+  else if constexpr (MASK == 8)
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(iv, 0x128, 0xf, 0xf, true));  // row_ror:8
+  else {
+    const WavePair p = wave_swap_pair<MASK>(v);
+    return (__lane_id() & MASK) ? p.a : p.b;
   }
 }
 
-__device__ __forceinline__ float wave_xor_max(float v, int mask)
+// v op (the value of lane l ^ MASK), op = maximum / sum.  For 16 and 32 the swap already yields both operands, and both
+// operations are commutative, so nothing has to be selected.
+template <int MASK>
+__device__ __forceinline__ float wave_xor_max(float v)
 {
-  return fmaxf(v, wave_xor_get(v, mask));
+  if constexpr (MASK >= 16) {
+    const WavePair p = wave_swap_pair<MASK>(v);
+    return fmaxf(p.a, p.b);
+  }
+  else
+    return fmaxf(v, wave_xor_get<MASK>(v));
 }
+template <int MASK>
+__device__ __forceinline__ float wave_xor_sum(float v)
+{
+  if constexpr (MASK >= 16) {
+    const WavePair p = wave_swap_pair<MASK>(v);
+    return p.a + p.b;
+  }
+  else
+    return v + wave_xor_get<MASK>(v);
+}
+// Maximum over the 32 lanes of each half of the wavefront; sums over them and over all 64 lanes, the distant lanes first (the
+// order the CPU oracle adds in).
+__device__ __forceinline__ float half_wave_max(float v) { return wave_xor_max<16>(wave_xor_max<8>(wave_xor_max<4>(wave_xor_max<2>(wave_xor_max<1>(v))))); }
+__device__ __forceinline__ float half_wave_sum(float v) { return wave_xor_sum<1>(wave_xor_sum<2>(wave_xor_sum<4>(wave_xor_sum<8>(wave_xor_sum<16>(v))))); }
+__device__ __forceinline__ float wave_sum(float v) { return half_wave_sum(wave_xor_sum<32>(v)); }
 
 // ---------------------------------------------------------------------------------------------
 // fp32 -> OCP e4m3, four codes per dword, as the reference's __nv_fp8_e4m3(float) gives them (round to nearest even,

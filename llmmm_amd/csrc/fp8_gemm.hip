@@ -282,8 +282,8 @@ __device__ __forceinline__ void swiglu_finish(const f32x4 (&acc)[8][MF], const f
         v[nf][q]         = IS_GATE ? silu_mul(mine, theirs) : silu_mul(theirs, mine);
         amax             = fmaxf(amax, __builtin_fabsf(v[nf][q]));
       }
-    amax              = wave_xor_max(amax, 16);
-    amax              = wave_xor_max(amax, 32);
+    amax              = wave_xor_max<16>(amax);
+    amax              = wave_xor_max<32>(amax);
     const float scale = amax / 448.f;
     const float inv   = requant_inv(amax);
     const int   r     = h * 16 + li;
@@ -358,8 +358,8 @@ __device__ __forceinline__ void qk_norm_rope_fragments(f32x4 (&acc)[8][MF], cons
         p[nf] = a;
       }
       float t = ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
-      t       = t + wave_xor_get(t, 32);
-      t       = t + wave_xor_get(t, 16);
+      t       = wave_xor_sum<32>(t);
+      t       = wave_xor_sum<16>(t);
       r[mf]   = 1.0f / __builtin_sqrtf(t / 128.0f + op.eps);
     }
 #pragma unroll
@@ -742,8 +742,8 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
       for (int nf = 0; nf < 8; ++nf)
 #pragma unroll
         for (int q = 0; q < 4; ++q) amax = fmaxf(amax, __builtin_fabsf(acc[nf][mf][q]));
-      amax              = wave_xor_max(amax, 16);
-      amax              = wave_xor_max(amax, 32);
+      amax              = wave_xor_max<16>(amax);
+      amax              = wave_xor_max<32>(amax);
       const float scale = amax / 448.f;
       const float inv   = requant_inv(amax);
       const int   r     = mf * 16 + li;
@@ -871,11 +871,7 @@ fp8_splitk_reduce_kernel(const float* __restrict__ planes, int S, void* __restri
     else {  // e4m3 codes + 1x128 scales, of C or (SwiGLU) of h, whose rows are N/2 wide
       const int ldc = OUT == OUT_SWIGLU ? (N >> 1) : N;
       float a = fmaxf(fmaxf(fmaxf(0.f, __builtin_fabsf(v[0])), __builtin_fabsf(v[1])), fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3])));
-      a       = wave_xor_max(a, 1);
-      a       = wave_xor_max(a, 2);
-      a       = wave_xor_max(a, 4);
-      a       = wave_xor_max(a, 8);
-      a       = wave_xor_max(a, 16);
+      a = half_wave_max(a);
       const float scale = a / 448.f;
       const float inv   = requant_inv(a);
       *(uint32_t*)((uint8_t*)Cv + (size_t)m * ldc + n) = pack_e4m3x4_in_range(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
@@ -926,8 +922,7 @@ fp8_planes_qk_norm_rope_kernel(const float* __restrict__ planes, int S, void* __
       float acc = 0.f;
 #pragma unroll
       for (int q = 0; q < 4; ++q) acc = __builtin_fmaf(v[q], v[q], acc);
-#pragma unroll
-      for (int step = 16; step >= 1; step >>= 1) acc = acc + wave_xor_get(acc, step);
+      acc = half_wave_sum(acc);
       const float r = 1.0f / __builtin_sqrtf(acc / 128.0f + eps);
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[q] = (v[q] * r) * w4[q];
@@ -935,7 +930,7 @@ fp8_planes_qk_norm_rope_kernel(const float* __restrict__ planes, int S, void* __
     if (rotate) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const float other = wave_xor_get(v[q], 16);
+        const float other = wave_xor_get<16>(v[q]);
         const float t     = other * sn[q];
         v[q]              = __builtin_fmaf(v[q], cs[q], lo ? -t : t);
       }
@@ -949,8 +944,7 @@ fp8_planes_qk_norm_rope_kernel(const float* __restrict__ planes, int S, void* __
     }
     else {
       float a = fmaxf(fmaxf(fmaxf(0.f, __builtin_fabsf(v[0])), __builtin_fabsf(v[1])), fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3])));
-#pragma unroll
-      for (int step = 1; step <= 16; step <<= 1) a = wave_xor_max(a, step);
+      a = half_wave_max(a);
       const float scale = a / 448.f;
       const float inv   = requant_inv(a);
       *(uint32_t*)((uint8_t*)Cv + (size_t)m * N + n) = pack_e4m3x4_in_range(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);

@@ -372,8 +372,7 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
       else
         held[u] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-#pragma unroll
-    for (int step = 32; step >= 1; step >>= 1) acc = acc + wave_xor_get(acc, step);
+    acc = wave_sum(acc);
     if (lane == 0) gen_sum[wave] = acc;
     __syncthreads();  // (also: the zero fill is complete)
     const float total = (gen_sum[4 * rsel] + gen_sum[4 * rsel + 1]) + (gen_sum[4 * rsel + 2] + gen_sum[4 * rsel + 3]);
@@ -388,8 +387,7 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
 #pragma unroll
         for (int e = 0; e < 4; ++e) held[u][e] = (held[u][e] * rn) * wv[u][e];
         float a = fmaxf(fmaxf(fmaxf(0.f, __builtin_fabsf(held[u][0])), __builtin_fabsf(held[u][1])), fmaxf(__builtin_fabsf(held[u][2]), __builtin_fabsf(held[u][3])));
-#pragma unroll
-        for (int step = 1; step <= 16; step <<= 1) a = wave_xor_max(a, step);
+        a = half_wave_max(a);
         const float sc = a / 448.f;
         uint32_t    cd = 0;
         if (sc != 0.f) cd = pack_e4m3x4_sat(held[u][0] / sc, held[u][1] / sc, held[u][2] / sc, held[u][3] / sc);
@@ -440,8 +438,7 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
 #pragma unroll
           for (int q = 0; q < 4; ++q) h[q] = silu_mul(gv[u][q], uv[u][q]);
           float a = fmaxf(fmaxf(fmaxf(0.f, __builtin_fabsf(h[0])), __builtin_fabsf(h[1])), fmaxf(__builtin_fabsf(h[2]), __builtin_fabsf(h[3])));
-#pragma unroll
-          for (int step = 1; step <= 16; step <<= 1) a = wave_xor_max(a, step);
+          a = half_wave_max(a);
           const float scale = a / 448.f;
           const float inv   = requant_inv(a);
           *(uint32_t LLMMM_LDS*)((char LLMMM_LDS*)a_stage + j * 2048 + kmajor_offset<SWZ_ROWS16>(r, l32 >> 2) + (l32 & 3) * 4) =
@@ -520,8 +517,8 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
     for (int mb = 0; mb < MBLK; ++mb) {
       float a = fmaxf(fmaxf(fmaxf(0.f, __builtin_fabsf(acc[mb][0])), __builtin_fabsf(acc[mb][1])),
                       fmaxf(__builtin_fabsf(acc[mb][2]), __builtin_fabsf(acc[mb][3])));
-      a       = wave_xor_max(a, 16);
-      a       = wave_xor_max(a, 32);
+      a       = wave_xor_max<16>(a);
+      a       = wave_xor_max<32>(a);
       if (g == 0) wave_amax[wave][mb][i] = a;
     }
     __syncthreads();
@@ -712,8 +709,8 @@ fp8_strip_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, co
     // width leave an area in the same state; rows beyond M take part with whatever their sums are: their maxima are
     // exchanged and never used)
     float a = fmaxf(fmaxf(fmaxf(0.f, __builtin_fabsf(v[0])), __builtin_fabsf(v[1])), fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3])));
-    a       = wave_xor_max(a, 16);
-    a       = wave_xor_max(a, 32);  // the fragment's maximum of row i, in all four lanes that hold the row
+    a       = wave_xor_max<16>(a);
+    a       = wave_xor_max<32>(a);  // the fragment's maximum of row i, in all four lanes that hold the row
     const int frag = blockIdx.x * CF + cf, grp = frag >> 3, strip = frag & 7;
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(own_mark)::"memory");  // long landed; ties the register to this point
     const int cur = own_mark != 0u ? 1 : 0;  // the buffer this fragment did not fill last time (both clean: buffer 0)
@@ -738,8 +735,7 @@ fp8_strip_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, co
       __builtin_amdgcn_s_sleep(1);
     }
     float r0 = __builtin_bit_cast(float, (unsigned)w - 1u), r1 = __builtin_bit_cast(float, (unsigned)(w >> 32) - 1u);
-#pragma unroll
-    for (int step = 8; step <= 32; step <<= 1) r0 = wave_xor_max(r0, step), r1 = wave_xor_max(r1, step);  // over the group's fragments
+    r0 = wave_xor_max<32>(wave_xor_max<16>(wave_xor_max<8>(r0))), r1 = wave_xor_max<32>(wave_xor_max<16>(wave_xor_max<8>(r1)));  // over the group's fragments
     const float e0 = __shfl(r0, i >> 1, 64), e1 = __shfl(r1, i >> 1, 64);
     const float amax = (i & 1) ? e1 : e0;  // the group's maximum of row i
     const float scale = amax / 448.f;

@@ -83,11 +83,7 @@ __global__ void __launch_bounds__(256) quant_1x128_kernel(const float* __restric
       if (m >= mend) break;  // uniform over the half-wavefront that shares the row
       float a = QUANT_AMAX_SEED;
       if (live) a = amax4(a, v[u]);
-      a       = wave_xor_max(a, 1);
-      a       = wave_xor_max(a, 2);
-      a       = wave_xor_max(a, 4);
-      a       = wave_xor_max(a, 8);
-      a       = wave_xor_max(a, 16);
+      a = half_wave_max(a);
       const float s = a / 448.f;
       uint32_t    c = 0;
       if (s != 0.f) c = q_pack_quotients_e4m3x4(v[u], s);
@@ -127,12 +123,8 @@ __global__ void __launch_bounds__(256) quant_128x128_kernel(const float* __restr
       a    = amax4(a, v[r]);
     }
   }
-  a = wave_xor_max(a, 1);
-  a = wave_xor_max(a, 2);
-  a = wave_xor_max(a, 4);
-  a = wave_xor_max(a, 8);
-  a = wave_xor_max(a, 16);
-  a = wave_xor_max(a, 32);
+  a = half_wave_max(a);
+  a = wave_xor_max<32>(a);
   if ((tid & 63) == 0) wmax[tid >> 6] = a;
   __syncthreads();
   a             = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
@@ -179,11 +171,7 @@ __device__ __forceinline__ void rmsnorm_quant_chunk(f32x4 v, float r, const floa
     for (int e = 0; e < 4; ++e) y[e] = (v[e] * r) * wv[e];
   }
   float a = amax4(0.f, y);
-  a       = wave_xor_max(a, 1);
-  a       = wave_xor_max(a, 2);
-  a       = wave_xor_max(a, 4);
-  a       = wave_xor_max(a, 8);
-  a       = wave_xor_max(a, 16);
+  a = half_wave_max(a);
   const float s  = a / 448.f;
   uint32_t    cd = 0;
   if (s != 0.f) cd = q_pack_quotients_e4m3x4(y, s);
@@ -217,9 +205,7 @@ __global__ void __launch_bounds__(256) rmsnorm_quant_1x128_kernel(const IN_T* __
     }
   }
 #pragma unroll
-  for (int step = 32; step >= 1; step >>= 1)
-#pragma unroll
-    for (int gidx = 0; gidx < 4; ++gidx) part[gidx] = part[gidx] + wave_xor_get(part[gidx], step);
+  for (int gidx = 0; gidx < 4; ++gidx) part[gidx] = wave_sum(part[gidx]);
   const float acc = (part[0] + part[1]) + (part[2] + part[3]);
   const float ms  = acc / (float)K;
   const float r   = 1.0f / __builtin_sqrtf(ms + eps);
@@ -245,24 +231,21 @@ __global__ void __launch_bounds__(256) rmsnorm_quant_row_kernel(const IN_T* __re
   const int   chunks = K >> 2;
   f32x4       held[NI], wv[NI];
   float       acc = 0.f;
+  // every load without a condition (threads past the end of the row load its last chunk and drop it): behind one, the bf16
+  // values are converted inside the branch, and each chunk's load waits for the one before it
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int c = t + 256 * i;
-    held[i]     = f32x4{0.f, 0.f, 0.f, 0.f};
-    wv[i]       = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (c < chunks) {
-      held[i] = load_row4<IN_T>(xr + 4 * c);
-      wv[i]   = *(const f32x4*)(w + 4 * c);
-    }
+    const int c = min(t + 256 * i, chunks - 1);
+    held[i]     = load_row4<IN_T>(xr + 4 * c);
+    wv[i]       = *(const f32x4*)(w + 4 * c);
   }
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
-    if (t + 256 * i < chunks) {
+  for (int i = 0; i < NI; ++i) {
+    if (t + 256 * i >= chunks) held[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = __builtin_fmaf(held[i][e], held[i][e], acc);
-    }
-#pragma unroll
-  for (int step = 32; step >= 1; step >>= 1) acc = acc + wave_xor_get(acc, step);
+    for (int e = 0; e < 4; ++e) acc = __builtin_fmaf(held[i][e], held[i][e], acc);
+  }
+  acc = wave_sum(acc);
   if ((t & 63) == 0) group_sum[t >> 6] = acc;
   __syncthreads();
   const float total = (group_sum[0] + group_sum[1]) + (group_sum[2] + group_sum[3]);
@@ -276,9 +259,7 @@ __global__ void __launch_bounds__(256) rmsnorm_quant_row_kernel(const IN_T* __re
     amax[i] = amax4(0.f, held[i]);
   }
 #pragma unroll
-  for (int step = 1; step <= 16; step <<= 1)
-#pragma unroll
-    for (int i = 0; i < NI; ++i) amax[i] = wave_xor_max(amax[i], step);
+  for (int i = 0; i < NI; ++i) amax[i] = half_wave_max(amax[i]);
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int   c  = t + 256 * i;
@@ -325,15 +306,18 @@ __global__ void __launch_bounds__(256) planes_add_rmsnorm_quant_kernel(const flo
     rv[i]       = load_row4<T>(residual + (size_t)m * N + 4 * c);
     wv[i]       = *(const f32x4*)(w + 4 * c);
   }
-  constexpr int W = NI <= 3 ? 8 : 2;
+  // W planes in flight, as many as about 128 registers hold; only the planes that exist are asked for.
+  constexpr int W = NI <= 4 ? 8 : 32 / NI;
   for (int s0 = 0; s0 < S; s0 += W) {
     f32x4 p[W][NI];
 #pragma unroll
     for (int u = 0; u < W; ++u)
+      if (s0 + u < S) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int c = min(t + 256 * i, chunks - 1);
-        p[u][i]     = __builtin_nontemporal_load((const f32x4*)(planes + (size_t)min(s0 + u, S - 1) * plane + (size_t)m * N + 4 * c));
+        for (int i = 0; i < NI; ++i) {
+          const int c = min(t + 256 * i, chunks - 1);
+          p[u][i]     = __builtin_nontemporal_load((const f32x4*)(planes + (size_t)(s0 + u) * plane + (size_t)m * N + 4 * c));
+        }
       }
 #pragma unroll
     for (int u = 0; u < W; ++u)
@@ -362,8 +346,7 @@ __global__ void __launch_bounds__(256) planes_add_rmsnorm_quant_kernel(const flo
     else
       held[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-#pragma unroll
-  for (int step = 32; step >= 1; step >>= 1) acc = acc + wave_xor_get(acc, step);
+  acc = wave_sum(acc);
   if ((t & 63) == 0) group_sum[t >> 6] = acc;
   __syncthreads();
   const float total = (group_sum[0] + group_sum[1]) + (group_sum[2] + group_sum[3]);
@@ -377,9 +360,7 @@ __global__ void __launch_bounds__(256) planes_add_rmsnorm_quant_kernel(const flo
     amax[i] = amax4(0.f, held[i]);
   }
 #pragma unroll
-  for (int step = 1; step <= 16; step <<= 1)
-#pragma unroll
-    for (int i = 0; i < NI; ++i) amax[i] = wave_xor_max(amax[i], step);
+  for (int i = 0; i < NI; ++i) amax[i] = half_wave_max(amax[i]);
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int   c  = t + 256 * i;
@@ -393,49 +374,67 @@ __global__ void __launch_bounds__(256) planes_add_rmsnorm_quant_kernel(const flo
   }
 }
 
+// Chunks a thread of the two row kernels holds: the smallest of these that covers the row.  With 3 and 10 only, a row of 4096
+// columns behind eight planes loaded ten chunks of every plane where it has four, two planes at a time: 16 rows
+// 13.2 us, now 5.9 (and 5.3 -> 3.7 for rmsnorm_quant_row_kernel on 16 rows of 4096, 3.0 -> 2.5 on one of 2560, with the loads and the
+// reductions below).
+#define LLMMM_ROW_CHUNKS(COLUMNS, GO) \
+  switch (((COLUMNS) + 1023) / 1024) { \
+    case 1:                           \
+    case 2: GO(2); break;             \
+    case 3: GO(3); break;             \
+    case 4: GO(4); break;             \
+    case 5: GO(5); break;             \
+    case 6:                           \
+    case 7:                           \
+    case 8: GO(8); break;             \
+    default: GO(10); break;           \
+  }
+
+template <typename T>
+static void launch_planes_add_rmsnorm_quant(const float* planes, int S, const void* residual, void* hidden, const float* w, float eps, void* q, float* scale,
+                                            int M, int N, hipStream_t stream)
+{
+#define LLMMM_GO(NI)                                                                                                                             \
+  hipLaunchKernelGGL((planes_add_rmsnorm_quant_kernel<T, NI>), dim3(M), dim3(256), 0, stream, planes, S, (const T*)residual, (T*)hidden, w, eps, \
+                     (uint8_t*)q, scale, M, N)
+  LLMMM_ROW_CHUNKS(N, LLMMM_GO)
+#undef LLMMM_GO
+}
+
 hipError_t planes_add_rmsnorm_quant_launch(int hidden_dtype, const float* planes, int S, const void* residual, void* hidden, const float* w,
                                            float eps, void* q, float* scale, int M, int N, hipStream_t stream)
 {
-#define LLMMM_GO(T)                                                                                                                        \
-  {                                                                                                                                        \
-    if (N <= 1024 * 3)                                                                                                                     \
-      hipLaunchKernelGGL((planes_add_rmsnorm_quant_kernel<T, 3>), dim3(M), dim3(256), 0, stream, planes, S, (const T*)residual, (T*)hidden, \
-                         w, eps, (uint8_t*)q, scale, M, N);                                                                                \
-    else                                                                                                                                   \
-      hipLaunchKernelGGL((planes_add_rmsnorm_quant_kernel<T, 10>), dim3(M), dim3(256), 0, stream, planes, S, (const T*)residual,           \
-                         (T*)hidden, w, eps, (uint8_t*)q, scale, M, N);                                                                    \
-  }
   if (N > 1024 * 10) return hipErrorInvalidValue;
   switch (hidden_dtype) {
-    case LLMMM_DTYPE_F16: LLMMM_GO(_Float16) break;
-    case LLMMM_DTYPE_BF16: LLMMM_GO(__bf16) break;
-    case LLMMM_DTYPE_F32: LLMMM_GO(float) break;
+    case LLMMM_DTYPE_F16: launch_planes_add_rmsnorm_quant<_Float16>(planes, S, residual, hidden, w, eps, q, scale, M, N, stream); break;
+    case LLMMM_DTYPE_BF16: launch_planes_add_rmsnorm_quant<__bf16>(planes, S, residual, hidden, w, eps, q, scale, M, N, stream); break;
+    case LLMMM_DTYPE_F32: launch_planes_add_rmsnorm_quant<float>(planes, S, residual, hidden, w, eps, q, scale, M, N, stream); break;
     default: return hipErrorInvalidValue;
   }
-#undef LLMMM_GO
   return hipGetLastError();
+}
+
+template <typename T>
+static void launch_rmsnorm_quant(const void* x, const float* w, float eps, void* q, float* scale, int M, int K, hipStream_t stream)
+{
+#define LLMMM_GO(NI) hipLaunchKernelGGL((rmsnorm_quant_row_kernel<T, NI>), dim3(M), dim3(256), 0, stream, (const T*)x, w, eps, (uint8_t*)q, scale, M, K)
+  if (K <= 1024 * 10)
+    LLMMM_ROW_CHUNKS(K, LLMMM_GO)
+  else
+    hipLaunchKernelGGL((rmsnorm_quant_1x128_kernel<T>), dim3((M + 3) / 4), dim3(256), 0, stream, (const T*)x, w, eps, (uint8_t*)q, scale, M, K);
+#undef LLMMM_GO
 }
 
 hipError_t rmsnorm_quant_launch(int in_dtype, const void* x, const float* w, float eps, void* q, float* scale, int M, int K,
                                 hipStream_t stream)
 {
-  const dim3 grid((M + 3) / 4), block(256);
-#define LLMMM_NORM_GO(T)                                                                                                               \
-  {                                                                                                                                    \
-    if (K <= 1024 * 3)                                                                                                                 \
-      hipLaunchKernelGGL((rmsnorm_quant_row_kernel<T, 3>), dim3(M), block, 0, stream, (const T*)x, w, eps, (uint8_t*)q, scale, M, K);   \
-    else if (K <= 1024 * 10)                                                                                                           \
-      hipLaunchKernelGGL((rmsnorm_quant_row_kernel<T, 10>), dim3(M), block, 0, stream, (const T*)x, w, eps, (uint8_t*)q, scale, M, K);  \
-    else                                                                                                                               \
-      hipLaunchKernelGGL((rmsnorm_quant_1x128_kernel<T>), grid, block, 0, stream, (const T*)x, w, eps, (uint8_t*)q, scale, M, K);       \
-  }
   switch (in_dtype) {
-    case LLMMM_DTYPE_F16: LLMMM_NORM_GO(_Float16) break;
-    case LLMMM_DTYPE_BF16: LLMMM_NORM_GO(__bf16) break;
-    case LLMMM_DTYPE_F32: LLMMM_NORM_GO(float) break;
+    case LLMMM_DTYPE_F16: launch_rmsnorm_quant<_Float16>(x, w, eps, q, scale, M, K, stream); break;
+    case LLMMM_DTYPE_BF16: launch_rmsnorm_quant<__bf16>(x, w, eps, q, scale, M, K, stream); break;
+    case LLMMM_DTYPE_F32: launch_rmsnorm_quant<float>(x, w, eps, q, scale, M, K, stream); break;
     default: return hipErrorInvalidValue;
   }
-#undef LLMMM_NORM_GO
   return hipGetLastError();
 }
 

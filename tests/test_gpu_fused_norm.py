@@ -61,6 +61,13 @@ def test_streaming_kernel(lib, oracle, M, N, K, split, dt):
     _check(lib, oracle, M, N, K, dt, TILES["skinny"], split)
 
 
+# the row kernel behind the planes: both sides of every step in the chunks a thread holds, planes in one batch, just more than
+# one batch, and a batch of one
+@pytest.mark.parametrize("N,split", [(2048, 8), (2176, 9), (3072, 8), (3200, 9), (4096, 8), (4224, 6), (5120, 7), (5248, 4), (8192, 5), (8320, 3), (10240, 4)])
+def test_chunk_edges(lib, oracle, N, split):
+    _check(lib, oracle, 7, N, 128 * split + 128, "bf16", TILES["skinny"], split)
+
+
 # the tile kernels in plane mode (one plane and split-K)
 @pytest.mark.parametrize("M,N,K,tile,split", [(256, 2560, 4096, "auto", 0), (128, 2560, 1024, "128x128", 1), (128, 2560, 1024, "128x128", 3),
                                               (512, 2560, 512, "256x256", 0), (256, 2560, 9728, "128x256", 2), (2048, 2560, 256, "auto", 0)])

@@ -29,6 +29,12 @@ def test_bit_exact_against_oracle(lib, oracle, M, K, dtype):
     assert np.array_equal(q.cpu().numpy(), rq), "codes differ"
 
 
+# a thread of the row kernel holds 2, 3, 4, 5, 8 or 10 chunks of 1024 columns: both sides of every such edge
+@pytest.mark.parametrize("K", [1024, 1152, 2048, 2176, 3072, 3200, 4096, 4224, 5120, 5248, 7168, 8192, 8320, 10240])
+def test_chunk_edges(lib, oracle, K):
+    test_bit_exact_against_oracle(lib, oracle, 9, K, torch.bfloat16)
+
+
 def test_feeds_the_gemm(lib, oracle):
     """End to end: rmsnorm + quant on the GPU, then the FP8 GEMM, against the oracle's chain."""
     from helpers import assert_fp8_gemm_close
