@@ -37,6 +37,20 @@ def test_bit_exact_against_oracle(lib, oracle, M, N, quant_m, transpose):
         assert (s.view(np.uint32) == rs.view(np.uint32)).all()
 
 
+@pytest.mark.parametrize("M,N", [(1, 4), (7, 132), (127, 124), (129, 260), (249, 252), (385, 1024)])
+def test_block_maximum_in_the_last_row_and_column(lib, oracle, M, N):
+    """128 x 128 blocks that the matrix cuts short: threads past its end read the last row or column again, so the maximum must be
+    each block's own wherever it sits."""
+    rng = np.random.default_rng(M + N)
+    x = rng.normal(0, 1, (M, N)).astype(np.float32)
+    x[M - 1, :] *= 7
+    x[:, N - 1] *= 11
+    x[M - 1, N - 1] = -300
+    rq, rs = oracle.quant_fp8(x, 128, False)
+    q, s = _run(lib, x, 128, False, rs.shape)
+    assert (q == rq).all() and (s.view(np.uint32) == rs.view(np.uint32)).all()
+
+
 def test_golden_fixture(lib):
     d = np.load(os.path.join(G, "quant_130x256.npz"))
     q, s = _run(lib, d["x"], 1, True, d["s_1x128_t"].shape)
