@@ -51,6 +51,18 @@ def test_block_maximum_in_the_last_row_and_column(lib, oracle, M, N):
     assert (q == rq).all() and (s.view(np.uint32) == rs.view(np.uint32)).all()
 
 
+@pytest.mark.parametrize("quant_m", [1, 128])
+def test_block_maximum_in_every_lane(lib, oracle, quant_m):
+    """Row m of block m % 2 has its maximum (of either sign) in column m: every lane's value crosses every step of the reduction."""
+    rng = np.random.default_rng(5)
+    x = rng.uniform(-1, 1, (128, 256)).astype(np.float32)
+    for m in range(128):
+        x[m, (m % 2) * 128 + m] = (2.0 + m) * (-1) ** (m // 2)
+    rq, rs = oracle.quant_fp8(x, quant_m, False)
+    q, s = _run(lib, x, quant_m, False, rs.shape)
+    assert (q == rq).all() and (s.view(np.uint32) == rs.view(np.uint32)).all()
+
+
 def test_golden_fixture(lib):
     d = np.load(os.path.join(G, "quant_130x256.npz"))
     q, s = _run(lib, d["x"], 1, True, d["s_1x128_t"].shape)
