@@ -85,37 +85,93 @@ bool as_bool(PyObject* o)
   return v != 0;
 }
 
-PyObject* current_raw_stream;  // torch._C._cuda_getCurrentRawStream(device index)
-
-// None: torch's current stream; a torch stream: its handle; anything else: the handle as an integer.
-void* as_stream(PyObject* o)
-{
-  if (o == Py_None) {
-    const long device = c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getDevice().index();
-    PyObject*  index  = PyLong_FromLong(device);
-    PyObject*  raw    = index ? PyObject_CallOneArg(current_raw_stream, index) : nullptr;
-    Py_XDECREF(index);
-    if (!raw) throw Refused();
-    void* p = PyLong_AsVoidPtr(raw);
-    Py_DECREF(raw);
-    if (!p && PyErr_Occurred()) throw Refused();
-    return p;
+// A Python object that is dropped with its scope; null: a Python exception has been set.
+struct Owned {
+  PyObject* o;
+  explicit Owned(PyObject* o) : o(o)
+  {
+    if (!o) throw Refused();
   }
-  PyObject* handle = PyLong_Check(o) ? nullptr : PyObject_GetAttrString(o, "cuda_stream");
-  if (!handle) PyErr_Clear();
-  PyObject* index = PyNumber_Long(handle ? handle : o);
-  Py_XDECREF(handle);
-  if (!index) throw Refused();
-  void* p = PyLong_AsVoidPtr(index);
-  Py_DECREF(index);
+  Owned(const Owned&) = delete;
+  ~Owned() { Py_DECREF(o); }
+};
+void* as_pointer(PyObject* o)
+{
+  void* p = PyLong_AsVoidPtr(o);
   if (!p && PyErr_Occurred()) throw Refused();
   return p;
 }
-
-at::Tensor empty(at::IntArrayRef sizes, at::ScalarType type, const at::Device& device)
+int64_t int_attribute(PyObject* o, const char* name)
 {
-  return at::empty(sizes, at::TensorOptions().dtype(type).device(device));
+  const Owned     a(PyObject_GetAttrString(o, name));
+  const long long v = PyLong_AsLongLong(a.o);
+  if (v == -1 && PyErr_Occurred()) throw Refused();
+  return v;
 }
+
+PyObject *current_raw_stream, *external_stream;  // torch._C._cuda_getCurrentRawStream(device index), torch.cuda.ExternalStream
+
+// The stream a call runs on.  Its tensors -- the private workspace, which the caller never sees and nobody else can protect, and the
+// returned outputs -- belong to that stream: the allocator hands a block freed there only to work ordered behind this call.  From the
+// current stream's blocks they would be taken while that stream may still use them, and given back while this call still runs.
+struct Launch {
+  void*       handle;
+  bool        foreign = false;                                                     // not torch's current stream
+  c10::Stream current = c10::Stream(c10::Stream::DEFAULT, c10::Device(c10::kCUDA, 0)), stream = current;  // set where foreign
+
+  template <typename Make>
+  at::Tensor allocate(Make&& make) const
+  {
+    if (!foreign) return make();
+    const c10::impl::VirtualGuardImpl impl(c10::DeviceType::CUDA);
+    struct Restore {
+      const c10::impl::VirtualGuardImpl& impl;
+      c10::Stream                        previous;
+      ~Restore() { impl.exchangeStream(previous); }
+    } restore{impl, impl.exchangeStream(stream)};
+    return make();
+  }
+  at::Tensor empty(at::IntArrayRef sizes, at::ScalarType type, const at::Device& device) const
+  {
+    return allocate([&] { return at::empty(sizes, at::TensorOptions().dtype(type).device(device)); });
+  }
+  // A tensor that goes back to the caller, who goes on with it on the current stream.
+  const at::Tensor& returned(const at::Tensor& t) const
+  {
+    if (foreign) t.record_stream(current);
+    return t;
+  }
+};
+// None: torch's current stream; a torch stream: its handle; anything else: the handle as an integer.
+Launch launch(PyObject* o)
+{
+  const c10::impl::VirtualGuardImpl impl(c10::DeviceType::CUDA);
+  const c10::Device                 device = impl.getDevice();
+  const Owned                       index(PyLong_FromLong(device.index())), raw(PyObject_CallOneArg(current_raw_stream, index.o));
+  Launch                            on{as_pointer(raw.o)};
+  if (o == Py_None) return on;
+  PyObject* attribute = PyLong_Check(o) ? nullptr : PyObject_GetAttrString(o, "cuda_stream");
+  if (!attribute) PyErr_Clear();
+  const bool named  = attribute != nullptr;
+  PyObject*  number = PyNumber_Long(named ? attribute : o);
+  Py_XDECREF(attribute);
+  const Owned handle(number);
+  void* const p = as_pointer(handle.o);
+  if (p == on.handle) return on;
+  on.handle  = p;
+  on.foreign = true;
+  on.current = impl.getStream(device);
+  if (named)
+    on.stream = c10::Stream::unpack3(int_attribute(o, "stream_id"), (c10::DeviceIndex)int_attribute(o, "device_index"), c10::DeviceType::CUDA);
+  else if ((uintptr_t)p > 1) {
+    const Owned s(PyObject_CallOneArg(external_stream, handle.o));
+    on.stream = c10::Stream::unpack3(int_attribute(s.o, "stream_id"), (c10::DeviceIndex)int_attribute(s.o, "device_index"), c10::DeviceType::CUDA);
+  }
+  else  // 0 and 1 (the legacy handle): the device's default stream
+    on.stream = c10::Stream(c10::Stream::DEFAULT, device);
+  return on;
+}
+
 int64_t blocks(int64_t n) { return (n + 127) / 128; }
 int64_t whole_blocks(int64_t n) { return n % 128 == 0 ? n / 128 : 0; }
 
@@ -191,19 +247,25 @@ struct Workspace {
   void*      p = nullptr;
   size_t     n = 0;
 };
-// The caller's workspace, or (`own` >= 0) one of that many bytes, at least 16.
-Workspace workspace(PyObject* o, int64_t own, const at::Device& device)
+// The caller's workspace, if there is one.
+Workspace workspace(PyObject* o)
 {
   Workspace w;
-  if (o != Py_None) {
-    if (!THPVariable_Check(o)) refuse(PyExc_TypeError, "workspace must be a tensor");
-    const at::Tensor& t = THPVariable_Unpack(o);
-    w.p = t.data_ptr(), w.n = (size_t)t.numel() * t.element_size();
-  }
-  else if (own >= 0) {
-    w.own = empty({own > 16 ? own : 16}, at::kByte, device);
-    w.p = w.own.data_ptr(), w.n = (size_t)w.own.numel();
-  }
+  if (o == Py_None) return w;
+  if (!THPVariable_Check(o)) refuse(PyExc_TypeError, "workspace must be a tensor");
+  const at::Tensor& t = THPVariable_Unpack(o);
+  w.p = t.data_ptr(), w.n = (size_t)t.numel() * t.element_size();
+  return w;
+}
+// The caller's workspace, or one of own() bytes, at least 16.
+template <typename Bytes>
+Workspace workspace(PyObject* o, Bytes&& own, const Launch& on, const at::Device& device)
+{
+  if (o != Py_None) return workspace(o);
+  Workspace     w;
+  const int64_t n = (int64_t)own();
+  w.own = on.empty({n > 16 ? n : 16}, at::kByte, device);
+  w.p = w.own.data_ptr(), w.n = (size_t)w.own.numel();
   return w;
 }
 
@@ -222,14 +284,16 @@ PyObject* fp16_gemm(Args v)
   const bool bt = as_bool(v[3]);
   const int  N  = bt ? b0 : b1;
   if ((bt ? b1 : b0) != K || B.scalar_type() != A.scalar_type()) refuse(PyExc_ValueError, "shape or dtype mismatch between A and B");
-  at::Tensor own;
-  if (v[2] == Py_None) own = empty({M, N}, A.scalar_type(), A.device());
   const llmmm_gemm_cfg cfg = {as_int(v[4]), 0, 0, 0};
   const void *         a = ptr(v[0], "A", T_ANY, 0), *b = ptr(v[1], "B", T_ANY, 0);
-  void*                c = own.defined() ? own.data_ptr() : ptr(v[2], "C", t, (int64_t)M * N);
-  void* const          s = as_stream(v[5]);
-  call([&] { return llmmm_fp16_gemm_ex(t == T_F16 ? LLMMM_DTYPE_F16 : LLMMM_DTYPE_BF16, a, b, c, M, N, K, bt ? LLMMM_B_TRANSPOSED : LLMMM_B_ROW_MAJOR, &cfg, s); });
-  if (own.defined()) return THPVariable_Wrap(own);
+  void*                c = v[2] == Py_None ? nullptr : ptr(v[2], "C", t, (int64_t)M * N);
+  const Launch         on = launch(v[5]);
+  at::Tensor           own;
+  if (!c) own = on.empty({M, N}, A.scalar_type(), A.device()), c = own.data_ptr();
+  call([&] {
+    return llmmm_fp16_gemm_ex(t == T_F16 ? LLMMM_DTYPE_F16 : LLMMM_DTYPE_BF16, a, b, c, M, N, K, bt ? LLMMM_B_TRANSPOSED : LLMMM_B_ROW_MAJOR, &cfg, on.handle);
+  });
+  if (own.defined()) return THPVariable_Wrap(on.returned(own));
   Py_INCREF(v[2]);
   return v[2];
 }
@@ -245,8 +309,8 @@ PyObject* fp16_mm(Args v)
   const void* a = ptr(v[0], "A", T_ANY, (int64_t)M * K);
   const void* b = ptr(v[1], "B", T_ANY, (int64_t)K * N);
   void*       c = ptr(v[2], "C", T_ANY, (int64_t)M * N);
-  void* const s = as_stream(v[6]);
-  call([&] { return llmmm_fp16_gemm(t == T_F16 ? LLMMM_DTYPE_F16 : LLMMM_DTYPE_BF16, a, b, c, M, N, K, LLMMM_B_ROW_MAJOR, s); });
+  const Launch on = launch(v[6]);
+  call([&] { return llmmm_fp16_gemm(t == T_F16 ? LLMMM_DTYPE_F16 : LLMMM_DTYPE_BF16, a, b, c, M, N, K, LLMMM_B_ROW_MAJOR, on.handle); });
   Py_RETURN_NONE;
 }
 
@@ -267,8 +331,8 @@ PyObject* quantize_into(Args v)
   const float* x = (const float*)ptr(v[0], "x", T_F32, (int64_t)M * N);
   void*        q = ptr(v[1], "q", T_FP8, (int64_t)M * N);
   float*       c = (float*)ptr(v[2], "scale", T_F32, scale_count(kind, M, N));
-  void* const  s = as_stream(v[6]);
-  call([&] { return llmmm_quant_fp8(kind, x, q, c, M, N, s); });
+  const Launch on = launch(v[6]);
+  call([&] { return llmmm_quant_fp8(kind, x, q, c, M, N, on.handle); });
   Py_RETURN_NONE;
 }
 
@@ -279,12 +343,13 @@ PyObject* quantize(Args v)
   const int         kind = as_int(v[1]);
   int               M, N;
   shape2(X, "x", M, N);
-  const at::Tensor q = empty({M, N}, at::kByte, X.device());
-  const at::Tensor c = kind == LLMMM_QUANT_1x128_T ? empty({blocks(N), M}, at::kFloat, X.device()) : empty({blocks(M), blocks(N)}, at::kFloat, X.device());
-  const float*     x = (const float*)ptr(v[0], "x", T_F32, (int64_t)M * N);
-  void* const      s = as_stream(v[2]);
-  call([&] { return llmmm_quant_fp8(kind, x, q.data_ptr(), (float*)c.data_ptr(), M, N, s); });
-  return tuple2(q, c);
+  const float*     x  = (const float*)ptr(v[0], "x", T_F32, (int64_t)M * N);
+  const Launch     on = launch(v[2]);
+  const at::Tensor q  = on.empty({M, N}, at::kByte, X.device());
+  const at::Tensor c =
+      kind == LLMMM_QUANT_1x128_T ? on.empty({blocks(N), M}, at::kFloat, X.device()) : on.empty({blocks(M), blocks(N)}, at::kFloat, X.device());
+  call([&] { return llmmm_quant_fp8(kind, x, q.data_ptr(), (float*)c.data_ptr(), M, N, on.handle); });
+  return tuple2(on.returned(q), on.returned(c));
 }
 
 // (x, weight, eps, stream) -> (codes, scales)
@@ -294,13 +359,13 @@ PyObject* rmsnorm_quantize(Args v)
   int               M, K;
   shape2(X, "x", M, K);
   const int        code = hidden_dtype(X);
-  const at::Tensor q = empty({M, K}, at::kByte, X.device()), c = empty({blocks(K), M}, at::kFloat, X.device());
-  const void*      x = ptr(v[0], "x", T_ANY, 0);
-  const float*     w = (const float*)ptr(v[1], "weight", T_F32, K);
-  const float      eps = as_float(v[2]);
-  void* const      s   = as_stream(v[3]);
-  call([&] { return llmmm_rmsnorm_quant_fp8(code, x, w, eps, q.data_ptr(), (float*)c.data_ptr(), M, K, s); });
-  return tuple2(q, c);
+  const void*      x    = ptr(v[0], "x", T_ANY, 0);
+  const float*     w    = (const float*)ptr(v[1], "weight", T_F32, K);
+  const float      eps  = as_float(v[2]);
+  const Launch     on   = launch(v[3]);
+  const at::Tensor q = on.empty({M, K}, at::kByte, X.device()), c = on.empty({blocks(K), M}, at::kFloat, X.device());
+  call([&] { return llmmm_rmsnorm_quant_fp8(code, x, w, eps, q.data_ptr(), (float*)c.data_ptr(), M, K, on.handle); });
+  return tuple2(on.returned(q), on.returned(c));
 }
 
 // (out_kind, A, As, Bt, Bs, C, Cs, M, N, K, workspace, tile, split_k, b_preshuffled, a_layout, stream)
@@ -315,10 +380,10 @@ PyObject* fp8_gemm(Args v)
   const float*   bs    = (const float*)ptr(v[4], "B_scale_transposed", T_F32, blocks(N) * whole_blocks(K));
   void*          c     = ptr(v[5], "C", types, M * n_out);
   float*         cs    = fp8 ? (float*)ptr(v[6], "C_scale_transposed", T_F32, blocks(n_out) * M) : nullptr;
-  const Workspace      w   = workspace(v[10], -1, at::Device(at::kCPU));
+  const Workspace      w   = workspace(v[10]);
   const llmmm_gemm_cfg cfg = {as_int(v[11]), as_int(v[12]), as_bool(v[13]) ? LLMMM_FP8_B_PRESHUFFLED : LLMMM_FP8_B_ROWS, layout};
-  void* const          s   = as_stream(v[15]);
-  call([&] { return llmmm_fp8_gemm_ex(kind, a.a, a.as, b, bs, c, cs, M, N, K, w.p, w.n, &cfg, s); });
+  const Launch         on  = launch(v[15]);
+  call([&] { return llmmm_fp8_gemm_ex(kind, a.a, a.as, b, bs, c, cs, M, N, K, w.p, w.n, &cfg, on.handle); });
   Py_RETURN_NONE;
 }
 
@@ -329,9 +394,6 @@ PyObject* fp8_gemm_add_rmsnorm_quant(Args v)
   const int         code = hidden_dtype(R);
   if (H.scalar_type() != R.scalar_type()) not_supported();
   const int        M = as_int(v[8]), N = as_int(v[9]), K = as_int(v[10]), layout = as_int(v[15]);
-  const Workspace  w = workspace(
-      v[11], v[11] == Py_None ? (int64_t)(llmmm_fp8_gemm_add_rmsnorm_quant_workspace(M, N, K) + a_workspace_bytes(layout, M, N, K)) : -1, R.device());
-  const at::Tensor q = empty({M, N}, at::kByte, R.device()), c = empty({blocks(N), M}, at::kFloat, R.device());
   const AOperand   a  = a_operand(v[0], v[1], layout, M, K);
   const void*      b  = ptr(v[2], "B_transposed", T_FP8, (int64_t)N * K);
   const float*     bs = (const float*)ptr(v[3], "B_scale_transposed", T_F32, blocks(N) * whole_blocks(K));
@@ -340,11 +402,14 @@ PyObject* fp8_gemm_add_rmsnorm_quant(Args v)
   const float*     nw = (const float*)ptr(v[6], "norm_weight", T_F32, N);
   const float      eps = as_float(v[7]);
   const llmmm_gemm_cfg cfg = {as_int(v[12]), as_int(v[13]), as_bool(v[14]) ? LLMMM_FP8_B_PRESHUFFLED : LLMMM_FP8_B_ROWS, layout};
-  void* const          s   = as_stream(v[16]);
+  const Launch         on  = launch(v[16]);
+  const Workspace  w = workspace(
+      v[11], [&] { return llmmm_fp8_gemm_add_rmsnorm_quant_workspace(M, N, K) + a_workspace_bytes(layout, M, N, K); }, on, R.device());
+  const at::Tensor q = on.empty({M, N}, at::kByte, R.device()), c = on.empty({blocks(N), M}, at::kFloat, R.device());
   call([&] {
-    return llmmm_fp8_gemm_add_rmsnorm_quant(a.a, a.as, b, bs, code, r, h, nw, eps, q.data_ptr(), (float*)c.data_ptr(), M, N, K, w.p, w.n, &cfg, s);
+    return llmmm_fp8_gemm_add_rmsnorm_quant(a.a, a.as, b, bs, code, r, h, nw, eps, q.data_ptr(), (float*)c.data_ptr(), M, N, K, w.p, w.n, &cfg, on.handle);
   });
-  return tuple2(q, c);
+  return tuple2(on.returned(q), on.returned(c));
 }
 
 // (A, As, Bt, Bs, q_norm, k_norm, eps, cos, sin, positions, n_q, n_kv, M, N, K, out_fp8, workspace, tile, split_k, b_preshuffled, a_layout, stream)
@@ -354,11 +419,6 @@ PyObject* fp8_gemm_qkv_rope(Args v)
   const at::Tensor &B = tensor(v[2], "B_transposed"), &T = tensor(v[7], "cos_table");
   const int         n_q = as_int(v[10]), n_kv = as_int(v[11]), M = as_int(v[12]), N = as_int(v[13]), K = as_int(v[14]), layout = as_int(v[20]);
   const bool        fp8 = as_bool(v[15]);
-  const Workspace   w = workspace(
-      v[16], v[16] == Py_None ? (int64_t)(llmmm_fp8_gemm_qkv_rope_workspace(M, N, K) + a_workspace_bytes(layout, M, N, K)) : -1, B.device());
-  const at::Tensor out = empty({M, N}, fp8 ? at::kByte : at::kBFloat16, B.device());
-  at::Tensor       sc;
-  if (fp8) sc = empty({blocks(N), M}, at::kFloat, B.device());
   if (T.dim() < 1 || T.size(0) > INT_MAX) refuse(PyExc_ValueError, "cos_table must have rows");
   const int      rows = (int)T.size(0);
   const AOperand a    = a_operand(v[0], v[1], layout, M, K);
@@ -371,12 +431,17 @@ PyObject* fp8_gemm_qkv_rope(Args v)
   const float*   st   = (const float*)ptr(v[8], "sin_table", T_F32, (int64_t)rows * 64);
   const int*     pos  = (const int*)ptr(v[9], "positions", T_I32, M);
   const llmmm_gemm_cfg cfg = {as_int(v[17]), as_int(v[18]), as_bool(v[19]) ? LLMMM_FP8_B_PRESHUFFLED : LLMMM_FP8_B_ROWS, layout};
-  void* const          s   = as_stream(v[21]);
+  const Launch         on  = launch(v[21]);
+  const Workspace  w   = workspace(
+      v[16], [&] { return llmmm_fp8_gemm_qkv_rope_workspace(M, N, K) + a_workspace_bytes(layout, M, N, K); }, on, B.device());
+  const at::Tensor out = on.empty({M, N}, fp8 ? at::kByte : at::kBFloat16, B.device());
+  at::Tensor       sc;
+  if (fp8) sc = on.empty({blocks(N), M}, at::kFloat, B.device());
   call([&] {
     return llmmm_fp8_gemm_qkv_rope(fp8 ? LLMMM_OUT_FP8Q : LLMMM_OUT_BF16, a.a, a.as, b, bs, out.data_ptr(), fp8 ? (float*)sc.data_ptr() : nullptr, qn, kn, eps, ct, st,
-                                   rows, pos, n_q, n_kv, M, N, K, w.p, w.n, &cfg, s);
+                                   rows, pos, n_q, n_kv, M, N, K, w.p, w.n, &cfg, on.handle);
   });
-  return fp8 ? tuple2(out, sc) : THPVariable_Wrap(out);
+  return fp8 ? tuple2(on.returned(out), on.returned(sc)) : THPVariable_Wrap(on.returned(out));
 }
 
 // (codes, stream) -> the pre-shuffled image, a new tensor of the same shape and type
@@ -385,11 +450,11 @@ PyObject* preshuffle(Args v)
   const at::Tensor& Q = tensor(v[0], "src_transposed");
   int               N, K;
   shape2(Q, "src_transposed", N, K);
-  const at::Tensor out = at::empty_like(Q);
   const void*      q   = ptr(v[0], "src_transposed", T_FP8, (int64_t)N * K);
-  void* const      s   = as_stream(v[1]);
-  call([&] { return llmmm_fp8_preshuffle_b(q, out.data_ptr(), N, K, s); });
-  return THPVariable_Wrap(out);
+  const Launch     on  = launch(v[1]);
+  const at::Tensor out = on.allocate([&] { return at::empty_like(Q); });
+  call([&] { return llmmm_fp8_preshuffle_b(q, out.data_ptr(), N, K, on.handle); });
+  return THPVariable_Wrap(on.returned(out));
 }
 
 template <PyObject* (*F)(Args), Py_ssize_t COUNT>
@@ -424,5 +489,8 @@ PyMODINIT_FUNC PyInit__native(void)
   PyObject* torch_c  = PyImport_ImportModule("torch._C");
   current_raw_stream = torch_c ? PyObject_GetAttrString(torch_c, "_cuda_getCurrentRawStream") : nullptr;
   Py_XDECREF(torch_c);
-  return current_raw_stream ? PyModule_Create(&module) : nullptr;
+  PyObject* cuda  = current_raw_stream ? PyImport_ImportModule("torch.cuda") : nullptr;
+  external_stream = cuda ? PyObject_GetAttrString(cuda, "ExternalStream") : nullptr;
+  Py_XDECREF(cuda);
+  return external_stream ? PyModule_Create(&module) : nullptr;
 }

@@ -5,7 +5,12 @@ Same names, argument order and error behaviour as the reference's C++ functions
 :547-549, :2467-2476), taking torch CUDA tensors where the reference takes raw device pointers.
 Everything goes through the C ABI of ``libllmmm.so``; torch only owns the memory and the stream.  The calls of a
 model's step check and marshal their arguments in ``_native.so`` (csrc/binding.cpp), the others through ctypes here.
+
+``stream``: None (torch's current stream), a torch stream or a raw handle.  What a call allocates itself -- private workspaces, returned
+tensors -- is allocated on that stream, and returned tensors are recorded on the current one; the caller orders the two streams where
+inputs or results cross them.
 """
+import contextlib
 import ctypes
 
 import torch
@@ -22,6 +27,18 @@ def _stream(stream):
     if isinstance(stream, torch.cuda.Stream):
         return ctypes.c_void_p(stream.cuda_stream)
     return ctypes.c_void_p(int(stream))
+
+
+def _launch_stream(stream):
+    """A stream argument as the torch stream to allocate on: None (nothing to do) where it is the current stream."""
+    if stream is None:
+        return None
+    handle = _stream(stream).value or 0
+    if handle == torch.cuda.current_stream().cuda_stream:
+        return None
+    if isinstance(stream, torch.cuda.Stream):
+        return stream
+    return torch.cuda.ExternalStream(handle) if handle > 1 else torch.cuda.default_stream()  # 1: the legacy handle
 
 
 def _ptr(t, what, dtypes=None, numel=None):
@@ -204,12 +221,16 @@ def fp8_gemm_planes(A, A_scale_transposed, B_transposed, B_scale_transposed, M, 
                     split_k=0, b_preshuffled=False, a_swiglu=False):
     """A projection that stops at its fp32 partial sums: returns (planes float32 [>= splits, M, N], splits).  Feed them to the next
     projection as a :class:`PlanesRmsnorm` (residual add, RMSNorm and quantisation then happen in that projection's kernel)."""
-    if planes is None:
-        planes = torch.empty(max(int(lib.llmmm_fp8_gemm_planes_bytes(M, N, K)) // 4, max(split_k, 1) * M * N), dtype=torch.float32,
-                             device=B_transposed.device)
     kb = K // 128 if K % 128 == 0 else 0
-    if workspace is None and _a_workspace_bytes(A, M, N, K, a_swiglu):
-        workspace = torch.empty(_a_workspace_bytes(A, M, N, K, a_swiglu), dtype=torch.uint8, device=B_transposed.device)
+    own_planes, launch = planes is None, _launch_stream(stream)
+    with contextlib.nullcontext() if launch is None else torch.cuda.stream(launch):  # the call's own tensors belong to the stream it runs on
+        if own_planes:
+            planes = torch.empty(max(int(lib.llmmm_fp8_gemm_planes_bytes(M, N, K)) // 4, max(split_k, 1) * M * N), dtype=torch.float32,
+                                 device=B_transposed.device)
+        if workspace is None and _a_workspace_bytes(A, M, N, K, a_swiglu):
+            workspace = torch.empty(_a_workspace_bytes(A, M, N, K, a_swiglu), dtype=torch.uint8, device=B_transposed.device)
+    if own_planes and launch is not None:
+        planes.record_stream(torch.cuda.current_stream())
     a_p, as_p, a_layout, _keep = _a_operand(A, A_scale_transposed, M, K, a_swiglu)
     cfg = GemmCfg(tile, split_k, _lib.FP8_B_PRESHUFFLED if b_preshuffled else _lib.FP8_B_ROWS, a_layout)
     splits = ctypes.c_int(0)

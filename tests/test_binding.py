@@ -78,3 +78,80 @@ def test_streams_and_code_types():
     for c, cs in results[1:]:
         assert torch.equal(c, results[0][0]) and torch.equal(cs, results[0][1])
     assert results[0][0].any()
+
+
+def _blocks(stream):
+    """(bytes allocated, states of the blocks) of torch's allocator on one stream."""
+    segments = [s for s in torch.cuda.memory_snapshot() if s["stream"] == stream]
+    return sum(s["allocated_size"] for s in segments), [b["state"] for s in segments for b in s["blocks"]]
+
+
+def _allocating_calls():
+    """name -> call(stream) of every entry point that allocates a workspace or an output itself, on inputs that exist already."""
+    M, N, K = 16, 2048, 4096
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x, wt = torch.randn((M, K), generator=g, device="cuda"), torch.randn((N, K), generator=g, device="cuda") * 0.02
+    (a, as_), (b, bs) = llmmm_amd.quantize_activation(x), llmmm_amd.quantize_weight(wt)
+    residual, w, wk = torch.randn((M, N), generator=g, device="cuda").bfloat16(), torch.ones(N, device="cuda"), torch.ones(K, device="cuda")
+    hidden = torch.empty_like(residual)
+    tab, pos = torch.randn((M, 64), generator=g, device="cuda"), torch.arange(M, dtype=torch.int32, device="cuda")
+    half, halfw = x[:1].expand(128, K).half().contiguous(), wt.half()
+    streaming = llmmm_amd._lib.TILE_SKINNY
+    return {
+        "add_rmsnorm_quant": lambda s: llmmm_amd.fp8_gemm_add_rmsnorm_quant(a, as_, b, bs, residual, hidden, w, 1e-6, M, N, K, tile=streaming, split_k=8, stream=s),
+        "qkv_rope": lambda s: (llmmm_amd.fp8_gemm_qkv_rope(a, as_, b, bs, None, None, 1e-6, tab, tab, pos, 8, 4, M, N, K, tile=streaming, split_k=8, stream=s),),
+        "qkv_rope_fp8": lambda s: llmmm_amd.fp8_gemm_qkv_rope(a, as_, b, bs, None, None, 1e-6, tab, tab, pos, 8, 4, M, N, K, out_fp8=True, stream=s),
+        "planes": lambda s: (llmmm_amd.fp8_gemm_planes(a, as_, b, bs, M, N, K, tile=streaming, split_k=4, stream=s)[0],),
+        "quantize_activation": lambda s: llmmm_amd.quantize_activation(x, s),
+        "quantize_weight": lambda s: llmmm_amd.quantize_weight(wt, s),
+        "rmsnorm": lambda s: llmmm_amd.rmsnorm_quantize_activation(x, wk, 1e-6, s),
+        "preshuffle": lambda s: (llmmm_amd.preshuffle_weight(b, s),),
+        "fp16_gemm": lambda s: (llmmm_amd.fp16_gemm(half, halfw, b_transposed=True, stream=s),),
+    }
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["stream", "handle", "external", "default"])
+def test_a_call_allocates_on_the_stream_it_runs_on(form):
+    """Private workspaces and returned tensors come from the launch stream's blocks -- from the current stream's they could be handed
+    on while the call still runs -- and a returned tensor dropped while the current stream still works is not given out again before."""
+    side, here = torch.cuda.Stream(), torch.cuda.Stream()
+    if form == "default":  # from a side stream onto the default one, named by its handle
+        side = torch.cuda.default_stream()
+    stream = {"stream": side, "handle": side.cuda_stream, "external": torch.cuda.ExternalStream(side.cuda_stream) if side.cuda_stream else side, "default": 0}[form]
+    calls = _allocating_calls()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(here):
+        for name, call in calls.items():
+            torch.cuda.synchronize()
+            torch.cuda.empty_cache()
+            before, before_here = _blocks(side.cuda_stream)[0], _blocks(here.cuda_stream)[0]
+            out = call(stream)
+            torch.cuda.synchronize()
+            assert torch.cuda.current_stream() == here, name
+            assert _blocks(here.cuda_stream)[0] == before_here, "%s took memory of the current stream" % name
+            size = sum(-(-t.numel() * t.element_size() // 512) * 512 for t in out)
+            assert _blocks(side.cuda_stream)[0] - before >= size, "%s: outputs are not the launch stream's" % name
+            torch.cuda._sleep(20_000_000)  # about 10 ms of work on the current stream that may still read the outputs
+            del out
+            assert "active_pending_free" in _blocks(side.cuda_stream)[1], "%s: an output is free before the current stream is done" % name
+
+
+@pytest.mark.gpu
+def test_results_on_another_stream_while_the_current_one_reuses_its_memory():
+    """The same bits as on the current stream, with the side stream busy at the call and every freed block of the current stream
+    overwritten as soon as the call has returned."""
+    calls = _allocating_calls()
+    expect = {name: [t.clone() for t in call(None)] for name, call in calls.items()}
+    side = torch.cuda.Stream()
+    for name, call in calls.items():
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(2_000_000)
+        out = call(side)
+        for n in (1 << 12, 1 << 17, 1 << 20, 1 << 22):
+            torch.empty(n, dtype=torch.uint8, device="cuda").fill_(0x7f)
+        torch.cuda.current_stream().wait_stream(side)
+        n = 4 * 16 * 2048 if name == "planes" else None  # (rows beyond the splits are not written)
+        for t, e in zip(out, expect[name]):
+            assert torch.equal(t.view(torch.uint8).flatten()[:n and 4 * n], e.view(torch.uint8).flatten()[:n and 4 * n]), name
