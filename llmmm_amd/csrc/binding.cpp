@@ -37,6 +37,15 @@ unsigned type_bit(const at::Tensor& t)
 
 struct Refused {};  // a Python exception has been set
 
+// Without the interpreter lock, as torch.empty and ctypes go about it: other Python threads run while the allocator has to go to
+// the device, and while a launch waits for a full hardware queue.
+struct Unlocked {
+  PyThreadState* const state = PyEval_SaveThread();
+  Unlocked() = default;
+  Unlocked(const Unlocked&) = delete;
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 [[noreturn]] void refuse(PyObject* type, const char* fmt, ...)
 {
   va_list ap;
@@ -122,6 +131,7 @@ struct Launch {
   template <typename Make>
   at::Tensor allocate(Make&& make) const
   {
+    const Unlocked unlocked;
     if (!foreign) return make();
     const c10::impl::VirtualGuardImpl impl(c10::DeviceType::CUDA);
     struct Restore {
@@ -184,15 +194,15 @@ PyObject* tuple2(const at::Tensor& a, const at::Tensor& b)
   return r;
 }
 
-// The call itself, without the interpreter lock (a full hardware queue makes a launch wait).  The text of a failure is the calling
-// thread's, so it is fetched before anything else runs.
+// The call itself.  The text of a failure is the calling thread's, so it is fetched before anything else runs on this thread.
 template <typename F>
 void call(F&& f)
 {
   int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = f();
-  Py_END_ALLOW_THREADS
+  {
+    const Unlocked unlocked;
+    rc = f();
+  }
   if (rc == LLMMM_OK) return;
   const char *text = llmmm_error_string(rc), *detail = llmmm_last_error();
   if (rc == LLMMM_ERR_NOT_ALIGNED || rc == LLMMM_ERR_UNSUPPORTED_TYPE)

@@ -1,4 +1,7 @@
 """The native side of the Python entry points (llmmm_amd/csrc/binding.cpp): what it refuses, how, and the streams it takes."""
+import ctypes
+import subprocess
+
 import pytest
 import torch
 
@@ -155,3 +158,40 @@ def test_results_on_another_stream_while_the_current_one_reuses_its_memory():
         n = 4 * 16 * 2048 if name == "planes" else None  # (rows beyond the splits are not written)
         for t, e in zip(out, expect[name]):
             assert torch.equal(t.view(torch.uint8).flatten()[:n and 4 * n], e.view(torch.uint8).flatten()[:n and 4 * n]), name
+
+
+GIL_PROBE = r"""
+#include <dlfcn.h>
+#include <stddef.h>
+int calls, held;  /* allocations, and those made with the interpreter lock held */
+static void* hip(const char* name) { return dlsym(dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_NOLOAD), name); }
+void* probe_alloc(size_t n, int device, void* stream)
+{
+  void* p = NULL;
+  ++calls;
+  held += ((int (*)(void))dlsym(RTLD_DEFAULT, "PyGILState_Check"))();
+  return ((int (*)(void**, size_t))hip("hipMalloc"))(&p, n) == 0 ? p : NULL;
+}
+void probe_free(void* p, size_t n, int device, void* stream) { ((int (*)(void*))hip("hipFree"))(p); }
+"""
+
+
+@pytest.mark.gpu
+def test_the_interpreter_lock_is_free_while_memory_is_allocated(tmp_path):
+    """An allocation that has to go to the device (here through an allocator of the test's own) does not hold up other Python threads."""
+    src, so = tmp_path / "gil_probe.c", str(tmp_path / "gil_probe.so")
+    src.write_text("#define _GNU_SOURCE\n" + GIL_PROBE)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", so, str(src), "-ldl"], check=True)
+    probe = ctypes.CDLL(so)
+    calls, held = ctypes.c_int.in_dll(probe, "calls"), ctypes.c_int.in_dll(probe, "held")
+    allocator = torch.cuda.memory.CUDAPluggableAllocator(so, "probe_alloc", "probe_free")
+    keep = test_the_interpreter_lock_is_free_while_memory_is_allocated.keep = [probe, allocator]  # (pools in use are not freed before the process ends)
+    for name, call in _allocating_calls().items():
+        torch.cuda.synchronize()
+        before, pool = calls.value, torch.cuda.MemPool(allocator.allocator())
+        with torch.cuda.use_mem_pool(pool):
+            out = call(None)
+        torch.cuda.synchronize()
+        assert calls.value > before, name
+        assert held.value == 0, "%s allocates with the interpreter lock held" % name
+        keep += [pool, out]
