@@ -288,9 +288,11 @@ PyObject* fp16_gemm(Args v)
   const at::Tensor &A = tensor(v[0], "A"), &B = tensor(v[1], "B");
   const unsigned    t = type_bit(A);
   if (t != T_F16 && t != T_BF16) not_supported();
-  int M, K, b0, b1;
+  int M, K;
   shape2(A, "A", M, K);
-  shape2(B, "B", b0, b1);
+  if (B.dim() < 2) refuse(PyExc_IndexError, "B must have two dimensions");  // (more are taken: the first two are its shape)
+  if (B.size(0) > INT_MAX || B.size(1) > INT_MAX) refuse(PyExc_OverflowError, "B is too large");
+  const int  b0 = (int)B.size(0), b1 = (int)B.size(1);
   const bool bt = as_bool(v[3]);
   const int  N  = bt ? b0 : b1;
   if ((bt ? b1 : b0) != K || B.scalar_type() != A.scalar_type()) refuse(PyExc_ValueError, "shape or dtype mismatch between A and B");
@@ -429,7 +431,8 @@ PyObject* fp8_gemm_qkv_rope(Args v)
   const at::Tensor &B = tensor(v[2], "B_transposed"), &T = tensor(v[7], "cos_table");
   const int         n_q = as_int(v[10]), n_kv = as_int(v[11]), M = as_int(v[12]), N = as_int(v[13]), K = as_int(v[14]), layout = as_int(v[20]);
   const bool        fp8 = as_bool(v[15]);
-  if (T.dim() < 1 || T.size(0) > INT_MAX) refuse(PyExc_ValueError, "cos_table must have rows");
+  if (T.dim() < 1) refuse(PyExc_IndexError, "cos_table must have rows");
+  if (T.size(0) > INT_MAX) refuse(PyExc_OverflowError, "cos_table is too large");
   const int      rows = (int)T.size(0);
   const AOperand a    = a_operand(v[0], v[1], layout, M, K);
   const void*    b    = ptr(v[2], "B_transposed", T_FP8, (int64_t)N * K);

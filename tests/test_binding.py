@@ -38,6 +38,26 @@ def test_host_tensors_are_refused_everywhere():
             llmmm_amd.quantize_activation(bad)
 
 
+def test_shapes_the_fp16_product_refuses():
+    half = torch.zeros((256, 256), dtype=torch.float16)
+    with pytest.raises(ValueError, match="two dimensions"):
+        llmmm_amd.fp16_gemm(half[None], half)
+    with pytest.raises(IndexError):
+        llmmm_amd.fp16_gemm(half, half[0])
+    with pytest.raises(ValueError, match="shape or dtype mismatch"):
+        llmmm_amd.fp16_gemm(half, half[:128])
+    with pytest.raises(TypeError, match="must be a CUDA tensor"):  # trailing dimensions of B are no reason
+        llmmm_amd.fp16_gemm(half, half[:, :, None])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bt", [False, True])
+def test_trailing_dimensions_of_b(bt):
+    g = torch.Generator(device="cuda").manual_seed(8)
+    a, b = (torch.randn(s, generator=g, device="cuda").half() for s in ((128, 256), (256, 256)))
+    assert torch.equal(llmmm_amd.fp16_gemm(a, b[:, :, None], b_transposed=bt), llmmm_amd.fp16_gemm(a, b, b_transposed=bt))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,make,error,match", [
     ("A", lambda t: t[:, :K // 2], ValueError, "A must be contiguous"),
