@@ -1,7 +1,7 @@
-"""Builds ``libllmmm.so`` (HIP kernels + C ABI) for gfx950 with hipcc and ``_native.so`` (the Python entry points' host work), in-tree.
+"""Builds ``libllmmm.so`` (HIP kernels + C ABI) for gfx950 with hipcc and ``_native.so`` (the Python entry points' host work) with g++, in-tree.
 
-``python llmmm_amd/build.py`` (run as a script: importing the package needs the libraries this
-builds).  hipcc cross-compiles without a GPU; the resulting libraries sit next to this file so
+``python llmmm_amd/build.py [--library]`` (run as a script: importing the package needs the libraries this
+builds; ``--library``: ``libllmmm.so`` alone, without torch and g++).  hipcc cross-compiles without a GPU; the resulting libraries sit next to this file so
 that they travel with the source tree.
 """
 import os
@@ -62,11 +62,18 @@ def _compile_binding():
 
 
 def build(verbose=False):
+    """Both libraries.  ``libllmmm.so`` needs hipcc only and is linked whether or not the Python side (g++, torch's headers) can be built."""
     os.makedirs(OBJ, exist_ok=True)
     with ThreadPoolExecutor(max_workers=5) as pool:
         binding = pool.submit(_compile_binding)
-        results = list(pool.map(_compile, SOURCES.items()))
-        binding = binding.result()
+        build_library(pool, verbose)
+        _link_binding(binding.result())
+    return LIB
+
+
+def build_library(pool, verbose=False):
+    """``libllmmm.so``: all that a user of the C ABI or the C++ shims needs."""
+    results = list(pool.map(_compile, SOURCES.items()))
     objs = [o for o, _ in results]
     if verbose:
         for _, out in results:
@@ -76,8 +83,6 @@ def build(verbose=False):
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + res.stdout)
-    _link_binding(binding)
-    return LIB
 
 
 def _link_binding(obj):
@@ -103,5 +108,11 @@ def build_dropin_test():
 
 
 if __name__ == "__main__":
-    print(build(verbose="-v" in sys.argv))
+    if "--library" in sys.argv:
+        os.makedirs(OBJ, exist_ok=True)
+        with ThreadPoolExecutor(max_workers=4) as library_pool:
+            build_library(library_pool, verbose="-v" in sys.argv)
+        print(LIB)
+    else:
+        print(build(verbose="-v" in sys.argv))
     print(build_dropin_test())
