@@ -6,7 +6,7 @@ of shapes on the GPU at hand and writes ``csrc/tune_table.h`` (compiled into ``l
 The reference only hints at such an interface (``tune(N, K)`` in src/mm/fp32/impl.h:20-23, a
 stub that throws).  Candidates: for M <= 128 the split-K factor of the weight-streaming kernel; for 32 < M < 128 also a
 single row of 128 x 128 tiles (a row tail) and its splits; for M % 128 == 0 the MFMA tiles (M = 128 tries both); for the
-FP16 / BF16 GEMM all five tiles.  Timing: HIP events around a HIP graph of back-to-back launches
+FP16 / BF16 GEMM every tile.  Timing: HIP events around a HIP graph of back-to-back launches
 that rotate over enough weight copies to defeat the caches -- at every M: in a model the weights of a
 projection are never in cache when its GEMM starts, and at prefill sizes the best tile for cached weights can be
 a quarter slower on cold ones (2560 x 9728 at M = 2048: 128 x 128 tiles 59.9 us cached / 84.7 cold, 256 x 128 tiles
@@ -114,7 +114,7 @@ def pick_best(results, tolerance=0.02):
 FP16_SHAPES = [(1024, 1024, 1024), (2048, 2048, 2048), (4096, 4096, 4096), (4096, 6144, 2048), (4096, 2048, 12288), (2048, 19456, 2560),
                (2048, 2560, 9728)]  # the benchmark shapes, those of test/fp16_mm_test.cc:96-103 and two Qwen3-4B prefill projections
 FP16_TILES = {_lib.TILE_256x256: (256, 256), _lib.TILE_128x256: (128, 256), _lib.TILE_256x128: (256, 128), _lib.TILE_128x128: (128, 128),
-              _lib.TILE_64x128: (64, 128)}
+              _lib.TILE_64x128: (64, 128), _lib.TILE_64x64: (64, 64)}  # every tile the FP16 / BF16 kernel has
 
 
 def tune_fp16_shape(M, N, K, iters=40, dtype=torch.float16, verbose=True):

@@ -137,3 +137,13 @@ def test_pick_best_prefers_fewer_splits_within_the_noise():
     assert tune.pick_best({(0, 1): 196.3, (0, 3): 194.3, (2, 1): 288.0}) == (0, 1)
     assert tune.pick_best({(3, 1): 85.0, (2, 1): 62.5, (1, 1): 66.5}) == (2, 1)          # a real difference is a real difference
     assert tune.pick_best({(8, 4): 6.65, (8, 5): 6.60, (8, 8): 7.4}) == (8, 4)
+
+
+def test_fp16_candidates_are_the_kernels_tiles():
+    """The tuner measures every tile the FP16 / BF16 dispatch has: a row takes precedence over the heuristic, which picks from all of them."""
+    import re
+    from llmmm_amd import _lib, tune
+    src = open(os.path.join(ROOT, "llmmm_amd", "csrc", "fp16_gemm.hip")).read()
+    names = re.findall(r"case LLMMM_TILE_(\d+x\d+):", src[src.index("static hipError_t dispatch_fp16"):])
+    assert len(names) == 6
+    assert tune.FP16_TILES == {getattr(_lib, "TILE_" + n): tuple(int(x) for x in n.split("x")) for n in names}
