@@ -622,13 +622,24 @@ def phase_accounting(kind, M=4096, N=4096, K=4096, launches=40):
     ms_plain, _ = _events_ms(plain, launches, 5, graph=True)
     ms_probe, _ = _events_ms(probe, launches, 5, graph=True)
     torch.cuda.synchronize()
-    rec = stamps.cpu().numpy().reshape(-1, 12).astype(np.float64)
+    return phase_summary(stamps.cpu().numpy(), kind, K, ms_plain, ms_probe)
+
+
+# How the two 256 x 256 kernels are built: waves per workgroup (one or two per SIMD), K per stage and the cycles a SIMD's matrix pipe needs
+# for a stage (FP8: two waves x 32 MFMAs 16x16x128 of 32 cycles; FP16: one wave x 2 x 64 MFMAs 16x16x32 of 16 cycles)
+PHASE_KERNELS = {"fp8": {"waves": 8, "stage": 128, "ideal_cycles": 2048.0}, "fp16": {"waves": 4, "stage": 64, "ideal_cycles": 2048.0}}
+
+
+def phase_summary(stamps, kind, K, ms_plain, ms_probe):
+    """The per-phase times in the stamps of one launch (eight records per workgroup; a kernel with fewer waves repeats its own)."""
+    shape = PHASE_KERNELS[kind]
+    rec = stamps.reshape(-1, 8, 12)[:, :shape["waves"]].reshape(-1, 12).astype(np.float64)
     t = rec[:, :10].reshape(-1, 5, 2)  # [wave, point, (100 MHz ticks, shader cycles)]
     real, cyc = t[:, :, 0], t[:, :, 1]
     wait_cy, load_wait_cy = rec[:, 10], rec[:, 11]
     t0 = real[:, 0].min()
     names = ["prologue (entry -> first operands in LDS)", "K loop", "epilogue (amax / convert / staging / stores issued)", "store drain (stores acknowledged)"]
-    out = {"kernel_us_uninstrumented": ms_plain * 1e3, "kernel_us_instrumented": ms_probe * 1e3, "waves": int(t.shape[0]),
+    out = {"kernel_us_uninstrumented": ms_plain * 1e3, "kernel_us_instrumented": ms_probe * 1e3, "waves": int(t.shape[0]), "waves_per_workgroup": shape["waves"],
            "first_wave_start_to_last_wave_end_us": (real[:, 4].max() - t0) / 100.0, "wave_start_spread_us": (real[:, 0].max() - t0) / 100.0, "phases": []}
     for p, name in enumerate(names):
         d_us = (real[:, p + 1] - real[:, p]) / 100.0
@@ -640,16 +651,16 @@ def phase_accounting(kind, M=4096, N=4096, K=4096, launches=40):
     out["wave_lifetime_us_median"] = float(np.median(whole_us))
     out["shader_mhz_from_stamps"] = float(np.median(whole_cy / whole_us))
     loop_cy = float(np.median(cyc[:, 2] - cyc[:, 1]))
-    slices = K // 128 if kind == "fp8" else K // 32
+    slices = K // shape["stage"]
     out["k_loop_cycles_per_stage"] = loop_cy / slices
-    # a SIMD holds two waves; per stage each issues 32 MFMAs of 32 cycles (fp8 16x16x128, a 128-K slice) or of 16 cycles (f16 16x16x32, K = 32)
     out["k_loop_wait_cycles_per_stage"] = float(np.median(wait_cy)) / slices
     out["k_loop_load_wait_cycles_per_stage"] = float(np.median(load_wait_cy)) / slices
-    # per SIMD (its two waves are records w and w + 4 of a workgroup: waves are dealt to the four SIMDs in turn): the cycles
-    # per stage in which BOTH of its waves sit in a wait cannot be read off the sums, but their minimum bounds it from above
-    w8 = wait_cy.reshape(-1, 8)
-    out["k_loop_wait_cycles_per_stage_less_waiting_wave_of_a_simd"] = float(np.median(np.minimum(w8[:, :4], w8[:, 4:]))) / slices
-    ideal = 2048.0 if kind == "fp8" else 1024.0
+    if shape["waves"] == 8:
+        # per SIMD (its two waves are records w and w + 4 of a workgroup: waves are dealt to the four SIMDs in turn): the cycles
+        # per stage in which BOTH of its waves sit in a wait cannot be read off the sums, but their minimum bounds it from above
+        w8 = wait_cy.reshape(-1, 8)
+        out["k_loop_wait_cycles_per_stage_less_waiting_wave_of_a_simd"] = float(np.median(np.minimum(w8[:, :4], w8[:, 4:]))) / slices
+    ideal = shape["ideal_cycles"]
     out["k_loop_ideal_cycles_per_stage"] = ideal
     out["k_loop_matrix_pipe_share"] = ideal / out["k_loop_cycles_per_stage"]
     return out
@@ -735,7 +746,7 @@ def main():
     if w in ("phases_fp8_4096", "phases_fp16_4096"):
         kind = "fp8" if "fp8" in w else "fp16"
         r = phase_accounting(kind)
-        print("phase accounting, %s 256 x 256 tile kernel, M = N = K = 4096 (one tile per CU, 8 waves per tile)" % ("FP8 fused-quant" if kind == "fp8" else "FP16"))
+        print("phase accounting, %s 256 x 256 tile kernel, M = N = K = 4096 (one tile per CU, %d waves per tile)" % ("FP8 fused-quant" if kind == "fp8" else "FP16", r["waves_per_workgroup"]))
         print("kernel time per launch (HIP events, graph of back-to-back launches): %.2f us; the instrumented build: %.2f us" %
               (r["kernel_us_uninstrumented"], r["kernel_us_instrumented"]))
         print("first wave's start to last wave's end: %.2f us; wave starts spread over %.2f us; median wave lifetime %.2f us; shader clock %.0f MHz" %
@@ -743,12 +754,14 @@ def main():
         print("%-62s %9s %9s %9s %9s %12s" % ("phase (per wave, %d waves)" % r["waves"], "median us", "mean us", "min us", "max us", "median cyc"))
         for p in r["phases"]:
             print("%-62s %9.2f %9.2f %9.2f %9.2f %12.0f" % (p["phase"], p["us_median"], p["us_mean"], p["us_min"], p["us_max"], p["cycles_median"]))
-        print("K loop: %.0f cycles per stage against %.0f with the matrix pipe always busy (two waves per SIMD, 32 MFMAs each per stage): %.1f %%" %
-              (r["k_loop_cycles_per_stage"], r["k_loop_ideal_cycles_per_stage"], 100 * r["k_loop_matrix_pipe_share"]))
+        print("K loop: %.0f cycles per stage of %d in K against %.0f with the matrix pipe always busy (%s): %.1f %%" %
+              (r["k_loop_cycles_per_stage"], PHASE_KERNELS[kind]["stage"], r["k_loop_ideal_cycles_per_stage"],
+               "two waves per SIMD, 32 MFMAs each" if kind == "fp8" else "one wave per SIMD, 128 MFMAs", 100 * r["k_loop_matrix_pipe_share"]))
         print("of which a wave waits %.0f cycles per stage (%.0f for its own loads to land, the rest for the other waves at the barrier);"
               % (r["k_loop_wait_cycles_per_stage"], r["k_loop_load_wait_cycles_per_stage"]))
-        print("the less-waiting wave of each SIMD's pair: %.0f cycles per stage (an upper bound on the time a SIMD has no wave to issue from)"
-              % r["k_loop_wait_cycles_per_stage_less_waiting_wave_of_a_simd"])
+        if kind == "fp8":
+            print("the less-waiting wave of each SIMD's pair: %.0f cycles per stage (an upper bound on the time a SIMD has no wave to issue from)"
+                  % r["k_loop_wait_cycles_per_stage_less_waiting_wave_of_a_simd"])
         print(json.dumps({"workload": w, **r}))
         return
     import re as _re

@@ -7,6 +7,7 @@ import math
 import os
 import re
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -67,3 +68,21 @@ def test_traffic_comes_from_a_profile_of_the_same_source(bench, tmp_path, monkey
     assert value is None and "another version" in why
     (fake / "profiles" / "fp16_gemm_kernel_4096.txt").unlink()
     assert bench.measured_traffic("fp16_gemm_4096")[0] is None
+
+
+@pytest.mark.parametrize("kind,waves,stage", [("fp8", 8, 128), ("fp16", 4, 64)])
+def test_phase_summary_counts_a_kernels_own_waves(bench, kind, waves, stage):
+    """Eight records per workgroup; the FP16 kernel has four waves, one per SIMD, and K stages of 64: a record's copy is no second wave."""
+    K, tiles, per_stage = 1024, 3, 2500
+    rec = np.zeros((tiles, 8, 12))
+    for w in range(8):
+        own = w % waves
+        cycles = [0, 1000, 1000 + per_stage * (K // stage), 50000, 51000]
+        rec[:, w, 0:10:2] = np.array([1, 2, 30, 33, 34]) + own
+        rec[:, w, 1:10:2] = np.array(cycles) + 7 * own
+        rec[:, w, 10], rec[:, w, 11] = (100 + own) * (K // stage), 10 * (K // stage)
+    r = bench.phase_summary(rec.astype(np.int64).reshape(-1), kind, K, 0.1, 0.11)
+    assert r["waves"] == tiles * waves and r["waves_per_workgroup"] == waves
+    assert r["k_loop_cycles_per_stage"] == per_stage and r["k_loop_matrix_pipe_share"] == 2048 / per_stage
+    assert r["k_loop_wait_cycles_per_stage"] == 100 + (waves - 1) / 2
+    assert ("k_loop_wait_cycles_per_stage_less_waiting_wave_of_a_simd" in r) == (kind == "fp8")
