@@ -116,13 +116,14 @@ __device__ __forceinline__ PhaseClock phase_clock()
 // (Any number of tiles: XCD x owns tiles/8 of them and one more if x < tiles%8.  Dealing the ids of a tile count that 8 does not
 // divide out in turn made every XCD read nearly all of both operands: FP8 384 x 3584 x 18944 in 84 tiles x 3 splits 45.4 us, 37.9 so;
 // FP16 1152 x 3456 x 2048 in 243 tiles of 128 x 128 22.4 us, 19.7 so.)
-__device__ __forceinline__ void tile_coords(int wg, int tiles_m, int tiles_n, int& tm, int& tn)
+// in_turn: tile ids in the hardware's order instead, in groups of four rows (see splits_in_turn in fp8_gemm.hip).
+__device__ __forceinline__ void tile_coords(int wg, int tiles_m, int tiles_n, int& tm, int& tn, bool in_turn = false)
 {
   const int tiles   = tiles_m * tiles_n;
   const int x       = wg & 7, rem = tiles & 7;
-  const int L       = x * (tiles >> 3) + (x < rem ? x : rem) + (wg >> 3);
+  const int L       = in_turn ? wg : x * (tiles >> 3) + (x < rem ? x : rem) + (wg >> 3);
   const int groups  = (tiles_m + 3) >> 2;
-  const int group_m = (tiles_m + groups - 1) / groups;
+  const int group_m = in_turn ? 4 : (tiles_m + groups - 1) / groups;
   const int per     = group_m * tiles_n;
   const int group   = L / per;
   const int first   = group * group_m;

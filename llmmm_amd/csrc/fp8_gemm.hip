@@ -393,6 +393,22 @@ constexpr int fp8_lds_bytes()
   return !deep ? 2 * TC::STAGE : (4 * stage_d <= 160 * 1024 ? 4 : 3) * stage_d;
 }
 
+// Where the tiles of a split run go out in turn instead of in contiguous runs per XCD: where the reduce kernel is a large part of
+// the call and finds the planes in its own XCD's L2 that way.  128-column tiles only: they are the reduce kernel's column groups
+// (256 columns: 6144 x 2560 at M = 256 in 4 splits 26.0 / 27.8).
+//  * One row of tiles: tiles share no weights, so contiguous runs gain nothing, and in turn tile n and the reduce kernel's group n
+//    sit on the same XCD for every split if 8 divides the tiles, for some otherwise (bf16 out, M = 128, us, contiguous / in turn:
+//    2560 x 9728 16.4 / 14.8, 2560 x 4096 12.7 / 11.5, 3072 x 8192 16.7 / 14.2, 4096 x 14336 23.4 / 20.7).
+//  * Up to 60 tiles that 8 does not divide, K <= 4096: 256 x 3456 x 4096 16.5 / 15.7, 384 x 1152 x 4096 12.6 / 12.1, 640 x 1152 x 4096
+//    14.75 / 14.1.  With a longer K or more tiles the operands' reuse wins (256 x 3456 x 8192 19.4 / 20.3, 384 x 1152 x 8192
+//    15.5 / 16.9, 384 x 3200 x 4096 17.2 / 18.5).
+template <int BN>
+__device__ __forceinline__ bool splits_in_turn(int splits, int tiles_m, int tiles_n, int K)
+{
+  const int tiles = tiles_m * tiles_n;
+  return BN == 128 && splits > 1 && (tiles_m == 1 || ((tiles & 7) != 0 && tiles <= 60 && K <= 4096));
+}
+
 // BMODE bit 0 (BPRE): Bt is the pre-shuffled image of the weights (layout.hip) instead of row-major [N, K].
 // BMODE bit 1 (BNT): the weight loads carry the non-temporal hint (one tile row: every weight byte is read once).
 // BMODE bit 2 (DEEP, 32-row-wave tiles only): the launch has at most one workgroup per CU, which then runs a deeper pipeline.
@@ -436,7 +452,7 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   const int wm   = wave % TC::WAVES_M;
   const int wn   = wave / TC::WAVES_M;
   int       tm, tn;
-  tile_coords(tile_index, tiles_m, tiles_n, tm, tn);
+  tile_coords(tile_index, tiles_m, tiles_n, tm, tn, splits_in_turn<BN>(gridDim.y, tiles_m, tiles_n, K));
   // SwiGLU output: the tile's two 128-column halves are the gate columns n0 .. n0+127 and the up columns
   // N/2 + n0 .. of the same 128 output columns, so the weight rows of the upper half start N/2 - 128 rows further on
   constexpr bool SWIGLU = OUT == OUT_SWIGLU;

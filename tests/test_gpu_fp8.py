@@ -86,6 +86,16 @@ def test_tile_kernels_split_k(lib, oracle, tile, split):
     assert all((a == b).all() for a, b in zip(out[1:], again[1:])) and (out[0].view(np.uint32) == again[0].view(np.uint32)).all()
 
 
+# both orders in which a split run deals its tiles out: one row of tiles (8 divides their number or not, more than 60), several rows on
+# both sides of 60 tiles and of K = 4096, five rows (groups of four and one / of three and two)
+@pytest.mark.parametrize("M,N,K,split", [(128, 1152, 512, 2), (128, 1024, 768, 3), (128, 8320, 256, 2), (256, 1152, 512, 2), (256, 3840, 256, 2), (384, 2560, 256, 2),
+                                         (384, 2688, 256, 2), (640, 640, 384, 3), (256, 128, 4224, 5), (384, 128, 4096, 4), (640, 1024, 256, 2)])
+def test_split_tile_orders(lib, oracle, M, N, K, split):
+    Aq, As, Bq, Bs = fp8_inputs(oracle, M, N, K, seed=11)
+    ref = oracle.fp8_gemm(Aq, As, Bq, Bs, promote=128)
+    _check_all(oracle, _run_all(lib, Aq, As, Bq, Bs, tile=TILES["128x128"], split_k=split), ref, "%d x %d x %d in %d splits" % (M, N, K, split))
+
+
 @pytest.mark.parametrize("K", [128, 256, 384, 512, 640])
 def test_short_k(lib, oracle, K):
     """1 to 5 slices through the 256x256 tile kernel: prologue-only, odd and even slice counts."""
