@@ -582,6 +582,23 @@ static __device__ unsigned   g_strip_xch_timeouts;
 
 enum { ST_OUT_F32 = 0, ST_OUT_BF16 = 1, ST_OUT_ADD = 2, ST_OUT_FP8Q = 3 };
 
+// The maximum with lane l ^ MASK around the exchange: LDS-crossbar swizzles and a selected half swap.  The register-only steps of
+// wave_xor_max are shorter and the launch gets longer with them, in either of the two places (6144 x 2560, us, this form /
+// wave_xor_max: 6.3 / 6.6 - 6.8 at M = 1, 6.3 - 6.5 / 6.7 - 7.0 at 2, 6.4 - 6.6 / 6.9 - 7.1 at 4; other shapes move by less than two
+// runs of one form differ).  What the polling fragments wait for is each other's store, not these steps.
+template <int MASK>
+__device__ __forceinline__ float exchange_max(float v)
+{
+  static_assert(MASK == 8 || MASK == 16 || MASK == 32, "the distances in use");
+  const int iv = __builtin_bit_cast(int, v);
+  if constexpr (MASK == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap((unsigned)iv, (unsigned)iv, false, false);  // r[0] = the lower half in both, r[1] = the upper
+    return fmaxf(v, __builtin_bit_cast(float, (__lane_id() < 32) ? r[1] : r[0]));
+  }
+  else
+    return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(iv, (MASK << 10) | 0x1f)));
+}
+
 // CF = 16-column fragments of a strip (1 or 2): with CF = 2 a workgroup owns 32 columns -- wave w takes fragment w % 2 and
 // the K range (w / 2) of four -- so that N / 32 workgroups cover outputs whose N / 16 strips would be more than the CUs
 // (a second round of workgroups costs more than the narrower K split: 6144 columns are 384 strips or 192 wide ones).
@@ -709,8 +726,8 @@ fp8_strip_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, co
     // width leave an area in the same state; rows beyond M take part with whatever their sums are: their maxima are
     // exchanged and never used)
     float a = fmaxf(fmaxf(fmaxf(0.f, __builtin_fabsf(v[0])), __builtin_fabsf(v[1])), fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3])));
-    a       = wave_xor_max<16>(a);
-    a       = wave_xor_max<32>(a);  // the fragment's maximum of row i, in all four lanes that hold the row
+    a       = exchange_max<16>(a);
+    a       = exchange_max<32>(a);  // the fragment's maximum of row i, in all four lanes that hold the row
     const int frag = blockIdx.x * CF + cf, grp = frag >> 3, strip = frag & 7;
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(own_mark)::"memory");  // long landed; ties the register to this point
     const int cur = own_mark != 0u ? 1 : 0;  // the buffer this fragment did not fill last time (both clean: buffer 0)
@@ -735,7 +752,7 @@ fp8_strip_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, co
       __builtin_amdgcn_s_sleep(1);
     }
     float r0 = __builtin_bit_cast(float, (unsigned)w - 1u), r1 = __builtin_bit_cast(float, (unsigned)(w >> 32) - 1u);
-    r0 = wave_xor_max<32>(wave_xor_max<16>(wave_xor_max<8>(r0))), r1 = wave_xor_max<32>(wave_xor_max<16>(wave_xor_max<8>(r1)));  // over the group's fragments
+    r0 = exchange_max<32>(exchange_max<16>(exchange_max<8>(r0))), r1 = exchange_max<32>(exchange_max<16>(exchange_max<8>(r1)));  // over the group's fragments
     const float e0 = __shfl(r0, i >> 1, 64), e1 = __shfl(r1, i >> 1, 64);
     const float amax = (i & 1) ? e1 : e0;  // the group's maximum of row i
     const float scale = amax / 448.f;
