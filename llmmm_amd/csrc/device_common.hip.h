@@ -157,12 +157,16 @@ __device__ __forceinline__ WavePair wave_swap_pair(float v)
   asm("" : "+v"(x), "+v"(y));
   return {__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
 }
-// The value lane (l ^ mask) holds, for mask = 1, 2, 4, 8, 16 or 32.  Register moves only, no trip through the LDS crossbar -- the reductions of the row kernels are chains of these,
-// eleven long, and with ds_swizzle for 4, 8 and 16 (about 60 cycles a step instead of 8) seven of the eleven waited on it:
+// The value lane (l ^ mask) holds, for mask = 1, 2, 4, 8, 16 or 32.  Register moves but for 16: the reductions of the row kernels are
+// chains of these, eleven long, and with ds_swizzle for 4, 8 and 16 (about 60 cycles a step instead of 8) seven of the eleven waited
+// on the LDS crossbar (sums and maxima over 16 take the row swap above, which yields both operands):
 //   1, 2     DPP quad permutes,
 //   4        lane l + 4 for the lanes with bit 2 clear, l - 4 for the others: two DPP row shifts with complementary bank masks,
 //   8        a DPP rotation of the 16-lane row by 8,
-//   16, 32   the row and half swaps above.
+//   16       ds_swizzle, through the LDS crossbar after all: the row swap and its selection hold two more registers per value, and
+//            in the kernel that fetches four values at once (the rotary embedding behind split-K planes) they cost the fifth wave
+//            per SIMD: 107 instead of 93 VGPRs, 10240 columns at M = 128 29.0 -> 29.9 us,
+//   32       the half swap above.
 template <int MASK>
 __device__ __forceinline__ float wave_xor_get(float v)
 {
@@ -177,6 +181,8 @@ __device__ __forceinline__ float wave_xor_get(float v)
   }
   else if constexpr (MASK == 8)
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(iv, 0x128, 0xf, 0xf, true));  // row_ror:8
+  else if constexpr (MASK == 16)
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(iv, (16 << 10) | 0x1f));
   else {
     const WavePair p = wave_swap_pair<MASK>(v);
     return (__lane_id() & MASK) ? p.a : p.b;
