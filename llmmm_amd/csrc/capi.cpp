@@ -131,31 +131,34 @@ int heuristic_tile(int M, int N)
 }
 
 // The FP16 / BF16 kernels' tile for shapes the table does not list.  A launch takes about
-//   fixed + K / 64 * (full rounds * all + (a round is left over) * one)   microseconds,
-// where a CU holds `per_cu` tiles side by side, works K = 64 of them all in `all` and of a lone one in `one`, and the busiest CU
-// gets ceil(tiles / CUs) tiles.  The constants are fitted to 56 shapes (M, N, K log-uniform in 256 .. 8192 and the benchmark's) x
-// both B layouts on the MI355X; the choice is within 1 % of the best tile on average and 15 % at worst there (the tile a
-// wave-count rule chose before cost 31 % on average with today's kernels' times, 3.4 x at worst: 64 x 64 tiles for 384 x 256 x 3648).
+//   fixed + rounds * setup + K / 64 * (full rounds * all + (a round is left over) * one)   microseconds,
+// where a CU holds `per_cu` tiles side by side, works K = 64 of them all in `all` and of a lone one in `one`, every round starts and
+// ends in `setup`, and the busiest CU gets ceil(tiles / CUs) tiles.  The constants are fitted to the measured times of every tile on
+// 1011 shapes x both B layouts on the MI355X (M, N log-uniform in 128 .. 8192, K in 16 .. 8192, 40 % of them below 512): the choice
+// is within 0.2 % of the best tile on average and 24 % at worst (256 x 384 x 6832), and a fit to two thirds of them is within 0.2 %
+// on the rest.  (Without the term in the rounds, and fitted from K = 256 up only, it took the largest tiles at short K: 17 % off on
+// average, 1408 x 256 x 160 5.7 us in 128 x 256 tiles for 3.3 in 64 x 64.)
 int heuristic_tile_fp16(int M, int N, int K)
 {
   static const struct {
     int    id, bm, bn, per_cu;
-    double fixed, one, all;
-  } cand[] = {{LLMMM_TILE_256x256, 256, 256, 1, 1.24, 1.295, 1.295}, {LLMMM_TILE_128x256, 128, 256, 1, 0.50, 0.777, 0.777},
-              {LLMMM_TILE_256x128, 256, 128, 1, 0.50, 0.797, 0.797}, {LLMMM_TILE_128x128, 128, 128, 2, 2.57, 0.526, 0.950},
-              {LLMMM_TILE_64x128, 64, 128, 2, 2.83, 0.295, 0.629},   {LLMMM_TILE_64x64, 64, 64, 2, 2.85, 0.182, 0.402}};
+    double fixed, setup, one, all;
+  } cand[] = {{LLMMM_TILE_256x256, 256, 256, 1, 0.00, 9.84, 1.048, 1.048}, {LLMMM_TILE_128x256, 128, 256, 1, 0.01, 4.21, 0.626, 0.626},
+              {LLMMM_TILE_256x128, 256, 128, 1, 0.00, 3.96, 0.665, 0.665}, {LLMMM_TILE_128x128, 128, 128, 2, 0.52, 3.04, 0.509, 0.760},
+              {LLMMM_TILE_64x128, 64, 128, 2, 0.61, 2.31, 0.286, 0.589},   {LLMMM_TILE_64x64, 64, 64, 2, 1.00, 1.67, 0.182, 0.466}};
   int    best    = -1;
   double best_us = 0.;
   for (const auto& c : cand) {
     if (M % c.bm || N % c.bn) continue;
-    const long tiles  = (long)(M / c.bm) * (N / c.bn);
-    const long per    = (tiles + NUM_CUS - 1) / NUM_CUS;  // tiles of the busiest CU
-    double     rounds = per / c.per_cu * c.all + (per % c.per_cu ? c.one : 0.);
+    const long tiles = (long)(M / c.bm) * (N / c.bn);
+    const long per   = (tiles + NUM_CUS - 1) / NUM_CUS;  // tiles of the busiest CU
+    const long full  = per / c.per_cu, left = per % c.per_cu ? 1 : 0;
+    double     round = 1.;  // of the last round, what it takes of a whole one
     if (c.id == LLMMM_TILE_256x256) {  // a partly filled last round runs in half-size tiles where launch_fp16 can arrange it
-      const long tm = M / 256, tn = N / 256, full = tiles / NUM_CUS * NUM_CUS;
-      if (tiles > NUM_CUS && tm > 1 && full % tm == 0 && tn - full / tm > 0 && (tn - full / tm) * tm * 2 <= NUM_CUS) rounds -= 0.4 * c.one;
+      const long tm = M / 256, tn = N / 256, whole = tiles / NUM_CUS * NUM_CUS;
+      if (tiles > NUM_CUS && tm > 1 && whole % tm == 0 && tn - whole / tm > 0 && (tn - whole / tm) * tm * 2 <= NUM_CUS) round = 0.6;
     }
-    const double us = c.fixed + K / 64. * rounds;
+    const double us = c.fixed + (full + left - 1 + round) * c.setup + K / 64. * ((full - 1 + round) * c.all + left * c.one);
     if (best < 0 || us < best_us) best = c.id, best_us = us;
   }
   return best;

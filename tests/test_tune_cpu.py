@@ -147,3 +147,20 @@ def test_fp16_candidates_are_the_kernels_tiles():
     names = re.findall(r"case LLMMM_TILE_(\d+x\d+):", src[src.index("static hipError_t dispatch_fp16"):])
     assert len(names) == 6
     assert tune.FP16_TILES == {getattr(_lib, "TILE_" + n): tuple(int(x) for x in n.split("x")) for n in names}
+
+
+def test_fp16_tile_rule(tmp_path):
+    """heuristic_tile_fp16 (capi.cpp) on shapes of every K range: small tiles where a short K leaves little but a tile's start and end, large
+    ones where the operands' bytes decide.  (The function alone, compiled here: the library has no query for this entry point.)"""
+    src = open(os.path.join(ROOT, "llmmm_amd", "csrc", "capi.cpp")).read()
+    at = src.index("int heuristic_tile_fp16(")
+    rule = src[at:src.index("\n}\n", at) + 3]
+    shapes = [(1408, 256, 160, "64x64"), (2048, 256, 160, "64x64"), (256, 2176, 80, "64x64"), (256, 256, 32, "64x64"), (1024, 1024, 1024, "64x64"),
+              (5504, 2048, 256, "128x128"), (7424, 1152, 240, "128x128"), (6912, 4352, 16, "128x128"), (1152, 3456, 2000, "128x128"),
+              (4096, 4096, 4096, "256x256"), (8192, 8192, 8192, "256x256"), (2048, 19456, 2560, "256x256")]
+    (tmp_path / "rule.cpp").write_text('#include "llmmm.h"\n#include <cstdio>\nconstexpr int NUM_CUS = 256;\n%sint main()\n{\n%s}\n' % (
+        rule, "".join('  std::printf("%%d\\n", heuristic_tile_fp16(%d, %d, %d));\n' % s[:3] for s in shapes)))
+    subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "include"), "-o", str(tmp_path / "rule"), str(tmp_path / "rule.cpp")], check=True)
+    got = subprocess.run([str(tmp_path / "rule")], stdout=subprocess.PIPE, check=True, text=True).stdout.split()
+    from llmmm_amd import _lib
+    assert [int(x) for x in got] == [getattr(_lib, "TILE_" + s[3]) for s in shapes]
