@@ -134,8 +134,8 @@ int heuristic_tile(int M, int N)
 //   fixed + rounds * setup + K / 64 * (full rounds * all + (a round is left over) * one)   microseconds,
 // where a CU holds `per_cu` tiles side by side, works K = 64 of them all in `all` and of a lone one in `one`, every round starts and
 // ends in `setup`, and the busiest CU gets ceil(tiles / CUs) tiles.  The constants are fitted to the measured times of every tile on
-// 1011 shapes x both B layouts on the MI355X (M, N log-uniform in 128 .. 8192, K in 16 .. 8192, 40 % of them below 512): the choice
-// is within 0.2 % of the best tile on average and 24 % at worst (256 x 384 x 6832), and a fit to two thirds of them is within 0.2 %
+// 1170 shapes x both B layouts on the MI355X (M, N log-uniform in 128 .. 8192, K in 16 .. 8192, half of them below 512): the choice
+// is within 0.2 % of the best tile on average and 24 % at worst (256 x 384 x 6832), and a fit to 70 % of them is within 0.2 %
 // on the rest.  (Without the term in the rounds, and fitted from K = 256 up only, it took the largest tiles at short K: 17 % off on
 // average, 1408 x 256 x 160 5.7 us in 128 x 256 tiles for 3.3 in 64 x 64.)
 int heuristic_tile_fp16(int M, int N, int K)
@@ -143,13 +143,15 @@ int heuristic_tile_fp16(int M, int N, int K)
   static const struct {
     int    id, bm, bn, per_cu;
     double fixed, setup, one, all;
-  } cand[] = {{LLMMM_TILE_256x256, 256, 256, 1, 0.00, 9.84, 1.048, 1.048}, {LLMMM_TILE_128x256, 128, 256, 1, 0.01, 4.21, 0.626, 0.626},
-              {LLMMM_TILE_256x128, 256, 128, 1, 0.00, 3.96, 0.665, 0.665}, {LLMMM_TILE_128x128, 128, 128, 2, 0.52, 3.04, 0.509, 0.760},
-              {LLMMM_TILE_64x128, 64, 128, 2, 0.61, 2.31, 0.286, 0.589},   {LLMMM_TILE_64x64, 64, 64, 2, 1.00, 1.67, 0.182, 0.466}};
+    int    form;  // 128 x 128: 1 = the shallow rings, 2 = the deep ones (llmmm::fp16_deep)
+  } cand[] = {{LLMMM_TILE_256x256, 256, 256, 1, 0.00, 9.14, 1.048, 1.048, 0}, {LLMMM_TILE_128x256, 128, 256, 1, 0.00, 5.14, 0.707, 0.707, 0},
+              {LLMMM_TILE_256x128, 256, 128, 1, 0.10, 4.60, 0.684, 0.684, 0}, {LLMMM_TILE_128x128, 128, 128, 2, 0.42, 3.05, 0.398, 0.999, 1},
+              {LLMMM_TILE_128x128, 128, 128, 1, 0.00, 3.92, 0.380, 0.380, 2}, {LLMMM_TILE_64x128, 64, 128, 2, 0.64, 2.28, 0.303, 0.673, 0},
+              {LLMMM_TILE_64x64, 64, 64, 2, 1.06, 1.71, 0.182, 0.397, 0}};
   int    best    = -1;
   double best_us = 0.;
   for (const auto& c : cand) {
-    if (M % c.bm || N % c.bn) continue;
+    if (M % c.bm || N % c.bn || (c.form && (c.form == 2) != llmmm::fp16_deep(M, N, K))) continue;
     const long tiles = (long)(M / c.bm) * (N / c.bn);
     const long per   = (tiles + NUM_CUS - 1) / NUM_CUS;  // tiles of the busiest CU
     const long full  = per / c.per_cu, left = per % c.per_cu ? 1 : 0;

@@ -482,6 +482,12 @@ static hipError_t launch_fp16(const void* A, const void* B, void* C, int M, int 
   return hipGetLastError();
 }
 
+// The rings of the 128 x 128 tile.  Up to one tile per CU and from K = 1024 on they take the whole LDS (1920 x 1536 x 5312, 180 tiles:
+// 38 us deep, 44 us shallow; at K = 1024 the two are even).  Beyond one tile two workgroups share a CU (3968 x 2944 x 576, 713 tiles:
+// 20.6 us shallow, 24.7 us deep), and a shorter K is over before the deep rings have paid for their start (1664 x 1408, us, shallow /
+// deep: K = 512 7.8 / 8.5, 640 8.7 / 9.3, 800 10.3 / 10.7).
+bool fp16_deep(int M, int N, int K) { return (long)(M / 128) * (N / 128) <= num_cus() && K >= 1024; }
+
 template <typename T, bool B_NK>
 static hipError_t dispatch_fp16(int tile, const void* A, const void* B, void* C, int M, int N, int K, hipStream_t stream)
 {
@@ -490,10 +496,8 @@ static hipError_t dispatch_fp16(int tile, const void* A, const void* B, void* C,
     // half tiles of eight 64 x 64 waves, two per SIMD: ahead of four 128 x 64 waves by 1-3 % (2048 x 2560 x 9728: 119 / 123 us)
     case LLMMM_TILE_128x256: return launch_fp16<T, 128, 256, 64, 64, 3, 3, B_NK>(A, B, C, M, N, K, stream);
     case LLMMM_TILE_256x128: return launch_fp16<T, 256, 128, 64, 64, 3, 3, B_NK>(A, B, C, M, N, K, stream);
-    // 128 x 128: up to one tile per CU the rings take the whole LDS (1920 x 1536 x 5312, 180 tiles: 38 us deep, 44 us shallow);
-    // beyond that two workgroups share a CU (3968 x 2944 x 576, 713 tiles: 20.6 us shallow, 24.7 us deep)
     case LLMMM_TILE_128x128:
-      return (long)(M / 128) * (N / 128) <= num_cus() ? launch_fp16<T, 128, 128, 64, 64, 5, 5, B_NK>(A, B, C, M, N, K, stream)
+      return fp16_deep(M, N, K) ? launch_fp16<T, 128, 128, 64, 64, 5, 5, B_NK>(A, B, C, M, N, K, stream)
                                                       : launch_fp16<T, 128, 128, 64, 64, 3, 2, B_NK>(A, B, C, M, N, K, stream);
     case LLMMM_TILE_64x128: return launch_fp16<T, 64, 128, 32, 64, 3, 3, B_NK>(A, B, C, M, N, K, stream);
     case LLMMM_TILE_64x64: return launch_fp16<T, 64, 64, 32, 32, 4, 4, B_NK>(A, B, C, M, N, K, stream);

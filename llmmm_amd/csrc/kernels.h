@@ -10,6 +10,7 @@
 namespace llmmm {
 
 // dtype: 0 = fp16, 1 = bf16.  b_layout: 0 = B[K,N] row-major, 1 = Bt[N,K].
+bool       fp16_deep(int M, int N, int K);  // whether the 128 x 128 FP16 / BF16 tile runs in its deep rings
 hipError_t fp16_gemm_launch(int dtype, int b_layout, int tile, const void* A, const void* B, void* C, int M, int N, int K,
                             hipStream_t stream);
 

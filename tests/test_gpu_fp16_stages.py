@@ -43,3 +43,10 @@ def test_tile_counts_that_eight_does_not_divide(lib, M, N, bt):
 def test_more_128x128_tiles_than_compute_units(lib):
     _check(lib, 2304, 2048, 80, torch.float16, False, TILES["128x128"][0])  # 288 tiles: the shallow rings, two workgroups per CU
     _check(lib, 2304, 2048, 192, torch.bfloat16, True, TILES["128x128"][0])
+
+
+@pytest.mark.parametrize("bt", [False, True])
+def test_deep_rings_around_their_first_k(lib, bt):
+    """128 x 128 tiles: the shallow rings up to K = 1008, the deep ones from 1024 on, at every kind of K tail."""
+    for K in (1008, 1024, 1040, 1056, 1072, 1088, 1136, 1152, 1200, 1264, 1328, 1360):
+        _check(lib, 256, 128, K, torch.float16, bt, TILES["128x128"][0])

@@ -155,11 +155,14 @@ def test_fp16_tile_rule(tmp_path):
     src = open(os.path.join(ROOT, "llmmm_amd", "csrc", "capi.cpp")).read()
     at = src.index("int heuristic_tile_fp16(")
     rule = src[at:src.index("\n}\n", at) + 3]
+    kernel = open(os.path.join(ROOT, "llmmm_amd", "csrc", "fp16_gemm.hip")).read()
+    at = kernel.index("bool fp16_deep(")
+    deep = kernel[at:kernel.index("\n", at) + 1]
     shapes = [(1408, 256, 160, "64x64"), (2048, 256, 160, "64x64"), (256, 2176, 80, "64x64"), (256, 256, 32, "64x64"), (1024, 1024, 1024, "64x64"),
               (5504, 2048, 256, "128x128"), (7424, 1152, 240, "128x128"), (6912, 4352, 16, "128x128"), (1152, 3456, 2000, "128x128"),
-              (4096, 4096, 4096, "256x256"), (8192, 8192, 8192, "256x256"), (2048, 19456, 2560, "256x256")]
-    (tmp_path / "rule.cpp").write_text('#include "llmmm.h"\n#include <cstdio>\nconstexpr int NUM_CUS = 256;\n%sint main()\n{\n%s}\n' % (
-        rule, "".join('  std::printf("%%d\\n", heuristic_tile_fp16(%d, %d, %d));\n' % s[:3] for s in shapes)))
+              (4096, 4096, 4096, "256x256"), (8192, 8192, 8192, "256x256"), (2048, 19456, 2560, "256x256"), (896, 4096, 384, "128x128"), (1024, 2560, 640, "128x128")]
+    (tmp_path / "rule.cpp").write_text('#include "llmmm.h"\n#include <cstdio>\nconstexpr int NUM_CUS = 256;\nnamespace llmmm {\nstatic int num_cus() { return 256; }\n%s}\n%sint main()\n{\n%s}\n' % (
+        deep, rule, "".join('  std::printf("%%d\\n", heuristic_tile_fp16(%d, %d, %d));\n' % s[:3] for s in shapes)))
     subprocess.run(["g++", "-std=c++17", "-I", os.path.join(ROOT, "include"), "-o", str(tmp_path / "rule"), str(tmp_path / "rule.cpp")], check=True)
     got = subprocess.run([str(tmp_path / "rule")], stdout=subprocess.PIPE, check=True, text=True).stdout.split()
     from llmmm_amd import _lib
