@@ -112,7 +112,7 @@ __device__ __forceinline__ PhaseClock phase_clock()
 
 // Logical tile id -> (tm, tn).  Hardware hands consecutive workgroup ids to the 8 XCDs in turn,
 // so ids congruent mod 8 share an L2: give each XCD a contiguous run of the grouped order
-// (groups of up to four tile rows of equal height swept along n), whose members reuse the same few A and B panels.
+// (groups of up to four tile rows swept along n, all of one height but the last: 5 rows as 3 + 2, 13 as 4 + 4 + 4 + 1), whose members reuse the same few A and B panels.
 // (Any number of tiles: XCD x owns tiles/8 of them and one more if x < tiles%8.  Dealing the ids of a tile count that 8 does not
 // divide out in turn made every XCD read nearly all of both operands: FP8 384 x 3584 x 18944 in 84 tiles x 3 splits 45.4 us, 37.9 so;
 // FP16 1152 x 3456 x 2048 in 243 tiles of 128 x 128 22.4 us, 19.7 so.)
@@ -215,7 +215,7 @@ __device__ __forceinline__ float wave_xor_sum(float v)
 // quantisers' one negative seed.  Such floats are ordered like their bits read as signed integers, and an integer maximum takes
 // its DPP operand in the same instruction, where fmaxf costs three (the move, a quieting of the moved value, the maximum).  What
 // bounds the row kernels on many rows is how many vector instructions a wave issues (2048 rows of 2560 bf16: about 500, eight
-// waves on each SIMD; 12 fewer per maximum: decoder layer of 2560 x 9728 at M = 2048 263.3 -> 261.5 us, at M = 100 70.2 -> 69.8).  After
+// waves on each SIMD); this form takes 12 fewer per maximum, less than the runs of a whole decoder layer differ by.  After
 // the steps 1 and 2 all lanes of a quad agree, so a mirrored half row serves for step 4.
 __device__ __forceinline__ float half_wave_max(float v)
 {

@@ -584,8 +584,8 @@ enum { ST_OUT_F32 = 0, ST_OUT_BF16 = 1, ST_OUT_ADD = 2, ST_OUT_FP8Q = 3 };
 
 // The maximum with lane l ^ MASK around the exchange: LDS-crossbar swizzles and a selected half swap.  The register-only steps of
 // wave_xor_max are shorter and the launch gets longer with them, in either of the two places (6144 x 2560, us, this form /
-// wave_xor_max: 6.3 / 6.6 - 6.8 at M = 1, 6.3 - 6.5 / 6.7 - 7.0 at 2, 6.4 - 6.6 / 6.9 - 7.1 at 4; other shapes move by less than two
-// runs of one form differ).  What the polling fragments wait for is each other's store, not these steps.
+// wave_xor_max: 6.3 / 6.6 - 6.8 at M = 1, 6.3 - 6.5 / 6.7 - 7.0 at 2, 6.4 - 6.6 / 6.9 - 7.1 at 4; 5120 x 5120 7.9 - 8.0 / 8.2 - 8.4 at M = 1;
+// others move by less than two runs of one form differ).  What the polling fragments wait for is each other's store, not these steps.
 template <int MASK>
 __device__ __forceinline__ float exchange_max(float v)
 {

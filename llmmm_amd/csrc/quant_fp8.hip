@@ -307,7 +307,11 @@ __global__ void __launch_bounds__(256) planes_add_rmsnorm_quant_kernel(const flo
     rv[i]       = load_row4<T>(residual + (size_t)m * N + 4 * c);
     wv[i]       = *(const f32x4*)(w + 4 * c);
   }
-  // W planes in flight, as many as about 128 registers hold; only the planes that exist are asked for.
+  // W planes in flight: 64 to 128 registers of loads beside the row's own; only the planes that exist are asked for.  That costs waves:
+  // 177 VGPRs and two per SIMD for three chunks, 256 and one for eight and ten, where a form that held eight planes of three chunks or
+  // two of ten, existing or not, took 126 and four, 170 and two.  With the GEMM in front of it that form was slower or even on
+  // 1 .. 2048 rows of 2048 .. 10240 columns behind 1 .. 8 planes (us, then / now: 640 x 2560 x 4096 25.6 / 25.1, 768 x 3072 x 8192
+  // 44.6 / 43.7, 16 x 8192 x 8192 24.5 / 22.0, 16 x 10240 x 2048 15.5 / 14.3).
   constexpr int W = NI <= 4 ? 8 : 32 / NI;
   for (int s0 = 0; s0 < S; s0 += W) {
     f32x4 p[W][NI];
