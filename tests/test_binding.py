@@ -215,3 +215,29 @@ def test_the_interpreter_lock_is_free_while_memory_is_allocated(tmp_path):
         assert calls.value > before, name
         assert held.value == 0, "%s allocates with the interpreter lock held" % name
         keep += [pool, out]
+
+
+@pytest.mark.gpu
+def test_calls_on_a_stream_that_takes_part_in_a_capture():
+    """Allocating calls on a forked side stream inside a capture: replayed results are the eager ones, every time."""
+    calls = _allocating_calls()
+    expect = {name: [t.clone() for t in call(None)] for name, call in calls.items()}
+    torch.cuda.synchronize()
+    side, outs = torch.cuda.Stream(), {}
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        side.wait_stream(torch.cuda.current_stream())
+        for name, call in calls.items():
+            outs[name] = call(side)
+        torch.cuda.current_stream().wait_stream(side)
+    for _ in range(3):
+        for out in outs.values():
+            for t in out:
+                t.view(torch.uint8).fill_(0x11)
+        graph.replay()
+        torch.cuda.synchronize()
+        for name, out in outs.items():
+            n = 4 * 16 * 2048 if name == "planes" else None
+            for t, e in zip(out, expect[name]):
+                assert torch.equal(t.view(torch.uint8).flatten()[:n and 4 * n], e.view(torch.uint8).flatten()[:n and 4 * n]), name
+        torch.empty(1 << 20, device="cuda").normal_()  # the program's own work between replays
