@@ -100,6 +100,14 @@ typedef struct llmmm_gemm_cfg {
 LLMMM_API int llmmm_fp16_gemm(int dtype, const void* A, const void* B, void* C, int M, int N, int K, int b_layout, void* stream);
 LLMMM_API int llmmm_fp16_gemm_ex(int dtype, const void* A, const void* B, void* C, int M, int N, int K, int b_layout,
                                  const llmmm_gemm_cfg* cfg, void* stream);
+/* The same with scratch memory: K may be split into up to 8 shares, whose fp32 partial sums (one M x N plane each) go through
+ * `workspace` and are added in a fixed order by a second kernel -- where the tiles alone would leave most of the chip idle and K is
+ * long.  llmmm_fp16_gemm_workspace: the bytes the library's own choice for a shape uses (0: it does not split).  Less, or none: no
+ * split, as in the two calls above.  cfg with a tile id (128x128, 64x128 or 64x64) and split_k > 1 asks for that split; the result does not depend
+ * on what the workspace held.  Calls that may overlap need workspaces of their own. */
+LLMMM_API size_t llmmm_fp16_gemm_workspace(int M, int N, int K);
+LLMMM_API int    llmmm_fp16_gemm_ws(int dtype, const void* A, const void* B, void* C, int M, int N, int K, int b_layout, void* workspace,
+                                    size_t workspace_bytes, const llmmm_gemm_cfg* cfg, void* stream);
 
 /* ---- FP8 blockwise GEMM -----------------------------------------------------------------
  * Replaces  fp8_gemm_blockwise_quant_A_1x128__B_128x128__output_fp32(A, A_scale_transposed,

@@ -42,6 +42,8 @@ _vp, _fp, _i, _sz = _c.c_void_p, _c.c_void_p, _c.c_int, _c.c_size_t
 SIGNATURES = {
     "llmmm_fp16_gemm": (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "llmmm_fp16_gemm_ex": (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _c.POINTER(GemmCfg), _vp]),
+    "llmmm_fp16_gemm_workspace": (_sz, [_i, _i, _i]),
+    "llmmm_fp16_gemm_ws": (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _sz, _c.POINTER(GemmCfg), _vp]),
     "llmmm_fp8_gemm": (_i, [_i, _vp, _fp, _vp, _fp, _vp, _fp, _i, _i, _i, _vp, _sz, _vp]),
     "llmmm_fp8_gemm_ex": (_i, [_i, _vp, _fp, _vp, _fp, _vp, _fp, _i, _i, _i, _vp, _sz, _c.POINTER(GemmCfg), _vp]),
     "llmmm_fp8_gemm_static_ws": (_i, [_i, _vp, _fp, _vp, _fp, _vp, _fp, _i, _i, _i, _vp]),

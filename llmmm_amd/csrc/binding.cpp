@@ -279,6 +279,15 @@ Workspace workspace(PyObject* o, Bytes&& own, const Launch& on, const at::Device
   return w;
 }
 
+// Planes for the split the library chooses for an FP16 / BF16 product, if it chooses one; dropped with the call, in stream order.
+Workspace fp16_workspace(bool automatic, int M, int N, int K, const Launch& on, const at::Device& device)
+{
+  Workspace    w;
+  const size_t n = automatic ? llmmm_fp16_gemm_workspace(M, N, K) : 0;
+  if (n) w.own = on.empty({(int64_t)n}, at::kByte, device), w.p = w.own.data_ptr(), w.n = n;
+  return w;
+}
+
 // ---------------------------------------------------------------------------------------------- entry points
 typedef PyObject* const* Args;
 
@@ -302,8 +311,10 @@ PyObject* fp16_gemm(Args v)
   const Launch         on = launch(v[5]);
   at::Tensor           own;
   if (!c) own = on.empty({M, N}, A.scalar_type(), A.device()), c = own.data_ptr();
+  const Workspace ws = fp16_workspace(cfg.tile == LLMMM_TILE_AUTO, M, N, K, on, A.device());
   call([&] {
-    return llmmm_fp16_gemm_ex(t == T_F16 ? LLMMM_DTYPE_F16 : LLMMM_DTYPE_BF16, a, b, c, M, N, K, bt ? LLMMM_B_TRANSPOSED : LLMMM_B_ROW_MAJOR, &cfg, on.handle);
+    return llmmm_fp16_gemm_ws(t == T_F16 ? LLMMM_DTYPE_F16 : LLMMM_DTYPE_BF16, a, b, c, M, N, K, bt ? LLMMM_B_TRANSPOSED : LLMMM_B_ROW_MAJOR, ws.p, ws.n, &cfg,
+                              on.handle);
   });
   if (own.defined()) return THPVariable_Wrap(on.returned(own));
   Py_INCREF(v[2]);
@@ -322,7 +333,10 @@ PyObject* fp16_mm(Args v)
   const void* b = ptr(v[1], "B", T_ANY, (int64_t)K * N);
   void*       c = ptr(v[2], "C", T_ANY, (int64_t)M * N);
   const Launch on = launch(v[6]);
-  call([&] { return llmmm_fp16_gemm(t == T_F16 ? LLMMM_DTYPE_F16 : LLMMM_DTYPE_BF16, a, b, c, M, N, K, LLMMM_B_ROW_MAJOR, on.handle); });
+  const Workspace ws = fp16_workspace(true, M, N, K, on, A.device());
+  call([&] {
+    return llmmm_fp16_gemm_ws(t == T_F16 ? LLMMM_DTYPE_F16 : LLMMM_DTYPE_BF16, a, b, c, M, N, K, LLMMM_B_ROW_MAJOR, ws.p, ws.n, nullptr, on.handle);
+  });
   Py_RETURN_NONE;
 }
 

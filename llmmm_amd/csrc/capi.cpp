@@ -138,7 +138,7 @@ int heuristic_tile(int M, int N)
 // is within 0.2 % of the best tile on average and 24 % at worst (256 x 384 x 6832), and a fit to 70 % of them is within 0.2 %
 // on the rest.  (Without the term in the rounds, and fitted from K = 256 up only, it took the largest tiles at short K: 17 % off on
 // average, 1408 x 256 x 160 5.7 us in 128 x 256 tiles for 3.3 in 64 x 64.)
-int heuristic_tile_fp16(int M, int N, int K)
+int heuristic_tile_fp16(int M, int N, int K, double* estimate = nullptr)
 {
   static const struct {
     int    id, bm, bn, per_cu;
@@ -163,7 +163,35 @@ int heuristic_tile_fp16(int M, int N, int K)
     const double us = c.fixed + (full + left - 1 + round) * c.setup + K / 64. * ((full - 1 + round) * c.all + left * c.one);
     if (best < 0 || us < best_us) best = c.id, best_us = us;
   }
+  if (estimate) *estimate = best_us;
   return best;
+}
+// Split-K of the FP16 / BF16 kernels: S shares of every tile, at most one workgroup per CU, their fp32 planes written and added by a
+// second kernel.  What that adds to a share's own time is fitted to every (tile, S) of 550 shapes with at most 1.2 tiles of 128 x 128
+// per CU (K 256 .. 8192); a split is taken where the estimate is 6 % ahead of the unsplit choice's (`unsplit`).  On those shapes it then never
+// lost, 99 took it, and the mean time is 0.94 of the unsplit choice's, 1.7 % above the best (tile, S) of each (us, unsplit / split:
+// 256 x 128 x 7504 20.6 / 9.4, 384 x 640 x 5264 24.6 / 12.7, 256 x 1408 x 7024 26.1 / 16.8, 512 x 128 x 2048 7.8 / 7.2).  The planes' way
+// through memory bounds it: 1024^3 in two shares takes 9.9 for 6.1.  Returns S (1: no split) and, if S > 1, the tile.
+int heuristic_split_fp16(int M, int N, int K, double unsplit, int* tile)
+{
+  static const struct {
+    int    id, bm, bn;
+    double start, stage, launch, per_share, per_mb;  // (the 128 x 128 tile in its deep rings)
+  } cand[] = {{LLMMM_TILE_128x128, 128, 128, 3.92, 0.380, 3.54, 0.440, 0.147},
+              {LLMMM_TILE_64x128, 64, 128, 2.92, 0.303, 2.50, 0.447, -0.490},
+              {LLMMM_TILE_64x64, 64, 64, 2.77, 0.182, 2.78, 0.451, -0.501}};
+  const double mb     = (double)M * N * 4e-6;
+  const int    stages = (K + 63) / 64;
+  double       limit  = unsplit * 0.94;
+  int          split  = 1;
+  for (const auto& c : cand) {
+    const long tiles = (long)(M / c.bm) * (N / c.bn);
+    for (int s = 2; s <= llmmm::FP16_MAX_SPLIT && s <= stages && (tiles + 7) / 8 * 8 * s <= NUM_CUS; ++s) {
+      const double us = c.start + (stages + s - 1) / s * c.stage + c.launch + mb * (c.per_share * s + c.per_mb);
+      if (us < limit) *tile = c.id, split = s, limit = us;
+    }
+  }
+  return split;
 }
 
 constexpr int MAX_TILE_SPLIT = 8;
@@ -514,7 +542,25 @@ const char* llmmm_last_error(void) { return g_last_error; }
 
 int llmmm_version(void) { return 100; }
 
-int llmmm_fp16_gemm_ex(int dtype, const void* A, const void* B, void* C, int M, int N, int K, int b_layout,
+// Kernel choice of a call without (or with AUTO) cfg; split > 1 needs split * M * N floats.
+static void choose_fp16(int M, int N, int K, bool may_split, int* tile, int* split)
+{
+  *split = 1;
+  if (lookup_fp16_tile(M, N, K, tile)) return;
+  double us;
+  *tile = heuristic_tile_fp16(M, N, K, &us);
+  if (may_split) *split = heuristic_split_fp16(M, N, K, us, tile);
+}
+
+size_t llmmm_fp16_gemm_workspace(int M, int N, int K)
+{
+  if (M <= 0 || N <= 0 || K <= 0 || M % 128 || N % 128 || K % 16) return 0;
+  int tile, split;
+  choose_fp16(M, N, K, true, &tile, &split);
+  return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
+}
+
+int llmmm_fp16_gemm_ws(int dtype, const void* A, const void* B, void* C, int M, int N, int K, int b_layout, void* workspace, size_t workspace_bytes,
                        const llmmm_gemm_cfg* cfg, void* stream)
 {
   if (dtype != LLMMM_DTYPE_F16 && dtype != LLMMM_DTYPE_BF16) return fail(LLMMM_ERR_UNSUPPORTED_TYPE, "T is not supported.");
@@ -526,17 +572,31 @@ int llmmm_fp16_gemm_ex(int dtype, const void* A, const void* B, void* C, int M, 
   if (!aligned16(A) || !aligned16(B) || !aligned16(C)) return fail(LLMMM_ERR_INVALID_ARGUMENT, "pointers must be 16-byte aligned");
   if ((long)M * K >= (1L << 31) || (long)N * K >= (1L << 31) || (long)M * N >= (1L << 31))
     return fail(LLMMM_ERR_INVALID_ARGUMENT, "matrix has 2^31 or more elements");
-  int tile = cfg ? cfg->tile : LLMMM_TILE_AUTO;
+  const size_t plane = (size_t)M * N * sizeof(float);
+  int          tile = cfg ? cfg->tile : LLMMM_TILE_AUTO, split = 1;
   if (tile == LLMMM_TILE_AUTO) {
-    if (!lookup_fp16_tile(M, N, K, &tile)) tile = LLMMM_TILE_AUTO;
-    if (tile == LLMMM_TILE_AUTO) tile = heuristic_tile_fp16(M, N, K);
+    choose_fp16(M, N, K, workspace != nullptr, &tile, &split);
+    if (split > 1 && workspace_bytes < split * plane) choose_fp16(M, N, K, false, &tile, &split);  // (documented: no room, no split)
   }
   int bm, bn;
   if (!tile_dims(tile, bm, bn) || tile == LLMMM_TILE_128x160) return fail(LLMMM_ERR_INVALID_ARGUMENT, "unknown tile id %d", tile);
   if (M % bm || N % bn) return fail(LLMMM_ERR_NOT_ALIGNED, "M or N or K are not aligned.");
-  const hipError_t e = llmmm::fp16_gemm_launch(dtype, b_layout, tile, A, B, C, M, N, K, (hipStream_t)stream);
+  if (cfg && cfg->tile != LLMMM_TILE_AUTO && cfg->split_k > 1 && workspace) {  // (ignored without a workspace, as llmmm_fp16_gemm_ex ignores it)
+    split = cfg->split_k;
+    if (split > llmmm::FP16_MAX_SPLIT || split > (K + 63) / 64 || (tile != LLMMM_TILE_128x128 && !fp16_only(tile)))
+      return fail(LLMMM_ERR_INVALID_ARGUMENT, "split-K %d: 128 x 128 and smaller tiles, at most %d shares and one per 64 of K", split, llmmm::FP16_MAX_SPLIT);
+    if (workspace_bytes < split * plane) return fail(LLMMM_ERR_WORKSPACE, "workspace holds %zu bytes, split-K %d needs %zu", workspace_bytes, split, split * plane);
+  }
+  if (split > 1 && !aligned16(workspace)) return fail(LLMMM_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
+  const hipError_t e = split > 1 ? llmmm::fp16_gemm_split_launch(dtype, b_layout, tile, A, B, C, M, N, K, split, (float*)workspace, (hipStream_t)stream)
+                                 : llmmm::fp16_gemm_launch(dtype, b_layout, tile, A, B, C, M, N, K, (hipStream_t)stream);
   if (e != hipSuccess) return fail(LLMMM_ERR_RUNTIME, "fp16 gemm launch: %s", hipGetErrorString(e));
   return LLMMM_OK;
+}
+
+int llmmm_fp16_gemm_ex(int dtype, const void* A, const void* B, void* C, int M, int N, int K, int b_layout, const llmmm_gemm_cfg* cfg, void* stream)
+{
+  return llmmm_fp16_gemm_ws(dtype, A, B, C, M, N, K, b_layout, nullptr, 0, cfg, stream);
 }
 
 int llmmm_fp16_gemm(int dtype, const void* A, const void* B, void* C, int M, int N, int K, int b_layout, void* stream)

@@ -253,9 +253,12 @@ struct Fp16Wave {
 // The kernel's body for tile `tile_index` of the tiles_m x tiles_n tiles of the column range that starts at n_base (0 and
 // the whole matrix for the plain kernel); lds: the workgroup's rings.
 // STAMP: the phase-accounting build -- clock readings at five points of every wave, stored to `stamps` at the end.
-template <typename T, int BM, int BN, int WM, int WN, int DA, int DB, bool B_NK, bool STAMP = false>
-__device__ __forceinline__ void fp16_gemm_body(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C, int M, int N, int K, int tiles_m,
-                                               int tiles_n, char LLMMM_LDS* lds, int tile_index, int n_base, unsigned long long* stamps = nullptr)
+// SPLIT: the workgroup takes share `sp` of `S` of the K stages (pitch = the matrices' K, K = its own range) and stores its partial
+// sums to plane sp of `planes` (fp16_splitk_reduce_kernel) instead of C.
+template <typename T, int BM, int BN, int WM, int WN, int DA, int DB, bool B_NK, bool STAMP = false, bool SPLIT = false>
+__device__ __forceinline__ void fp16_gemm_body(const T* __restrict__ A, const T* __restrict__ B, T* __restrict__ C, int M, int N, int pitch, int tiles_m,
+                                               int tiles_n, char LLMMM_LDS* lds, int tile_index, int n_base, unsigned long long* stamps = nullptr,
+                                               float* __restrict__ planes = nullptr, int sp = 0, int S = 1)
 {
   typedef Fp16Tile<BM, BN, WM, WN, DA, DB> TC;
   typedef typename Vec16<T>::vec           vec;
@@ -273,11 +276,15 @@ __device__ __forceinline__ void fp16_gemm_body(const T* __restrict__ A, const T*
   tile_coords(tile_index, tiles_m, tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = n_base + tn * BN;
 
+  const int stages = (pitch + TC::BK - 1) / TC::BK, first = SPLIT ? sp * stages / S : 0;  // whole stages: a share ends on a multiple of BK or with K
+  const int K      = SPLIT ? min(pitch, (sp + 1) * stages / S * TC::BK) - first * TC::BK : pitch;
+
   Fp16Wave<T, BM, BN, WM, WN, DA, DB, B_NK> w;
   w.K = K, w.wave = wave, w.lane = lane, w.lds = lds, w.lds_addr = (unsigned)(size_t)lds;
-  w.Ag     = A + (size_t)m0 * K;
-  w.Bg     = B_NK ? B + (size_t)n0 * K : B + n0;
+  w.Ag     = A + (size_t)m0 * pitch;
+  w.Bg     = B_NK ? B + (size_t)n0 * pitch : B + n0;
   w.b_step = B_NK ? (size_t)TC::BK : (size_t)TC::BK * N;
+  if constexpr (SPLIT) w.Ag += (size_t)first * TC::BK, w.Bg += (size_t)first * w.b_step;
   // ---- loader: lane -> what the 16 bytes at (1 KB load base + 16*lane) must hold.  (The byte offsets fit 32 bits: BM rows of
   // A or BN of Bt are part of matrices below 2^31 elements, and so are the k rows below K.)
   {
@@ -285,11 +292,11 @@ __device__ __forceinline__ void fp16_gemm_body(const T* __restrict__ A, const T*
     const int c = (lane & 7) ^ k128_swz(r);         // logical chunk placed at physical chunk lane%8
     w.a_k       = c * 8;
 #pragma unroll
-    for (int i = 0; i < TC::A_LOADS; ++i) w.a_off[i] = ((unsigned)(r + i * TC::ROWS_PER_LOAD) * (unsigned)K + c * 8) * 2u;
+    for (int i = 0; i < TC::A_LOADS; ++i) w.a_off[i] = ((unsigned)(r + i * TC::ROWS_PER_LOAD) * (unsigned)pitch + c * 8) * 2u;
 #pragma unroll
     for (int i = 0; i < TC::B_LOADS; ++i) {
       if constexpr (B_NK) {
-        w.b_off[i] = ((unsigned)(r + i * TC::ROWS_PER_LOAD) * (unsigned)K + c * 8) * 2u;
+        w.b_off[i] = ((unsigned)(r + i * TC::ROWS_PER_LOAD) * (unsigned)pitch + c * 8) * 2u;
         w.b_k[i]   = c * 8;
       }
       else {
@@ -374,6 +381,18 @@ __device__ __forceinline__ void fp16_gemm_body(const T* __restrict__ A, const T*
   for (int nf = 0; nf < NF; ++nf)
 #pragma unroll
     for (int mf = 0; mf < MF; ++mf) asm volatile("" : "+a"(w.acc[nf][mf]));
+  if constexpr (SPLIT) {
+    // a plane is a row of 1 KB blocks, one per 16 x 16 fragment, in the accumulators' own lane order: every store is one linear
+    // kilobyte, whatever the tile, and the reduce kernel finds 8 rows x 16 bytes of a fragment in one cache line
+    float* plane = planes + (size_t)sp * M * N;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (nothing is left in flight; the compiler counts its own stores from here)
+#pragma unroll
+    for (int mf = 0; mf < MF; ++mf)
+#pragma unroll
+      for (int nf = 0; nf < NF; ++nf)
+        *(f32x4*)(plane + ((size_t)((m0 + wm * WM) / 16 + mf) * (N / 16) + (n0 + wn * WN) / 16 + nf) * 256 + lane * 4) = w.acc[nf][mf];
+    return;
+  }
   if constexpr (STAMP) ph[2] = phase_clock();
   __builtin_amdgcn_s_barrier();  // every wave is through with the operands: the rings are free
   asm volatile("" ::: "memory");
@@ -440,6 +459,61 @@ fp16_gemm_kernel(const T* __restrict__ A, const T* __restrict__ B, T* __restrict
   fp16_gemm_body<T, BM, BN, WM, WN, DA, DB, B_NK>(A, B, C, M, N, K, tiles_m, tiles_n, (char LLMMM_LDS*)lds, blockIdx.x, 0);
 }
 
+// split-K: S workgroups per tile, each over its share of the K stages, and a second kernel that adds their planes (where it pays:
+// heuristic_split_fp16 in capi.cpp).  What bounds it besides the product is the planes' way through memory, so both kernels deal the
+// tiles to the XCDs alike -- XCD x (workgroup ids = x mod 8) owns a contiguous run of tiles with all S shares of each -- and the reduce
+// kernel finds the planes in its own L2.
+// Workgroup wg of 8 * ceil(tiles / 8) * per: item 0 .. tiles * per - 1 of XCD-contiguous tiles with `per` items each; false: none.
+__device__ __forceinline__ bool split_item(int wg, int tiles, int per, int& tile_id, int& item)
+{
+  const int x = wg & 7, j = wg >> 3, mine = (tiles >> 3) + (x < (tiles & 7) ? 1 : 0);
+  if (j >= mine * per) return false;
+  const int t = j % mine;
+  item        = j / mine;
+  tile_id     = t * 8 + x;  // tile_coords takes the ids = x mod 8 for XCD x's run
+  return true;
+}
+
+template <typename T, int BM, int BN, int WM, int WN, int DA, int DB, bool B_NK>
+__global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64)
+fp16_split_gemm_kernel(const T* __restrict__ A, const T* __restrict__ B, float* __restrict__ planes, int M, int N, int K, int tiles_m, int tiles_n, int S)
+{
+  __shared__ __attribute__((aligned(1024))) char lds[Fp16Tile<BM, BN, WM, WN, DA, DB>::LDS];
+  int tile_id, sp;
+  if (!split_item(blockIdx.x, tiles_m * tiles_n, S, tile_id, sp)) return;
+  fp16_gemm_body<T, BM, BN, WM, WN, DA, DB, B_NK, false, true>(A, B, nullptr, M, N, K, tiles_m, tiles_n, (char LLMMM_LDS*)lds, tile_id, 0, nullptr, planes, sp, S);
+}
+
+// Adds the S planes in order and rounds to T.  A wave takes 8 rows x 64 columns: lane l row l / 8, columns 8 (l % 8) .. +7, i.e. two
+// 16-byte pieces of a fragment whose eight rows lie in one cache line, and its stores are eight whole 128-byte lines.
+// All loads of a lane go out together (a launch of this size is one latency long): S is a constant.
+template <typename T, int S, int BM, int BN>
+__global__ void __launch_bounds__(256)
+fp16_splitk_reduce_kernel(const float* __restrict__ planes, T* __restrict__ C, int M, int N, int tiles_m, int tiles_n)
+{
+  constexpr int UNITS = BM * BN / 2048;  // workgroups per tile
+  int           tile_id, unit, tm, tn;
+  if (!split_item(blockIdx.x, tiles_m * tiles_n, UNITS, tile_id, unit)) return;
+  tile_coords(tile_id, tiles_m, tiles_n, tm, tn);
+  const int    lane = threadIdx.x & 63, w = unit * 4 + (threadIdx.x >> 6);
+  const int    row = tm * BM + w / (BN / 64) * 8 + (lane >> 3), col = tn * BN + w % (BN / 64) * 64 + (lane & 7) * 8;
+  const float* p = planes + ((size_t)(row >> 4) * (N >> 4) + (col >> 4)) * 256 + ((col & 8) * 4 + (row & 15)) * 4;
+  f32x4        v[S][2];
+#pragma unroll
+  for (int s = 0; s < S; ++s) v[s][0] = *(const f32x4*)(p + (size_t)s * M * N), v[s][1] = *(const f32x4*)(p + (size_t)s * M * N + 64);
+  typedef T tx8 __attribute__((ext_vector_type(8)));
+  tx8       o;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    f32x4 t = v[0][h];
+#pragma unroll
+    for (int s = 1; s < S; ++s) t += v[s][h];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[4 * h + e] = (T)t[e];
+  }
+  *(tx8*)(C + (size_t)row * N + col) = o;
+}
+
 // 256 x 256 tiles whose number is not a multiple of the 256 CUs end with a round that keeps part of the chip busy for a
 // whole tile's time (2048 x 19456: 608 tiles, the third round 96 of them).  One launch of both shapes: the columns that fill
 // whole rounds go to 256 x 256 tiles (workgroups 0 .. tiles_m_big * cols_big - 1, dispatched first), the remaining columns
@@ -481,6 +555,53 @@ static hipError_t launch_fp16(const void* A, const void* B, void* C, int M, int 
   hipLaunchKernelGGL((fp16_gemm_kernel<T, BM, BN, WM, WN, DA, DB, B_NK>), dim3(tiles_m * tiles_n), dim3(Fp16Tile<BM, BN, WM, WN, DA, DB>::NT), 0, stream,
                      (const T*)A, (const T*)B, (T*)C, M, N, K, tiles_m, tiles_n);
   return hipGetLastError();
+}
+
+template <typename T, int BM, int BN, int WM, int WN, int DA, int DB>
+static hipError_t launch_fp16_split(bool b_nk, const void* A, const void* B, void* C, int M, int N, int K, int S, float* planes, hipStream_t stream)
+{
+  const int  tiles_m = M / BM, tiles_n = N / BN, runs = (tiles_m * tiles_n + 7) / 8 * 8;
+  const dim3 grid(runs * S), block(Fp16Tile<BM, BN, WM, WN, DA, DB>::NT), reduce_grid(runs * (BM * BN / 2048));
+  if (b_nk)
+    hipLaunchKernelGGL((fp16_split_gemm_kernel<T, BM, BN, WM, WN, DA, DB, true>), grid, block, 0, stream, (const T*)A, (const T*)B, planes, M, N, K, tiles_m, tiles_n, S);
+  else
+    hipLaunchKernelGGL((fp16_split_gemm_kernel<T, BM, BN, WM, WN, DA, DB, false>), grid, block, 0, stream, (const T*)A, (const T*)B, planes, M, N, K, tiles_m, tiles_n, S);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  switch (S) {
+#define LLMMM_GO(n) \
+  case n: hipLaunchKernelGGL((fp16_splitk_reduce_kernel<T, n, BM, BN>), reduce_grid, dim3(256), 0, stream, planes, (T*)C, M, N, tiles_m, tiles_n); break
+    LLMMM_GO(2);
+    LLMMM_GO(3);
+    LLMMM_GO(4);
+    LLMMM_GO(5);
+    LLMMM_GO(6);
+    LLMMM_GO(7);
+    LLMMM_GO(8);
+#undef LLMMM_GO
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+template <typename T>
+static hipError_t fp16_split(bool b_nk, int tile, const void* A, const void* B, void* C, int M, int N, int K, int S, float* planes, hipStream_t stream)
+{
+  switch (tile) {
+    case LLMMM_TILE_128x128: return launch_fp16_split<T, 128, 128, 64, 64, 5, 5>(b_nk, A, B, C, M, N, K, S, planes, stream);
+    case LLMMM_TILE_64x128: return launch_fp16_split<T, 64, 128, 32, 64, 3, 3>(b_nk, A, B, C, M, N, K, S, planes, stream);
+    case LLMMM_TILE_64x64: return launch_fp16_split<T, 64, 64, 32, 32, 4, 4>(b_nk, A, B, C, M, N, K, S, planes, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// K in S shares through fp32 planes (S * M * N floats), 2 <= S <= FP16_MAX_SPLIT, S <= the number of 64-wide K stages.
+hipError_t fp16_gemm_split_launch(int dtype, int b_layout, int tile, const void* A, const void* B, void* C, int M, int N, int K, int S, float* planes,
+                                  hipStream_t stream)
+{
+  if (S < 2 || S > FP16_MAX_SPLIT || S > (K + 63) / 64 || !planes || M % 128 || N % 128) return hipErrorInvalidValue;
+  return dtype == 0 ? fp16_split<_Float16>(b_layout != 0, tile, A, B, C, M, N, K, S, planes, stream)
+                    : fp16_split<__bf16>(b_layout != 0, tile, A, B, C, M, N, K, S, planes, stream);
 }
 
 // The rings of the 128 x 128 tile.  Up to one tile per CU and from K = 1024 on they take the whole LDS (1920 x 1536 x 5312, 180 tiles:

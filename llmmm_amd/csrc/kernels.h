@@ -13,6 +13,9 @@ namespace llmmm {
 bool       fp16_deep(int M, int N, int K);  // whether the 128 x 128 FP16 / BF16 tile runs in its deep rings
 hipError_t fp16_gemm_launch(int dtype, int b_layout, int tile, const void* A, const void* B, void* C, int M, int N, int K,
                             hipStream_t stream);
+constexpr int FP16_MAX_SPLIT = 8;
+hipError_t    fp16_gemm_split_launch(int dtype, int b_layout, int tile, const void* A, const void* B, void* C, int M, int N, int K, int S, float* planes,
+                                     hipStream_t stream);
 
 // out_kind: 0 = fp32, 1 = bf16, 2 = e4m3 codes + per-1x128 scales, 3 = SwiGLU (silu(C[:, :N/2]) * C[:, N/2:]) as codes + scales.  S > 1 splits K over S
 // workgroups per tile (S <= K/128): `planes` then holds S * M * N floats of partial sums, added

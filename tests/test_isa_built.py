@@ -153,6 +153,19 @@ def test_fp16_loop_hazards(objects):
         _check_m0(name, code)
 
 
+def test_fp16_split_loop_hazards(objects):
+    """The same loop over a share of K (fp16_split_gemm_kernel): its plane stores read the accumulators straight behind it."""
+    path = next(o for o in objects if any("fp16_split_gemm_kernel" in n for n in _kernels(o)))
+    meta = _kernels(path)
+    functions = {n: c for n, c in _functions(_tool("llvm-objdump", "-d", path)).items() if "fp16_split_gemm_kernel" in n and not n.endswith(".kd")}
+    assert len(functions) == 12  # three tiles x 2 types x 2 layouts
+    for name, code in functions.items():
+        assert int(meta[name]["private_segment_fixed_size"]) == 0 and int(meta[name]["vgpr_spill_count"]) == 0, name
+        assert sum(c[1].startswith("v_mfma") for c in code) > 0 and sum(c[1] == "s_add_u32" and c[2][0] == "m0" for c in code) > 0, name
+        _check_mfma_reads(name, code)
+        _check_m0(name, code)
+
+
 def test_the_checks_see_a_missing_wait_and_a_second_m0_write(objects):
     path = next(o for o in objects if any("fp16_gemm_kernel" in n for n in _kernels(o)))
     name, code = next((n, c) for n, c in _functions(_tool("llvm-objdump", "-d", path)).items() if "fp16_gemm_kernelIDF16_Li64ELi64E" in n and not n.endswith(".kd"))
