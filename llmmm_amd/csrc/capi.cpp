@@ -480,6 +480,16 @@ int strip_exchange_area(void* stream)
   return used++;
 }
 
+// The SwiGLU output of the weight-streaming kernel in one launch (64 gate + 64 up columns per workgroup, K unsplit; figures in
+// fp8_skinny.hip).  Its N / 128 workgroups have to fill the chip or a good part of its last round: with fewer, splitting K pulls more
+// (12288 x 2048, 96 workgroups, M = 24: 9.4 in two splits + reduce / 9.9 so), and 272 or 296 run a nearly empty second round
+// (34816 x 5120 at M = 1: 36.8 / 43.6; 51200 x 5120, 400 of them: 48.9 / 47.9 at M = 1, 54.6 / 49.2 at 16).
+bool swiglu_pair_pays(int M, int N, int K)
+{
+  const int groups = N / 128, last = groups % NUM_CUS;
+  return llmmm::fp8_skinny_swiglu_fits(M, N, K) && groups >= (M <= 16 ? 96 : 128) && (groups <= NUM_CUS || last == 0 || last >= NUM_CUS / 2);
+}
+
 // The split the weight-streaming kernel runs this shape in when it is the split-K form after all (tune table, then heuristic).
 int skinny_split_for(int M, int N, int K)
 {
@@ -793,6 +803,7 @@ int llmmm_fp8_gemm_ex(int out_kind, const void* A, const float* As, const void* 
       split = min_split;
     }
     float* partial = nullptr;
+    int    pair_area;
     if (swiglu && !workspace) return fail(LLMMM_ERR_WORKSPACE, "the SwiGLU output at M <= %d needs a workspace of at least M * N floats", SKINNY_MAX_M);
     if (split > 1 && !(user && user->split_k > 0)) {
       // a split the library chose itself shrinks to what the caller's workspace holds
@@ -807,7 +818,10 @@ int llmmm_fp8_gemm_ex(int out_kind, const void* A, const float* As, const void* 
       if (!aligned16(workspace)) return fail(LLMMM_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
       partial = (float*)workspace;
     }
-    if (agen == 2)
+    const bool pair = swiglu && !agen && !(user && user->split_k > 0) && swiglu_pair_pays(M, N, K) && (pair_area = strip_exchange_area(stream)) >= 0;
+    if (pair)
+      e = llmmm::fp8_skinny_swiglu_launch(cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, pair_area, (hipStream_t)stream), partial = nullptr;
+    else if (agen == 2)
       e = llmmm::fp8_skinny_rmsnorm_a_launch(prep.hidden_dtype, cfg.b_layout, prep.ag, Bt, Bs, (float*)C, M, N, K, split, partial, (hipStream_t)stream);
     else if (agen)
       e = llmmm::fp8_skinny_swiglu_a_launch(partial ? LLMMM_OUT_F32 : out_kind, cfg.b_layout, (const float*)A, Bt, Bs, C, Cs, M, N, K, split, partial,

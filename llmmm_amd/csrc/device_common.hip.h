@@ -316,6 +316,51 @@ __device__ __forceinline__ void store_row4<_Float16>(_Float16* p, f32x4 v)
   *(f16x4*)p = f16x4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
 }
 
+// ---------------------------------------------------------------------------------------------
+// The hand-over of row maxima between the two workgroups that hold the halves of one 1x128 quantisation group (the SwiGLU outputs:
+// 64 gate and the matching 64 up columns per workgroup).  `area` is [buffer 2][group][16-row block][half 2][16 rows] words of device
+// memory, zero when the library is loaded, one per stream.  A slot holds (bits of the maximum) + 1 -- never 0, maxima of absolute
+// values being neither negative nor NaN -- or 0 for "not written in this launch".  Two buffers take turns: a launch works in the one
+// that holds zeros and clears its own slots of the other.  Which is which, a workgroup reads off its own row-0 slot of buffer 0 at kernel
+// entry: written by nobody else, and both halves of a block take part in every launch that touches it, so they agree.  The state
+// is kept per block of 16 rows, so launches with other row counts may follow each other.
+// Device-scope relaxed atomics and no fence: the slots are all that is shared.  Waiting is safe because the halves' workgroup ids
+// are 2j and 2j + 1 and ids are dispatched in order: the smallest incomplete pair always makes progress.  The wait is bounded
+// all the same (20 ms of the 100 MHz clock); a wave that gives up counts itself in *timeouts and goes on with what it has.
+// ---------------------------------------------------------------------------------------------
+constexpr int PAIR_BLOCKS = 8;  // 16-row blocks of an area: M <= 128
+struct PairSlots {
+  unsigned* area;
+  int       groups, group, half;
+  __device__ __forceinline__ unsigned* slot(int buffer, int block, int h) const
+  {
+    return area + ((((size_t)buffer * groups + group) * PAIR_BLOCKS + block) * 2 + h) * 16;
+  }
+  // lane i < 16 of a 16-lane row: row i's maximum over this half
+  __device__ __forceinline__ void publish(int cur, int block, int i, float a) const
+  {
+    __hip_atomic_store(slot(cur ^ 1, block, half) + i, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(slot(cur, block, half) + i, __builtin_bit_cast(unsigned, a) + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  // row i's maximum over the other half
+  __device__ __forceinline__ float other(int cur, int block, int i, unsigned* timeouts) const
+  {
+    const unsigned*          src = slot(cur, block, half ^ 1) + i;
+    const unsigned long long t0  = __builtin_amdgcn_s_memrealtime();
+    unsigned                 w;
+    for (;;) {
+      w = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__builtin_amdgcn_ballot_w64(w == 0u) == 0ull) break;
+      if (__builtin_amdgcn_s_memrealtime() - t0 > 2000000ull) {
+        if (__lane_id() == 0) atomicAdd(timeouts, 1u);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    return __builtin_bit_cast(float, w - 1u);
+  }
+};
+
 // silu(g) * u with the hardware's exp2 and reciprocal (each within about one ulp of fp32): far below the
 // resolution of the e4m3 codes the result is quantised to.  g -> -inf gives -0, g -> +inf gives g * u.
 __device__ __forceinline__ float silu_mul(float g, float u)

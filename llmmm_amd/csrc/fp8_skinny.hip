@@ -16,6 +16,10 @@
 //    (fixed order, independent of arrival) and runs the epilogue.  An in-kernel "last arriver
 //    reduces" scheme was measured slower: its device-scope stores, counter and re-reads put three
 //    dependent memory round trips on the critical path of every column group.
+//  * SwiGLU (SK_OUT_SWIGLU, M <= 32): a workgroup takes 64 gate and the matching 64 up columns over all of K, applies the activation
+//    itself and agrees on the 1x128 groups' row maxima with the one other workgroup of the group (PairSlots).  That costs 1.2 us and
+//    saves the fp32 planes and the reduce launch (us, planes + reduce / so: 19456 x 2560 13.5 / 12.2 at M = 1, 13.3 / 11.8 at 16, 14.0 / 12.7
+//    at 24; 28672 x 4096 25.5 / 22.7; 12288 x 2048, split in two before, 8.9 / 9.4, 8.8 / 8.8 and 9.15 / 9.1 -- and a launch, 3 us of host time, less).
 //  * The activation rows a workgroup needs (16..64 rows x the K range of its split) are staged
 //    in LDS once, before the loop, whenever they fit beside the ring; every wave then reads its
 //    operand fragments from there instead of re-fetching them from L2 slice by slice.
@@ -24,7 +28,12 @@
 
 namespace llmmm {
 
-enum { SK_OUT_F32 = 0, SK_OUT_BF16 = 1, SK_OUT_FP8Q = 2 };
+enum { SK_OUT_F32 = 0, SK_OUT_BF16 = 1, SK_OUT_FP8Q = 2,
+       SK_OUT_SWIGLU = 3 };  // h = silu(gate) * up, quantised 1x128, in one launch: K unsplit, 64 gate + 64 up columns per workgroup
+
+// Where the workgroups of a SwiGLU output exchange their row maxima (PairSlots).
+static __device__ unsigned g_pair_xch[STRIP_XCH_AREAS][2 * STRIP_XCH_MAX_GROUPS * PAIR_BLOCKS * 2 * 16];
+static __device__ unsigned g_pair_xch_timeouts;
 
 // What one 128-K slice needs besides the weights: the activation rows (straight into the MFMA
 // operand registers) and both scales.  Rows beyond M are clamped to M-1 (a valid address, no
@@ -161,8 +170,10 @@ template <int MBLK, int OUT, int D, int ASTG, int AGEN = 0, typename HT = float>
 __global__ void __launch_bounds__(512)
 fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Bt,
                   const float* __restrict__ Bs, void* __restrict__ Cv, float* __restrict__ Cs, int M, int N, int K, int S,
-                  float* __restrict__ partial, int bpre, SkinnyGenA ag)
+                  float* __restrict__ partial, int bpre, SkinnyGenA ag, int xarea)
 {
+  constexpr bool SWIGLU = OUT == SK_OUT_SWIGLU;
+  static_assert(!SWIGLU || (AGEN == 0 && MBLK <= 2), "the SwiGLU output: given activations, at most 32 rows");
   constexpr bool APRE  = ASTG > 0;
   static_assert(AGEN == 0 || (MBLK == 1 && APRE), "generated activations: 16 rows, staged in LDS");
   constexpr int  LOADS = SKINNY_LOADS_PER_SLOT_BASE + (AGEN != 0 ? 0 : (APRE ? 1 : 3) * MBLK);  // vector-memory loads per slot, issued in slot order
@@ -179,6 +190,7 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
   __shared__ __attribute__((aligned(1024))) char ring6[D > 4 ? 8 * 2048 : 16];
   __shared__ __attribute__((aligned(1024))) char ring7[D > 4 ? 8 * 2048 : 16];
   __shared__ float    wave_amax[8][MBLK][16];
+  __shared__ f32x4    up_part[SWIGLU ? 4 : 1][SWIGLU ? MBLK : 1][SWIGLU ? 64 : 1];  // SwiGLU: the up waves' results, lane for lane
   __shared__ float    a_scale[AGEN != 0 ? (ASTG / 2048) * 16 : 1];  // AGEN: the generated row scales, [slice][row]
   __shared__ float    gen_sum[AGEN == 2 ? 8 : 1];                        // AGEN == 2: sums of squares of the 64-lane groups, two rows
 
@@ -205,14 +217,16 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
   // weights: loader lane -> (row, chunk) of the 1 KB group it fills; reader lane (g, i) -> row i, chunks 2g, 2g+1
   // pre-shuffled weights (bpre, layout.hip): the wave's 16 rows x 128 bytes of a slice are one 2 KB block that
   // already is the ring slot's image, and the blocks of consecutive slices follow each other
-  const uint8_t*   wrow = Bt + (size_t)(ng * 128 + wave * 16) * K;
+  // (SwiGLU: waves 0 .. 3 take the 64 gate columns, waves 4 .. 7 the up columns of the same outputs)
+  const int        n_wave = SWIGLU ? ng * 64 + (wave & 3) * 16 + (wave >> 2) * (N >> 1) : ng * 128 + wave * 16;
+  const uint8_t*   wrow = Bt + (size_t)n_wave * K;
   const KMajorLane l0   = kmajor_lane<SWZ_ROWS16>(0, lane);
   const KMajorLane l1   = kmajor_lane<SWZ_ROWS16>(1, lane);
   const unsigned   w_off0   = bpre ? (unsigned)lane * 16u : (unsigned)(l0.row * K + l0.chunk * 16);
   const unsigned   w_off1   = bpre ? 1024u + (unsigned)lane * 16u : (unsigned)(l1.row * K + l1.chunk * 16);
   const int        w_kstep  = bpre ? 2048 : 128;
   const int        w_rd   = kmajor_offset<SWZ_ROWS16>(i, 2 * g);
-  const float*     bsp    = Bs + (size_t)ng * KB;
+  const float*     bsp    = Bs + (size_t)(SWIGLU ? n_wave >> 7 : ng) * KB;
   const uint8_t*   ap[MBLK];
   const float*     asp[MBLK];
 #pragma unroll
@@ -226,6 +240,11 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
 #pragma unroll
   for (int mb = 0; mb < MBLK; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  // SwiGLU: which exchange buffer is next, per 16-row block (lane l: block l % MBLK); the oldest load in flight, looked at in the epilogue
+  unsigned        own_mark = 0u;
+  const PairSlots pair     = {SWIGLU ? &g_pair_xch[xarea][0] : nullptr, STRIP_XCH_MAX_GROUPS, ng >> 1, ng & 1};
+  if constexpr (SWIGLU) asm volatile("global_load_dword %0, %1, off sc1" : "=v"(own_mark) : "v"(pair.slot(0, lane & (MBLK - 1), ng & 1)) : "memory");
+
   // Activation staging: the 16*MBLK rows x (kb1 - kb0) slices this workgroup needs, as one
   // SWZ_ROWS16 tile of MBLK x 2 KB per slice, fetched once by LDS-direct loads of 8 whole rows
   // (1 KB units dealt round-robin to the waves) instead of once per wave and slice.  They are
@@ -235,14 +254,25 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
   const int                   a_rd   = kmajor_offset<SWZ_ROWS16>(i, 2 * g);
   if constexpr (APRE && AGEN == 0) {
     const unsigned a_addr = (unsigned)(size_t)(char LLMMM_LDS*)a_stage;
-    const int      units  = (kb1 - kb0) * 2 * MBLK;
-    for (int u = wave; u < units; u += 8) {
-      const int j = u / (2 * MBLK), within = u - j * (2 * MBLK);
+    auto fetch_unit = [&](int j, int within) {  // 8 rows of slice j
       const int r = within * 8 + (lane >> 3);
       const int c = (lane & 7) ^ kmajor_swz<SWZ_ROWS16>(r);
       const int m = min(m0 + r, M - 1);
       asm_load_lds_16B(A + (size_t)m * K + (size_t)(kb0 + j) * 128 + c * 16, a_addr + j * (MBLK * 2048) + within * 1024);
+    };
+    // K is not split for SwiGLU: whole slices in turn, without the units that hold no row below M (their products are computed and never
+    // stored) -- 12288 x 2048 at M = 4: 9.4 us in single units, 8.8 so.  The short K ranges of the other outputs would leave waves
+    // without a slice (6144 x 2560 in five splits at M = 1: 6.55 / 6.65): single units in turn.
+    if constexpr (SWIGLU) {
+      const int units = min(2 * MBLK, (M - m0 + 7) >> 3);
+      for (int j = wave; j < kb1 - kb0; j += 8) {
+#pragma unroll
+        for (int within = 0; within < 2 * MBLK; ++within)
+          if (within < units) fetch_unit(j, within);
+      }
     }
+    else
+      for (int u = wave; u < (kb1 - kb0) * 2 * MBLK; u += 8) fetch_unit(u / (2 * MBLK), u % (2 * MBLK));
   }
 
   // Software pipeline, D slices in flight per wave, all vector-memory loads issued strictly in
@@ -475,6 +505,50 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
   }
   LLMMM_LAST(0) LLMMM_LAST(1) LLMMM_LAST(2) LLMMM_LAST(3) LLMMM_LAST(4) LLMMM_LAST(5) LLMMM_LAST(6) LLMMM_LAST(7)
 #undef LLMMM_LAST
+
+  if constexpr (SWIGLU) {
+    if (wave >= 4) {
+#pragma unroll
+      for (int mb = 0; mb < MBLK; ++mb) up_part[wave & 3][mb][lane] = acc[mb];
+    }
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll
+      for (int mb = 0; mb < MBLK; ++mb) {
+        const f32x4 up = up_part[wave & 3][mb][lane];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[mb][q] = silu_mul(acc[mb][q], up[q]);
+        float a = fmaxf(fmaxf(fmaxf(0.f, __builtin_fabsf(acc[mb][0])), __builtin_fabsf(acc[mb][1])),
+                        fmaxf(__builtin_fabsf(acc[mb][2]), __builtin_fabsf(acc[mb][3])));
+        a       = wave_xor_max<16>(a);
+        a       = wave_xor_max<32>(a);
+        if (g == 0) wave_amax[wave][mb][i] = a;
+      }
+    }
+    __syncthreads();
+    if (wave >= 4) return;
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(own_mark)::"memory");  // long landed; ties the register to this point
+    const unsigned long long marks = __builtin_amdgcn_ballot_w64(own_mark != 0u);
+    float                    amax[MBLK];
+#pragma unroll
+    for (int mb = 0; mb < MBLK; ++mb) {
+      amax[mb] = fmaxf(fmaxf(wave_amax[0][mb][i], wave_amax[1][mb][i]), fmaxf(wave_amax[2][mb][i], wave_amax[3][mb][i]));
+      if (wave == mb && g == 0) pair.publish((int)(marks >> mb) & 1, mb, i, amax[mb]);
+    }
+    const int n = ng * 64 + wave * 16 + 4 * g;
+#pragma unroll
+    for (int mb = 0; mb < MBLK; ++mb) {
+      const int   m     = m0 + mb * 16 + i;
+      const float a     = fmaxf(amax[mb], pair.other((int)(marks >> mb) & 1, mb, i, &g_pair_xch_timeouts));
+      const float scale = a / 448.f;
+      const float inv   = requant_inv(a);
+      if (m < M) {
+        *(uint32_t*)((uint8_t*)Cv + (size_t)m * (N >> 1) + n) = pack_e4m3x4_in_range(acc[mb][0] * inv, acc[mb][1] * inv, acc[mb][2] * inv, acc[mb][3] * inv);
+        if (wave == 0 && g == 0 && (ng & 1) == 0) Cs[(size_t)(ng >> 1) * M + m] = scale;
+      }
+    }
+    return;
+  }
 
   // lane (g, i): row m = mb*16 + i, columns ncol .. ncol+3
   const int ncol = ng * 128 + wave * 16 + 4 * g;
@@ -851,7 +925,12 @@ hipError_t fp8_strip_fp8q_launch(int b_layout, const void* A, const float* As, c
 // Waves that gave up waiting in the exchange since the library was loaded (0 on a healthy device); synchronises.
 hipError_t strip_exchange_timeouts(unsigned* out)
 {
-  return hipMemcpyFromSymbol(out, HIP_SYMBOL(g_strip_xch_timeouts), sizeof(unsigned), 0, hipMemcpyDeviceToHost);
+  unsigned         n[2] = {0, 0};
+  const hipError_t e    = hipMemcpyFromSymbol(&n[0], HIP_SYMBOL(g_strip_xch_timeouts), sizeof(unsigned), 0, hipMemcpyDeviceToHost);
+  if (e != hipSuccess) return e;
+  const hipError_t f = hipMemcpyFromSymbol(&n[1], HIP_SYMBOL(g_pair_xch_timeouts), sizeof(unsigned), 0, hipMemcpyDeviceToHost);
+  *out               = n[0] + n[1];
+  return f;
 }
 
 template <typename HT>
@@ -877,10 +956,10 @@ hipError_t fp8_strip_add_residual_launch(int hidden_dtype, int b_layout, const v
 
 template <int MBLK, int OUT, int D, int ASTG>
 static hipError_t launch_skinny(const void* A, const float* As, const void* Bt, const float* Bs, void* C, float* Cs, int M,
-                                int N, int K, int S, float* partial, int bpre, hipStream_t stream)
+                                int N, int K, int S, float* partial, int bpre, hipStream_t stream, int xarea = 0)
 {
   hipLaunchKernelGGL((fp8_skinny_kernel<MBLK, OUT, D, ASTG>), dim3(N / 128, S, (M + 16 * MBLK - 1) / (16 * MBLK)), dim3(512), 0, stream,
-                     (const uint8_t*)A, As, (const uint8_t*)Bt, Bs, C, Cs, M, N, K, S, partial, bpre, SkinnyGenA{});
+                     (const uint8_t*)A, As, (const uint8_t*)Bt, Bs, C, Cs, M, N, K, S, partial, bpre, SkinnyGenA{}, xarea);
   return hipGetLastError();
 }
 
@@ -894,7 +973,7 @@ static hipError_t dispatch_skinny_agen(const float* G, const void* Bt, const flo
 #define LLMMM_GO(D, ASTG)                                                                                                                   \
   {                                                                                                                                         \
     hipLaunchKernelGGL((fp8_skinny_kernel<1, OUT, D, ASTG, 1>), dim3(N / 128, S, 1), dim3(512), 0, stream, (const uint8_t*)G, (const float*)nullptr, \
-                       (const uint8_t*)Bt, Bs, C, Cs, M, N, K, S, partial, bpre, SkinnyGenA{});                                            \
+                       (const uint8_t*)Bt, Bs, C, Cs, M, N, K, S, partial, bpre, SkinnyGenA{}, 0);                                            \
     return hipGetLastError();                                                                                                               \
   }
   if (slices >= 8 && need <= 28672) LLMMM_GO(8, 28672);
@@ -924,7 +1003,7 @@ static hipError_t dispatch_skinny_gen2(const SkinnyGenA& ag, const void* Bt, con
 #define LLMMM_GO(D, ASTG)                                                                                                                       \
   {                                                                                                                                             \
     hipLaunchKernelGGL((fp8_skinny_kernel<1, SK_OUT_F32, D, ASTG, 2, HT>), dim3(N / 128, S, 1), dim3(512), 0, stream, (const uint8_t*)nullptr,  \
-                       (const float*)nullptr, (const uint8_t*)Bt, Bs, (void*)C, (float*)nullptr, M, N, K, S, partial, bpre, ag);                \
+                       (const float*)nullptr, (const uint8_t*)Bt, Bs, (void*)C, (float*)nullptr, M, N, K, S, partial, bpre, ag, 0);                \
     return hipGetLastError();                                                                                                                   \
   }
   if (slices >= 8 && need <= 28672) LLMMM_GO(8, 28672);
@@ -990,6 +1069,27 @@ static hipError_t dispatch_skinny(const void* A, const float* As, const void* Bt
   }
 #undef LLMMM_GO
   return hipErrorInvalidValue;
+}
+
+// The SwiGLU output in one launch: K unsplit, the workgroups of a group agreeing on its row maxima through exchange area `xarea`.
+// The activation rows of all of K have to fit the staging area: K <= 5120 up to 16 rows, 2560 up to 32.
+bool fp8_skinny_swiglu_fits(int M, int N, int K)
+{
+  return M >= 1 && N % 256 == 0 && N / 256 <= STRIP_XCH_MAX_GROUPS && K % 128 == 0 && K >= 512 && (M <= 16 ? K <= 5120 : M <= 32 && K <= 2560);
+}
+hipError_t fp8_skinny_swiglu_launch(int b_layout, const void* A, const float* As, const void* Bt, const float* Bs, void* C, float* Cs, int M, int N, int K,
+                                    int xarea, hipStream_t stream)
+{
+  if (!fp8_skinny_swiglu_fits(M, N, K) || xarea < 0 || xarea >= STRIP_XCH_AREAS || !Cs) return hipErrorInvalidValue;
+  const int bpre = b_layout == LLMMM_FP8_B_PRESHUFFLED, KB = K / 128;
+#define LLMMM_GO(MBLK, D, ASTG) return launch_skinny<MBLK, SK_OUT_SWIGLU, D, ASTG>(A, As, Bt, Bs, C, Cs, M, N, K, 1, nullptr, bpre, stream, xarea)
+  if (M <= 16) {
+    if (KB * 2048 <= 65536) LLMMM_GO(1, 4, 65536);
+    LLMMM_GO(1, 4, 81920);
+  }
+  if (KB * 4096 <= 65536) LLMMM_GO(2, 4, 65536);
+  LLMMM_GO(2, 4, 81920);
+#undef LLMMM_GO
 }
 
 hipError_t fp8_skinny_launch(int out_kind, int b_layout, const void* A, const float* As, const void* Bt, const float* Bs, void* C,

@@ -1,0 +1,103 @@
+"""The SwiGLU output of the weight-streaming kernel in one launch (64 gate + 64 up columns per workgroup, row maxima exchanged between
+the two workgroups of a 1x128 group) against the same kernel through an fp32 plane and the reduce kernel: the same sums and the same
+arithmetic, so the same bits."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import fp8_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(t, M, N, K, pre, split=0, out=None, ws=None):
+    from llmmm_amd import _lib
+    C, Cs = out if out else (torch.full((M, N // 2), 0x55, dtype=torch.uint8, device="cuda"), torch.full((N // 256, M), -1.0, device="cuda"))
+    ws = torch.empty(M * N, device="cuda") if ws is None else ws
+    cfg = _lib.GemmCfg(_lib.TILE_AUTO if not split else _lib.TILE_SKINNY, split, 1 if pre else 0, 0)
+    rc = _lib.lib.llmmm_fp8_gemm_ex(_lib.OUT_FP8Q_SWIGLU, t[0].data_ptr(), t[1].data_ptr(), t[2].data_ptr(), t[3].data_ptr(), C.data_ptr(), Cs.data_ptr(), M, N,
+                                    K, ws.data_ptr(), ws.numel() * 4, ctypes.byref(cfg), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.lib.llmmm_last_error().decode()
+    return C, Cs
+
+
+def _same(a, b):
+    return torch.equal(a[0], b[0]) and torch.equal(a[1].view(torch.int32), b[1].view(torch.int32))
+
+
+def _inputs(oracle, M, N, K, seed, pre):
+    import llmmm_amd
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in fp8_inputs(oracle, M, N, K, seed=seed)]
+    return [t[0], t[1], llmmm_amd.preshuffle_weight(t[2]) if pre else t[2], t[3]], t
+
+
+def _timeouts():
+    from llmmm_amd import _lib
+    n = ctypes.c_uint(7)
+    assert _lib.lib.llmmm_probe_strip_exchange_timeouts(ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("N,K", [(12288, 512), (19456, 2560), (32768, 640), (12288, 5120)])
+@pytest.mark.parametrize("pre", [False, True])
+def test_bits_of_the_plane_route(oracle, N, K, pre):
+    t, _ = _inputs(oracle, 32, N, K, 5, pre)
+    for M in (1, 2, 8, 9, 15, 16, 17, 24, 25, 32):
+        s = [t[0][:M].contiguous(), t[1][:, :M].contiguous(), t[2], t[3]]
+        if M <= 16 or K <= 2560:
+            assert _same(_call(s, M, N, K, pre), _call(s, M, N, K, pre, split=1)), M
+    assert _timeouts() == 0
+
+
+def test_launches_that_change_rows_and_shapes(oracle):
+    """Exchange slots are kept per block of 16 rows: launches of other row counts and widths on one stream, other maxima each time."""
+    cases = []
+    for i, (M, N, K) in enumerate([(1, 12288, 512), (32, 19456, 512), (16, 12288, 640), (17, 32768, 512), (3, 19456, 512), (32, 12288 + 4096, 512)]):
+        t, _ = _inputs(oracle, M, N, K, 10 + i, False)
+        t[1] = t[1] * (2.0 ** i)
+        cases.append((t, M, N, K, _call(t, M, N, K, False, split=1)))
+    outs = [[(torch.empty_like(c[4][0]), torch.empty_like(c[4][1])) for c in cases] for _ in range(4)]
+    ws = torch.empty(32 * 32768, device="cuda")
+    for o in outs:
+        for c, out in zip(cases, o):
+            _call(c[0], c[1], c[2], c[3], False, out=out, ws=ws)
+    for o in outs:
+        assert all(_same(x, c[4]) for x, c in zip(o, cases))
+    assert _timeouts() == 0
+
+
+def test_captured_with_other_work_between_replays(oracle):
+    M, N, K = 16, 12288, 512
+    t, _ = _inputs(oracle, M, N, K, 3, False)
+    out, ws = (torch.empty((M, N // 2), dtype=torch.uint8, device="cuda"), torch.empty((N // 256, M), device="cuda")), torch.empty(M * N, device="cuda")
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        _call(t, M, N, K, False, out=out, ws=ws)
+    side.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        for _ in range(3):
+            _call(t, M, N, K, False, out=out, ws=ws)
+    for rep in range(4):
+        t[1].mul_(3.0)
+        want = _call(t, M, N, K, False, split=1)
+        out[0].fill_(0)
+        out[1].fill_(0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert _same(out, want), rep
+    assert _timeouts() == 0
+
+
+def test_non_finite_operands(oracle):
+    M, N, K = 5, 12288, 512
+    t, _ = _inputs(oracle, M, N, K, 4, False)
+    t[0][1, 7] = 0x7F            # NaN code
+    t[1][2, 3] = float("inf")
+    t[1][:, 4] = 0.0             # a row of zeros
+    t[0][2] = 0
+    a, b = _call(t, M, N, K, False), _call(t, M, N, K, False, split=1)
+    assert torch.equal(a[0], b[0]) and torch.equal(torch.nan_to_num(a[1], nan=-2.0), torch.nan_to_num(b[1], nan=-2.0))
