@@ -866,7 +866,12 @@ int llmmm_fp8_gemm_ex(int out_kind, const void* A, const float* As, const void* 
       if (!aligned16(workspace)) return fail(LLMMM_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
       planes = (float*)workspace;
     }
-    e = llmmm::fp8_gemm_launch(out_kind, cfg.tile, cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, split, planes, (hipStream_t)stream);
+    int pair_area;
+    if (swiglu && cfg.tile == LLMMM_TILE_128x128 && split <= 1 && !(user && user->split_k > 0) && llmmm::fp8_gemm_swiglu_pair_fits(M, N, K) &&
+        (pair_area = strip_exchange_area(stream)) >= 0)
+      e = llmmm::fp8_gemm_swiglu_pair_launch(cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, pair_area, (hipStream_t)stream);
+    else
+      e = llmmm::fp8_gemm_launch(out_kind, cfg.tile, cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, split, planes, (hipStream_t)stream);
   }
   if (e != hipSuccess) return fail(LLMMM_ERR_RUNTIME, "fp8 gemm launch: %s", hipGetErrorString(e));
   return LLMMM_OK;

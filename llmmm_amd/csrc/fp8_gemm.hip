@@ -37,7 +37,13 @@ enum { OUT_F32 = 0, OUT_BF16 = 1, OUT_FP8Q = 2, OUT_SWIGLU = 3,
        // internal: the bf16 / e4m3 epilogues behind the per-head RMSNorm + RoPE of a QKV projection (Fp8HeadOp)
        OUT_ROPE_BF16 = 4, OUT_ROPE_FP8Q = 5,
        // internal: hidden = T(C + residual), T = float / bf16 / fp16 (Fp8HeadOp::residual, the output goes to Cv)
-       OUT_ADD_F32 = 6, OUT_ADD_BF16 = 7, OUT_ADD_F16 = 8 };
+       OUT_ADD_F32 = 6, OUT_ADD_BF16 = 7, OUT_ADD_F16 = 8,
+       // internal: OUT_SWIGLU from 128 x 128 tiles of 64 gate and the matching 64 up columns (one tile row, deep pipeline)
+       OUT_SWIGLU_PAIR = 9 };
+
+// Where the workgroups of OUT_SWIGLU_PAIR exchange their row maxima (PairSlots).
+static __device__ unsigned g_tile_pair_xch[STRIP_XCH_AREAS][2 * STRIP_XCH_MAX_GROUPS * PAIR_BLOCKS * 2 * 16];
+static __device__ unsigned g_tile_pair_timeouts;
 
 __device__ __forceinline__ f32x4 mfma_fp8_k128(i32x8 x, i32x8 y)
 {
@@ -180,7 +186,8 @@ __device__ __forceinline__ void fp8_scale_load_lds(const char* lane_ptr, unsigne
 // steps (spread, so that no wave sits in the memory pipeline's issue queue while its matrix
 // work waits, and early enough to land within the slice), its scales during the fifth.
 // 160-column waves (NF = 10): fragments nf < nfb lie in the first weight-scale block and take s, the others s2.
-template <int BM, int BN, int WM, bool BNT, bool LOAD, bool SCALE_LDS = false, bool MT = false>
+// PAIR: 64 gate and 64 up columns, fragments 0 .. 3 and 4 .. 7: s and s2 likewise.
+template <int BM, int BN, int WM, bool BNT, bool LOAD, bool SCALE_LDS = false, bool MT = false, bool PAIR = false>
 __device__ __forceinline__ void fp8_compute_stage(const char LLMMM_LDS* lds, int a_rd0, int a_rd1, int b_rd0, int b_rd1,
                                                   const float (&s)[WM / 16], f32x4 (&acc)[Fp8Tile<BM, BN, WM>::NF][WM / 16], const Fp8Next& nx, unsigned lane_off,
                                                   unsigned b_lane_off, unsigned row_off, unsigned zero, int K, size_t b_hi, int wave, float (&sa_next)[WM / 16],
@@ -189,7 +196,8 @@ __device__ __forceinline__ void fp8_compute_stage(const char LLMMM_LDS* lds, int
   constexpr int MF = WM / 16;
   typedef Fp8Tile<BM, BN, WM> TC;
   constexpr int  NF  = TC::NF;
-  constexpr bool TWO = NF != 8;
+  constexpr bool TWO = NF != 8 || PAIR;
+  static_assert(!PAIR || SCALE_LDS, "the pair's scales travel with the stage");
   constexpr int           NL   = TC::A_LOADS + TC::B_LOADS;
   constexpr int           LPG  = (NL + 3) / 4;
   const char LLMMM_LDS*   ldsA = lds;
@@ -423,6 +431,8 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   constexpr int  MF   = TC::MF;
   constexpr int  NF   = TC::NF;
   constexpr bool TWO  = NF != 8;  // 160-column waves straddle two weight-scale blocks
+  constexpr bool PAIR = OUT == OUT_SWIGLU_PAIR;
+  static_assert(!PAIR || (BM == 128 && BN == 128 && WM == 32 && (BMODE & 4) != 0), "gate / up pairs: deep 128 x 128 tiles");
   static_assert(!TWO || (OUT == OUT_F32 || OUT == OUT_BF16 || OUT == OUT_ADD_F32 || OUT == OUT_ADD_BF16 || OUT == OUT_ADD_F16),
                 "the 160-column tile has no 1x128-grouped epilogues");
   constexpr bool BPRE = (BMODE & 1) != 0, BNT = (BMODE & 2) != 0;
@@ -441,7 +451,7 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   unsigned long long wait_cycles = 0;  // STAMP: shader cycles this wave spent in the K loop's "loads landed + barrier" waits (slices 1 ..)
   unsigned long long load_wait_cycles = 0;  // ... of which for its own loads (the rest: for the other waves at the barrier)
   if constexpr (STAMP) ph[0] = phase_clock();
-  static_assert(!MT || (DEEP && BM == 128 && BN == 128 && (OUT == OUT_F32 || OUT == OUT_BF16 || OUT == OUT_FP8Q)), "row tails: deep 128 x 128 tiles only");
+  static_assert(!MT || (DEEP && BM == 128 && BN == 128 && (OUT == OUT_F32 || OUT == OUT_BF16 || OUT == OUT_FP8Q || PAIR)), "row tails: deep 128 x 128 tiles only");
   constexpr int  STAGE_D = TC::STAGE + TC::NW * 256;                 // operands + 256 bytes of scales per wave
   constexpr int  NST     = !DEEP ? 2 : (4 * STAGE_D <= 160 * 1024 ? 4 : 3);
   static_assert(fp8_lds_bytes<BM, BN, WM, BMODE>() == (DEEP ? NST * STAGE_D : 2 * TC::STAGE), "the kernels size the buffers with fp8_lds_bytes");
@@ -452,13 +462,14 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   const int wm   = wave % TC::WAVES_M;
   const int wn   = wave / TC::WAVES_M;
   int       tm, tn;
-  tile_coords(tile_index, tiles_m, tiles_n, tm, tn, splits_in_turn<BN>(gridDim.y, tiles_m, tiles_n, K));
+  tile_coords(tile_index, tiles_m, tiles_n, tm, tn, PAIR || splits_in_turn<BN>(gridDim.y, tiles_m, tiles_n, K));
+  // (PAIR: tile = workgroup id, one tile row -- a pair's ids are 2j and 2j + 1, which PairSlots relies on)
   // SwiGLU output: the tile's two 128-column halves are the gate columns n0 .. n0+127 and the up columns
   // N/2 + n0 .. of the same 128 output columns, so the weight rows of the upper half start N/2 - 128 rows further on
   constexpr bool SWIGLU = OUT == OUT_SWIGLU;
   static_assert(!SWIGLU || BN == 256, "the SwiGLU epilogue pairs the two 128-column halves of a 256-wide tile");
-  const int    m0   = tm * BM, n0 = n_base + (SWIGLU ? tn * 128 : tn * BN);
-  const size_t b_hi = SWIGLU ? (size_t)((N >> 1) - 128) * K : 0;
+  const int    m0   = tm * BM, n0 = n_base + (SWIGLU ? tn * 128 : PAIR ? tn * 64 : tn * BN);
+  const size_t b_hi = SWIGLU || PAIR ? (size_t)((N >> 1) - BN / 2) * K : 0;
   const int    KB   = K >> 7;
   // split-K: gridDim.y workgroups share a tile, each taking a contiguous run of slices and (the
   // host only splits the fp32 instantiation) writing its partial sums to its own [M, N] plane
@@ -495,8 +506,8 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   const float*   Bsp     = Bs + (size_t)((n0 >> 7) + (SWIGLU ? wn * (N >> 8) : wn)) * KB + kb0;
   // 160-column waves: columns n0 .. n0+159 lie in weight-scale blocks n0/128 and n0/128 + 1; the first nfb fragments
   // (16 columns each) belong to the former
-  const float*   Bsp2    = Bsp + (TWO ? KB : 0);
-  const int      nfb     = TWO ? (128 - (n0 & 127)) >> 4 : NF;
+  const float*   Bsp2    = Bsp + (TWO ? KB : PAIR ? (size_t)(N >> 8) * KB : 0);
+  const int      nfb     = TWO ? (128 - (n0 & 127)) >> 4 : PAIR ? 4 : NF;
   const float*   Asl     = As + (size_t)kb0 * M;
   unsigned       zero    = 0;
   asm volatile("" : "+v"(zero));  // a VGPR holding 0: the per-lane offset of the wave-uniform Bs load
@@ -504,6 +515,11 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
 
   const unsigned lds0 = (unsigned)(size_t)(char LLMMM_LDS*)lds;
   char LLMMM_LDS* const s0 = (char LLMMM_LDS*)lds;
+
+  // PAIR: which exchange buffer is next, lane l for the wave's 16-row block l % 2; the oldest load in flight, looked at in the epilogue
+  unsigned        own_mark = 0u;
+  const PairSlots pair     = {PAIR ? &g_tile_pair_xch[op.xarea][0] : nullptr, STRIP_XCH_MAX_GROUPS, tn >> 1, tn & 1};
+  if constexpr (PAIR) asm volatile("global_load_dword %0, %1, off sc1" : "=v"(own_mark) : "v"(pair.slot(0, wm * MF + (lane & 1), tn & 1)) : "memory");
 
   if constexpr (DEEP) {
     constexpr int PER = TC::A_LOADS + TC::B_LOADS + 1;  // vector-memory loads of a wave per slice
@@ -513,7 +529,7 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
     static_assert((NST - 2) * PER < 64, "vmcnt is a 6-bit counter");
     // this lane's scale source: a row scale (stride M floats per slice) or the column-group scale (stride 1)
     const bool     row_lane = lane < WM;
-    const char*    sc_ptr   = row_lane ? (const char*)(Asl + (MT ? min(m0 + wm * WM + lane, M - 1) : m0 + wm * WM + lane)) : (const char*)(TWO && lane >= 48 ? Bsp2 : Bsp);
+    const char*    sc_ptr   = row_lane ? (const char*)(Asl + (MT ? min(m0 + wm * WM + lane, M - 1) : m0 + wm * WM + lane)) : (const char*)((TWO || PAIR) && lane >= 48 ? Bsp2 : Bsp);
     const unsigned sc_step  = row_lane ? (unsigned)M * 4u : 4u;
     // prologue: slices 0 .. NST-2 (a K range shorter than that repeats its last slice into the spare stages)
 #pragma unroll
@@ -545,7 +561,7 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
     nx.Bs_elem   = nullptr;                                                                                                       \
     nx.Bs_elem2  = nullptr;                                                                                                       \
     nx.sc_ptr    = sc_next;                                                                                                       \
-    fp8_compute_stage<BM, BN, WM, BNT, LOAD, true, MT>(s0 + cur, a_rd0, a_rd1, b_rd0, b_rd1, s, acc, nx, lane_off, b_lane_off, row_off, zero, K, \
+    fp8_compute_stage<BM, BN, WM, BNT, LOAD, true, MT, PAIR>(s0 + cur, a_rd0, a_rd1, b_rd0, b_rd1, s, acc, nx, lane_off, b_lane_off, row_off, zero, K, \
                                                        b_hi, wave, sa_next, sb_next, s2, nfb, sb2_next, a_tail);                  \
     cur = cur + STAGE_D == NST * STAGE_D ? 0 : cur + STAGE_D;                                                                     \
   }
@@ -721,6 +737,52 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
       const int   r = 4 * j + (lane >> 4), c = lane & 15;
       const i32x4 v = *(const i32x4 LLMMM_LDS*)(stg + r * 256 + ((c ^ (r & 15)) << 4));
       if (!MT || row0 + r < M) *(i32x4*)(C + (size_t)(row0 + r) * N + col0 + c * 8) = v;
+    }
+  }
+  else if constexpr (PAIR) {
+    // What bounded the SwiGLU output of one row of 128 x 128 tiles behind its K loop was the fp32 plane: 7.8 MB written and read again and a second
+    // launch at 100 x 19456.  us, plane + reduce / this: 19456 x 2560 21.7 / 18.4 at M = 48, 25.4 / 20.3 at 100, 25.9 / 20.6 at 128; 28672 x 4096
+    // 35.8 / 28.1 at 100; 12288 x 2048 17.7 / 14.2 at 100.
+    // Lane (g, li) holds the gate value of column nf*16 + 4g + q in acc[nf] and the up value of the same output in acc[nf + 4]: nothing
+    // moves between waves; the group's other 64 columns are the neighbouring workgroup's.
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(own_mark)::"memory");  // long landed; ties the register to this point
+    const unsigned long long marks = __builtin_amdgcn_ballot_w64(own_mark != 0u);
+    float                    amax[MF];
+#pragma unroll
+    for (int mf = 0; mf < MF; ++mf) {
+      if (row0 + mf * 16 >= M) continue;  // (wave-uniform: no row of the block exists, in either half)
+      float a = 0.f;
+#pragma unroll
+      for (int nf = 0; nf < 4; ++nf)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          acc[nf][mf][q] = silu_mul(acc[nf][mf][q], acc[nf + 4][mf][q]);
+          a              = fmaxf(a, __builtin_fabsf(acc[nf][mf][q]));
+        }
+      a        = wave_xor_max<16>(a);
+      amax[mf] = wave_xor_max<32>(a);
+      if (g == 0) pair.publish((int)(marks >> mf) & 1, wm * MF + mf, li, amax[mf]);
+    }
+    uint8_t* C = (uint8_t*)Cv;
+#pragma unroll
+    for (int mf = 0; mf < MF; ++mf) {
+      if (row0 + mf * 16 >= M) continue;
+      const float a     = fmaxf(amax[mf], pair.other((int)(marks >> mf) & 1, wm * MF + mf, li, &g_tile_pair_timeouts));
+      const float scale = a / 448.f;
+      const float inv   = requant_inv(a);
+      const int   r     = mf * 16 + li;
+#pragma unroll
+      for (int nf = 0; nf < 4; ++nf) {
+        const f32x4 v = acc[nf][mf];
+        *(uint32_t LLMMM_LDS*)(stg + r * 64 + ((nf ^ ((r >> 2) & 3)) << 4) + 4 * g) = pack_e4m3x4_in_range(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
+      }
+      if (g == 0 && (tn & 1) == 0 && (!MT || row0 + r < M)) Cs[(size_t)(tn >> 1) * M + row0 + r] = scale;
+    }
+#pragma unroll
+    for (int j = 0; j < WM / 16; ++j) {
+      const int   r = 16 * j + (lane >> 2), c = lane & 3;
+      const i32x4 v = *(const i32x4 LLMMM_LDS*)(stg + r * 64 + ((c ^ ((r >> 2) & 3)) << 4));
+      if (!MT || row0 + r < M) *(i32x4*)(C + (size_t)(row0 + r) * (N >> 1) + n0 + c * 16) = v;
     }
   }
   else if constexpr (OUT == OUT_SWIGLU) {
@@ -1094,6 +1156,21 @@ hipError_t fp8_gemm_launch(int out_kind, int tile, int b_layout, const void* A, 
     default: return hipErrorInvalidValue;
   }
 }
+
+bool fp8_gemm_swiglu_pair_fits(int M, int N, int K) { return M >= 1 && M <= 128 && N % 256 == 0 && N / 256 <= STRIP_XCH_MAX_GROUPS && K % 128 == 0 && K >= 128; }
+hipError_t fp8_gemm_swiglu_pair_launch(int b_layout, const void* A, const float* As, const void* Bt, const float* Bs, void* C, float* Cs, int M, int N, int K,
+                                       int xarea, hipStream_t stream)
+{
+  if (!fp8_gemm_swiglu_pair_fits(M, N, K) || xarea < 0 || xarea >= STRIP_XCH_AREAS || !Cs) return hipErrorInvalidValue;
+  const bool bpre   = b_layout == LLMMM_FP8_B_PRESHUFFLED;
+  const auto kernel = M == 128 ? (bpre ? fp8_gemm_kernel<128, 128, 32, OUT_SWIGLU_PAIR, 7> : fp8_gemm_kernel<128, 128, 32, OUT_SWIGLU_PAIR, 6>)
+                               : (bpre ? fp8_gemm_kernel<128, 128, 32, OUT_SWIGLU_PAIR, 15> : fp8_gemm_kernel<128, 128, 32, OUT_SWIGLU_PAIR, 14>);
+  Fp8HeadOp op;
+  op.xarea = xarea;
+  hipLaunchKernelGGL(kernel, dim3(N / 128), dim3(Fp8Tile<128, 128, 32>::NT), 0, stream, (const uint8_t*)A, As, (const uint8_t*)Bt, Bs, C, Cs, M, N, K, 1, N / 128, op);
+  return hipGetLastError();
+}
+hipError_t tile_pair_timeouts(unsigned* out) { return hipMemcpyFromSymbol(out, HIP_SYMBOL(g_tile_pair_timeouts), sizeof(unsigned), 0, hipMemcpyDeviceToHost); }
 
 hipError_t fp8_gemm_phases_launch(const void* A, const float* As, const void* Bt, const float* Bs, void* C, float* Cs, int M, int N, int K,
                                   unsigned long long* stamps, hipStream_t stream)

@@ -925,12 +925,12 @@ hipError_t fp8_strip_fp8q_launch(int b_layout, const void* A, const float* As, c
 // Waves that gave up waiting in the exchange since the library was loaded (0 on a healthy device); synchronises.
 hipError_t strip_exchange_timeouts(unsigned* out)
 {
-  unsigned         n[2] = {0, 0};
-  const hipError_t e    = hipMemcpyFromSymbol(&n[0], HIP_SYMBOL(g_strip_xch_timeouts), sizeof(unsigned), 0, hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return e;
-  const hipError_t f = hipMemcpyFromSymbol(&n[1], HIP_SYMBOL(g_pair_xch_timeouts), sizeof(unsigned), 0, hipMemcpyDeviceToHost);
-  *out               = n[0] + n[1];
-  return f;
+  unsigned   n[3] = {0, 0, 0};
+  hipError_t e    = hipMemcpyFromSymbol(&n[0], HIP_SYMBOL(g_strip_xch_timeouts), sizeof(unsigned), 0, hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = hipMemcpyFromSymbol(&n[1], HIP_SYMBOL(g_pair_xch_timeouts), sizeof(unsigned), 0, hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = tile_pair_timeouts(&n[2]);
+  *out = n[0] + n[1] + n[2];
+  return e;
 }
 
 template <typename HT>

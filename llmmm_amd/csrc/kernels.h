@@ -39,8 +39,15 @@ struct Fp8HeadOp {
   int          n_q        = 0;
   int          n_kv       = 0;
   const void*  residual   = nullptr;  // fp8_gemm_add_residual_launch only: [M, N] of the hidden dtype
+  int          xarea      = 0;        // fp8_gemm_swiglu_pair_launch only: the exchange area
   unsigned long long* stamps = nullptr;  // fp8_gemm_phases_launch only: PHASE_STAMPS clock readings per wave (see there)
 };
+// One row of 128 x 128 tiles, each 64 gate and the matching 64 up columns, with the SwiGLU output in its epilogue: the two workgroups of
+// a 1x128 group exchange row maxima through area `xarea` (0 .. STRIP_XCH_AREAS - 1; launches that share one must not overlap).  M <= 128.
+bool       fp8_gemm_swiglu_pair_fits(int M, int N, int K);
+hipError_t fp8_gemm_swiglu_pair_launch(int b_layout, const void* A, const float* As, const void* Bt, const float* Bs, void* C, float* Cs, int M, int N, int K,
+                                       int xarea, hipStream_t stream);
+hipError_t tile_pair_timeouts(unsigned* out);
 // A tile kernel (no split) with the head op in its epilogue; out_kind LLMMM_OUT_BF16 or LLMMM_OUT_FP8Q.
 hipError_t fp8_gemm_qk_rope_launch(int out_kind, int tile, int b_layout, const void* A, const float* As, const void* Bt, const float* Bs, void* C,
                                    float* Cs, int M, int N, int K, const Fp8HeadOp& op, hipStream_t stream);
