@@ -480,6 +480,16 @@ int strip_exchange_area(void* stream)
   return used++;
 }
 
+// The QKV projection with per-head norm and rotary embedding (bf16) in column strips, one launch (ST_OUT_ROPE in fp8_skinny.hip): one
+// strip of 32 columns per CU at most -- 10240 columns are 320, 5120 of K at M = 1: 12.8 split + second kernel / 14.3 so -- and few rows, every strip
+// reading all of them (us, split + second kernel / so: 6144 x 2560 6.9 / 6.3 at M = 1, 7.4 / 7.1 at 8, 7.3 / 8.2 at 12; 4096 x 2048 5.9 / 5.4,
+// 6.0 / 6.1, 6.2 / 6.0; 7168 x 5120 11.4 / 9.4, 11.8 / 10.0, 11.6 / 11.0 and 11.8 / 12.4 at 16; 6144 x 4096 9.2 / 8.1, 9.4 / 8.5, 9.3 / 8.8, 9.7 / 9.0).
+bool rope_strips_pay(int M, int N, int K)
+{
+  return K / 128 >= 8 && N / 128 <= llmmm::STRIP_XCH_MAX_GROUPS && N / 32 <= NUM_CUS &&
+         (M <= 8 || (M <= 16 && (long)M * K <= 65536 && (long)N * K >= 24000000L));
+}
+
 // The SwiGLU output of the weight-streaming kernel in one launch (64 gate + 64 up columns per workgroup, K unsplit; figures in
 // fp8_skinny.hip).  Its N / 128 workgroups have to fill the chip or a good part of its last round: with fewer, splitting K pulls more
 // (12288 x 2048, 96 workgroups, M = 24: 9.4 in two splits + reduce / 9.9 so), and 272 or 296 run a nearly empty second round
@@ -1209,6 +1219,16 @@ int llmmm_fp8_gemm_qkv_rope(int out_kind, const void* A, const float* As, const 
   PlaneCfg pc;
   int      rc = resolve_plane_cfg(A, As, Bt, Bs, M, N, K, workspace, workspace_bytes, user, true, &pc, stream, false);
   if (rc) return rc;
+  int area;
+  if (out_kind == LLMMM_OUT_BF16 && pc.skinny && !pc.prep.agen && !(user && (user->split_k > 0 || user->tile != LLMMM_TILE_AUTO)) && rope_strips_pay(M, N, K) &&
+      (area = strip_exchange_area(stream)) >= 0) {
+    llmmm::Fp8HeadOp op;
+    op.qw = q_norm_weight, op.kw = k_norm_weight, op.cos_t = cos_table, op.sin_t = sin_table, op.pos = positions;
+    op.eps = eps, op.table_rows = table_rows, op.n_q = n_q_heads, op.n_kv = n_kv_heads;
+    const hipError_t e = llmmm::fp8_strip_rope_launch(pc.b_layout, A, As, Bt, Bs, out, M, N, K, op, area, (hipStream_t)stream);
+    if (e != hipSuccess) return fail(LLMMM_ERR_RUNTIME, "fp8 gemm + qk-norm + rope launch: %s", hipGetErrorString(e));
+    return LLMMM_OK;
+  }
   if (pc.tile == LLMMM_TILE_128x160) return fail(LLMMM_ERR_INVALID_ARGUMENT, "the 128 x 160 tile cannot hold whole heads");
   if (pc.split == 0) {  // a tile kernel without split: norm and rope run on the accumulators, no planes
     llmmm::Fp8HeadOp op;

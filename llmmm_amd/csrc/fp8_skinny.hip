@@ -654,7 +654,16 @@ constexpr unsigned long long XCH_SPIN_TICKS = 2000000ull;  // 20 ms
 static __device__ unsigned   g_strip_xch[XCH_AREAS][2][XCH_GROUPS][8][16];
 static __device__ unsigned   g_strip_xch_timeouts;
 
-enum { ST_OUT_F32 = 0, ST_OUT_BF16 = 1, ST_OUT_ADD = 2, ST_OUT_FP8Q = 3 };
+// ST_OUT_ROPE: the bf16 output behind a QKV projection's per-head RMSNorm and rotary embedding (Fp8HeadOp).  A strip is then the 16 columns
+// 16 f .. of a head and their rotation partners 64 further on (f = 0 .. 3), so the rotation stays inside the workgroup, and the norm's sum of
+// squares -- a butterfly over the head's 32 four-column chunks in the order 16, 8, 4, 2, 1 -- needs the other three strips only for the
+// steps 8 and 4: every strip publishes its four sums behind step 16 (16 rows x 4 floats) and adds the others' in the fixed order, so
+// the bits are those of the kernel behind planes.  Slots, buffers and waiting as above, in an area of their own; strips of a value head
+// or without norm weights exchange nothing, and then none of the head's four does.
+// Against the split-K form with its second kernel: one launch, no planes (us, device: see rope_strips_pay in capi.cpp).
+static __device__ unsigned g_rope_xch[XCH_AREAS][2][XCH_GROUPS][4][64];
+
+enum { ST_OUT_F32 = 0, ST_OUT_BF16 = 1, ST_OUT_ADD = 2, ST_OUT_FP8Q = 3, ST_OUT_ROPE = 4 };
 
 // The maximum with lane l ^ MASK around the exchange: LDS-crossbar swizzles and a selected half swap.  The register-only steps of
 // wave_xor_max are shorter and the launch gets longer with them, in either of the two places (6144 x 2560, us, this form /
@@ -679,8 +688,10 @@ __device__ __forceinline__ float exchange_max(float v)
 template <int MBLK, int OUT, int D, bool TAIL, typename HT, int CF = 1>
 __global__ void __launch_bounds__(512)
 fp8_strip_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Bt, const float* __restrict__ Bs,
-                 void* __restrict__ Cv, const HT* __restrict__ residual, int M, int N, int K, int bpre, float* __restrict__ Cs, int xarea)
+                 void* __restrict__ Cv, const HT* __restrict__ residual, int M, int N, int K, int bpre, float* __restrict__ Cs, int xarea, Fp8HeadOp op)
 {
+  constexpr bool ROPE = OUT == ST_OUT_ROPE;
+  static_assert(!ROPE || (MBLK == 1 && CF == 2), "a rotary strip: 16 rows, two fragments of one head");
   static_assert(OUT != ST_OUT_FP8Q || MBLK == 1, "the exchange handles one 16-row block");
   static_assert(CF == 1 || CF == 2, "16 or 32 columns per workgroup");
   constexpr int KS = 8 / CF;  // K ranges per column fragment
@@ -701,7 +712,7 @@ fp8_strip_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, co
   const int i    = lane & 15;
   const int cf   = wave % CF;            // the wave's column fragment
   const int ks   = wave / CF;            // ... and its K range
-  const int n0   = blockIdx.x * 16 * CF + 16 * cf;  // the wave's first column
+  const int n0   = ROPE ? (blockIdx.x >> 2) * 128 + (blockIdx.x & 3) * 16 + 64 * cf : blockIdx.x * 16 * CF + 16 * cf;  // the wave's first column
   const int KB   = K >> 7;
   // K is dealt in whole slices: every wave takes q = KB / KS consecutive slices through its ring (q >= 1: the host checks
   // KB >= 8), and the KB % KS slices behind them go one each to the first K ranges as a "tail" slice, requested before
@@ -749,6 +760,8 @@ fp8_strip_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, co
     asm volatile("global_load_dword %0, %1, off sc1" : "=v"(own_mark) : "v"(&g_strip_xch[xarea][0][frag >> 3][frag & 7][0]) : "memory");
   }
 
+  if constexpr (ROPE) asm volatile("global_load_dword %0, %1, off sc1" : "=v"(own_mark) : "v"(&g_rope_xch[xarea][0][blockIdx.x >> 2][blockIdx.x & 3][0]) : "memory");
+
   // the tail slice first (the oldest loads in flight: landed whenever a ring slot has), then the wave's q slices through
   // its ring, D in flight (the pipeline of fp8_skinny_kernel)
   SkinnySlot<MBLK, false> tslot;
@@ -789,6 +802,77 @@ fp8_strip_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, co
 #pragma unroll
   for (int mb = 0; mb < MBLK; ++mb) part[wave][mb][lane] = acc[mb];
   __syncthreads();
+  if constexpr (ROPE) {
+    if (wave != 0) return;
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(own_mark)::"memory");  // long landed; ties the register to this point
+    f32x4 x[2];  // the lane's four columns and their rotation partners, row i
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      x[c] = part[c][0][lane];
+#pragma unroll
+      for (int w = 1; w < KS; ++w) x[c] += part[w * CF + c][0][lane];
+    }
+    const int  head = blockIdx.x >> 2, f = blockIdx.x & 3, row = min(i, M - 1);
+    const bool rotate = head < op.n_q + op.n_kv;
+    const int  angle = 16 * f + 4 * g;
+    f32x4      cs = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
+    if (rotate) {
+      const int p = min(max(op.pos[row], 0), op.table_rows - 1);
+      cs = *(const f32x4*)(op.cos_t + (size_t)p * 64 + angle), sn = *(const f32x4*)(op.sin_t + (size_t)p * 64 + angle);
+    }
+    const float* nw = head < op.n_q ? op.qw : (rotate ? op.kw : nullptr);
+    if (nw != nullptr) {
+      const f32x4 w0 = *(const f32x4*)(nw + angle), w1 = *(const f32x4*)(nw + 64 + angle);
+      float       s16[2];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        s16[c] = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s16[c] = __builtin_fmaf(x[c][q], x[c][q], s16[c]);
+      }
+      const float mine = s16[0] + s16[1];
+      const int   cur  = own_mark != 0u ? 1 : 0;  // (lane-uniform)
+      __hip_atomic_store(&g_rope_xch[xarea][cur ^ 1][head][f][lane], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // (one NaN for all of them: a slot must not become 0)
+      __hip_atomic_store(&g_rope_xch[xarea][cur][head][f][lane], (mine != mine ? 0x7fc00000u : __builtin_bit_cast(unsigned, mine)) + 1u, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+      unsigned                 u[4];
+      const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+      for (;;) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) u[k] = __hip_atomic_load(&g_rope_xch[xarea][cur][head][k][lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_ballot_w64(u[0] == 0u || u[1] == 0u || u[2] == 0u || u[3] == 0u) == 0ull) break;
+        if (__builtin_amdgcn_s_memrealtime() - t0 > XCH_SPIN_TICKS) {
+          if (lane == 0) atomicAdd(&g_strip_xch_timeouts, 1u);
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      float q[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) q[k] = __builtin_bit_cast(float, u[k] - 1u);
+      float t = (q[0] + q[2]) + (q[1] + q[3]);  // steps 8 and 4
+      t       = wave_xor_sum<32>(t);            // 2
+      t       = wave_xor_sum<16>(t);            // 1
+      const float r = 1.0f / __builtin_sqrtf(t / 128.0f + op.eps);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[0][e] = (x[0][e] * r) * w0[e], x[1][e] = (x[1][e] * r) * w1[e];
+    }
+    if (rotate) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float lo = x[0][e], hi = x[1][e], t1 = hi * sn[e], t2 = lo * sn[e];
+        x[0][e] = __builtin_fmaf(lo, cs[e], -t1);
+        x[1][e] = __builtin_fmaf(hi, cs[e], t2);
+      }
+    }
+    if (i < M) {
+      __bf16* o = (__bf16*)Cv + (size_t)i * N + head * 128 + angle;
+      store_row4<__bf16>(o, x[0]);
+      store_row4<__bf16>(o + 64, x[1]);
+    }
+    return;
+  }
   if (wave >= MBLK * CF) return;  // wave mb * CF + c finishes column fragment c of the 16-row block mb
   const int mb = wave / CF;       // (wave % CF = cf: the fragment whose K ranges this wave summed one of)
   f32x4     v  = part[cf][mb][lane];
@@ -861,7 +945,7 @@ int strip_fragments(int N, int K)
 }
 template <int MBLK, int OUT, typename HT, int CF>
 static hipError_t launch_strip_cf(const void* A, const float* As, const void* Bt, const float* Bs, void* C, const void* residual, int M, int N, int K, int bpre,
-                                  hipStream_t stream, float* Cs, int xarea)
+                                  hipStream_t stream, float* Cs, int xarea, const Fp8HeadOp& op = Fp8HeadOp{})
 {
   constexpr int KS = 8 / CF;
   const int  q = (K / 128) / KS;
@@ -875,10 +959,10 @@ static hipError_t launch_strip_cf(const void* A, const float* As, const void* Bt
 #define LLMMM_GO(D)                                                                                                                                         \
   if (tail)                                                                                                                                                 \
     hipLaunchKernelGGL((fp8_strip_kernel<MBLK, OUT, D, true, HT, CF>), grid, block, 0, stream, (const uint8_t*)A, As, (const uint8_t*)Bt, Bs, C, (const HT*)residual, \
-                       M, N, K, bpre, Cs, xarea);                                                                                                           \
+                       M, N, K, bpre, Cs, xarea, op);                                                                                                       \
   else                                                                                                                                                      \
     hipLaunchKernelGGL((fp8_strip_kernel<MBLK, OUT, D, false, HT, CF>), grid, block, 0, stream, (const uint8_t*)A, As, (const uint8_t*)Bt, Bs, C, (const HT*)residual, \
-                       M, N, K, bpre, Cs, xarea)
+                       M, N, K, bpre, Cs, xarea, op)
   if (best == 4) {
     LLMMM_GO(4);
   }
@@ -920,6 +1004,15 @@ hipError_t fp8_strip_fp8q_launch(int b_layout, const void* A, const float* As, c
 {
   if (M < 1 || M > 16 || N % 128 || N / 128 > XCH_GROUPS || K % 128 || K / 128 < 8 || xarea < 0 || xarea >= XCH_AREAS || !Cs) return hipErrorInvalidValue;
   return launch_strip<1, ST_OUT_FP8Q, float>(A, As, Bt, Bs, C, nullptr, M, N, K, b_layout == LLMMM_FP8_B_PRESHUFFLED, stream, Cs, xarea);
+}
+
+// The bf16 output behind per-head RMSNorm and rotary embedding (M <= 16, at most STRIP_XCH_MAX_GROUPS heads).
+hipError_t fp8_strip_rope_launch(int b_layout, const void* A, const float* As, const void* Bt, const float* Bs, void* C, int M, int N, int K, const Fp8HeadOp& op,
+                                 int xarea, hipStream_t stream)
+{
+  if (M < 1 || M > 16 || N != (op.n_q + 2 * op.n_kv) * 128 || N / 128 > XCH_GROUPS || K % 128 || K / 128 < 8 || xarea < 0 || xarea >= XCH_AREAS)
+    return hipErrorInvalidValue;
+  return launch_strip_cf<1, ST_OUT_ROPE, float, 2>(A, As, Bt, Bs, C, nullptr, M, N, K, b_layout == LLMMM_FP8_B_PRESHUFFLED, stream, nullptr, xarea, op);
 }
 
 // Waves that gave up waiting in the exchange since the library was loaded (0 on a healthy device); synchronises.
