@@ -490,6 +490,20 @@ bool rope_strips_pay(int M, int N, int K)
          (M <= 8 || (M <= 16 && (long)M * K <= 65536 && (long)N * K >= 24000000L));
 }
 
+// The same beyond 16 rows: a workgroup holds whole heads of 16 or 32 rows over all of K and rotates them itself (0: planes and a second
+// kernel).  Where the split form would not split, the launch is saved at the same sums; 16-row groups while they fit one round of the chip
+// -- every group streams its heads' weights again, from the L2 -- and 32-row ones beyond (us, plane + second kernel / groups of 16 / 32:
+// 4096 x 2048 9.9 / 7.5 / 8.2 at M = 80, 10.0 / 7.5 / 8.4 at 128; 6144 x 2560 12.1 / 9.2 / 10.2 at M = 80, 12.3 / 16.6 / 10.2 at 100).  Against a split
+// run from 48 rows on, where its planes have grown (6144 x 2560 in five splits 8.0 / 9.3 / 10.6 at M = 32, 9.3 / 9.1 at 48, 10.0 / 9.2 at 64;
+// 6144 x 4096 in four 11.8 / 12.5 at 64).
+int rope_row_group(int M, int N, int K, int split)
+{
+  if (M <= 16 || M > SKINNY_MAX_M || K < 512 || (split > 1 && (M < 48 || K > 2560))) return 0;
+  const int heads = N / 128;
+  if ((M + 15) / 16 * heads <= NUM_CUS && K <= 5120) return 16;
+  return split <= 1 && (M + 31) / 32 * heads <= NUM_CUS && K <= 2560 ? 32 : 0;
+}
+
 // The SwiGLU output of the weight-streaming kernel in one launch (64 gate + 64 up columns per workgroup, K unsplit; figures in
 // fp8_skinny.hip).  Its N / 128 workgroups have to fill the chip or a good part of its last round: with fewer, splitting K pulls more
 // (12288 x 2048, 96 workgroups, M = 24: 9.4 in two splits + reduce / 9.9 so), and 272 or 296 run a nearly empty second round
@@ -1219,15 +1233,20 @@ int llmmm_fp8_gemm_qkv_rope(int out_kind, const void* A, const float* As, const 
   PlaneCfg pc;
   int      rc = resolve_plane_cfg(A, As, Bt, Bs, M, N, K, workspace, workspace_bytes, user, true, &pc, stream, false);
   if (rc) return rc;
-  int area;
-  if (out_kind == LLMMM_OUT_BF16 && pc.skinny && !pc.prep.agen && !(user && (user->split_k > 0 || user->tile != LLMMM_TILE_AUTO)) && rope_strips_pay(M, N, K) &&
-      (area = strip_exchange_area(stream)) >= 0) {
-    llmmm::Fp8HeadOp op;
-    op.qw = q_norm_weight, op.kw = k_norm_weight, op.cos_t = cos_table, op.sin_t = sin_table, op.pos = positions;
-    op.eps = eps, op.table_rows = table_rows, op.n_q = n_q_heads, op.n_kv = n_kv_heads;
-    const hipError_t e = llmmm::fp8_strip_rope_launch(pc.b_layout, A, As, Bt, Bs, out, M, N, K, op, area, (hipStream_t)stream);
-    if (e != hipSuccess) return fail(LLMMM_ERR_RUNTIME, "fp8 gemm + qk-norm + rope launch: %s", hipGetErrorString(e));
-    return LLMMM_OK;
+  if (pc.skinny && !pc.prep.agen && !(user && (user->split_k > 0 || user->tile != LLMMM_TILE_AUTO))) {
+    // one launch where it is the faster form: column strips, or whole heads per workgroup in row groups
+    const int  group  = rope_row_group(M, N, K, pc.split);
+    int        area   = -1;
+    const bool strips = out_kind == LLMMM_OUT_BF16 && rope_strips_pay(M, N, K) && (area = strip_exchange_area(stream)) >= 0;
+    if (strips || group) {
+      llmmm::Fp8HeadOp op;
+      op.qw = q_norm_weight, op.kw = k_norm_weight, op.cos_t = cos_table, op.sin_t = sin_table, op.pos = positions;
+      op.eps = eps, op.table_rows = table_rows, op.n_q = n_q_heads, op.n_kv = n_kv_heads;
+      const hipError_t e = strips ? llmmm::fp8_strip_rope_launch(pc.b_layout, A, As, Bt, Bs, out, M, N, K, op, area, (hipStream_t)stream)
+                                  : llmmm::fp8_skinny_rope_launch(out_kind, group, pc.b_layout, A, As, Bt, Bs, out, out_scale, M, N, K, op, (hipStream_t)stream);
+      if (e != hipSuccess) return fail(LLMMM_ERR_RUNTIME, "fp8 gemm + qk-norm + rope launch: %s", hipGetErrorString(e));
+      return LLMMM_OK;
+    }
   }
   if (pc.tile == LLMMM_TILE_128x160) return fail(LLMMM_ERR_INVALID_ARGUMENT, "the 128 x 160 tile cannot hold whole heads");
   if (pc.split == 0) {  // a tile kernel without split: norm and rope run on the accumulators, no planes

@@ -29,6 +29,8 @@
 namespace llmmm {
 
 enum { SK_OUT_F32 = 0, SK_OUT_BF16 = 1, SK_OUT_FP8Q = 2,
+       // the output of a QKV projection behind per-head RMSNorm and rotary embedding (Fp8HeadOp), K unsplit: a workgroup holds whole heads
+       SK_OUT_ROPE_BF16 = 4, SK_OUT_ROPE_FP8Q = 5,
        SK_OUT_SWIGLU = 3 };  // h = silu(gate) * up, quantised 1x128, in one launch: K unsplit, 64 gate + 64 up columns per workgroup
 
 // Where the workgroups of a SwiGLU output exchange their row maxima (PairSlots).
@@ -170,9 +172,11 @@ template <int MBLK, int OUT, int D, int ASTG, int AGEN = 0, typename HT = float>
 __global__ void __launch_bounds__(512)
 fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Bt,
                   const float* __restrict__ Bs, void* __restrict__ Cv, float* __restrict__ Cs, int M, int N, int K, int S,
-                  float* __restrict__ partial, int bpre, SkinnyGenA ag, int xarea)
+                  float* __restrict__ partial, int bpre, SkinnyGenA ag, int xarea, Fp8HeadOp op)
 {
   constexpr bool SWIGLU = OUT == SK_OUT_SWIGLU;
+  constexpr bool ROPE   = OUT == SK_OUT_ROPE_BF16 || OUT == SK_OUT_ROPE_FP8Q;
+  static_assert(!ROPE || (AGEN == 0 && ASTG >= 16 * MBLK * 528), "the rotary output: given activations; the result is laid out where they were staged");
   static_assert(!SWIGLU || (AGEN == 0 && MBLK <= 2), "the SwiGLU output: given activations, at most 32 rows");
   constexpr bool APRE  = ASTG > 0;
   static_assert(AGEN == 0 || (MBLK == 1 && APRE), "generated activations: 16 rows, staged in LDS");
@@ -260,10 +264,10 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
       const int m = min(m0 + r, M - 1);
       asm_load_lds_16B(A + (size_t)m * K + (size_t)(kb0 + j) * 128 + c * 16, a_addr + j * (MBLK * 2048) + within * 1024);
     };
-    // K is not split for SwiGLU: whole slices in turn, without the units that hold no row below M (their products are computed and never
+    // K is not split for SwiGLU and the rotary output: whole slices in turn, without the units that hold no row below M (their products are computed and never
     // stored) -- 12288 x 2048 at M = 4: 9.4 us in single units, 8.8 so.  The short K ranges of the other outputs would leave waves
     // without a slice (6144 x 2560 in five splits at M = 1: 6.55 / 6.65): single units in turn.
-    if constexpr (SWIGLU) {
+    if constexpr (SWIGLU || ROPE) {
       const int units = min(2 * MBLK, (M - m0 + 7) >> 3);
       for (int j = wave; j < kb1 - kb0; j += 8) {
 #pragma unroll
@@ -505,6 +509,68 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
   }
   LLMMM_LAST(0) LLMMM_LAST(1) LLMMM_LAST(2) LLMMM_LAST(3) LLMMM_LAST(4) LLMMM_LAST(5) LLMMM_LAST(6) LLMMM_LAST(7)
 #undef LLMMM_LAST
+
+  if constexpr (ROPE) {
+    // The head's rows go out through LDS, half a wavefront per row, lane l the columns 4l .. 4l + 3: from here on the arithmetic, and its
+    // order, of fp8_planes_qk_norm_rope_kernel.  The angles are on their way before the barrier.
+    constexpr int PASSES = MBLK;  // 16 half-waves, 16 * MBLK rows
+    const int     l32 = tid & 31, angle = (l32 & 15) * 4;
+    const bool    rotate = ng < op.n_q + op.n_kv, lo = l32 < 16;
+    const float*  nw     = ng < op.n_q ? op.qw : (rotate ? op.kw : nullptr);
+    f32x4         w4 = {1.f, 1.f, 1.f, 1.f}, cs[PASSES], sn[PASSES];
+    if (nw != nullptr) w4 = *(const f32x4*)(nw + l32 * 4);
+#pragma unroll
+    for (int u = 0; u < PASSES; ++u) {
+      cs[u] = f32x4{1.f, 1.f, 1.f, 1.f}, sn[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (rotate) {
+        const int p = min(max(op.pos[min(m0 + u * 16 + (tid >> 5), M - 1)], 0), op.table_rows - 1);
+        cs[u]       = *(const f32x4*)(op.cos_t + (size_t)p * 64 + angle);
+        sn[u]       = *(const f32x4*)(op.sin_t + (size_t)p * 64 + angle);
+      }
+    }
+    constexpr int RS = 132;  // floats per row: the 16 rows of a store lie 4 banks apart
+    float LLMMM_LDS* const rows = (float LLMMM_LDS*)a_stage;
+    __syncthreads();  // the activations have been read
+#pragma unroll
+    for (int mb = 0; mb < MBLK; ++mb) *(f32x4 LLMMM_LDS*)(rows + (mb * 16 + i) * RS + wave * 16 + 4 * g) = acc[mb];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PASSES; ++u) {
+      const int r = u * 16 + (tid >> 5), m = m0 + r;
+      f32x4     v = *(const f32x4 LLMMM_LDS*)(rows + r * RS + l32 * 4);
+      if (nw != nullptr) {
+        float a = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a = __builtin_fmaf(v[q], v[q], a);
+        a = half_wave_sum(a);
+        const float rn = 1.0f / __builtin_sqrtf(a / 128.0f + op.eps);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = (v[q] * rn) * w4[q];
+      }
+      if (rotate) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float other = wave_xor_get<16>(v[q]);
+          const float t     = other * sn[u][q];
+          v[q]              = __builtin_fmaf(v[q], cs[u][q], lo ? -t : t);
+        }
+      }
+      if constexpr (OUT == SK_OUT_ROPE_BF16) {
+        if (m < M) store_row4<__bf16>((__bf16*)Cv + (size_t)m * N + ng * 128 + l32 * 4, v);
+      }
+      else {
+        float a = fmaxf(fmaxf(fmaxf(0.f, __builtin_fabsf(v[0])), __builtin_fabsf(v[1])), fmaxf(__builtin_fabsf(v[2]), __builtin_fabsf(v[3])));
+        a = half_wave_max(a);
+        const float scale = a / 448.f;
+        const float inv   = requant_inv(a);
+        if (m < M) {
+          *(uint32_t*)((uint8_t*)Cv + (size_t)m * N + ng * 128 + l32 * 4) = pack_e4m3x4_in_range(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
+          if (l32 == 0) Cs[(size_t)ng * M + m] = scale;
+        }
+      }
+    }
+    return;
+  }
 
   if constexpr (SWIGLU) {
     if (wave >= 4) {
@@ -1049,10 +1115,10 @@ hipError_t fp8_strip_add_residual_launch(int hidden_dtype, int b_layout, const v
 
 template <int MBLK, int OUT, int D, int ASTG>
 static hipError_t launch_skinny(const void* A, const float* As, const void* Bt, const float* Bs, void* C, float* Cs, int M,
-                                int N, int K, int S, float* partial, int bpre, hipStream_t stream, int xarea = 0)
+                                int N, int K, int S, float* partial, int bpre, hipStream_t stream, int xarea = 0, const Fp8HeadOp& op = Fp8HeadOp{})
 {
   hipLaunchKernelGGL((fp8_skinny_kernel<MBLK, OUT, D, ASTG>), dim3(N / 128, S, (M + 16 * MBLK - 1) / (16 * MBLK)), dim3(512), 0, stream,
-                     (const uint8_t*)A, As, (const uint8_t*)Bt, Bs, C, Cs, M, N, K, S, partial, bpre, SkinnyGenA{}, xarea);
+                     (const uint8_t*)A, As, (const uint8_t*)Bt, Bs, C, Cs, M, N, K, S, partial, bpre, SkinnyGenA{}, xarea, op);
   return hipGetLastError();
 }
 
@@ -1066,7 +1132,7 @@ static hipError_t dispatch_skinny_agen(const float* G, const void* Bt, const flo
 #define LLMMM_GO(D, ASTG)                                                                                                                   \
   {                                                                                                                                         \
     hipLaunchKernelGGL((fp8_skinny_kernel<1, OUT, D, ASTG, 1>), dim3(N / 128, S, 1), dim3(512), 0, stream, (const uint8_t*)G, (const float*)nullptr, \
-                       (const uint8_t*)Bt, Bs, C, Cs, M, N, K, S, partial, bpre, SkinnyGenA{}, 0);                                            \
+                       (const uint8_t*)Bt, Bs, C, Cs, M, N, K, S, partial, bpre, SkinnyGenA{}, 0, Fp8HeadOp{});                                            \
     return hipGetLastError();                                                                                                               \
   }
   if (slices >= 8 && need <= 28672) LLMMM_GO(8, 28672);
@@ -1096,7 +1162,7 @@ static hipError_t dispatch_skinny_gen2(const SkinnyGenA& ag, const void* Bt, con
 #define LLMMM_GO(D, ASTG)                                                                                                                       \
   {                                                                                                                                             \
     hipLaunchKernelGGL((fp8_skinny_kernel<1, SK_OUT_F32, D, ASTG, 2, HT>), dim3(N / 128, S, 1), dim3(512), 0, stream, (const uint8_t*)nullptr,  \
-                       (const float*)nullptr, (const uint8_t*)Bt, Bs, (void*)C, (float*)nullptr, M, N, K, S, partial, bpre, ag, 0);                \
+                       (const float*)nullptr, (const uint8_t*)Bt, Bs, (void*)C, (float*)nullptr, M, N, K, S, partial, bpre, ag, 0, Fp8HeadOp{});                \
     return hipGetLastError();                                                                                                                   \
   }
   if (slices >= 8 && need <= 28672) LLMMM_GO(8, 28672);
@@ -1183,6 +1249,22 @@ hipError_t fp8_skinny_swiglu_launch(int b_layout, const void* A, const float* As
   if (KB * 4096 <= 65536) LLMMM_GO(2, 4, 65536);
   LLMMM_GO(2, 4, 81920);
 #undef LLMMM_GO
+}
+
+// A QKV projection with norm and rotary embedding in one launch: K unsplit, row groups of `group` = 16 or 32 rows whose activations fit the
+// staging area (K <= 5120 / 2560).
+hipError_t fp8_skinny_rope_launch(int out_kind, int group, int b_layout, const void* A, const float* As, const void* Bt, const float* Bs, void* C, float* Cs, int M,
+                                  int N, int K, const Fp8HeadOp& op, hipStream_t stream)
+{
+  const int bpre = b_layout == LLMMM_FP8_B_PRESHUFFLED;
+  if (M < 1 || M > 128 || N != (op.n_q + 2 * op.n_kv) * 128 || K % 128 || K < 512 || (group != 16 && group != 32) || group * K > 81920) return hipErrorInvalidValue;
+#define LLMMM_GO(OUT)                                                                                                                                           \
+  return group == 16 ? launch_skinny<1, OUT, 4, 81920>(A, As, Bt, Bs, C, Cs, M, N, K, 1, nullptr, bpre, stream, 0, op)                                          \
+                     : launch_skinny<2, OUT, 4, 81920>(A, As, Bt, Bs, C, Cs, M, N, K, 1, nullptr, bpre, stream, 0, op)
+  if (out_kind == LLMMM_OUT_BF16) LLMMM_GO(SK_OUT_ROPE_BF16);
+  if (out_kind == LLMMM_OUT_FP8Q && Cs) LLMMM_GO(SK_OUT_ROPE_FP8Q);
+#undef LLMMM_GO
+  return hipErrorInvalidValue;
 }
 
 hipError_t fp8_skinny_launch(int out_kind, int b_layout, const void* A, const float* As, const void* Bt, const float* Bs, void* C,

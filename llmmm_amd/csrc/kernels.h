@@ -78,6 +78,8 @@ hipError_t fp8_splitk_reduce_launch(int out_kind, const float* planes, int S, vo
 
 // M <= 128 (row groups of 64); S splits of K.  partial == nullptr (S must be 1): complete result in C / Cs.
 // Otherwise only the S partial planes `partial` [S][M][N] fp32 are written; run fp8_splitk_reduce_launch behind it.
+hipError_t fp8_skinny_rope_launch(int out_kind, int group, int b_layout, const void* A, const float* As, const void* Bt, const float* Bs, void* C, float* Cs, int M,
+                                  int N, int K, const Fp8HeadOp& op, hipStream_t stream);
 hipError_t fp8_strip_rope_launch(int b_layout, const void* A, const float* As, const void* Bt, const float* Bs, void* C, int M, int N, int K, const Fp8HeadOp& op,
                                  int xarea, hipStream_t stream);
 bool       fp8_skinny_swiglu_fits(int M, int N, int K);

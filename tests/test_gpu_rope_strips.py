@@ -9,7 +9,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _case(lib, oracle, M, K, n_q, n_kv, seed, norm=True, pre=False, rows=512):
+def _case(lib, oracle, M, K, n_q, n_kv, seed, norm=True, pre=False, rows=512, fp8=False):
     N = (n_q + 2 * n_kv) * 128
     rng = np.random.default_rng(seed)
     X = rng.standard_normal((M, K)).astype(np.float32)
@@ -26,10 +26,12 @@ def _case(lib, oracle, M, K, n_q, n_kv, seed, norm=True, pre=False, rows=512):
     qw, kw = (rng.uniform(0.5, 1.5, 128).astype(np.float32) for _ in range(2)) if norm else (None, None)
     g = lambda a: None if a is None else torch.from_numpy(a).cuda()
     C = torch.empty((M, N), dtype=torch.float32, device="cuda")
-    lib.fp8_gemm_blockwise_quant_A_1x128__B_128x128__output_fp32(t[0], t[1], b, bs, C, M, N, K, tile=lib._lib.TILE_STRIP, b_preshuffled=pre)
-    want = oracle.f32_to_bf16_bits(oracle.qk_norm_rope(C.cpu().numpy(), qw, kw, 1e-6, cos, sin, pos, n_q, n_kv))
+    how = {"tile": lib._lib.TILE_STRIP} if M <= 16 else {"tile": lib._lib.TILE_SKINNY, "split_k": 1}  # (beyond 16 rows: K in one range)
+    lib.fp8_gemm_blockwise_quant_A_1x128__B_128x128__output_fp32(t[0], t[1], b, bs, C, M, N, K, b_preshuffled=pre, **how)
+    want = oracle.qk_norm_rope(C.cpu().numpy(), qw, kw, 1e-6, cos, sin, pos, n_q, n_kv)
+    want = oracle.requant_c_1x128(want) if fp8 else oracle.f32_to_bf16_bits(want)
     args = (t[0], t[1], b, bs, g(qw), g(kw), 1e-6, g(cos), g(sin), g(pos), n_q, n_kv, M, N, K)
-    return (lambda: lib.fp8_gemm_qkv_rope(*args, b_preshuffled=pre)), want, t
+    return (lambda: lib.fp8_gemm_qkv_rope(*args, b_preshuffled=pre, out_fp8=fp8)), want, t
 
 
 def _bits(out):
@@ -51,6 +53,17 @@ def test_oracle_bits(lib, oracle, K, n_q, n_kv, pre):
     call, want, _ = _case(lib, oracle, 3, K, n_q, n_kv, K, norm=False, pre=pre)
     assert np.array_equal(_bits(call()), want)
     assert _timeouts(lib) == 0
+
+
+# (heads, K) whose 16-row groups, or only whose 32-row ones, fit one round of the chip; the first and last rows of a group
+@pytest.mark.parametrize("M,K,n_q,n_kv", [(48, 2560, 32, 8), (49, 2560, 32, 8), (64, 2560, 32, 8), (65, 2560, 32, 8), (80, 2560, 32, 8), (81, 2560, 32, 8), (100, 2560, 32, 8),
+                                          (128, 2560, 32, 8), (17, 2048, 16, 8), (33, 2048, 16, 8), (127, 2048, 16, 8), (128, 2048, 16, 8)])
+def test_whole_heads_in_row_groups(lib, oracle, M, K, n_q, n_kv):
+    call, want, _ = _case(lib, oracle, M, K, n_q, n_kv, M, pre=M % 2 == 0)
+    assert np.array_equal(_bits(call()), want)
+    call, (codes, scales), _ = _case(lib, oracle, M, K, n_q, n_kv, M, norm=M % 3 != 0, fp8=True)
+    q, s = call()
+    assert np.array_equal(q.cpu().numpy(), codes) and np.array_equal(s.cpu().numpy().view(np.uint32), scales.view(np.uint32))
 
 
 def test_back_to_back_and_captured(lib, oracle):
