@@ -514,6 +514,16 @@ bool swiglu_pair_pays(int M, int N, int K)
   return llmmm::fp8_skinny_swiglu_fits(M, N, K) && groups >= (M <= 16 ? 96 : 128) && (groups <= NUM_CUS || last == 0 || last >= NUM_CUS / 2);
 }
 
+// The SwiGLU output of fewer than 128 rows in 256-column tiles (a row tail; each holds whole 1x128 groups, so nothing is exchanged): from
+// 33 rows on where the 128-column ones would be more than one round of the chip, from 17 -- against the weight-streaming kernel -- where they
+// fill three quarters of a round (us, pre-shuffled, before / so: 37888 x 3584 43.4 / 35.8 at M = 48, 49.2 / 38.3 at 100; 34816 x 5120 63.8 / 50.9 at 100;
+// 57344 x 8192 115 / 83.7 at 100; 51200 x 5120, 200 tiles, 63.4 / 50.1 at 32, 59.0 / 48.9 at 20 -- but 148 tiles of 37888 x 3584 33.5 / 34.7 at 20).
+bool swiglu_wide_tail(int M, int N)
+{
+  if (M >= 128 || N % 256) return false;
+  return M > 32 ? N / 128 > NUM_CUS : M > 16 && N / 256 >= NUM_CUS * 3 / 4 && N / 256 <= NUM_CUS;
+}
+
 // The split the weight-streaming kernel runs this shape in when it is the split-K form after all (tune table, then heuristic).
 int skinny_split_for(int M, int N, int K)
 {
@@ -842,8 +852,11 @@ int llmmm_fp8_gemm_ex(int out_kind, const void* A, const float* As, const void* 
       if (!aligned16(workspace)) return fail(LLMMM_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
       partial = (float*)workspace;
     }
-    const bool pair = swiglu && !agen && !(user && user->split_k > 0) && swiglu_pair_pays(M, N, K) && (pair_area = strip_exchange_area(stream)) >= 0;
-    if (pair)
+    const bool wide = swiglu && !agen && !(user && (user->split_k > 0 || user->tile != LLMMM_TILE_AUTO)) && swiglu_wide_tail(M, N);
+    const bool pair = swiglu && !wide && !agen && !(user && user->split_k > 0) && swiglu_pair_pays(M, N, K) && (pair_area = strip_exchange_area(stream)) >= 0;
+    if (wide)
+      e = llmmm::fp8_gemm_launch(out_kind, LLMMM_TILE_128x256, cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, 1, nullptr, (hipStream_t)stream), partial = nullptr;
+    else if (pair)
       e = llmmm::fp8_skinny_swiglu_launch(cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, pair_area, (hipStream_t)stream), partial = nullptr;
     else if (agen == 2)
       e = llmmm::fp8_skinny_rmsnorm_a_launch(prep.hidden_dtype, cfg.b_layout, prep.ag, Bt, Bs, (float*)C, M, N, K, split, partial, (hipStream_t)stream);
@@ -891,7 +904,9 @@ int llmmm_fp8_gemm_ex(int out_kind, const void* A, const float* As, const void* 
       planes = (float*)workspace;
     }
     int pair_area;
-    if (swiglu && cfg.tile == LLMMM_TILE_128x128 && split <= 1 && !(user && user->split_k > 0) && llmmm::fp8_gemm_swiglu_pair_fits(M, N, K) &&
+    if (swiglu && cfg.tile == LLMMM_TILE_128x128 && split <= 1 && !(user && (user->split_k > 0 || user->tile != LLMMM_TILE_AUTO)) && swiglu_wide_tail(M, N))
+      e = llmmm::fp8_gemm_launch(out_kind, LLMMM_TILE_128x256, cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, 1, nullptr, (hipStream_t)stream);
+    else if (swiglu && cfg.tile == LLMMM_TILE_128x128 && split <= 1 && !(user && user->split_k > 0) && llmmm::fp8_gemm_swiglu_pair_fits(M, N, K) &&
         (pair_area = strip_exchange_area(stream)) >= 0)
       e = llmmm::fp8_gemm_swiglu_pair_launch(cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, pair_area, (hipStream_t)stream);
     else

@@ -272,9 +272,10 @@ __device__ __forceinline__ void swiglu_send(const f32x4 (&acc)[8][MF], char LLMM
 // The kept fragments mf = KEEP0 .. (own values: gate if IS_GATE, else up) meet the partner's values of the same
 // rows and columns: h = silu(gate) * up, then the fused 1x128 quantisation of h exactly as for plain C
 // (examples/005.fp8.mm.opt.cu:401-462), staged row-major in `stg` and stored as whole 128-byte rows.
-template <int MF, int KEEP0, bool IS_GATE>
+// MT: only rows below M are stored.
+template <int MF, int KEEP0, bool IS_GATE, bool MT>
 __device__ __forceinline__ void swiglu_finish(const f32x4 (&acc)[8][MF], const f32x4 (&other)[8][MF / 2], char LLMMM_LDS* stg, uint8_t* C,
-                                              float* Cs_col, int ldc, int row0, int col0, int lane)
+                                              float* Cs_col, int ldc, int row0, int col0, int lane, int M)
 {
   constexpr int MH = MF / 2;
   const int     g = lane >> 4, li = lane & 15;
@@ -299,13 +300,13 @@ __device__ __forceinline__ void swiglu_finish(const f32x4 (&acc)[8][MF], const f
     for (int nf = 0; nf < 8; ++nf)
       *(uint32_t LLMMM_LDS*)(stg + r * 128 + ((nf ^ ((r >> 1) & 7)) << 4) + 4 * g) =
         pack_e4m3x4_in_range(v[nf][0] * inv, v[nf][1] * inv, v[nf][2] * inv, v[nf][3] * inv);
-    if (g == 0) Cs_col[row0 + KEEP0 * 16 + r] = scale;
+    if (g == 0 && (!MT || row0 + KEEP0 * 16 + r < M)) Cs_col[row0 + KEEP0 * 16 + r] = scale;
   }
 #pragma unroll
   for (int j = 0; j < MH * 2; ++j) {
     const int   r = 8 * j + (lane >> 3), c = lane & 7;
     const i32x4 x = *(const i32x4 LLMMM_LDS*)(stg + r * 128 + ((c ^ ((r >> 1) & 7)) << 4));
-    *(i32x4*)(C + (size_t)(row0 + KEEP0 * 16 + r) * ldc + col0 + c * 16) = x;
+    if (!MT || row0 + KEEP0 * 16 + r < M) *(i32x4*)(C + (size_t)(row0 + KEEP0 * 16 + r) * ldc + col0 + c * 16) = x;
   }
 }
 
@@ -442,7 +443,7 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   // scales travelling with the stage.  (With two workgroups per CU the two-stage form is faster: 29 vs 38 us on
   // 2048 x 2560 x 4096 in 128 x 128 tiles.)
   constexpr bool DEEP    = (BMODE & 4) != 0 && WM == 32;
-  // BMODE bit 3 (MT, deep 128 x 128 tiles with the fp32 / bf16 / fp8 outputs only): M is not a multiple of BM; the rows
+  // BMODE bit 3 (MT, deep 128 x 128 tiles with the fp32 / bf16 / fp8 outputs and both SwiGLU forms of 128 rows): M is not a multiple of BM; the rows
   // of the last tile row beyond the matrix are computed from copies of its last row and never stored.
   constexpr bool MT      = (BMODE & 8) != 0;
   // BMODE bit 4 (STAMP): the phase-accounting build -- clock readings at five points of every wave, stored to op.stamps at the end
@@ -451,7 +452,8 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   unsigned long long wait_cycles = 0;  // STAMP: shader cycles this wave spent in the K loop's "loads landed + barrier" waits (slices 1 ..)
   unsigned long long load_wait_cycles = 0;  // ... of which for its own loads (the rest: for the other waves at the barrier)
   if constexpr (STAMP) ph[0] = phase_clock();
-  static_assert(!MT || (DEEP && BM == 128 && BN == 128 && (OUT == OUT_F32 || OUT == OUT_BF16 || OUT == OUT_FP8Q || PAIR)), "row tails: deep 128 x 128 tiles only");
+  static_assert(!MT || (DEEP && BM == 128 && ((BN == 128 && (OUT == OUT_F32 || OUT == OUT_BF16 || OUT == OUT_FP8Q || PAIR)) || (BN == 256 && OUT == OUT_SWIGLU))),
+                "row tails: deep 128-row tiles only");
   constexpr int  STAGE_D = TC::STAGE + TC::NW * 256;                 // operands + 256 bytes of scales per wave
   constexpr int  NST     = !DEEP ? 2 : (4 * STAGE_D <= 160 * 1024 ? 4 : 3);
   static_assert(fp8_lds_bytes<BM, BN, WM, BMODE>() == (DEEP ? NST * STAGE_D : 2 * TC::STAGE), "the kernels size the buffers with fp8_lds_bytes");
@@ -807,9 +809,9 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
     uint8_t*  C    = (uint8_t*)Cv;
     const int half = N >> 1;
     if (wn == 0)
-      swiglu_finish<MF, 0, true>(acc, other, xmine, C, Cs + (size_t)(n0 >> 7) * M, half, row0, n0, lane);
+      swiglu_finish<MF, 0, true, MT>(acc, other, xmine, C, Cs + (size_t)(n0 >> 7) * M, half, row0, n0, lane, M);
     else
-      swiglu_finish<MF, MH, false>(acc, other, xmine, C, Cs + (size_t)(n0 >> 7) * M, half, row0, n0, lane);
+      swiglu_finish<MF, MH, false, MT>(acc, other, xmine, C, Cs + (size_t)(n0 >> 7) * M, half, row0, n0, lane, M);
   }
   else {
     uint8_t* C = (uint8_t*)Cv;
@@ -1046,8 +1048,10 @@ static hipError_t launch_reduce(const float* planes, int S, void* C, float* Cs, 
 template <int BM, int BN, int WM, int OUT>
 static auto pick_kernel(int bmode) -> decltype(&fp8_gemm_kernel<BM, BN, WM, OUT, 0>)
 {
-  if (bmode & 8) {  // a row tail: deep 128 x 128 tiles with the fp32 / bf16 / fp8 outputs
+  if (bmode & 8) {  // a row tail: deep 128 x 128 tiles with the fp32 / bf16 / fp8 outputs, 128 x 256 ones with SwiGLU
     if constexpr (BM == 128 && BN == 128 && WM == 32 && (OUT == OUT_F32 || OUT == OUT_BF16 || OUT == OUT_FP8Q))
+      return (bmode & 1) ? fp8_gemm_kernel<BM, BN, WM, OUT, 15> : fp8_gemm_kernel<BM, BN, WM, OUT, 14>;
+    else if constexpr (BM == 128 && BN == 256 && WM == 32 && OUT == OUT_SWIGLU)
       return (bmode & 1) ? fp8_gemm_kernel<BM, BN, WM, OUT, 15> : fp8_gemm_kernel<BM, BN, WM, OUT, 14>;
     else
       return nullptr;

@@ -66,6 +66,17 @@ def test_bits_of_the_plane_route_tiles(oracle, N, K, pre):
     assert _timeouts() == 0
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 49152, 128), (20, 49152, 384), (32, 51200, 256), (33, 33024, 640), (64, 33024, 256), (65, 33024, 128), (100, 37888, 512), (127, 33024, 384)])
+@pytest.mark.parametrize("pre", [False, True])
+def test_row_tails_in_wide_tiles(oracle, M, N, K, pre):
+    """More 128-column tiles than CUs: 256-column tiles of fewer than 128 rows, which hold whole groups."""
+    t, _ = _inputs(oracle, M, N, K, M, pre)
+    guard = torch.full((M + 4, N // 2), 0x55, dtype=torch.uint8, device="cuda"), torch.full((N // 256 + 1, M), -1.0, device="cuda")
+    got, want = _call(t, M, N, K, pre, out=guard), _call(t, M, N, K, pre, split=1)
+    assert _same((got[0][:M], got[1][:-1]), want)
+    assert (guard[0][M:] == 0x55).all() and (guard[1][-1] == -1.0).all()
+
+
 def test_launches_that_change_rows_and_shapes(oracle):
     """Exchange slots are kept per block of 16 rows: launches of other row counts and widths on one stream, other maxima each time."""
     from llmmm_amd import _lib
