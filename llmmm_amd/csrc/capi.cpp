@@ -88,44 +88,67 @@ int heuristic_split(int M, int N, int K)
   return s;
 }
 
-// Tile for the MFMA kernels: fewest "waves" of workgroups over the 256 CUs, weighted by tile
-// area and a mild efficiency penalty for the smaller tiles (less operand reuse per byte of LDS).
-int heuristic_tile(int M, int N)
+constexpr int MAX_TILE_SPLIT = 8;
+
+// The FP8 tile kernels' time in microseconds: a CU holds `per_cu` tiles side by side and works a 128-wide slice of them all in `all` and of
+// a lone one in `one`; every round of tiles starts and ends in `setup`.  Launches of at most one workgroup per CU (and a single tile row)
+// run in the deep rings and have constants of their own.  S > 1 shares of K add a second kernel (`launch`) and S fp32 planes on their way
+// through memory (per MB of a plane).  Fitted to every (tile, S) of 644 shapes on the MI355X -- 128 .. 4096 rows, N 1024 .. 57344, K 1024 .. 28672,
+// half of them the tuned families' projections at other M -- each on weights from the caches and from HBM (geometric mean of the two).  The
+// smallest estimate is within 0.6 % of the best (tile, S) on average, 12 % at worst.  (Rounds weighted by tile area, and a split
+// only where the tiles leave most of the chip idle, were 6.9 % off, 31 % at worst: 1408 x 26624 x 9216 468 us in 128 x 256 tiles for 381 in 128 x 128;
+// 1024 x 2688 x 22016 103 unsplit for 70 in three shares; 896 x 10240 x 8192 126 for 83 in 128 x 160 tiles; 128 x 10496 x 1536
+// 16.7 streaming for 11.4 in 128 x 128 tiles.)
+double fp8_tile_estimate(int tile, int M, int N, int K, int S)
 {
   static const struct {
-    int   id, bm, bn, per_cu;
-    float eff;
-  } cand[] = {{LLMMM_TILE_256x256, 256, 256, 1, 1.00f},
-              {LLMMM_TILE_128x256, 128, 256, 1, 0.85f},
-              {LLMMM_TILE_256x128, 256, 128, 1, 0.85f},
-              {LLMMM_TILE_128x128, 128, 128, 2, 0.90f}};
-  int   best      = -1;
-  float best_cost = 0.f;
-  for (const auto& c : cand) {
-    if (M % c.bm || N % c.bn) continue;
-    const long  tiles = (long)(M / c.bm) * (N / c.bn);
-    const long  slots = (long)NUM_CUS * c.per_cu;
-    float       waves = (float)((tiles + slots - 1) / slots);
-    if (c.id == LLMMM_TILE_256x256) {
-      // a launch of 256 x 256 tiles fills a partly empty last round with half-size tiles where it can (the same
-      // conditions as launch_fp8 / launch_fp16 in the kernel files): that round then costs half
-      const long tm = M / 256, tn = N / 256, full = tiles / NUM_CUS * NUM_CUS;
-      if (tiles > NUM_CUS && tm > 1 && full % tm == 0 && tn - full / tm > 0 && (tn - full / tm) * tm * 2 <= NUM_CUS) waves -= 0.5f;
-    }
-    // More 128 x 128 tiles than CUs put two on some CUs, and on weights that come from HBM -- as a layer's weights do in a
-    // model -- that costs 6-32 % against half as many 256 x 128 tiles, one per CU, whose tile rows re-read the weights half
-    // as often (us, weights rotated over more copies than the caches hold / one copy; 128 x 128 | 256 x 128 | 128 x 256:
-    // 2048 x 2560 x 9728 85.3 / 64.0 | 64.5 / 62.6 | 66.4 / 62.2; 1024 x 6144 x 2560 27.9 / 21.3 | 22.4 / 21.6 | 23.6 / 21.4;
-    // 512 x 10240 x 8192 73.0 / 55.0 | 57.9 / 53.3 | 59.7 / 53.0; 256 x 19456 x 2560 29.1 / 20.5 | 25.8 / 24.0 | 26.0 / 20.9).
-    // Up to one tile per CU the small tile stays ahead (1024 x 4096 x 4096: 26.8 | 31.7 | 30.6 cold).
-    float eff = c.eff;
-    if (c.id == LLMMM_TILE_128x128 && tiles > NUM_CUS) eff = 0.74f;
-    if (c.id == LLMMM_TILE_256x128) eff = 0.86f;  // (ahead of 128 x 256 on weights from HBM: 256 x 22016 x 4096 34.0 against 40.0 us)
-    const float cost  = waves * c.per_cu * c.bm * c.bn / eff;
-    if (best < 0 || cost < best_cost) {
-      best      = c.id;
-      best_cost = cost;
-    }
+    int    id, bm, bn, per_cu;
+    double setup, one, all, deep_setup, deep_slice, launch, per_share, per_mb;
+  } form[] = {{LLMMM_TILE_256x256, 256, 256, 1, 5.85, 1.393, 1.393, 5.85, 1.393, 4.05, 0.253, 0.052},
+              {LLMMM_TILE_128x256, 128, 256, 1, 2.81, 1.100, 1.100, 4.05, 0.804, 3.59, 0.306, 0.042},
+              {LLMMM_TILE_256x128, 256, 128, 1, 3.59, 1.032, 1.032, 4.23, 0.768, 2.78, 0.285, 0.228},
+              {LLMMM_TILE_128x128, 128, 128, 2, 2.55, 0.677, 1.045, 4.41, 0.538, 2.21, 0.425, 0.056},
+              {LLMMM_TILE_128x160, 128, 160, 2, 2.41, 0.743, 1.302, 4.40, 0.679, 2.21, 0.425, 0.056}};
+  for (const auto& f : form) {
+    if (f.id != tile) continue;
+    const long   tiles_m = (M + f.bm - 1) / f.bm, groups = tiles_m * (N / f.bn) * S;
+    const int    slices = (K / 128 + S - 1) / S;
+    const bool   deep   = groups <= NUM_CUS || tiles_m == 1;
+    const long   per = (groups + NUM_CUS - 1) / NUM_CUS, side = deep ? 1 : f.per_cu, full = per / side, left = per % side ? 1 : 0;
+    const double us  = (full + left) * (deep ? f.deep_setup : f.setup) + slices * (full * (deep ? f.deep_slice : f.all) + left * f.one);
+    return S > 1 ? us + f.launch + (double)M * N * 4e-6 * (f.per_share * S + f.per_mb) : us;
+  }
+  return 1e30;
+}
+bool tile_dims(int tile, int& bm, int& bn);
+bool fp16_only(int tile) { return tile == LLMMM_TILE_64x128 || tile == LLMMM_TILE_64x64; }
+
+// Split-K factor for a given tile: the smallest estimate, with at most one workgroup per CU and shares of two slices or more.
+int heuristic_tile_split(int tile, int M, int N, int K)
+{
+  int bm, bn;
+  if (!tile_dims(tile, bm, bn)) return 1;
+  const long tiles   = (long)((M + bm - 1) / bm) * (N / bn);
+  int        best    = 1;
+  double     best_us = fp8_tile_estimate(tile, M, N, K, 1);
+  for (int s = 2; s <= MAX_TILE_SPLIT && tiles * s <= NUM_CUS && s <= K / 256; ++s) {
+    const double us = fp8_tile_estimate(tile, M, N, K, s);
+    if (us < best_us) best = s, best_us = us;
+  }
+  return best;
+}
+// Tile for a shape the table does not list, each in its best split.  (The 128 x 160 tile serves some outputs only: prefer_wide_tile.)
+int heuristic_tile(int M, int N, int K)
+{
+  static const int cand[] = {LLMMM_TILE_256x256, LLMMM_TILE_128x256, LLMMM_TILE_256x128, LLMMM_TILE_128x128};
+  int              best   = -1;
+  double           best_us = 0.;
+  for (int tile : cand) {
+    int bm, bn;
+    tile_dims(tile, bm, bn);
+    if (M % bm || N % bn) continue;
+    const double us = fp8_tile_estimate(tile, M, N, K, heuristic_tile_split(tile, M, N, K));
+    if (best < 0 || us < best_us) best = tile, best_us = us;
   }
   return best;
 }
@@ -194,35 +217,6 @@ int heuristic_split_fp16(int M, int N, int K, double unsplit, int* tile)
   return split;
 }
 
-constexpr int MAX_TILE_SPLIT = 8;
-
-bool tile_dims(int tile, int& bm, int& bn);
-bool fp16_only(int tile) { return tile == LLMMM_TILE_64x128 || tile == LLMMM_TILE_64x64; }
-
-// Split-K factor for the MFMA tile kernels: only when the tiles alone leave most of the chip idle -- at most about one
-// workgroup per CU, every split at least two slices long -- and only when the shorter K loop pays for the fp32 planes'
-// round trip and the second launch.  The estimate (microseconds): a 128 x 128 x 128 slice of a lone workgroup takes
-// about 0.5 us (measured: 2048..19456-column outputs at M = 128..512), larger tiles in proportion; the reduce launch
-// costs about 3 us and S planes are written and read at about 4 TB/s.  (M = 256, N = 6144, K = 2560 in 96 tiles:
-// 14.3 us unsplit, 18.9 us in two splits; M = 256, N = 2560, K = 9728 in 40 tiles: 40 us unsplit, 18.6 us in six.)
-int heuristic_tile_split(int tile, int M, int N, int K)
-{
-  int bm, bn;
-  if (!tile_dims(tile, bm, bn)) return 1;
-  const int tiles = (M / bm) * (N / bn), kb = K / 128;
-  int       smax  = NUM_CUS / tiles;
-  if (smax > kb / 2) smax = kb / 2;
-  if (smax > MAX_TILE_SPLIT) smax = MAX_TILE_SPLIT;
-  const double t_slice  = 0.5 * (double)bm * bn / (128.0 * 128.0);
-  const double plane_us = (double)M * N * 4.0 * 2.0 / 4.0e6;  // one plane written and read
-  int          best     = 1;
-  double       best_us  = kb * t_slice;
-  for (int s = 2; s <= smax; ++s) {
-    const double us = ((kb + s - 1) / s) * t_slice + 3.0 + s * plane_us;
-    if (us < best_us) best = s, best_us = us;
-  }
-  return best;
-}
 bool tile_dims(int tile, int& bm, int& bn)
 {
   switch (tile) {
@@ -390,11 +384,12 @@ int choose_fp8(int M, int N, int K, llmmm_gemm_cfg* cfg)
   if (cfg->tile < 0) {
     if (M % 128) return fail(LLMMM_ERR_NOT_ALIGNED, "M or N or K are not aligned.");
     // an (N, K) that was tuned at other M: the tile of the nearest tuned M; otherwise the heuristic
+    // -- unless the estimates are 10 % apart (1536 x 4608 x 3584: 41 us in the 256 x 256 tiles of M = 2048, 30 in 256 x 128 ones)
     int t, sp;
-    if (lookup_tile(M, N, K, &t, &sp))
+    cfg->tile = heuristic_tile(M, N, K);
+    if (lookup_tile(M, N, K, &t, &sp) &&
+        fp8_tile_estimate(t, M, N, K, sp > 0 ? sp : heuristic_tile_split(t, M, N, K)) * 0.9 <= fp8_tile_estimate(cfg->tile, M, N, K, heuristic_tile_split(cfg->tile, M, N, K)))
       cfg->tile = t, cfg->split_k = sp;
-    else
-      cfg->tile = heuristic_tile(M, N);
   }
   if (cfg->tile == LLMMM_TILE_SKINNY) {
     if (cfg->split_k <= 0) cfg->split_k = heuristic_split(M, N, K);
@@ -411,16 +406,13 @@ int choose_fp8(int M, int N, int K, llmmm_gemm_cfg* cfg)
 // most of the chip idle (decode-sized M).
 constexpr size_t SWIGLU_PLANE_LIMIT = 16u << 20;
 
-// Outputs without 1x128 groups (fp32, bf16, residual add) may use the 160-column tile: when 128 x 128 tiles were chosen,
-// are not split, and 160-column ones need fewer rounds of the chip -- 2560 columns at M = 2048: 320 tiles (two rounds,
-// the second a quarter full) against 256 (one).  Measured on O / down at M = 2048: 30.0 -> 26.9 us, 64.0 -> 55.8 us.
-void prefer_wide_tile(llmmm_gemm_cfg* cfg, int M, int N)
+// Outputs without 1x128 groups (fp32, bf16, residual add) may use the 160-column tile, unsplit, where its estimate is the smaller: 2560
+// columns at M = 2048 are 256 such tiles, one per CU (O / down in 320 tiles of 128 x 128: 30.0 -> 26.9 us, 64.0 -> 55.8).
+void prefer_wide_tile(llmmm_gemm_cfg* cfg, int M, int N, int K)
 {
-  // (or 256 x 128 tiles, which the table and the heuristic name where 128 x 128 ones would sit two to a CU: one 128 x 160 tile
-  // per CU is as fast on weights from HBM and faster on cached ones -- 1024 x 5120 x 2560, us: 19.8 / 19.0 against 21.3 / 20.9)
-  if ((cfg->tile != LLMMM_TILE_128x128 && cfg->tile != LLMMM_TILE_256x128) || cfg->split_k > 1 || N % 640 || M % 128) return;
-  const long t128 = (long)(M / 128) * (N / 128), t160 = (long)(M / 128) * (N / 160);
-  if ((t160 + NUM_CUS - 1) / NUM_CUS < (t128 + NUM_CUS - 1) / NUM_CUS) cfg->tile = LLMMM_TILE_128x160;
+  int bm, bn;
+  if (N % 640 || M % 128 || !tile_dims(cfg->tile, bm, bn)) return;
+  if (fp8_tile_estimate(LLMMM_TILE_128x160, M, N, K, 1) < fp8_tile_estimate(cfg->tile, M, N, K, cfg->split_k < 1 ? 1 : cfg->split_k)) cfg->tile = LLMMM_TILE_128x160, cfg->split_k = 1;
 }
 
 // The weight-streaming kernel in column strips (one launch, the K split inside the workgroup) takes what the split-K
@@ -547,7 +539,7 @@ int choose_fp8_out(int out_kind, int M, int N, int K, llmmm_gemm_cfg* cfg)
 {
   const int rc = choose_fp8(M, N, K, cfg);
   if (rc) return rc;
-  if (out_kind == LLMMM_OUT_F32 || out_kind == LLMMM_OUT_BF16) prefer_wide_tile(cfg, M, N), prefer_strip(cfg, M, N, K);
+  if (out_kind == LLMMM_OUT_F32 || out_kind == LLMMM_OUT_BF16) prefer_wide_tile(cfg, M, N, K), prefer_strip(cfg, M, N, K);
   if (out_kind == LLMMM_OUT_FP8Q) prefer_strip_fp8q(cfg, M, N, K);
   if (out_kind == LLMMM_OUT_FP8Q_SWIGLU) {
     if (N % 256) return fail(LLMMM_ERR_NOT_ALIGNED, "M or N or K are not aligned.");
@@ -559,7 +551,8 @@ int choose_fp8_out(int out_kind, int M, int N, int K, llmmm_gemm_cfg* cfg)
         if (!narrow) cfg->tile = LLMMM_TILE_128x128;  // through one fp32 plane, twice the workgroups
       }
       else if (narrow && M % 128 == 0)  // (a row tail stays with the 128 x 128 tiles and the plane)
-        cfg->tile = (M % 256 == 0 && (long)(M / 256) * (N / 256) >= NUM_CUS) ? LLMMM_TILE_256x256 : LLMMM_TILE_128x256;
+        cfg->tile = M % 256 == 0 && fp8_tile_estimate(LLMMM_TILE_256x256, M, N, K, 1) < fp8_tile_estimate(LLMMM_TILE_128x256, M, N, K, 1) ? LLMMM_TILE_256x256
+                                                                                                                                          : LLMMM_TILE_128x256;
     }
   }
   return LLMMM_OK;
@@ -986,7 +979,7 @@ static size_t plane_route_workspace(int M, int N, int K, bool wide_ok)
   if (M <= 0 || N <= 0 || K <= 0 || N % 128 || K % 128) return 0;
   llmmm_gemm_cfg cfg;
   if (choose_fp8(M, N, K, &cfg) != LLMMM_OK) return 0;
-  if (wide_ok) prefer_wide_tile(&cfg, M, N), prefer_strip(&cfg, M, N, K);
+  if (wide_ok) prefer_wide_tile(&cfg, M, N, K), prefer_strip(&cfg, M, N, K);
   if (cfg.tile == LLMMM_TILE_STRIP) return strip_fallback_plane_bytes(M, N, K);  // strips need none (epilogue inside the kernel); a call with generated activations leaves them
   int split = cfg.split_k < 1 ? 1 : cfg.split_k;
   if (split > max_split_for(K)) split = max_split_for(K);
@@ -1053,7 +1046,7 @@ static int resolve_plane_cfg(const void*& A, const float*& As, const void* Bt, c
   llmmm_gemm_cfg cfg;
   const int      rc = choose_fp8(M, N, K, &cfg);
   if (rc) return rc;
-  if (wide_ok) prefer_wide_tile(&cfg, M, N);
+  if (wide_ok) prefer_wide_tile(&cfg, M, N, K);
   // (wide_ok also stands for "no 1x128-grouped epilogue behind the GEMM": the callers that may take column strips.  Not with
   // activations the kernel has to make itself, nor against an explicit split.)
   if (wide_ok && !(user && (user->a_layout != LLMMM_FP8_A_QUANTISED || user->split_k > 0 || user->tile != LLMMM_TILE_AUTO))) prefer_strip(&cfg, M, N, K);
