@@ -93,9 +93,11 @@ constexpr int MAX_TILE_SPLIT = 8;
 // The FP8 tile kernels' time in microseconds: a CU holds `per_cu` tiles side by side and works a 128-wide slice of them all in `all` and of
 // a lone one in `one`; every round of tiles starts and ends in `setup`.  Launches of at most one workgroup per CU (and a single tile row)
 // run in the deep rings and have constants of their own.  S > 1 shares of K add a second kernel (`launch`) and S fp32 planes on their way
-// through memory (per MB of a plane).  Fitted to every (tile, S) of 644 shapes on the MI355X -- 128 .. 4096 rows, N 1024 .. 57344, K 1024 .. 28672,
+// through memory (per MB of a plane; 0.1 on top of what was fitted, for what the planes displace in the caches).  Fitted to every (tile, S) of 644 shapes on the MI355X -- 128 .. 4096 rows, N 1024 .. 57344, K 1024 .. 28672,
 // half of them the tuned families' projections at other M -- each on weights from the caches and from HBM (geometric mean of the two).  The
-// smallest estimate is within 0.6 % of the best (tile, S) on average, 12 % at worst.  (Rounds weighted by tile area, and a split
+// choice (best_fp8_tile) takes 0.939 of the time of the rules before it on the 600 with more
+// than 128 rows; the smallest estimate by itself 0.936, within 0.6 % of the best (tile, S), but on weights that just fit the caches it loses by
+// its planes (384 x 3584 x 18944, three sets of weights in turn: 39.0 us in three shares of 128 x 128 tiles, 40.3 in six of 128 x 256).  (Rounds weighted by tile area, and a split
 // only where the tiles leave most of the chip idle, were 6.9 % off, 31 % at worst: 1408 x 26624 x 9216 468 us in 128 x 256 tiles for 381 in 128 x 128;
 // 1024 x 2688 x 22016 103 unsplit for 70 in three shares; 896 x 10240 x 8192 126 for 83 in 128 x 160 tiles; 128 x 10496 x 1536
 // 16.7 streaming for 11.4 in 128 x 128 tiles.)
@@ -116,41 +118,59 @@ double fp8_tile_estimate(int tile, int M, int N, int K, int S)
     const bool   deep   = groups <= NUM_CUS || tiles_m == 1;
     const long   per = (groups + NUM_CUS - 1) / NUM_CUS, side = deep ? 1 : f.per_cu, full = per / side, left = per % side ? 1 : 0;
     const double us  = (full + left) * (deep ? f.deep_setup : f.setup) + slices * (full * (deep ? f.deep_slice : f.all) + left * f.one);
-    return S > 1 ? us + f.launch + (double)M * N * 4e-6 * (f.per_share * S + f.per_mb) : us;
+    return S > 1 ? us + f.launch + (double)M * N * 4e-6 * ((f.per_share + 0.1) * S + f.per_mb) : us;
   }
   return 1e30;
 }
 bool tile_dims(int tile, int& bm, int& bn);
 bool fp16_only(int tile) { return tile == LLMMM_TILE_64x128 || tile == LLMMM_TILE_64x64; }
 
-// Split-K factor for a given tile: the smallest estimate, with at most one workgroup per CU and shares of two slices or more.
+// The choice among `tiles` (the largest first), with at most one workgroup per CU in a split and shares of two slices or more; returns the
+// tile, -1 if none divides the shape (fewer than 128 rows count as a row tail of a 128-row tile).  Each tile with the split it is fastest
+// in; of tiles within 3 % of the fastest the one with the fewest shares, and of unsplit ones beyond one workgroup per CU the largest (it
+// reads the least: 1024 x 18176 x 18560 takes 420 us in 256 x 256 tiles, 444 in 128 x 128 ones, 2 % below them by estimate).
+int best_fp8_tile(const int* tiles, int n, int M, int N, int K, int* split)
+{
+  constexpr double NEAR = 1.03;
+  constexpr int    MAX_TILES = 8;
+  struct {
+    double us;
+    int    split, area;  // area: of an unsplit launch beyond one workgroup per CU, otherwise 0
+  } of[MAX_TILES];
+  double smallest = 1e30;
+  if (n > MAX_TILES) n = MAX_TILES;
+  for (int i = 0; i < n; ++i) {
+    int bm, bn;
+    of[i] = {1e30, 1, 0};
+    if (!tile_dims(tiles[i], bm, bn) || (M % bm && !(M < 128 && bm == 128)) || N % bn) continue;
+    const long count = (long)((M + bm - 1) / bm) * (N / bn);
+    for (int s = 1; s == 1 || (s <= MAX_TILE_SPLIT && count * s <= NUM_CUS && s <= K / 256); ++s) {
+      const double us = fp8_tile_estimate(tiles[i], M, N, K, s);
+      if (us < of[i].us) of[i] = {us, s, s == 1 && count > NUM_CUS ? bm * bn : 0};
+    }
+    if (of[i].us < smallest) smallest = of[i].us;
+  }
+  int best = -1;
+  for (int i = 0; i < n; ++i) {
+    if (of[i].us >= 1e30 || of[i].us > smallest * NEAR) continue;
+    if (best < 0 || of[i].split < of[best].split || (of[i].split == of[best].split && of[i].us < of[best].us && of[i].area >= of[best].area)) best = i;
+  }
+  if (best < 0) return -1;
+  *split = of[best].split;
+  return tiles[best];
+}
+// Split-K factor for a given tile.
 int heuristic_tile_split(int tile, int M, int N, int K)
 {
-  int bm, bn;
-  if (!tile_dims(tile, bm, bn)) return 1;
-  const long tiles   = (long)((M + bm - 1) / bm) * (N / bn);
-  int        best    = 1;
-  double     best_us = fp8_tile_estimate(tile, M, N, K, 1);
-  for (int s = 2; s <= MAX_TILE_SPLIT && tiles * s <= NUM_CUS && s <= K / 256; ++s) {
-    const double us = fp8_tile_estimate(tile, M, N, K, s);
-    if (us < best_us) best = s, best_us = us;
-  }
-  return best;
+  int split = 1;
+  best_fp8_tile(&tile, 1, M, N, K, &split);
+  return split;
 }
-// Tile for a shape the table does not list, each in its best split.  (The 128 x 160 tile serves some outputs only: prefer_wide_tile.)
-int heuristic_tile(int M, int N, int K)
+// Tile and split for a shape the table does not list.  (The 128 x 160 tile serves some outputs only: prefer_wide_tile.)
+int heuristic_tile(int M, int N, int K, int* split)
 {
   static const int cand[] = {LLMMM_TILE_256x256, LLMMM_TILE_128x256, LLMMM_TILE_256x128, LLMMM_TILE_128x128};
-  int              best   = -1;
-  double           best_us = 0.;
-  for (int tile : cand) {
-    int bm, bn;
-    tile_dims(tile, bm, bn);
-    if (M % bm || N % bn) continue;
-    const double us = fp8_tile_estimate(tile, M, N, K, heuristic_tile_split(tile, M, N, K));
-    if (best < 0 || us < best_us) best = tile, best_us = us;
-  }
-  return best;
+  return best_fp8_tile(cand, 4, M, N, K, split);
 }
 
 // The FP16 / BF16 kernels' tile for shapes the table does not list.  A launch takes about
@@ -374,22 +394,31 @@ int choose_fp8(int M, int N, int K, llmmm_gemm_cfg* cfg)
   if (cfg->tile < 0 && M <= SKINNY_MAX_M) {
     int sp;
     if (lookup_skinny(M, N, K, &sp)) cfg->tile = LLMMM_TILE_SKINNY, cfg->split_k = sp;
-    // untuned shapes: the weight-streaming kernel up to 64 rows; above that only while the weight matrix is small -- its
-    // eight 16-row blocks per wave and its fp32 planes grow with M, and from about 20 MB of weights on, one row of 128 x 128
-    // tiles (a row tail for M < 128) is faster (measured at M = 96, us, streaming / tiles: N x K = 4096 x 4096 12.4 / 14.2,
-    // 6144 x 4096 19.9 / 16.0, 4096 x 14336 39.4 / 22.1, 28672 x 4096 66.7 / 27.1)
-    // (from 40 MB on the tiles win from 33 rows on, as on the tuned 19456 x 2560)
-    if (cfg->tile < 0) cfg->tile = (M <= 32 || (long)N * K < 20000000L || (M <= 64 && (long)N * K < 40000000L)) ? LLMMM_TILE_SKINNY : LLMMM_TILE_128x128;
+    // untuned shapes: the weight-streaming kernel up to 32 rows; its 16-row blocks per wave and its fp32 planes grow with M, and
+    // one row of 128-row tiles (128 x 128 as a row tail for M < 128) is the faster from 65 rows on at every size (167 shapes with 65 .. 128
+    // rows, N 1024 .. 32768, K 1024 .. 28672: 0.59 of the streaming time on average, 1.02 at most; us: 128 x 10496 x 1536 16.7 / 11.4, 128 x 2304 x 7808
+    // 21.7 / 14.7, 96 x 28672 x 4096 66.7 / 27.1).  Between, on large matrices and on medium ones with many columns (137 shapes: 0.865 of
+    // streaming alone; 40 x 16512 x 1408 15.1 / 9.2, 64 x 12416 x 1152 12.1 / 8.3 -- but 64 x 1152 x 17920 12.5 / 14.9).
+    const long nk = (long)N * K;
+    if (cfg->tile < 0) {
+      if (M <= 32 || (M <= 64 && nk < 40000000L && (N < 7000 || nk < 12000000L)))
+        cfg->tile = LLMMM_TILE_SKINNY;
+      else if (M == 128)
+        cfg->tile = heuristic_tile(M, N, K, &cfg->split_k);
+      else
+        cfg->tile = LLMMM_TILE_128x128;
+    }
   }
   if (cfg->tile < 0) {
     if (M % 128) return fail(LLMMM_ERR_NOT_ALIGNED, "M or N or K are not aligned.");
     // an (N, K) that was tuned at other M: the tile of the nearest tuned M; otherwise the heuristic
-    // -- unless the estimates are 10 % apart (1536 x 4608 x 3584: 41 us in the 256 x 256 tiles of M = 2048, 30 in 256 x 128 ones)
+    // -- unless the estimates are 15 % apart (1536 x 4608 x 3584: 41 us in the 256 x 256 tiles of M = 2048, 30 in 256 x 128 ones)
     int t, sp;
-    cfg->tile = heuristic_tile(M, N, K);
-    if (lookup_tile(M, N, K, &t, &sp) &&
-        fp8_tile_estimate(t, M, N, K, sp > 0 ? sp : heuristic_tile_split(t, M, N, K)) * 0.9 <= fp8_tile_estimate(cfg->tile, M, N, K, heuristic_tile_split(cfg->tile, M, N, K)))
-      cfg->tile = t, cfg->split_k = sp;
+    cfg->tile = heuristic_tile(M, N, K, &cfg->split_k);
+    if (lookup_tile(M, N, K, &t, &sp)) {
+      if (sp <= 0) sp = heuristic_tile_split(t, M, N, K);
+      if (fp8_tile_estimate(t, M, N, K, sp) * 0.85 <= fp8_tile_estimate(cfg->tile, M, N, K, cfg->split_k)) cfg->tile = t, cfg->split_k = sp;
+    }
   }
   if (cfg->tile == LLMMM_TILE_SKINNY) {
     if (cfg->split_k <= 0) cfg->split_k = heuristic_split(M, N, K);
