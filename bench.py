@@ -331,7 +331,7 @@ def bench_mlp_chain(M, steps, warmup, hidden=2560, inter=9728, rotate_bytes=768 
     ms, _ = _events_ms(step, steps, warmup, graph=True)
     return {"name": "qwen3_4b_mlp_block_m%d" % M, "M": M, "hidden": hidden, "intermediate": inter, "us": ms * 1e3,
             "hbm_gbs": per_copy / ms * 1e-6, "frac_of_hbm_peak": per_copy / ms * 1e-6 / PEAK_HBM_GBS, "weight_copies": copies,
-            "launches": "rmsnorm+quant, gate_up+swiglu (+reduce), down (+reduce)"}
+            "launches": "rmsnorm+quant, gate_up+swiglu, down (+reduce)"}
 
 
 def bench_proj_add_norm(name, M, steps, warmup, rotate_bytes=768 << 20):
@@ -483,9 +483,9 @@ def bench_decoder_layer(M, steps, warmup, rotate_bytes=768 << 20, consumer_side=
     if consumer_side:
         launches = "qkv on norm(down planes + residual) +norm+rope (2 kernels), o planes (1), gate_up fp32 on norm(o planes + residual) (1), down planes on silu(gate)*up (1)"
     elif M <= 4:
-        launches = "qkv+norm+rope (2 kernels), o+add+norm+quant (2), gate_up fp32 (1), down on silu(gate)*up +add+norm+quant (2)"
+        launches = "qkv+norm+rope (1 kernel), o+add+norm+quant (2), gate_up fp32 (1), down on silu(gate)*up +add+norm+quant (2)"
     else:
-        launches = "qkv+norm+rope (2 kernels), o+add+norm+quant (2), gate_up+swiglu (2), down+add+norm+quant (2)"
+        launches = "qkv+norm+rope (%d), o+add+norm+quant (2), gate_up+swiglu (1), down+add+norm+quant (2)" % (1 if M <= 8 else 2)
     return {"name": "qwen3_4b_decoder_layer_gemms_m%d%s" % (M, "_consumer_side" if consumer_side else ""), "M": M, "us": ms * 1e3, "weight_bytes": per_copy,
             "hbm_gbs": per_copy / ms * 1e-6, "frac_of_hbm_peak": per_copy / ms * 1e-6 / PEAK_HBM_GBS, "weight_copies": copies,
             "launches": launches + "; attention not included"}
