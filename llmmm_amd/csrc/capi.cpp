@@ -525,24 +525,33 @@ int rope_row_group(int M, int N, int K, int split)
   return split <= 1 && (M + 31) / 32 * heads <= NUM_CUS && K <= 2560 ? 32 : 0;
 }
 
+// A SwiGLU launch of exchanging workgroups that fills every CU (249 .. 256 of them, pair_place) loses at K = 4096, where the columns that an
+// XCD reads side by side meet on the same channels (32768 columns pre-shuffled, us, with planes / so: 27.7 / 32.2 at M = 1, 29.3 / 31.1 at 16,
+// 31.5 / 33.9 at 48 -- but 36.4 / 33.7 at 100, and K = 2048 15.7 / 14.8 at M = 1).
+bool swiglu_pair_camps(int N, int K) { return N / 128 > NUM_CUS - 8 && N / 128 <= NUM_CUS && K % 4096 == 0; }
+
 // The SwiGLU output of the weight-streaming kernel in one launch (64 gate + 64 up columns per workgroup, K unsplit; figures in
 // fp8_skinny.hip).  Its N / 128 workgroups have to fill the chip or a good part of its last round: with fewer, splitting K pulls more
 // (12288 x 2048, 96 workgroups, M = 24: 9.4 in two splits + reduce / 9.9 so), and 272 or 296 run a nearly empty second round
-// (34816 x 5120 at M = 1: 36.8 / 43.6; 51200 x 5120, 400 of them: 48.9 / 47.9 at M = 1, 54.6 / 49.2 at 16).
-bool swiglu_pair_pays(int M, int N, int K)
+// (34816 x 5120 at M = 1: 36.8 / 43.6; 51200 x 5120, 400 of them: 48.9 / 47.9 at M = 1, 54.6 / 49.2 at 16). 
+// Row-major weights, which stream less evenly, need more of them (12288 x 2048: 8.5 / 9.2 at M = 1, 9.3 / 10.6 at 16; 16384 x 3072 at M = 1
+// 13.9 / 14.7; pre-shuffled 8.7 / 8.8, 9.3 / 9.5 and 13.2 / 13.4 for a launch less).
+bool swiglu_pair_pays(int M, int N, int K, bool pre)
 {
   const int groups = N / 128, last = groups % NUM_CUS;
-  return llmmm::fp8_skinny_swiglu_fits(M, N, K) && groups >= (M <= 16 ? 96 : 128) && (groups <= NUM_CUS || last == 0 || last >= NUM_CUS / 2);
+  if (swiglu_pair_camps(N, K)) return false;
+  return llmmm::fp8_skinny_swiglu_fits(M, N, K) && groups >= (!pre ? 144 : M <= 16 ? 96 : 128) && (groups <= NUM_CUS || last == 0 || last >= NUM_CUS / 2);
 }
 
 // The SwiGLU output of fewer than 128 rows in 256-column tiles (a row tail; each holds whole 1x128 groups, so nothing is exchanged): from
 // 33 rows on where the 128-column ones would be more than one round of the chip, from 17 -- against the weight-streaming kernel -- where they
 // fill three quarters of a round (us, pre-shuffled, before / so: 37888 x 3584 43.4 / 35.8 at M = 48, 49.2 / 38.3 at 100; 34816 x 5120 63.8 / 50.9 at 100;
 // 57344 x 8192 115 / 83.7 at 100; 51200 x 5120, 200 tiles, 63.4 / 50.1 at 32, 59.0 / 48.9 at 20 -- but 148 tiles of 37888 x 3584 33.5 / 34.7 at 20).
-bool swiglu_wide_tail(int M, int N)
+// Up to 32 rows only with a long K: 65536 x 2048 30.4 / 32.5 at 24.
+bool swiglu_wide_tail(int M, int N, int K)
 {
   if (M >= 128 || N % 256) return false;
-  return M > 32 ? N / 128 > NUM_CUS : M > 16 && N / 256 >= NUM_CUS * 3 / 4 && N / 256 <= NUM_CUS;
+  return M > 32 ? N / 128 > NUM_CUS : M > 16 && K >= 4096 && N / 256 >= NUM_CUS * 3 / 4 && N / 256 <= NUM_CUS;
 }
 
 // The split the weight-streaming kernel runs this shape in when it is the split-K form after all (tune table, then heuristic).
@@ -874,8 +883,8 @@ int llmmm_fp8_gemm_ex(int out_kind, const void* A, const float* As, const void* 
       if (!aligned16(workspace)) return fail(LLMMM_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned");
       partial = (float*)workspace;
     }
-    const bool wide = swiglu && !agen && !(user && (user->split_k > 0 || user->tile != LLMMM_TILE_AUTO)) && swiglu_wide_tail(M, N);
-    const bool pair = swiglu && !wide && !agen && !(user && user->split_k > 0) && swiglu_pair_pays(M, N, K) && (pair_area = strip_exchange_area(stream)) >= 0;
+    const bool wide = swiglu && !agen && !(user && (user->split_k > 0 || user->tile != LLMMM_TILE_AUTO)) && swiglu_wide_tail(M, N, K);
+    const bool pair = swiglu && !wide && !agen && !(user && user->split_k > 0) && swiglu_pair_pays(M, N, K, cfg.b_layout == LLMMM_FP8_B_PRESHUFFLED) && (pair_area = strip_exchange_area(stream)) >= 0;
     if (wide)
       e = llmmm::fp8_gemm_launch(out_kind, LLMMM_TILE_128x256, cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, 1, nullptr, (hipStream_t)stream), partial = nullptr;
     else if (pair)
@@ -926,10 +935,10 @@ int llmmm_fp8_gemm_ex(int out_kind, const void* A, const float* As, const void* 
       planes = (float*)workspace;
     }
     int pair_area;
-    if (swiglu && cfg.tile == LLMMM_TILE_128x128 && split <= 1 && !(user && (user->split_k > 0 || user->tile != LLMMM_TILE_AUTO)) && swiglu_wide_tail(M, N))
+    if (swiglu && cfg.tile == LLMMM_TILE_128x128 && split <= 1 && !(user && (user->split_k > 0 || user->tile != LLMMM_TILE_AUTO)) && swiglu_wide_tail(M, N, K))
       e = llmmm::fp8_gemm_launch(out_kind, LLMMM_TILE_128x256, cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, 1, nullptr, (hipStream_t)stream);
     else if (swiglu && cfg.tile == LLMMM_TILE_128x128 && split <= 1 && !(user && user->split_k > 0) && llmmm::fp8_gemm_swiglu_pair_fits(M, N, K) &&
-        (pair_area = strip_exchange_area(stream)) >= 0)
+             !(M <= 64 && cfg.b_layout == LLMMM_FP8_B_PRESHUFFLED && swiglu_pair_camps(N, K)) && (pair_area = strip_exchange_area(stream)) >= 0)
       e = llmmm::fp8_gemm_swiglu_pair_launch(cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, pair_area, (hipStream_t)stream);
     else
       e = llmmm::fp8_gemm_launch(out_kind, cfg.tile, cfg.b_layout, A, As, Bt, Bs, C, Cs, M, N, K, split, planes, (hipStream_t)stream);

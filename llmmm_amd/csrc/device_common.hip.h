@@ -324,11 +324,30 @@ __device__ __forceinline__ void store_row4<_Float16>(_Float16* p, f32x4 v)
 // that holds zeros and clears its own slots of the other.  Which is which, a workgroup reads off its own row-0 slot of buffer 0 at kernel
 // entry: written by nobody else, and both halves of a block take part in every launch that touches it, so they agree.  The state
 // is kept per block of 16 rows, so launches with other row counts may follow each other.
-// Device-scope relaxed atomics and no fence: the slots are all that is shared.  Waiting is safe because the halves' workgroup ids
-// are 2j and 2j + 1 and ids are dispatched in order: the smallest incomplete pair always makes progress.  The wait is bounded
-// all the same (20 ms of the 100 MHz clock); a wave that gives up counts itself in *timeouts and goes on with what it has.
+// Device-scope relaxed atomics and no fence: the slots are all that is shared.  Waiting is safe because of where the halves sit
+// (pair_place).  The wait is bounded all the same (20 ms of the 100 MHz clock); a wave that gives up counts itself in *timeouts
+// and goes on with what it has.
 // ---------------------------------------------------------------------------------------------
 constexpr int PAIR_BLOCKS = 8;  // 16-row blocks of an area: M <= 128
+
+// The group and half of a workgroup of `total` (an even number).  Ids go to the eight XCDs in turn and each XCD dispatches its share in order.
+// Up to 31 workgroups per XCD the halves are neighbours by id: the smallest incomplete pair makes progress, and a second launch that waits
+// like this one cannot take an XCD whole, even where two XCDs begin the two in different order.  A larger launch can (32 CUs, one workgroup
+// on each), so its halves are eight ids apart, neighbours on one XCD, which then holds at most one incomplete pair of it.
+// (Of the last ids, fewer than 16, the halves lie closer: a workgroup or two of each XCD.)  Not for all launches, because it moves what the XCDs
+// read at a time: 28672 x 4096 pre-shuffled 22.5 us at M = 16 as neighbours by id, 25.4 on one XCD; other shapes differ by -3 .. +2 %.
+__device__ __forceinline__ void pair_place(int id, int total, int& group, int& half)
+{
+  if (total <= 8 * 31) {
+    group = id >> 1, half = id & 1;
+    return;
+  }
+  const int first = id & ~15, r = id - first;
+  const int apart = total - first >= 16 ? 8 : (total - first) >> 1;
+  half  = r >= apart ? 1 : 0;
+  group = (first >> 1) + r - half * apart;
+}
+
 struct PairSlots {
   unsigned* area;
   int       groups, group, half;

@@ -465,7 +465,11 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   const int wn   = wave / TC::WAVES_M;
   int       tm, tn;
   tile_coords(tile_index, tiles_m, tiles_n, tm, tn, PAIR || splits_in_turn<BN>(gridDim.y, tiles_m, tiles_n, K));
-  // (PAIR: tile = workgroup id, one tile row -- a pair's ids are 2j and 2j + 1, which PairSlots relies on)
+  if constexpr (PAIR) {  // one tile row; the two tiles of a 1x128 group wait for each other
+    int group, half;
+    pair_place(tile_index, tiles_n, group, half);
+    tn = 2 * group + half;
+  }
   // SwiGLU output: the tile's two 128-column halves are the gate columns n0 .. n0+127 and the up columns
   // N/2 + n0 .. of the same 128 output columns, so the weight rows of the upper half start N/2 - 128 rows further on
   constexpr bool SWIGLU = OUT == OUT_SWIGLU;

@@ -203,7 +203,12 @@ fp8_skinny_kernel(const uint8_t* __restrict__ A, const float* __restrict__ As, c
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g    = lane >> 4;
   const int i    = lane & 15;
-  const int ng   = blockIdx.x;
+  int       ng   = blockIdx.x;
+  if constexpr (OUT == SK_OUT_SWIGLU) {
+    int group, half;
+    pair_place(ng, gridDim.x, group, half);
+    ng = 2 * group + half;
+  }
   const int sp   = blockIdx.y;
   const int m0   = blockIdx.z * (16 * MBLK);  // row groups of 16 * MBLK rows: gridDim.z = number of groups
   const int KB   = K >> 7;

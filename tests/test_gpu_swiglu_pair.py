@@ -40,7 +40,7 @@ def _timeouts():
     return n.value
 
 
-@pytest.mark.parametrize("N,K", [(12288, 512), (19456, 2560), (32768, 640), (12288, 5120)])
+@pytest.mark.parametrize("N,K", [(12288, 512), (19456, 2560), (31744, 512), (32256, 512), (32768, 640), (12288, 5120)])
 @pytest.mark.parametrize("pre", [False, True])
 def test_bits_of_the_plane_route(oracle, N, K, pre):
     t, _ = _inputs(oracle, 32, N, K, 5, pre)
@@ -51,7 +51,7 @@ def test_bits_of_the_plane_route(oracle, N, K, pre):
     assert _timeouts() == 0
 
 
-@pytest.mark.parametrize("N,K", [(256, 128), (512, 256), (768, 384), (12288, 640), (19456, 2560), (65536, 128)])
+@pytest.mark.parametrize("N,K", [(256, 128), (512, 256), (768, 384), (12288, 640), (19456, 2560), (32000, 128), (65536, 128)])
 @pytest.mark.parametrize("pre", [False, True])
 def test_bits_of_the_plane_route_tiles(oracle, N, K, pre):
     from llmmm_amd import _lib
@@ -66,11 +66,15 @@ def test_bits_of_the_plane_route_tiles(oracle, N, K, pre):
     assert _timeouts() == 0
 
 
-@pytest.mark.parametrize("M,N,K", [(17, 49152, 128), (20, 49152, 384), (32, 51200, 256), (33, 33024, 640), (64, 33024, 256), (65, 33024, 128), (100, 37888, 512), (127, 33024, 384)])
+@pytest.mark.parametrize("M,N,K", [(17, 49152, 4096), (20, 51200, 4224), (32, 65536, 4096), (33, 33024, 640), (64, 33024, 256), (65, 33024, 128), (100, 37888, 512), (127, 33024, 384)])
 @pytest.mark.parametrize("pre", [False, True])
 def test_row_tails_in_wide_tiles(oracle, M, N, K, pre):
     """More 128-column tiles than CUs: 256-column tiles of fewer than 128 rows, which hold whole groups."""
-    t, _ = _inputs(oracle, M, N, K, M, pre)
+    if K < 4096:
+        t, _ = _inputs(oracle, M, N, K, M, pre)
+    else:  # (the weights of 1024 columns over and over, told apart by their scales)
+        t, _ = _inputs(oracle, M, 1024, K, M, pre)
+        t[2], t[3] = t[2].repeat(N // 1024, 1), t[3].repeat(N // 1024, 1) * torch.linspace(0.5, 1.5, N // 128, device="cuda")[:, None]
     guard = torch.full((M + 4, N // 2), 0x55, dtype=torch.uint8, device="cuda"), torch.full((N // 256 + 1, M), -1.0, device="cuda")
     got, want = _call(t, M, N, K, pre, out=guard), _call(t, M, N, K, pre, split=1)
     assert _same((got[0][:M], got[1][:-1]), want)
@@ -83,14 +87,14 @@ def test_launches_that_change_rows_and_shapes(oracle):
     cases = []
     for i, (M, N, K) in enumerate([(1, 12288, 512), (32, 19456, 512), (16, 12288, 640), (17, 32768, 512), (3, 19456, 512), (32, 12288 + 4096, 512),
                                    (48, 12288, 512), (128, 19456, 256), (100, 12288, 256), (33, 24576, 128)]):
-        t, _ = _inputs(oracle, M, N, K, 10 + i, False)
+        t, _ = _inputs(oracle, M, N, K, 10 + i, True)
         t[1] = t[1] * (2.0 ** i)
-        cases.append((t, M, N, K, _call(t, M, N, K, False, split=1)))
+        cases.append((t, M, N, K, _call(t, M, N, K, True, split=1)))
     outs = [[(torch.empty_like(c[4][0]), torch.empty_like(c[4][1])) for c in cases] for _ in range(4)]
     ws = torch.empty(128 * 32768, device="cuda")
     for o in outs:
         for c, out in zip(cases, o):
-            _call(c[0], c[1], c[2], c[3], False, out=out, ws=ws, tile=_lib.TILE_128x128 if c[1] > 32 else None)
+            _call(c[0], c[1], c[2], c[3], True, out=out, ws=ws, tile=_lib.TILE_128x128 if c[1] > 32 else None)
     for o in outs:
         for x, c in zip(o, cases):
             assert _same(x, c[4]), c[1:4]
@@ -100,7 +104,7 @@ def test_launches_that_change_rows_and_shapes(oracle):
 @pytest.mark.parametrize("M", [16, 100])
 def test_captured_with_other_work_between_replays(oracle, M):
     from llmmm_amd import _lib
-    N, K = 12288, 512
+    N, K = 19456, 512
     tile = _lib.TILE_128x128 if M > 32 else None
     t, _ = _inputs(oracle, M, N, K, 3, False)
     out, ws = (torch.empty((M, N // 2), dtype=torch.uint8, device="cuda"), torch.empty((N // 256, M), device="cuda")), torch.empty(M * N, device="cuda")
@@ -127,7 +131,7 @@ def test_captured_with_other_work_between_replays(oracle, M):
 @pytest.mark.parametrize("M", [5, 40])
 def test_non_finite_operands(oracle, M):
     from llmmm_amd import _lib
-    N, K = 12288, 512
+    N, K = 19456, 512
     t, _ = _inputs(oracle, M, N, K, 4, False)
     t[0][1, 7] = 0x7F            # NaN code
     t[1][2, 3] = float("inf")
