@@ -75,13 +75,17 @@ __device__ __forceinline__ void fp8_load_lds_16B(const void* sbase, unsigned vof
 {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
 }
-// The same load with the non-temporal hint, for weights that only one workgroup reads (a single
+// The loads of the K loop: to lds + AT.  NT: the non-temporal hint, for weights that only one workgroup reads (a single
 // tile row): streamed through, they do not displace the activations and scales every workgroup
 // shares.  Measured: about 1 us faster at M = 128 on the N = 19456 and K = 9728 shapes -- and 10-50 %
 // slower wherever several tile rows re-read the weights from the L2, so only used for one row.
-__device__ __forceinline__ void fp8_load_lds_16B_nt(const void* sbase, unsigned voff, unsigned lds_addr)
+template <bool NT, int AT>
+__device__ __forceinline__ void fp8_load_lds_16B_at(const void* sbase, unsigned voff, unsigned lds)
 {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+  if constexpr (NT)
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(sbase), "s"(lds), "n"(AT) : "memory", "scc");
+  else
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds), "n"(AT) : "memory", "scc");
 }
 template <int IMM>
 __device__ __forceinline__ void fp8_load_f32(float& dst, const void* sbase, unsigned voff)
@@ -89,46 +93,39 @@ __device__ __forceinline__ void fp8_load_f32(float& dst, const void* sbase, unsi
   asm volatile("global_load_dword %0, %1, %2 offset:%3" : "=v"(dst) : "v"(voff), "s"(sbase), "n"(IMM) : "memory");
 }
 
-// Load i (0 .. A_LOADS + B_LOADS - 1) of a wave for one stage.  All loads of a wave share one
-// per-lane offset: load i covers tile rows 8*(wave + i*NW) .. +7, and the SWZ_ROWS16 placement
-// only looks at row bits 0..3, so moving by 8*NW (>= 16) rows changes nothing but the
-// wave-uniform row base.
+// Load i (0 .. A_LOADS + B_LOADS - 1) of a wave for one stage covers tile rows 8*(wave + i*NW) .. +7 of A or of Bt; its lanes' byte offsets from the tile's
+// first row are constants of the kernel (off), its place in LDS is a constant behind the wave's first (lds_wave = stage + 1024 * wave).  What is left per load
+// is one scalar addition: the K loops are short of instruction slots.  (With the rows' distance added to a 64-bit base for every load, 266 instructions per
+// slice and wave of the 256 x 256 tile instead of 252 and 233 instead of 218 of the deep 128 x 160 one; us, then / now: 384 x 3584 x 18944 35.7 / 34.9,
+// 4096^3 54.5 / 54.3, 4096 rows through a layer of hidden 8192 2914 / 2903.  One scalar instruction more per load, a mask on EXEC, cost 2 .. 5 %.)
 //
 // Pre-shuffled weights (layout.hip) hold the same LDS image as consecutive 1 KB half blocks: half
 // block h of row group rg and slice kb at ((rg * K/128 + kb) * 2 + h) * 1024.  Rows 8*NW apart
-// are then 8*NW*K bytes apart as well, so only the per-lane offset (16 * lane instead of
+// are then 8*NW*K bytes apart as well, so only the lane's own offset (16 * lane instead of
 // row * K + chunk * 16, the wave's own rows folded into the base) and the step from slice to
 // slice (2048 instead of 128 bytes) differ between the two layouts.
-//
-// MT (a last tile row with fewer than BM rows of A): the lanes of load i whose row lies beyond the matrix fetch its
-// last row instead, so the per-lane offset differs from load to load -- a_tail[i], relative to the tile's first row.
-template <int BM, int BN, int WM, bool BNT, int I, bool MT = false>
-__device__ __forceinline__ void fp8_issue_load(unsigned lds_stage, const uint8_t* Ag, const uint8_t* Bg, unsigned a_off, unsigned b_off, int K, size_t b_hi, int wave,
-                                               const unsigned* a_tail = nullptr)
+template <int NLOADS>
+struct Fp8Offsets {
+  unsigned off[NLOADS];
+};
+template <int BM, int BN, int WM, bool BNT, int I>
+__device__ __forceinline__ void fp8_issue_load(unsigned lds_wave, const uint8_t* Ag, const uint8_t* Bg, const uint8_t* Bg_hi,
+                                               const Fp8Offsets<Fp8Tile<BM, BN, WM>::A_LOADS + Fp8Tile<BM, BN, WM>::B_LOADS>& o)
 {
   typedef Fp8Tile<BM, BN, WM> TC;
-  // b_hi: extra byte offset of the tile's upper half of weight rows (0 unless the two halves come from different row ranges)
-  const size_t b_skip = I - TC::A_LOADS >= TC::B_LOADS / 2 ? b_hi : 0;
-  if constexpr (I < TC::A_LOADS) {
-    if constexpr (MT)
-      fp8_load_lds_16B(Ag, a_tail[I], lds_stage + (wave + I * TC::NW) * 1024);
-    else
-      fp8_load_lds_16B(Ag + (size_t)(8 * TC::NW * I) * K, a_off, lds_stage + (wave + I * TC::NW) * 1024);
-  }
-  else if constexpr (I < TC::A_LOADS + TC::B_LOADS) {
-    if constexpr (BNT)
-      fp8_load_lds_16B_nt(Bg + (size_t)(8 * TC::NW * (I - TC::A_LOADS)) * K + b_skip, b_off, lds_stage + TC::A_BYTES + (wave + (I - TC::A_LOADS) * TC::NW) * 1024);
-    else
-      fp8_load_lds_16B(Bg + (size_t)(8 * TC::NW * (I - TC::A_LOADS)) * K + b_skip, b_off, lds_stage + TC::A_BYTES + (wave + (I - TC::A_LOADS) * TC::NW) * 1024);
-  }
+  // Bg_hi: the base of the tile's upper half of weight rows (Bg unless the two halves come from different row ranges)
+  if constexpr (I < TC::A_LOADS)
+    fp8_load_lds_16B_at<false, I * TC::NW * 1024>(Ag, o.off[I], lds_wave);
+  else if constexpr (I < TC::A_LOADS + TC::B_LOADS)
+    fp8_load_lds_16B_at<BNT, TC::A_BYTES + (I - TC::A_LOADS) * TC::NW * 1024>(I - TC::A_LOADS >= TC::B_LOADS / 2 ? Bg_hi : Bg, o.off[I], lds_wave);
 }
-template <int BM, int BN, int WM, bool BNT, int FIRST, int COUNT, bool MT = false>
-__device__ __forceinline__ void fp8_issue_loads(unsigned lds_stage, const uint8_t* Ag, const uint8_t* Bg, unsigned a_off, unsigned b_off, int K, size_t b_hi, int wave,
-                                                const unsigned* a_tail = nullptr)
+template <int BM, int BN, int WM, bool BNT, int FIRST, int COUNT>
+__device__ __forceinline__ void fp8_issue_loads(unsigned lds_wave, const uint8_t* Ag, const uint8_t* Bg, const uint8_t* Bg_hi,
+                                                const Fp8Offsets<Fp8Tile<BM, BN, WM>::A_LOADS + Fp8Tile<BM, BN, WM>::B_LOADS>& o)
 {
   if constexpr (COUNT > 0) {
-    fp8_issue_load<BM, BN, WM, BNT, FIRST, MT>(lds_stage, Ag, Bg, a_off, b_off, K, b_hi, wave, a_tail);
-    fp8_issue_loads<BM, BN, WM, BNT, FIRST + 1, COUNT - 1, MT>(lds_stage, Ag, Bg, a_off, b_off, K, b_hi, wave, a_tail);
+    fp8_issue_load<BM, BN, WM, BNT, FIRST>(lds_wave, Ag, Bg, Bg_hi, o);
+    fp8_issue_loads<BM, BN, WM, BNT, FIRST + 1, COUNT - 1>(lds_wave, Ag, Bg, Bg_hi, o);
   }
 }
 // The slice scales of the lane's four 16-row fragments and of the wave's column group.
@@ -162,9 +159,10 @@ __device__ __forceinline__ i32x8 fp8_read_frag(const char LLMMM_LDS* tile, int r
 
 // What a slice issues for its successor while it computes.
 struct Fp8Next {
-  unsigned       lds_stage;  // LDS byte address of the stage buffer to fill
+  unsigned       lds_stage;  // LDS byte address of the stage buffer to fill, plus 1024 * wave
   const uint8_t* Ag;         // tile's A rows / Bt rows at the next slice's k offset
   const uint8_t* Bg;
+  const uint8_t* Bg_hi;
   const float*   As_slice;   // As + kb_next * M
   const float*   Bs_elem;    // &Bs[nb, kb_next]
   const float*   Bs_elem2;   // 160-column waves: &Bs[nb + 1, kb_next]
@@ -185,11 +183,11 @@ __device__ __forceinline__ void fp8_scale_load_lds(const char* lane_ptr, unsigne
 // work waits, and early enough to land within the slice), its scales during the fifth.
 // 160-column waves (NF = 10): fragments nf < nfb lie in the first weight-scale block and take s, the others s2.
 // PAIR: 64 gate and 64 up columns, fragments 0 .. 3 and 4 .. 7: s and s2 likewise.
-template <int BM, int BN, int WM, bool BNT, bool LOAD, bool SCALE_LDS = false, bool MT = false, bool PAIR = false>
+template <int BM, int BN, int WM, bool BNT, bool LOAD, bool SCALE_LDS = false, bool PAIR = false>
 __device__ __forceinline__ void fp8_compute_stage(const char LLMMM_LDS* lds, int a_rd0, int a_rd1, int b_rd0, int b_rd1,
-                                                  const float (&s)[WM / 16], f32x4 (&acc)[Fp8Tile<BM, BN, WM>::NF][WM / 16], const Fp8Next& nx, unsigned lane_off,
-                                                  unsigned b_lane_off, unsigned row_off, unsigned zero, int K, size_t b_hi, int wave, float (&sa_next)[WM / 16],
-                                                  float& sb_next, const float (&s2)[WM / 16], int nfb, float& sb2_next, const unsigned* a_tail = nullptr)
+                                                  const float (&s)[WM / 16], f32x4 (&acc)[Fp8Tile<BM, BN, WM>::NF][WM / 16], const Fp8Next& nx,
+                                                  const Fp8Offsets<Fp8Tile<BM, BN, WM>::A_LOADS + Fp8Tile<BM, BN, WM>::B_LOADS>& off, unsigned row_off, unsigned zero,
+                                                  int wave, float (&sa_next)[WM / 16], float& sb_next, const float (&s2)[WM / 16], int nfb, float& sb2_next)
 {
   constexpr int MF = WM / 16;
   typedef Fp8Tile<BM, BN, WM> TC;
@@ -214,13 +212,13 @@ __device__ __forceinline__ void fp8_compute_stage(const char LLMMM_LDS* lds, int
     const int cur = nf & 1;
     if (nf + 1 < NF) b[cur ^ 1] = fp8_read_frag(ldsB, b_rd0, b_rd1, (nf + 1) * 2048);
     if constexpr (LOAD) {
-      if (nf == 0) fp8_issue_loads<BM, BN, WM, BNT, 0, LPG, MT>(nx.lds_stage, nx.Ag, nx.Bg, lane_off, b_lane_off, K, b_hi, wave, a_tail);
-      if (nf == 1) fp8_issue_loads<BM, BN, WM, BNT, LPG, LPG, MT>(nx.lds_stage, nx.Ag, nx.Bg, lane_off, b_lane_off, K, b_hi, wave, a_tail);
-      if (nf == 2) fp8_issue_loads<BM, BN, WM, BNT, 2 * LPG, LPG, MT>(nx.lds_stage, nx.Ag, nx.Bg, lane_off, b_lane_off, K, b_hi, wave, a_tail);
-      if (nf == 3) fp8_issue_loads<BM, BN, WM, BNT, 3 * LPG, LPG, MT>(nx.lds_stage, nx.Ag, nx.Bg, lane_off, b_lane_off, K, b_hi, wave, a_tail);
+      if (nf == 0) fp8_issue_loads<BM, BN, WM, BNT, 0, LPG>(nx.lds_stage, nx.Ag, nx.Bg, nx.Bg_hi, off);
+      if (nf == 1) fp8_issue_loads<BM, BN, WM, BNT, LPG, LPG>(nx.lds_stage, nx.Ag, nx.Bg, nx.Bg_hi, off);
+      if (nf == 2) fp8_issue_loads<BM, BN, WM, BNT, 2 * LPG, LPG>(nx.lds_stage, nx.Ag, nx.Bg, nx.Bg_hi, off);
+      if (nf == 3) fp8_issue_loads<BM, BN, WM, BNT, 3 * LPG, LPG>(nx.lds_stage, nx.Ag, nx.Bg, nx.Bg_hi, off);
       if (nf == 4) {
         if constexpr (SCALE_LDS)
-          fp8_scale_load_lds(nx.sc_ptr, nx.lds_stage + TC::STAGE + wave * 256);
+          fp8_scale_load_lds(nx.sc_ptr, nx.lds_stage + TC::STAGE - wave * 768);
         else
           fp8_issue_scales<MF, TWO>(sa_next, sb_next, nx.As_slice, row_off, nx.Bs_elem, zero, &sb2_next, nx.Bs_elem2);
       }
@@ -492,6 +490,14 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   const uint8_t*   Bg         = BPRE ? Bt + (size_t)(n0 + 16 * (wave >> 1)) * K + (wave & 1) * 1024 + (size_t)kb0 * 2048
                                      : Bt + (size_t)n0 * K + (size_t)kb0 * 128;
 
+  const uint8_t*   Bh         = Bg + b_hi;
+  // MT (a last tile row with fewer than BM rows of A): the lanes whose row lies beyond the matrix fetch its last row instead
+  Fp8Offsets<TC::A_LOADS + TC::B_LOADS> off;
+#pragma unroll
+  for (int i = 0; i < TC::A_LOADS; ++i) off.off[i] = (unsigned)((MT ? min(lp.row + 8 * TC::NW * i, M - 1 - m0) : lp.row + 8 * TC::NW * i) * K + lp.chunk * 16);
+#pragma unroll
+  for (int i = 0; i < TC::B_LOADS; ++i) off.off[TC::A_LOADS + i] = b_lane_off + (unsigned)(8 * TC::NW * i) * (unsigned)K;
+
   // operand reads: lane = (g = lane/16, i = lane%16) takes row i of a 16-row fragment and the
   // 32 bytes k = 32g .. 32g+31 (chunks 2g and 2g+1)
   const int g     = lane >> 4;
@@ -518,15 +524,13 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   float sa_next[MF], sb_next, sb2_next = 0.f;
 
   const unsigned lds0 = (unsigned)(size_t)(char LLMMM_LDS*)lds;
+  const unsigned ldsw = lds0 + wave * 1024;  // of the wave's first load
   char LLMMM_LDS* const s0 = (char LLMMM_LDS*)lds;
 
   const PairSlots pair = {op.xch.slots, op.xch.tag, op.xch.wait, 1, M, tn >> 1, tn & 1};  // PAIR: one wave reads a row
 
   if constexpr (DEEP) {
     constexpr int PER = TC::A_LOADS + TC::B_LOADS + 1;  // vector-memory loads of a wave per slice
-    unsigned a_tail[TC::A_LOADS];  // MT: per-load offsets with the row clamped to the matrix
-#pragma unroll
-    for (int i = 0; i < TC::A_LOADS; ++i) a_tail[i] = MT ? (unsigned)(min(lp.row + 8 * TC::NW * i, M - 1 - m0) * K + lp.chunk * 16) : 0u;
     static_assert((NST - 2) * PER < 64, "vmcnt is a 6-bit counter");
     // this lane's scale source: a row scale (stride M floats per slice) or the column-group scale (stride 1)
     const bool     row_lane = lane < WM;
@@ -536,8 +540,7 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
 #pragma unroll
     for (int u = 0; u < NST - 1; ++u) {
       const int kk = min(u, KBL - 1);
-      fp8_issue_loads<BM, BN, WM, BNT, 0, TC::A_LOADS + TC::B_LOADS, MT>(lds0 + u * STAGE_D, Ag + (size_t)kk * 128, Bg + (size_t)kk * B_KSTEP, lane_off,
-                                                                         b_lane_off, K, b_hi, wave, a_tail);
+      fp8_issue_loads<BM, BN, WM, BNT, 0, TC::A_LOADS + TC::B_LOADS>(ldsw + u * STAGE_D, Ag + (size_t)kk * 128, Bg + (size_t)kk * B_KSTEP, Bh + (size_t)kk * B_KSTEP, off);
       fp8_scale_load_lds(sc_ptr + (size_t)kk * sc_step, lds0 + u * STAGE_D + TC::STAGE + wave * 256);
     }
     const char* sc_next = sc_ptr + (size_t)(NST - 1) * sc_step;
@@ -555,15 +558,16 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
       s[mf] = sa_ * sb_, s2[mf] = sa_ * sb2_;                                                                                     \
     }                                                                                                                             \
     Fp8Next nx;                                                                                                                   \
-    nx.lds_stage = lds0 + (cur == 0 ? (NST - 1) * STAGE_D : cur - STAGE_D);                                                       \
+    nx.lds_stage = ldsw + (cur == 0 ? (NST - 1) * STAGE_D : cur - STAGE_D);                                                       \
     nx.Ag        = Ag + (size_t)(kc + NST - 1) * 128;                                                                             \
     nx.Bg        = Bg + (size_t)(kc + NST - 1) * B_KSTEP;                                                                         \
+    nx.Bg_hi     = Bh + (size_t)(kc + NST - 1) * B_KSTEP;                                                                         \
     nx.As_slice  = nullptr;                                                                                                       \
     nx.Bs_elem   = nullptr;                                                                                                       \
     nx.Bs_elem2  = nullptr;                                                                                                       \
     nx.sc_ptr    = sc_next;                                                                                                       \
-    fp8_compute_stage<BM, BN, WM, BNT, LOAD, true, MT, PAIR>(s0 + cur, a_rd0, a_rd1, b_rd0, b_rd1, s, acc, nx, lane_off, b_lane_off, row_off, zero, K, \
-                                                       b_hi, wave, sa_next, sb_next, s2, nfb, sb2_next, a_tail);                  \
+    fp8_compute_stage<BM, BN, WM, BNT, LOAD, true, PAIR>(s0 + cur, a_rd0, a_rd1, b_rd0, b_rd1, s, acc, nx, off, row_off, zero, wave, sa_next, sb_next, s2, nfb, \
+                                                         sb2_next);                                                               \
     cur = cur + STAGE_D == NST * STAGE_D ? 0 : cur + STAGE_D;                                                                     \
   }
     int kc = 0;
@@ -580,7 +584,7 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
     wait_vmcnt<0>();  // repeats of the last slice that a short K range left in flight
   }
   else {
-  fp8_issue_loads<BM, BN, WM, BNT, 0, TC::A_LOADS + TC::B_LOADS>(lds0, Ag, Bg, lane_off, b_lane_off, K, b_hi, wave);
+  fp8_issue_loads<BM, BN, WM, BNT, 0, TC::A_LOADS + TC::B_LOADS>(ldsw, Ag, Bg, Bh, off);
   fp8_issue_scales<MF, TWO>(sa_next, sb_next, Asl, row_off, Bsp, zero, &sb2_next, Bsp2);
 
   // One slice: wait for this wave's loads of the slice (all of them were issued at least half a
@@ -609,17 +613,17 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
     Fp8Next nx;                                                                                                                   \
     nx.lds_stage = NXT_LDS;                                                                                                       \
     nx.Ag        = Ag + (size_t)((KC) + 1) * 128;                                                                                 \
-    nx.Bg        = Bg + (size_t)((KC) + 1) * B_KSTEP;                                                                               \
+    nx.Bg        = Bg + (size_t)((KC) + 1) * B_KSTEP;                                                                             \
+    nx.Bg_hi     = Bh + (size_t)((KC) + 1) * B_KSTEP;                                                                             \
     nx.As_slice  = Asl + (size_t)((KC) + 1) * M;                                                                                  \
     nx.Bs_elem   = Bsp + (KC) + 1;                                                                                                \
     nx.Bs_elem2  = Bsp2 + (KC) + 1;                                                                                               \
-    fp8_compute_stage<BM, BN, WM, BNT, LOAD>(CUR, a_rd0, a_rd1, b_rd0, b_rd1, s, acc, nx, lane_off, b_lane_off, row_off, zero, K, b_hi, wave, sa_next, \
-                                    sb_next, s2, nfb, sb2_next);                                                                  \
+    fp8_compute_stage<BM, BN, WM, BNT, LOAD>(CUR, a_rd0, a_rd1, b_rd0, b_rd1, s, acc, nx, off, row_off, zero, wave, sa_next, sb_next, s2, nfb, sb2_next); \
   }
 
   unsigned cur = 0;  // byte offset of the stage being computed: 0 or STAGE
   for (int kc = 0; kc < KBL - 1; ++kc) {
-    LLMMM_FP8_SLICE(true, s0 + cur, lds0 + (TC::STAGE - cur), kc)
+    LLMMM_FP8_SLICE(true, s0 + cur, ldsw + (TC::STAGE - cur), kc)
     cur = TC::STAGE - cur;
   }
   LLMMM_FP8_SLICE(false, s0 + cur, 0u, KBL - 1)
