@@ -87,6 +87,20 @@ __device__ __forceinline__ void fp8_load_lds_16B_at(const void* sbase, unsigned 
   else
     asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds), "n"(AT) : "memory", "scc");
 }
+// The same in two halves, M0 and the load, with another instruction between them in place of the wait state.
+template <int AT>
+__device__ __forceinline__ void fp8_set_m0(unsigned lds)
+{
+  asm volatile("s_add_u32 m0, %0, %1" ::"s"(lds), "n"(AT) : "memory", "scc");
+}
+template <bool NT>
+__device__ __forceinline__ void fp8_load_lds_16B_m0(const void* sbase, unsigned voff)
+{
+  if constexpr (NT)
+    asm volatile("global_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(sbase) : "memory");
+  else
+    asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase) : "memory");
+}
 template <int IMM>
 __device__ __forceinline__ void fp8_load_f32(float& dst, const void* sbase, unsigned voff)
 {
@@ -118,6 +132,23 @@ __device__ __forceinline__ void fp8_issue_load(unsigned lds_wave, const uint8_t*
     fp8_load_lds_16B_at<false, I * TC::NW * 1024>(Ag, o.off[I], lds_wave);
   else if constexpr (I < TC::A_LOADS + TC::B_LOADS)
     fp8_load_lds_16B_at<BNT, TC::A_BYTES + (I - TC::A_LOADS) * TC::NW * 1024>(I - TC::A_LOADS >= TC::B_LOADS / 2 ? Bg_hi : Bg, o.off[I], lds_wave);
+}
+// ... in two halves (loads past the last: nothing)
+template <int BM, int BN, int WM, int I>
+__device__ __forceinline__ void fp8_issue_m0(unsigned lds_wave)
+{
+  typedef Fp8Tile<BM, BN, WM> TC;
+  if constexpr (I < TC::A_LOADS + TC::B_LOADS) fp8_set_m0<I < TC::A_LOADS ? I * TC::NW * 1024 : TC::A_BYTES + (I - TC::A_LOADS) * TC::NW * 1024>(lds_wave);
+}
+template <int BM, int BN, int WM, bool BNT, int I>
+__device__ __forceinline__ void fp8_issue_behind_m0(const uint8_t* Ag, const uint8_t* Bg, const uint8_t* Bg_hi,
+                                                    const Fp8Offsets<Fp8Tile<BM, BN, WM>::A_LOADS + Fp8Tile<BM, BN, WM>::B_LOADS>& o)
+{
+  typedef Fp8Tile<BM, BN, WM> TC;
+  if constexpr (I < TC::A_LOADS)
+    fp8_load_lds_16B_m0<false>(Ag, o.off[I]);
+  else if constexpr (I < TC::A_LOADS + TC::B_LOADS)
+    fp8_load_lds_16B_m0<BNT>(I - TC::A_LOADS >= TC::B_LOADS / 2 ? Bg_hi : Bg, o.off[I]);
 }
 template <int BM, int BN, int WM, bool BNT, int FIRST, int COUNT>
 __device__ __forceinline__ void fp8_issue_loads(unsigned lds_wave, const uint8_t* Ag, const uint8_t* Bg, const uint8_t* Bg_hi,
@@ -207,15 +238,45 @@ __device__ __forceinline__ void fp8_compute_stage(const char LLMMM_LDS* lds, int
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int mf = 1; mf < MF; ++mf) a[mf] = fp8_read_frag(ldsA, a_rd0, a_rd1, mf * 2048);
+  constexpr bool HALVES = MF == 2;
+  static_assert(NF >= 5 && (LPG == 2 || LPG == 3), "two or three loads in each of the first four fragment steps");
 #pragma unroll
   for (int nf = 0; nf < NF; ++nf) {
     const int cur = nf & 1;
-    if (nf + 1 < NF) b[cur ^ 1] = fp8_read_frag(ldsB, b_rd0, b_rd1, (nf + 1) * 2048);
-    if constexpr (LOAD) {
+    // 32-row waves (HALVES): a step's first load has the fragment's LDS reads between M0 and itself, its second the step's MFMAs.  Eight wait states fewer per
+    // slice: a prefill layer of 2048 rows (O and down in deep 128 x 160 tiles) 1.0 % faster, 257.6 us before this and the constant offsets, 254.2 with
+    // both; 384 x 3584 x 18944 0.3 .. 1.5 %, 35.7 / 34.8 likewise.  64-row waves gain 0.6 % at 4096^3 and lose 0.9 % where a launch is long enough for the
+    // power limit to decide (a layer of 4096 rows, hidden 8192), and keep the wait states.
+#define LLMMM_FP8_STEP_HEAD(S)                                                          \
+  if (nf == S) {                                                                        \
+    fp8_issue_m0<BM, BN, WM, S * LPG>(nx.lds_stage);                                    \
+    __builtin_amdgcn_sched_barrier(0);                                                  \
+    b[cur ^ 1] = fp8_read_frag(ldsB, b_rd0, b_rd1, (nf + 1) * 2048);                    \
+    __builtin_amdgcn_sched_barrier(0);                                                  \
+    fp8_issue_behind_m0<BM, BN, WM, BNT, S * LPG>(nx.Ag, nx.Bg, nx.Bg_hi, off);         \
+    fp8_issue_m0<BM, BN, WM, S * LPG + 1>(nx.lds_stage);                                \
+  }
+#define LLMMM_FP8_STEP_TAIL(S)                                                          \
+  if (nf == S) {                                                                        \
+    fp8_issue_behind_m0<BM, BN, WM, BNT, S * LPG + 1>(nx.Ag, nx.Bg, nx.Bg_hi, off);     \
+    fp8_issue_loads<BM, BN, WM, BNT, S * LPG + 2, LPG - 2>(nx.lds_stage, nx.Ag, nx.Bg, nx.Bg_hi, off); \
+  }
+    if (!LOAD || !HALVES || nf >= 4) {
+      if (nf + 1 < NF) b[cur ^ 1] = fp8_read_frag(ldsB, b_rd0, b_rd1, (nf + 1) * 2048);
+    }
+    if constexpr (LOAD && !HALVES) {
       if (nf == 0) fp8_issue_loads<BM, BN, WM, BNT, 0, LPG>(nx.lds_stage, nx.Ag, nx.Bg, nx.Bg_hi, off);
       if (nf == 1) fp8_issue_loads<BM, BN, WM, BNT, LPG, LPG>(nx.lds_stage, nx.Ag, nx.Bg, nx.Bg_hi, off);
       if (nf == 2) fp8_issue_loads<BM, BN, WM, BNT, 2 * LPG, LPG>(nx.lds_stage, nx.Ag, nx.Bg, nx.Bg_hi, off);
       if (nf == 3) fp8_issue_loads<BM, BN, WM, BNT, 3 * LPG, LPG>(nx.lds_stage, nx.Ag, nx.Bg, nx.Bg_hi, off);
+    }
+    if constexpr (LOAD && HALVES) {
+      LLMMM_FP8_STEP_HEAD(0)
+      LLMMM_FP8_STEP_HEAD(1)
+      LLMMM_FP8_STEP_HEAD(2)
+      LLMMM_FP8_STEP_HEAD(3)
+    }
+    if constexpr (LOAD) {
       if (nf == 4) {
         if constexpr (SCALE_LDS)
           fp8_scale_load_lds(nx.sc_ptr, nx.lds_stage + TC::STAGE - wave * 768);
@@ -244,7 +305,15 @@ __device__ __forceinline__ void fp8_compute_stage(const char LLMMM_LDS* lds, int
       }
     }
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (LOAD && HALVES) {
+      LLMMM_FP8_STEP_TAIL(0)
+      LLMMM_FP8_STEP_TAIL(1)
+      LLMMM_FP8_STEP_TAIL(2)
+      LLMMM_FP8_STEP_TAIL(3)
+    }
   }
+#undef LLMMM_FP8_STEP_HEAD
+#undef LLMMM_FP8_STEP_TAIL
 #pragma unroll
   for (int mf = 0; mf < MF; ++mf) {
     const float sc = TWO ? (NF - 1 < nfb ? s[mf] : s2[mf]) : s[mf];
