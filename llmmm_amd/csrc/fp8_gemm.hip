@@ -386,29 +386,41 @@ __device__ __forceinline__ void swiglu_finish(const f32x4 (&acc)[8][MF], const f
 // rotation reads them back in.  Half of the rows per pass, every load of a pass in flight at once and none of them
 // holding registers: fetched into registers instead, the 128 accumulator registers leave room for a few pieces at a
 // time and the epilogue pays one L2 round trip after the other (2048 x 6144 x 2560: 43 us with, 33.6 us without rope).
-template <int MF>
-__device__ __forceinline__ void qk_norm_rope_fragments(f32x4 (&acc)[8][MF], const Fp8HeadOp& op, int head, int row0, int lane, char LLMMM_LDS* tab)
+// SHARED (two heads per tile): waves wave0 and wave0 + partner hold the same rows of two heads and need the same angles.  Each fetches those of one half of
+// the rows, all at once, and reads both halves behind a barrier: half the table bytes through the CU's load path and one round trip instead of two.
+// (2048 x 6144 x 2560 45.4 us, now 42.5; 4096 x 6144 x 4096 103.7 / 101.0; 1024 x 6144 x 2560 28.4 / 28.1, these with the loads of the K loop.)
+// (`tab`: the piece of wave 0; head0: the tile's first head.)
+template <int MF, bool SHARED>
+__device__ __forceinline__ void qk_norm_rope_fragments(f32x4 (&acc)[8][MF], const Fp8HeadOp& op, int head0, int wn, int row0, int lane, char LLMMM_LDS* tab, int wave0, int partner)
 {
-  if (head >= op.n_q + op.n_kv) return;  // value head (wave-uniform)
-  constexpr int MFP = MF / 2;            // 16-row fragments per pass
+  const int heads = op.n_q + op.n_kv, head = head0 + wn;
+  if ((SHARED ? head0 : head) >= heads) return;  // value heads only (wave-uniform; SHARED: the whole workgroup)
+  constexpr int MFP = MF / 2;  // 16-row fragments per pass
   static_assert(MF % 2 == 0, "two passes");
-  const int      g = lane >> 4, li = lane & 15;
-  const unsigned tab_addr = (unsigned)(size_t)tab;
-  unsigned       toff[MF];  // byte offset of the lane's first piece in either table
+  const int                   g = lane >> 4, li = lane & 15;
+  constexpr int               PIECE = MF * 4096;
+  char LLMMM_LDS* const       mine  = tab + (wave0 + (SHARED ? wn * partner : 0)) * PIECE;
+  const char LLMMM_LDS* const at0   = tab + wave0 * PIECE;
+  const char LLMMM_LDS* const at1   = SHARED ? at0 + partner * PIECE : at0;
+  // pass h: pieces (m, nf, table) of fragments mf = h * MFP + m at + ((m * 4 + nf) * 2 + table) * 1024
+  const auto fetch = [&](int h) {
+    const unsigned to = (unsigned)(size_t)mine;
 #pragma unroll
-  for (int mf = 0; mf < MF; ++mf) toff[mf] = (unsigned)min(max(op.pos[row0 + mf * 16 + li], 0), op.table_rows - 1) * 256u + 16u * g;
-  // pass h: pieces (m, nf, table) of fragments mf = h * MFP + m at tab + ((m * 4 + nf) * 2 + table) * 1024
-#define LLMMM_ROPE_FETCH(H)                                                                                  \
-  _Pragma("unroll") for (int m = 0; m < MFP; ++m) _Pragma("unroll") for (int nf = 0; nf < 4; ++nf) {         \
-    fp8_load_lds_16B(op.cos_t, toff[(H) * MFP + m] + 64u * nf, tab_addr + ((m * 4 + nf) * 2 + 0) * 1024);    \
-    fp8_load_lds_16B(op.sin_t, toff[(H) * MFP + m] + 64u * nf, tab_addr + ((m * 4 + nf) * 2 + 1) * 1024);    \
-  }
-#define LLMMM_ROPE_ROTATE(H)                                                                                 \
+    for (int m = 0; m < MFP; ++m) {
+      const unsigned toff = (unsigned)min(max(op.pos[row0 + (h * MFP + m) * 16 + li], 0), op.table_rows - 1) * 256u + 16u * g;  // the lane's first piece
+#pragma unroll
+      for (int nf = 0; nf < 4; ++nf) {
+        fp8_load_lds_16B(op.cos_t, toff + 64u * nf, to + ((m * 4 + nf) * 2 + 0) * 1024);
+        fp8_load_lds_16B(op.sin_t, toff + 64u * nf, to + ((m * 4 + nf) * 2 + 1) * 1024);
+      }
+    }
+  };
+#define LLMMM_ROPE_ROTATE(H, AT)                                                                             \
   _Pragma("unroll") for (int m = 0; m < MFP; ++m) {                                                          \
     const int mf = (H) * MFP + m;                                                                            \
     _Pragma("unroll") for (int nf = 0; nf < 4; ++nf) {                                                       \
-      const f32x4 cs = *(const f32x4 LLMMM_LDS*)(tab + ((m * 4 + nf) * 2 + 0) * 1024 + lane * 16);           \
-      const f32x4 sn = *(const f32x4 LLMMM_LDS*)(tab + ((m * 4 + nf) * 2 + 1) * 1024 + lane * 16);           \
+      const f32x4 cs = *(const f32x4 LLMMM_LDS*)((AT) + ((m * 4 + nf) * 2 + 0) * 1024 + lane * 16);          \
+      const f32x4 sn = *(const f32x4 LLMMM_LDS*)((AT) + ((m * 4 + nf) * 2 + 1) * 1024 + lane * 16);          \
       _Pragma("unroll") for (int q = 0; q < 4; ++q) {                                                        \
         const float lo = acc[nf][mf][q], hi = acc[nf + 4][mf][q];                                            \
         const float t1 = hi * sn[q], t2 = lo * sn[q];                                                        \
@@ -417,9 +429,9 @@ __device__ __forceinline__ void qk_norm_rope_fragments(f32x4 (&acc)[8][MF], cons
       }                                                                                                      \
     }                                                                                                        \
   }
-  LLMMM_ROPE_FETCH(0)
+  fetch(SHARED ? wn : 0);
   const float* nw = head < op.n_q ? op.qw : op.kw;
-  if (nw != nullptr) {
+  if (head < heads && nw != nullptr) {
     float r[MF];
 #pragma unroll
     for (int mf = 0; mf < MF; ++mf) {
@@ -446,13 +458,16 @@ __device__ __forceinline__ void qk_norm_rope_fragments(f32x4 (&acc)[8][MF], cons
     }
   }
   wait_vmcnt<0>();
-  LLMMM_ROPE_ROTATE(0)
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the first pass has been read: its slots may be refilled
-  LLMMM_ROPE_FETCH(1)
-  wait_vmcnt<0>();
-  LLMMM_ROPE_ROTATE(1)
+  if constexpr (SHARED) __syncthreads();  // both halves are there
+  if (head < heads) { LLMMM_ROPE_ROTATE(0, at0) }
+  if constexpr (!SHARED) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the first pass has been read: its slots may be refilled
+    fetch(1);
+    wait_vmcnt<0>();
+  }
+  if (head < heads) { LLMMM_ROPE_ROTATE(1, at1) }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the caller stages its output in the same memory
-#undef LLMMM_ROPE_FETCH
+  if constexpr (SHARED) __syncthreads();
 #undef LLMMM_ROPE_ROTATE
 }
 
@@ -713,7 +728,7 @@ __device__ __forceinline__ void fp8_gemm_body(const uint8_t* __restrict__ A, con
   const int             row0 = m0 + wm * WM;
   const int             col0 = n0 + wn * TC::WN;
   const int             li   = lane & 15;
-  if constexpr (OUT == OUT_ROPE_BF16 || OUT == OUT_ROPE_FP8Q) qk_norm_rope_fragments<MF>(acc, op, col0 >> 7, row0, lane, stg);
+  if constexpr (OUT == OUT_ROPE_BF16 || OUT == OUT_ROPE_FP8Q) qk_norm_rope_fragments<MF, TC::WAVES_N == 2>(acc, op, n0 >> 7, wn, row0, lane, s0, TC::WAVES_N == 2 ? wm : wave, TC::WAVES_M);
   if constexpr (TWO) {
     // 160-column waves: the same staging with padded rows instead of the chunk XOR (a row is 40 or 20 chunks, not a power
     // of two), 16-byte chunks dealt to the lanes in row-major order
