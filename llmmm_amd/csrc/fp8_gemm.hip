@@ -387,8 +387,9 @@ __device__ __forceinline__ void swiglu_finish(const f32x4 (&acc)[8][MF], const f
 // holding registers: fetched into registers instead, the 128 accumulator registers leave room for a few pieces at a
 // time and the epilogue pays one L2 round trip after the other (2048 x 6144 x 2560: 43 us with, 33.6 us without rope).
 // SHARED (two heads per tile): waves wave0 and wave0 + partner hold the same rows of two heads and need the same angles.  Each fetches those of one half of
-// the rows, all at once, and reads both halves behind a barrier: half the table bytes through the CU's load path and one round trip instead of two.
-// (2048 x 6144 x 2560 45.4 us, now 42.5; 4096 x 6144 x 4096 103.7 / 101.0; 1024 x 6144 x 2560 28.4 / 28.1, these with the loads of the K loop.)
+// the rows, all at once, and reads both halves behind a barrier: half the table bytes through the CU's load path and one pass instead of two.
+// (By itself, on pre-shuffled weights in the caches: 256 x 256 tiles 2048 x 6144 x 2560 44.7 us, now 42.8; 4096 x 6144 x 4096 101.0 / 99.9;
+// 128 x 256 tiles 384 x 6144 x 2560 22.7 / 21.4, 512 x 7168 x 5120 40.6 / 39.2.)
 // (`tab`: the piece of wave 0; head0: the tile's first head.)
 template <int MF, bool SHARED>
 __device__ __forceinline__ void qk_norm_rope_fragments(f32x4 (&acc)[8][MF], const Fp8HeadOp& op, int head0, int wn, int row0, int lane, char LLMMM_LDS* tab, int wave0, int partner)
@@ -402,18 +403,28 @@ __device__ __forceinline__ void qk_norm_rope_fragments(f32x4 (&acc)[8][MF], cons
   char LLMMM_LDS* const       mine  = tab + (wave0 + (SHARED ? wn * partner : 0)) * PIECE;
   const char LLMMM_LDS* const at0   = tab + wave0 * PIECE;
   const char LLMMM_LDS* const at1   = SHARED ? at0 + partner * PIECE : at0;
-  // pass h: pieces (m, nf, table) of fragments mf = h * MFP + m at + ((m * 4 + nf) * 2 + table) * 1024
-  const auto fetch = [&](int h) {
+  // byte offsets of the lane's first piece in either table, of every fragment the wave fetches.  All positions are here before the first LDS-direct load:
+  // one loaded between those waits for the pieces ahead of it, a round trip more in each pass (2048 x 6144 x 2560 42.7 us with it, 42.8 without: too
+  // short to measure here).
+  constexpr int FETCHED = SHARED ? MFP : MF;
+  unsigned      toff[FETCHED];
+#pragma unroll
+  for (int i = 0; i < FETCHED; ++i) {
+    const int mf = SHARED ? wn * MFP + i : i;
+    toff[i]      = (unsigned)min(max(op.pos[row0 + mf * 16 + li], 0), op.table_rows - 1) * 256u + 16u * g;
+  }
+#pragma unroll
+  for (int i = 0; i < FETCHED; ++i) asm volatile("" : "+v"(toff[i]));
+  // pieces (m, nf, table) of MFP fragments, m = 0 .. MFP - 1, from toff[m0] on: at + ((m * 4 + nf) * 2 + table) * 1024
+  const auto fetch = [&](int m0) {
     const unsigned to = (unsigned)(size_t)mine;
 #pragma unroll
-    for (int m = 0; m < MFP; ++m) {
-      const unsigned toff = (unsigned)min(max(op.pos[row0 + (h * MFP + m) * 16 + li], 0), op.table_rows - 1) * 256u + 16u * g;  // the lane's first piece
+    for (int m = 0; m < MFP; ++m)
 #pragma unroll
       for (int nf = 0; nf < 4; ++nf) {
-        fp8_load_lds_16B(op.cos_t, toff + 64u * nf, to + ((m * 4 + nf) * 2 + 0) * 1024);
-        fp8_load_lds_16B(op.sin_t, toff + 64u * nf, to + ((m * 4 + nf) * 2 + 1) * 1024);
+        fp8_load_lds_16B(op.cos_t, toff[m0 + m] + 64u * nf, to + ((m * 4 + nf) * 2 + 0) * 1024);
+        fp8_load_lds_16B(op.sin_t, toff[m0 + m] + 64u * nf, to + ((m * 4 + nf) * 2 + 1) * 1024);
       }
-    }
   };
 #define LLMMM_ROPE_ROTATE(H, AT)                                                                             \
   _Pragma("unroll") for (int m = 0; m < MFP; ++m) {                                                          \
@@ -429,7 +440,7 @@ __device__ __forceinline__ void qk_norm_rope_fragments(f32x4 (&acc)[8][MF], cons
       }                                                                                                      \
     }                                                                                                        \
   }
-  fetch(SHARED ? wn : 0);
+  fetch(0);
   const float* nw = head < op.n_q ? op.qw : op.kw;
   if (head < heads && nw != nullptr) {
     float r[MF];
@@ -462,7 +473,7 @@ __device__ __forceinline__ void qk_norm_rope_fragments(f32x4 (&acc)[8][MF], cons
   if (head < heads) { LLMMM_ROPE_ROTATE(0, at0) }
   if constexpr (!SHARED) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the first pass has been read: its slots may be refilled
-    fetch(1);
+    fetch(MFP);
     wait_vmcnt<0>();
   }
   if (head < heads) { LLMMM_ROPE_ROTATE(1, at1) }
