@@ -2,8 +2,8 @@
 //
 // Replaces fp8_blockwise_symmetric_quantization<QUANT_M, 128, SCALE_TRANSPOSE>
 // (reference: examples/005.fp8.mm.cu:439-563): per block amax -> s = amax / 448.f ->
-// q = e4m3(s ? x / s : 0), the code of the IEEE-correct fp32 quotient (q_pack_quotients_e4m3x4 below
-// finds it without dividing wherever the rounding is not in doubt), round-to-nearest-even and
+// q = e4m3(s ? x / s : 0), the code of the IEEE-correct fp32 quotient (quotient_codes below
+// finds it without dividing), round-to-nearest-even and
 // saturation to +-448; a block of zeros gives s = 0 and q = 0.  Scale layouts:
 //   QUANT_M == 1:   transposed s[(n/128)*M + m]      plain s[m*ceil(N/128) + n/128]
 //   QUANT_M == 128: transposed s[(n/128)*M + m/128]  plain s[(m/128)*ceil(N/128) + n/128]
@@ -13,55 +13,105 @@
 // Rows may be ragged (any M); N must be a multiple of 4 (float4 accesses, as in the reference).
 #include "device_common.hip.h"
 #include "kernels.h"
+#include "quotient.hip.h"
 
 namespace llmmm {
 
-// e4m3 codes of v[0..3] / s (s != 0, |v[e]| <= 448 s up to rounding), equal bit for bit to converting the correctly
-// rounded fp32 quotients -- without dividing, almost always.  An IEEE fp32 division costs about ten vector instructions
-// per element and made the quantisers ALU-bound (the same element rate from bf16 and from fp32 inputs).  Instead:
-// v * (rcp(s) (1 - 2^-21)) and v * (rcp(s) (1 + 2^-21)): rcp(s) is within 2^-23 (relative) of 1 / s, its product with the
+// e4m3 codes of v[0..3] / s, s = amax / 448, equal bit for bit to converting the correctly rounded fp32 quotients by the correctly rounded scale -- almost
+// always without computing those.  An IEEE fp32 division per element made the quantisers ALU-bound (the same element rate from bf16 and from fp32 inputs).
+// Instead: v * (rcp(s) (1 - 2^-21)) and v * (rcp(s) (1 + 2^-21)): rcp(s) is within 2^-23 (relative) of 1 / s, its product with the
 // factor and the product with v add 2^-24 each, so both are within 2^-22 of the quotient times its factor and bracket the quotient
 // and its fp32 rounding; if they convert to the same code, then -- the conversion being monotone -- so does the
-// correctly rounded quotient.  Otherwise (a quotient within 2^-20 of a rounding boundary of the 3-bit mantissa: about
-// 3 in 10^5 elements), or when s is so small or large that rcp(s) leaves the normal range, the lane divides.
-// No clamp on the fast path: |v rcp(s)| < 448 (1 + 2^-20), and everything below 464 converts to 448.
-// Non-finite values follow the reference's arithmetic: a NaN element converts to the hardware's NaN code 0xFF in both brackets, the
-// only code with all of its low seven bits set, and the lane divides (pack_e4m3x4_sat writes 0x7F); an infinite or negative scale
-// (a block that holds an infinity, or nothing but NaN) fails the range test likewise.
-// What bounds the row kernels on many rows is the vector instructions they issue; this form and scale_of take about 25 fewer per four elements and
-// row block than scaling first and dividing for the scale (device time of a prefill layer of 2048 rows, three row kernels and a quantiser: 1.2 us of 272 less;
-// 19456 x 2560 in 128 x 128 blocks, with the pre-shuffle behind it, 58.4 us, now 58.1; a layer of one row 38.3, now 38.1).
-struct QuotientScale {
-  float dn, up;  // rcp(s) (1 -+ 2^-21); both NaN where the lane has to divide
-  float s;
+// correctly rounded quotient (`plain`).
+// No clamp there: |v rcp(s)| < 448 (1 + 2^-20), and everything below 464 converts to 448.
+// Otherwise the lane computes the quotients (rounded_codes): where one lies within 2^-20 of a rounding boundary of the 3-bit mantissa (about 3 in 10^5
+// elements), where an element is NaN -- the hardware's code 0xFF in both brackets, the only one with all of its low seven bits set; the code becomes
+// 0x7F --, and where amax lies outside 2^-60 .. 2^100 (a block that holds an infinity or nothing but NaN, one so small or large that something on the
+// way leaves the normal range), here by division.  A block of zeros has the codes 0.
+struct BlockScale {
+  float s;       // amax / 448
+  float dn, up;  // rcp(s) (1 -+ 2^-21)
+  bool  plain;   // they hold
+  bool  zero;    // a block of zeros: codes 0
 };
-__device__ __forceinline__ QuotientScale quotient_scale(float s)
+__device__ __forceinline__ BlockScale block_scale(float amax)
 {
-  float y = __builtin_amdgcn_rcpf(s);
-  if (!(s >= 0x1p-100f && s <= 0x1p100f)) y = __builtin_nanf("");  // every code then reads as NaN: the division
-  return {y * (1.0f - 0x1p-21f), y * (1.0f + 0x1p-21f), s};
+  const float s = scale_of_amax(amax), r = __builtin_amdgcn_rcpf(s);
+  return {s, r * (1.0f - 0x1p-21f), r * (1.0f + 0x1p-21f), amax >= 0x1p-60f && amax <= 0x1p100f, amax == 0.f};
 }
-__device__ __forceinline__ uint32_t q_pack_quotients_e4m3x4(f32x4 v, const QuotientScale& k)
+__device__ __forceinline__ uint32_t bracketed_codes(f32x4 v, const BlockScale& k, bool& plain)
 {
   int lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0] * k.dn, v[1] * k.dn, 0, false);
   lo     = __builtin_amdgcn_cvt_pk_fp8_f32(v[2] * k.dn, v[3] * k.dn, lo, true);
   int hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[0] * k.up, v[1] * k.up, 0, false);
   hi     = __builtin_amdgcn_cvt_pk_fp8_f32(v[2] * k.up, v[3] * k.up, hi, true);
   const uint32_t nan = (((uint32_t)lo & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u;
-  if (__builtin_expect((((uint32_t)lo ^ (uint32_t)hi) | nan) == 0u, 1)) return (uint32_t)lo;
-  if (k.s == 0.f) return 0u;  // a block of zeros
-  return pack_e4m3x4_sat(v[0] / k.s, v[1] / k.s, v[2] / k.s, v[3] / k.s);
+  plain = (((((uint32_t)lo ^ (uint32_t)hi) | nan) == 0u) & k.plain) | k.zero;
+  return k.zero ? 0u : (uint32_t)lo;
+}
+__device__ __forceinline__ uint32_t divided_codes(f32x4 v, float amax, float& s)
+{
+  s = amax / 448.0f;
+  if (s == 0.f) return 0u;
+  return pack_e4m3x4_sat(v[0] / s, v[1] / s, v[2] / s, v[3] / s);
+}
+__device__ __forceinline__ uint32_t rounded_codes(f32x4 v, float amax, float& s)
+{
+  if (__builtin_expect(!(amax >= 0x1p-60f && amax <= 0x1p100f), 0)) return divided_codes(v, amax, s);
+  s             = scale_of_amax(amax);
+  const float y = refined_reciprocal(s, __builtin_amdgcn_rcpf(s));
+  return pack_e4m3x4_in_range(rounded_quotient(v[0], s, y), rounded_quotient(v[1], s, y), rounded_quotient(v[2], s, y), rounded_quotient(v[3], s, y));
+}
+__device__ __forceinline__ uint32_t quotient_codes(f32x4 v, float amax, const BlockScale& k, float& s)
+{
+  bool     plain;
+  uint32_t c = bracketed_codes(v, k, plain);
+  s          = k.s;
+  if (__builtin_expect(!plain, 0)) c = divided_codes(v, amax, s);
+  return c;
 }
 
-// amax / 448, correctly rounded (Markstein: the quotient from the rounded reciprocal, corrected once by its exact remainder) where nothing
-// underflows or overflows on the way, by division elsewhere.
-__device__ __forceinline__ float scale_of(float a)
+// The NI chunks of a thread of the row kernels (t, t + 256, ..; those past the row's end dropped): codes, and the scales from the first lane of each block.
+// On many rows these kernels are bound by the vector instructions they issue, on few by the one pass a workgroup makes through code that is not in the
+// instruction cache yet.  So the chunks run side by side without a branch, and the chunks in doubt go one after the other through one piece of code, instead
+// of each through a copy of its own behind a branch of its own.  us, RMSNorm and quantiser on bf16 rows, with a division for the scale and for each chunk in
+// doubt / with the scale by scale_of_amax, behind branches of every chunk / now: 1 x 2560 2.55 / 2.73 / 2.40, 1 x 8192 4.40 / 4.66 / 3.65,
+// 16 x 4096 3.4 / 3.5 / 3.0, 2048 x 2560 8.2 / 8.0 / 7.3, 4096 x 8192 30.7 / 29.8 / 26.8; rows of zeros, for which the first did nothing at all,
+// 2048 x 2560 5.3 / 6.4 / 6.0.
+template <int NI>
+__device__ __forceinline__ void quantise_row(const f32x4 (&v)[NI], const float (&amax)[NI], unsigned t, unsigned chunks, uint8_t* __restrict__ q,
+                                             float* __restrict__ scale, int M, int m)
 {
-  constexpr float y = 1.0f / 448.0f;
-  const float     q = a * y;
-  const float     s = __builtin_fmaf(__builtin_fmaf(-448.0f, q, a), y, q);
-  if (__builtin_expect(a >= 0x1p-90f && a <= 0x1p120f, 1)) return s;
-  return a / 448.0f;
+  uint32_t code[NI];
+  float    s[NI];
+  unsigned doubt = 0;  // bit i: chunk i
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const BlockScale k = block_scale(amax[i]);
+    bool             plain;
+    code[i] = bracketed_codes(v[i], k, plain);
+    s[i]    = k.s;
+    doubt |= (plain | (t + 256u * i >= chunks)) ? 0u : 1u << i;
+  }
+  while (doubt != 0u) {
+    const int i = __builtin_ctz(doubt);
+    doubt &= doubt - 1u;
+    f32x4 vi = v[0];
+    float ai = amax[0], si;
+#pragma unroll
+    for (int j = 1; j < NI; ++j) vi = i == j ? v[j] : vi, ai = i == j ? amax[j] : ai;
+    const uint32_t ci = rounded_codes(vi, ai, si);
+#pragma unroll
+    for (int j = 0; j < NI; ++j) code[j] = i == j ? ci : code[j], s[j] = i == j ? si : s[j];
+  }
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const unsigned c = t + 256u * i;
+    if (c < chunks) {
+      *(uint32_t*)(q + 4 * c) = code[i];
+      if ((t & 31) == 0) scale[(c >> 5) * (unsigned)M + m] = s[i];
+    }
+  }
 }
 
 // The reference starts its block maximum from (float)INT_MIN (examples/005.fp8.mm.cu:456) and its comparison never
@@ -106,8 +156,8 @@ __global__ void __launch_bounds__(256) quant_1x128_kernel(const float* __restric
       float a = QUANT_AMAX_SEED;
       if (live) a = amax4(a, v[u]);
       a = half_wave_max(a);
-      const float    s = scale_of(a);
-      const uint32_t c = q_pack_quotients_e4m3x4(v[u], quotient_scale(s));
+      float          s;
+      const uint32_t c = quotient_codes(v[u], a, block_scale(a), s);
       if (live) *(uint32_t*)(q + (size_t)m * N + n) = c;
       if (l32 == 0) {
         if (TRANSPOSE)
@@ -150,12 +200,12 @@ __global__ void __launch_bounds__(256) quant_128x128_kernel(const float* __restr
   if ((tid & 63) == 0) wmax[tid >> 6] = a;
   __syncthreads();
   a             = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-  const float         s = scale_of(a);
-  const QuotientScale k = quotient_scale(s);
+  const BlockScale k = block_scale(a);
+  float            s = k.s;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int      m = mb * 128 + r * 8 + sub;
-    const uint32_t c = q_pack_quotients_e4m3x4(v[r], k);
+    const uint32_t c = quotient_codes(v[r], a, k, s);
     if (live && m < M) *(uint32_t*)(q + (size_t)m * N + n) = c;
   }
   if (tid == 0) {
@@ -194,8 +244,8 @@ __device__ __forceinline__ void rmsnorm_quant_chunk(f32x4 v, float r, const floa
   }
   float a = amax4(0.f, y);
   a = half_wave_max(a);
-  const float    s  = scale_of(a);
-  const uint32_t cd = q_pack_quotients_e4m3x4(y, quotient_scale(s));
+  float          s;
+  const uint32_t cd = quotient_codes(y, a, block_scale(a), s);
   if (live) {
     *(uint32_t*)(q + (size_t)m * K + 4 * c) = cd;
     if ((lane & 31) == 0) scale[(size_t)(c >> 5) * M + m] = s;
@@ -282,15 +332,7 @@ __global__ void __launch_bounds__(256) rmsnorm_quant_row_kernel(const IN_T* __re
   }
 #pragma unroll
   for (int i = 0; i < NI; ++i) amax[i] = half_wave_max(amax[i]);
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const unsigned c = t + 256u * i;
-    if (c < chunks) {
-      const float sc                           = scale_of(amax[i]);
-      *(uint32_t*)(qr + 4 * c) = q_pack_quotients_e4m3x4(held[i], quotient_scale(sc));
-      if ((t & 31) == 0) scale[(c >> 5) * (unsigned)M + m] = sc;
-    }
-  }
+  quantise_row<NI>(held, amax, t, chunks, qr, scale, M, m);
 }
 
 // The decoder-block epilogue behind a projection back to the hidden size (O, down), in one kernel behind the GEMM's
@@ -388,15 +430,7 @@ __global__ void __launch_bounds__(256) planes_add_rmsnorm_quant_kernel(const flo
   }
 #pragma unroll
   for (int i = 0; i < NI; ++i) amax[i] = half_wave_max(amax[i]);
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const unsigned c = t + 256u * i;
-    if (c < chunks) {
-      const float sc                           = scale_of(amax[i]);
-      *(uint32_t*)(qr + 4 * c) = q_pack_quotients_e4m3x4(held[i], quotient_scale(sc));
-      if ((t & 31) == 0) scale[(c >> 5) * (unsigned)M + m] = sc;
-    }
-  }
+  quantise_row<NI>(held, amax, t, chunks, qr, scale, M, m);
 }
 
 // Chunks a thread of the two row kernels holds: the smallest of these that covers the row.  With 3 and 10 only, a row of 4096
