@@ -68,7 +68,7 @@ struct Fp8Tile {
 };
 
 // Operand and scale loads of the main loop are written as inline assembly, with a wave-uniform
-// base in SGPRs and one constant per-lane byte offset, and the kernel places its own s_waitcnt:
+// base in SGPRs and per-lane byte offsets that are constants of the kernel, and the kernel places its own s_waitcnt:
 // the compiler then never sees an LDS-direct load in flight (it would turn every wait it
 // inserts into "all loads done"), and no vector ALU work goes into addresses.
 __device__ __forceinline__ void fp8_load_lds_16B(const void* sbase, unsigned voff, unsigned lds_addr)
@@ -109,9 +109,10 @@ __device__ __forceinline__ void fp8_load_f32(float& dst, const void* sbase, unsi
 
 // Load i (0 .. A_LOADS + B_LOADS - 1) of a wave for one stage covers tile rows 8*(wave + i*NW) .. +7 of A or of Bt; its lanes' byte offsets from the tile's
 // first row are constants of the kernel (off), its place in LDS is a constant behind the wave's first (lds_wave = stage + 1024 * wave).  What is left per load
-// is one scalar addition: the K loops are short of instruction slots.  (With the rows' distance added to a 64-bit base for every load, 266 instructions per
+// is one scalar addition.  (With the rows' distance added to a 64-bit base for every load, 266 instructions per
 // slice and wave of the 256 x 256 tile instead of 252 and 233 instead of 218 of the deep 128 x 160 one; us, then / now: 384 x 3584 x 18944 35.7 / 34.9,
-// 4096^3 54.5 / 54.3, 4096 rows through a layer of hidden 8192 2914 / 2903.  One scalar instruction more per load, a mask on EXEC, cost 2 .. 5 %.)
+// 4096 rows through a layer of hidden 8192 2914 / 2903, 4096^3 54.5 / 54.3, which is within the spread.  One scalar instruction more per load, a mask on EXEC,
+// cost 2 .. 5 %.)
 //
 // Pre-shuffled weights (layout.hip) hold the same LDS image as consecutive 1 KB half blocks: half
 // block h of row group rg and slice kb at ((rg * K/128 + kb) * 2 + h) * 1024.  Rows 8*NW apart
@@ -246,7 +247,8 @@ __device__ __forceinline__ void fp8_compute_stage(const char LLMMM_LDS* lds, int
     // 32-row waves (HALVES): a step's first load has the fragment's LDS reads between M0 and itself, its second the step's MFMAs.  Eight wait states fewer per
     // slice: a prefill layer of 2048 rows (O and down in deep 128 x 160 tiles) 1.0 % faster, 257.6 us before this and the constant offsets, 254.2 with
     // both; 384 x 3584 x 18944 0.3 .. 1.5 %, 35.7 / 34.8 likewise.  64-row waves gain 0.6 % at 4096^3 and lose 0.9 % where a launch is long enough for the
-    // power limit to decide (a layer of 4096 rows, hidden 8192), and keep the wait states.
+    // power limit to decide (a layer of 4096 rows, hidden 8192), and keep the wait states.  Offsets per load and halves take 130 .. 134 VGPRs where one offset
+    // took 126 .. 128, three waves per SIMD instead of four; LDS admits two.
 #define LLMMM_FP8_STEP_HEAD(S)                                                          \
   if (nf == S) {                                                                        \
     fp8_issue_m0<BM, BN, WM, S * LPG>(nx.lds_stage);                                    \
