@@ -44,3 +44,24 @@ def test_scales_and_codes_over_magnitudes(exponents, quant_m):
     q, s = llmmm_amd.quantize_activation(t) if quant_m == 1 else llmmm_amd.quantize_weight(t)
     assert np.array_equal(s.cpu().numpy().view(np.uint32).ravel(), rs.view(np.uint32).ravel())
     assert np.array_equal(q.cpu().numpy(), rq)
+
+
+@pytest.mark.parametrize("M,N", [(1, 4), (127, 132), (128, 128), (129, 260), (300, 384)])
+@pytest.mark.parametrize("quant_m", [1, 128])
+def test_scales_of_zero(M, N, quant_m):
+    """Zeros of both signs, blocks that hold NaN beside them, values so small that their scale rounds to zero: codes 0, next to blocks that have a scale."""
+    import torch
+
+    import llmmm_amd
+    rng = np.random.default_rng(M + N + quant_m)
+    x = rng.choice(np.float32([0, -0.0]), (M, N))
+    x[M // 2, N // 2] = np.nan
+    if N > 256:
+        x[:, 128:256] = rng.choice(np.float32([2.0 ** -149, -2.0 ** -147, 0]), (M, 128))
+        x[:, 256:] = rng.standard_normal((M, N - 256))
+    rq, rs = oracle.quant_fp8(x, quant_m, quant_m == 1)
+    t = torch.from_numpy(x).cuda()
+    q, s = llmmm_amd.quantize_activation(t) if quant_m == 1 else llmmm_amd.quantize_weight(t)
+    assert not rq[:, :min(N, 256)].any()
+    assert np.array_equal(s.cpu().numpy().view(np.uint32).ravel(), rs.view(np.uint32).ravel())
+    assert np.array_equal(q.cpu().numpy(), rq)
