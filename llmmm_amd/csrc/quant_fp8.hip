@@ -74,10 +74,10 @@ __device__ __forceinline__ uint32_t quotient_codes(f32x4 v, float amax, const Bl
 // The NI chunks of a thread of the row kernels (t, t + 256, ..; those past the row's end dropped): codes, and the scales from the first lane of each block.
 // On many rows these kernels are bound by the vector instructions they issue, on few by the one pass a workgroup makes through code that is not in the
 // instruction cache yet.  So the chunks run side by side without a branch, and the chunks in doubt go one after the other through one piece of code, instead
-// of each through a copy of its own behind a branch of its own.  us, RMSNorm and quantiser on bf16 rows, with a division for the scale and for each chunk in
-// doubt / with the scale by scale_of_amax, behind branches of every chunk / now: 1 x 2560 2.55 / 2.73 / 2.40, 1 x 8192 4.40 / 4.66 / 3.65,
-// 16 x 4096 3.4 / 3.5 / 3.0, 2048 x 2560 8.2 / 8.0 / 7.3, 4096 x 8192 30.7 / 29.8 / 26.8; rows of zeros, for which the first did nothing at all,
-// 2048 x 2560 5.3 / 6.4 / 6.0.
+// of each through a copy of its own behind a branch of its own.  us per launch, RMSNorm and quantiser on bf16 rows that are not in the caches, with a division
+// for the scale and for each chunk in doubt / with the scale by scale_of_amax, behind branches of every chunk / now: 1 x 2560 2.17 / 2.14 / 2.04,
+// 1 x 8192 3.76 / 3.67 / 3.11, 16 x 4096 2.83 / 2.75 / 2.54, 2048 x 2560 8.1 / 7.9 / 7.9, 4096 x 8192 30.5 / 29.3 / 28.5; rows of zeros, for which the first
+// did nothing at all, 2048 x 2560 5.5 / 6.5 / 6.2.
 template <int NI>
 __device__ __forceinline__ void quantise_row(const f32x4 (&v)[NI], const float (&amax)[NI], unsigned t, unsigned chunks, uint8_t* __restrict__ q,
                                              float* __restrict__ scale, int M, int m)
